@@ -552,3 +552,37 @@ def test_every_bf16_configuration_with_bf16_copies(gpu, M, N, K):
     ref = np.maximum(a16 @ w16.T + bias.astype(np.float64), 0.0)
     bound = np.abs(a16) @ np.abs(w16).T + np.abs(bias.astype(np.float64))
     assert (np.abs(outs[0] - ref) / bound).max() <= (K + 2) * 2.0 ** -24
+
+
+# The pipelined tiles: one to three k slices (64 deep in BF16 mode, 32 in
+# split mode), output edges just below, at and past a tile, odd leading
+# dimensions (16-byte stores at 4-byte alignment, 1 to 3 columns past the last
+# whole group), both epilogues (straight from the accumulators; staged, taken
+# for the activation derivative).  Integer-valued operands make every product
+# and sum exact, so the results must equal NumPy's bit for bit.
+@pytest.mark.parametrize("mode", ["bf16", "bf16x3"])
+@pytest.mark.parametrize("M,N,K", [(17, 17, 17), (63, 65, 64), (64, 64, 65), (129, 127, 128), (257, 255, 129),
+                                   (256, 256, 192), (300, 515, 33), (511, 513, 200), (130, 66, 4160)])
+def test_pipelined_tile_edges(gpu, mode, M, N, K):
+    rng = np.random.default_rng(M + 3 * N + 7 * K)
+    h, md = gpu._handle, _lib.GEMM_MODE[mode]
+    A = rng.integers(-3, 4, (M, K)).astype(np.float32)
+    B = rng.integers(-3, 4, (N, K)).astype(np.float32)
+    C0 = rng.integers(-9, 10, (M, N)).astype(np.float32)
+    bias = rng.integers(-9, 10, N).astype(np.float32)
+    aux = np.maximum(rng.integers(-2, 3, (M, N)), 0).astype(np.float32)
+    P = A @ B.T
+    gA, gB, gX = (vk.Array(gpu, data=v) for v in (A, B, aux))
+    try:
+        for i in range(len(vk.gemm_configs(mode))):
+            _lib.call("vkh_gemm_set_config", h, md, 0, 1, M, N, K, i)
+            np.testing.assert_array_equal(run_gemm(gpu, mode, 0, 1, A, B), P)
+            got = run_gemm(gpu, mode, 0, 1, A, B, C0=C0, alpha=2.0, beta=-1.0, bias=bias, act="relu")
+            np.testing.assert_array_equal(got, np.maximum(2 * P - C0 + bias, 0))
+            gC = vk.Array(gpu, shape=(M, N))
+            _lib.call("vkh_gemm_ex", h, md, 0, 1, M, N, K, 1.0, gA._ptr, K, gB._ptr, K, 0.0, gC._ptr, N,
+                      None, 0, None, gX._ptr, N, _lib.ACT["relu"])
+            gC._set_job([gA, gB, gX])
+            np.testing.assert_array_equal(np.asarray(gC), P * (aux > 0))
+    finally:
+        _lib.call("vkh_gemm_set_config", h, md, 0, 1, M, N, K, -1)

@@ -2,14 +2,12 @@
 //
 // The reference computes every output with one thread looping over K from
 // global memory (vulkpy/shader/matmul.comp:23-33, batch_affine.comp:25-39).
-// Here a 256-thread block computes a BM x BN tile: operands are staged through
-// LDS (K-contiguous rows, padded against bank conflicts), the next K slice is
-// prefetched into registers while the current one is multiplied, and four
-// waves (2 x 2) each own a (BM/2) x (BN/2) sub-tile built from 32 x 32 MFMA
+// Here a block computes a BM x BN tile: operand slices are staged through LDS
+// ahead of their use, and each wave owns a sub-tile of 32 x 32 or 16 x 16 MFMA
 // blocks:
 //   FP32    v_mfma_f32_32x32x2_f32    (operands as stored)
-//   BF16    v_mfma_f32_32x32x16_bf16  (operands rounded to nearest-even BF16)
-//   BF16X3  the same instruction three times: hi*hi + hi*lo + lo*hi, where
+//   BF16    v_mfma_f32_16x16x32_bf16  (operands rounded to nearest-even BF16)
+//   BF16X3  the same instruction three times: lo*hi + hi*lo + hi*hi, where
 //           x = hi + lo + O(2^-16 |x|) with hi = bf16(x), lo = bf16(x - hi)
 // Accumulation is FP32 in every mode.  The epilogue applies alpha, beta*C,
 // bias[n] and an activation, and can also emit a BF16 copy of the result.
@@ -25,10 +23,6 @@ namespace vkh {
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
 typedef __attribute__((ext_vector_type(16))) float f32x16_t;
-// register staging of 8 BF16 values; a native vector (unlike HIP's uint4
-// struct) stays in VGPRs when held in arrays across the K loop
-typedef __attribute__((ext_vector_type(4))) uint32_t u32x4_t;
-
 // f(integral_constant<int, 0>), ..., f(integral_constant<int, N - 1>): a
 // loop unrolled by construction
 template <typename F, int... I>
@@ -42,6 +36,9 @@ __device__ __forceinline__ void static_for(F&& f) {
 
 
 typedef __attribute__((ext_vector_type(4))) float f32x4_t;
+// the same in memory at any 4-byte alignment (global accesses of 16 bytes need
+// no more on this hardware)
+typedef __attribute__((ext_vector_type(4), aligned(4))) float f32x4u_t;
 
 struct GemmArgs {
   const float* A;
@@ -133,54 +130,44 @@ constexpr int PK_TK = 128;     // transpose tile k in k_pack_cols
 
 // dst[r][k] = bf16(op(src)[r][k]) for r < Rp, k < Kp, zero outside [R, K);
 // op(src)[r][k] = src[r*ld + k] (TRANS = false) or src[k*ld + r] (TRANS = true).
-template <bool SPLIT>
-__device__ __forceinline__ void pack8(const float v[8], uint16_t* hi, uint16_t* lo) {
-  uint16_t h[8], l[8];
-#pragma unroll
-  for (int q = 0; q < 8; ++q) {
-    h[q] = f2bf(v[q]);
-    if (SPLIT) l[q] = f2bf(v[q] - bf2f(h[q]));
-  }
-  uint4 hv, lv;
-  hv.x = h[0] | ((uint32_t)h[1] << 16); hv.y = h[2] | ((uint32_t)h[3] << 16);
-  hv.z = h[4] | ((uint32_t)h[5] << 16); hv.w = h[6] | ((uint32_t)h[7] << 16);
-  *reinterpret_cast<uint4*>(hi) = hv;
-  if (SPLIT) {
-    lv.x = l[0] | ((uint32_t)l[1] << 16); lv.y = l[2] | ((uint32_t)l[3] << 16);
-    lv.z = l[4] | ((uint32_t)l[5] << 16); lv.w = l[6] | ((uint32_t)l[7] << 16);
-    *reinterpret_cast<uint4*>(lo) = lv;
-  }
+// With PARTS > 1 an element is the sum of PARTS BF16 values, each the rounding
+// of what the ones before it leave, and a row holds groups of 32 k, the parts
+// of a group one after another (so a k slice of a row is contiguous in memory
+// in every mode).
+template <int PARTS>
+__device__ __forceinline__ uint64_t pack_off(uint64_t r, uint64_t k, uint64_t Kp) {
+  return PARTS == 1 ? r * Kp + k : r * Kp * PARTS + (k / 32) * (32 * PARTS) + k % 32;
 }
+
+__device__ __forceinline__ uint32_t bf2x(float a, float b) { return f2bf(a) | ((uint32_t)f2bf(b) << 16); }
 
 // Row-major source: 4 consecutive elements a thread, one thread per 4 of
 // the padded [Rp][Kp] (Rp * Kp / 4 < 2^31: the row from one 32-bit
 // multiply-high division), so that each load instruction reads one contiguous
-// 1 KB run and each store writes 512 B.
-__device__ __forceinline__ uint32_t bf2x(float a, float b) { return f2bf(a) | ((uint32_t)f2bf(b) << 16); }
-
-template <bool SPLIT>
+// 1 KB run and each store writes 512 B (64-byte runs with PARTS > 1).
+template <int PARTS>
 __global__ void __launch_bounds__(256)
-k_pack_rows(const float* src, uint64_t ld, uint64_t R, uint64_t K, uint16_t* hi, uint16_t* lo,
-            uint32_t total4, FastDiv kq, uint64_t Kp, int vec) {
+k_pack_rows(const float* src, uint64_t ld, uint64_t R, uint64_t K, uint16_t* dst, uint32_t total4, FastDiv kq,
+            uint64_t Kp) {
   const uint32_t t = blockIdx.x * 256 + threadIdx.x;
   if (t >= total4) return;
   const uint32_t r = kq.div(t);
   const uint64_t k = (uint64_t)(t - r * kq.d) * 4;
   float v[4];
-  if (r < R && vec && k + 3 < K) {
-    const float4 a = ld_stream(reinterpret_cast<const float4*>(src + r * ld + k));
-    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
+  if (r < R && k + 3 < K) {
+    const f32x4u_t a = __builtin_nontemporal_load(reinterpret_cast<const f32x4u_t*>(src + r * ld + k));
+#pragma unroll
+    for (int q = 0; q < 4; ++q) v[q] = a[q];
   } else {
 #pragma unroll
     for (int q = 0; q < 4; ++q) v[q] = (r < R && k + q < K) ? src[r * ld + k + q] : 0.f;
   }
-  const uint64_t off = (uint64_t)r * Kp + k;
-  *reinterpret_cast<uint2*>(hi + off) = make_uint2(bf2x(v[0], v[1]), bf2x(v[2], v[3]));
-  if constexpr (SPLIT) {
-    float l[4];
+  const uint64_t off = pack_off<PARTS>(r, k, Kp);
 #pragma unroll
-    for (int q = 0; q < 4; ++q) l[q] = v[q] - bf2f(f2bf(v[q]));
-    *reinterpret_cast<uint2*>(lo + off) = make_uint2(bf2x(l[0], l[1]), bf2x(l[2], l[3]));
+  for (int part = 0; part < PARTS; ++part) {
+    *reinterpret_cast<uint2*>(dst + off + part * 32) = make_uint2(bf2x(v[0], v[1]), bf2x(v[2], v[3]));
+#pragma unroll
+    for (int q = 0; q < 4; ++q) v[q] = v[q] - bf2f(f2bf(v[q]));
   }
 }
 
@@ -190,10 +177,9 @@ k_pack_rows(const float* src, uint64_t ld, uint64_t R, uint64_t K, uint16_t* hi,
 // 16-byte loads along r (512-byte row segments) and the writes 16-byte
 // stores along k (256-byte row segments of the packed buffer).  Rp is a
 // multiple of PK_TR; the last k tile may pass Kp.
-template <bool SPLIT>
+template <int PARTS>
 __global__ void __launch_bounds__(256)
-k_pack_cols(const float* src, uint64_t ld, uint64_t R, uint64_t K, uint16_t* hi, uint16_t* lo,
-            uint64_t Rp, uint64_t Kp, int vec) {
+k_pack_cols(const float* src, uint64_t ld, uint64_t R, uint64_t K, uint16_t* dst, uint64_t Rp, uint64_t Kp) {
   const uint64_t r0 = (uint64_t)blockIdx.x * PK_TR, k0 = (uint64_t)blockIdx.y * PK_TK;
   constexpr int R4 = PK_TR / 4;
   constexpr int NL = PK_TK * R4 / 256;  // 16-byte loads per thread, all issued before the LDS writes
@@ -203,14 +189,14 @@ k_pack_cols(const float* src, uint64_t ld, uint64_t R, uint64_t K, uint16_t* hi,
     const int f = threadIdx.x + i * 256;
     const int kk = f / R4, rr = (f % R4) * 4;
     const uint64_t r = r0 + rr, k = k0 + kk;
-    if (vec && k < K && r + 3 < R) {
-      v[i] = *reinterpret_cast<const vkh_f4v*>(src + k * ld + r);
+    if (k < K && r + 3 < R) {
+      v[i] = *reinterpret_cast<const f32x4u_t*>(src + k * ld + r);
     } else {
 #pragma unroll
       for (int q = 0; q < 4; ++q) v[i][q] = (k < K && r + q < R) ? src[k * ld + r + q] : 0.f;
     }
   }
-  if constexpr (!SPLIT) {
+  if constexpr (PARTS == 1) {
     // BF16 tile: the values are rounded on the way in (the rounding the
     // packed row would apply), so the tile takes 33 KB and four blocks fit
     // a compute unit.  Word w of row kk holds r = 2w (low half) and 2w + 1;
@@ -240,10 +226,10 @@ k_pack_cols(const float* src, uint64_t ld, uint64_t R, uint64_t K, uint16_t* hi,
       ev.z = (wd[4] & 0xffffu) | (wd[5] << 16); od.z = (wd[4] >> 16) | (wd[5] & 0xffff0000u);
       ev.w = (wd[6] & 0xffffu) | (wd[7] << 16); od.w = (wd[6] >> 16) | (wd[7] & 0xffff0000u);
       const uint64_t off = (r0 + 2 * rp) * Kp + k;
-      *reinterpret_cast<uint4*>(hi + off) = ev;
-      *reinterpret_cast<uint4*>(hi + off + Kp) = od;
+      *reinterpret_cast<uint4*>(dst + off) = ev;
+      *reinterpret_cast<uint4*>(dst + off + Kp) = od;
     }
-  } else {  // FP32 tile: the split needs each value's low part too
+  } else {  // FP32 tile: the lower parts need the values
     __shared__ float t[PK_TK][PK_TR + 1];
 #pragma unroll
     for (int i = 0; i < NL; ++i) {
@@ -261,17 +247,21 @@ k_pack_cols(const float* src, uint64_t ld, uint64_t R, uint64_t K, uint16_t* hi,
       float v[8];
 #pragma unroll
       for (int q = 0; q < 8; ++q) v[q] = t[kc * 8 + q][rr];
-      const uint64_t off = (r0 + rr) * Kp + k;
-      pack8<SPLIT>(v, hi + off, SPLIT ? lo + off : nullptr);
+      const uint64_t off = pack_off<PARTS>(r0 + rr, k, Kp);
+#pragma unroll
+      for (int part = 0; part < PARTS; ++part) {
+        *reinterpret_cast<uint4*>(dst + off + part * 32) =
+            make_uint4(bf2x(v[0], v[1]), bf2x(v[2], v[3]), bf2x(v[4], v[5]), bf2x(v[6], v[7]));
+#pragma unroll
+        for (int q = 0; q < 8; ++q) v[q] = v[q] - bf2f(f2bf(v[q]));
+      }
     }
   }
 }
 
 struct PackedArgs {
-  const uint16_t* Ah;
-  const uint16_t* Al;
-  const uint16_t* Bh;
-  const uint16_t* Bl;
+  const uint16_t* A;
+  const uint16_t* B;
   uint64_t Kp;
   // split k: block (tile, blockIdx.y = s) accumulates k in [s*kc, (s+1)*kc)
   // and writes its raw accumulators to part[s][M][N]; k_splitk_combine then
@@ -279,40 +269,6 @@ struct PackedArgs {
   uint64_t kc;
   float* part;
   GemmArgs e;
-};
-
-// Register stage of one packed operand's ROWS x BK slice: 16-byte loads of
-// K-contiguous BF16 rows (both parts in split mode), stored to LDS rows of
-// LDK = BK + 8 elements (the pad keeps rows 16-byte aligned and spreads the
-// rows of a 16-lane LDS access over distinct banks).
-template <int ROWS, int BK, bool SPLIT, int THREADS>
-struct PackedStager {
-  static constexpr int LDK = BK + 8;
-  static constexpr int NV = ROWS * BK / 8 / THREADS;  // 16-byte vectors per thread
-  static_assert(ROWS * BK / 8 % THREADS == 0, "whole 16-byte vectors per thread");
-  static constexpr int PARTS = SPLIT ? 2 : 1;
-  u32x4_t r[PARTS][NV];
-
-  __device__ __forceinline__ void load(const uint16_t* hi, const uint16_t* lo, uint64_t row0,
-                                       uint64_t Kp, uint64_t k0) {
-#pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      const int idx = threadIdx.x + i * THREADS;
-      const int row = idx / (BK / 8), c = idx % (BK / 8);
-      const uint64_t off = (row0 + row) * Kp + k0 + c * 8;
-      r[0][i] = *reinterpret_cast<const u32x4_t*>(hi + off);
-      if constexpr (SPLIT) r[1][i] = *reinterpret_cast<const u32x4_t*>(lo + off);
-    }
-  }
-  __device__ __forceinline__ void store(uint16_t* hi, uint16_t* lo) const {
-#pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      const int idx = threadIdx.x + i * THREADS;
-      const int row = idx / (BK / 8), c = idx % (BK / 8);
-      *reinterpret_cast<u32x4_t*>(hi + row * LDK + c * 8) = r[0][i];
-      if constexpr (SPLIT) *reinterpret_cast<u32x4_t*>(lo + row * LDK + c * 8) = r[1][i];
-    }
-  }
 };
 
 // 4 consecutive floats p[0 .. cnt) (one 16-byte load when `full`), zeros beyond.
@@ -427,10 +383,10 @@ __device__ __forceinline__ void store_part4(float* part, uint64_t N, uint64_t m,
   }
 }
 
-// Epilogue of a block whose waves each hold TM x TN 32 x 32 accumulator
-// blocks of a WM x WN sub-tile at (wm, wn): acc[i][j][r] is C[m, n] with
+// Epilogue of a block whose waves each hold the accumulator blocks of a
+// WM x WN sub-tile at (wm, wn): with 32 x 32 blocks acc[i][j][r] is C[m, n],
 // m = m0 + wm*WM + i*32 + (r/4)*8 + lhi*4 + r%4 and n = n0 + wn*WN + j*32 +
-// l32.  Each wave writes rows i*32 .. i*32+31 of its sub-tile to its own
+// l32 (l32 = lane % 32, lhi = lane / 32).  Each wave writes rows i*32 .. i*32+31 of its sub-tile to its own
 // 32 x (WN+4) float staging slice of `smem`, then reads them back as 4-float
 // row segments (WN/4 lanes per row), so C is accessed in whole row segments.
 // With `part` the raw sums go to that k chunk's partial matrix instead.  The
@@ -446,14 +402,36 @@ constexpr int TT_PITCH = 72;  // transposed tile row: 64 rows of C + 8, 16-byte 
 template <int WAVES, int WN>
 constexpr int tt_bytes() { return WAVES * WN * TT_PITCH * 2; }
 
-template <int TM, int TN, int WM, int WN, bool TST = false>
-__device__ __forceinline__ void staged_epilogue(float* smem, f32x16_t (&acc)[TM][TN], const GemmArgs& e,
+// rows i*32 .. i*32+31 of a wave's accumulators into its staging slice: 32 x 32
+// blocks (acc[i][j][r] as above), or 16 x 16 blocks, where acc[i][j][r] is
+// row i*16 + (lane/16)*4 + r, column j*16 + lane%16
+template <int I, int SROW, int TM, int TN>
+__device__ __forceinline__ void stage_pass(float* st, const f32x16_t (&acc)[TM][TN]) {
+  const int l32 = threadIdx.x & 31, lhi = (threadIdx.x >> 5) & 1;
+#pragma unroll
+  for (int j = 0; j < TN; ++j)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) st[((r / 4) * 8 + lhi * 4 + (r % 4)) * SROW + j * 32 + l32] = acc[I][j][r];
+}
+template <int I, int SROW, int TM, int TN>
+__device__ __forceinline__ void stage_pass(float* st, const f32x4_t (&acc)[TM][TN]) {
+  const int l16 = threadIdx.x & 15, lq = (threadIdx.x >> 4) & 3;
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) st[(i * 16 + lq * 4 + r) * SROW + j * 16 + l16] = acc[2 * I + i][j][r];
+}
+
+template <int WM, int WN, bool TST, typename Acc>
+__device__ __forceinline__ void staged_epilogue(float* smem, const Acc& acc, const GemmArgs& e,
                                                 float* part, uint64_t m0, uint64_t n0, int wm, int wn,
                                                 uint16_t* tbase = nullptr) {
+  constexpr int TM = WM / 32;  // passes of 32 rows
   constexpr int SROW = WN + 4, F4R = WN / 4, RPI = 64 / F4R;
   static_assert(64 % F4R == 0, "whole rows per wave pass");
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int l32 = lane & 31, lhi = lane >> 5;
   float* st = smem + wave * 32 * SROW;
   const uint64_t nb = n0 + wn * WN;
   const bool tr = e.Cbft && !part;
@@ -531,10 +509,12 @@ __device__ __forceinline__ void staged_epilogue(float* smem, f32x16_t (&acc)[TM]
       }
     }
   }
-  // ReLU' of segment seg's aux values, as act_deriv_mul finds it: 1
-  // (positive), NaN (NaN) or 0
-  auto relu_x = [&](int seg) {
-    const uint32_t byte = (cw[seg / 4] >> (8 * (seg % 4))) & 0xffu;
+  // ReLU' of the aux values of the pass's row segment k, as act_deriv_mul finds
+  // it: 1 (positive), NaN (NaN) or 0
+  constexpr int WPP = (ITER + 3) / 4;  // code words of a pass
+  uint32_t cwp[WPP];
+  auto relu_x = [&](int k) {
+    const uint32_t byte = (cwp[k / 4] >> (8 * (k % 4))) & 0xffu;
     f32x4_t xv;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
@@ -554,15 +534,20 @@ __device__ __forceinline__ void staged_epilogue(float* smem, f32x16_t (&acc)[TM]
     }
   };
   if (xpre && AHEAD) load_aux(0, 0);
-  // pass i: rows i*32 .. i*32+31 of the sub-tile (a compile-time i, so the
-  // accumulators stay in registers however large the pass's code)
-  auto pass = [&](auto ic) __attribute__((always_inline)) {
-    constexpr int i = decltype(ic)::value;
+  // Pass i: rows i*32 .. i*32+31 of the sub-tile.  One copy of the pass's code:
+  // only the staging of its accumulators (whose registers need constant
+  // indices) is unrolled.  With every pass unrolled the kernels took 64-128 KB,
+  // more than the instruction cache holds, and a block's epilogue waited for
+  // its instructions: a single 256 x 256 tile with K = 256 took 30-40 us.
+#pragma unroll 1
+  for (int i = 0; i < TM; ++i) {
+    static_for<TM>([&](auto ic) __attribute__((always_inline)) {
+      if (i == decltype(ic)::value) {
+        stage_pass<decltype(ic)::value, SROW>(st, acc);
 #pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r)
-        st[((r / 4) * 8 + lhi * 4 + (r % 4)) * SROW + j * 32 + l32] = acc[i][j][r];
+        for (int w = 0; w < WPP; ++w) cwp[w] = cw[decltype(ic)::value * ITER / 4 + w];
+      }
+    });
     __syncthreads();
     const uint64_t mb = m0 + wm * WM + i * 32;
     if (lane_fast && mb + 31 < e.M) {
@@ -576,7 +561,7 @@ __device__ __forceinline__ void staged_epilogue(float* smem, f32x16_t (&acc)[TM]
           const f32x4_t c = e.beta != 0.f ? *reinterpret_cast<const f32x4_t*>(e.C + (mb + rr) * e.ldc + n) : z;
           uint2 hb = make_uint2(0u, 0u);
           const float4 f = relu_codes
-                               ? finish4<false, true>(e, mb + rr, n, v, true, 4, c, bq, relu_x(i * ITER + k0 + k), false,
+                               ? finish4<false, true>(e, mb + rr, n, v, true, 4, c, bq, relu_x(k0 + k), false,
                                                       &hb, tst)
                                : finish4<false>(e, mb + rr, n, v, true, 4, c, bq, xq[k], false, &hb, tst);
           if (tst) put_t_bf(i, rr, cc, hb);
@@ -661,11 +646,93 @@ __device__ __forceinline__ void staged_epilogue(float* smem, f32x16_t (&acc)[TM]
       }
       __syncthreads();
     }
-  };
-  static_for<TM>(pass);
+  }
   if (csum && lane < WN) {
     const uint64_t m = m0 + wm * WM, nc = nb + lane;
     if (m < e.M && nc < e.N) e.cs[(m / CS_ROWS) * e.N + nc] = csacc;
+  }
+}
+
+// Epilogue straight from the accumulators, for kernels that multiply with the
+// operands exchanged (each block of the accumulators is then C^T's, so a lane
+// holds 4 consecutive columns of a row): no LDS, 16-byte accesses, 64-byte runs
+// of a row an instruction.  For alpha, beta, bias and ReLU (and the split-k
+// partial sums); anything else takes the staged epilogue.  acc[i][j] is the
+// 16 x 16 block (i, j) of the wave's sub-tile: row l16 = lane % 16, columns
+// 4 (lane / 16) .. + 3.  65536 x 1024 x 1024 151 us against 200 us staged.
+static bool direct_ok(const GemmArgs& e) {
+  return !e.Cbft && !e.cs && !e.Cbf && !e.no_c && !e.aux && !e.aux16 && e.act != VKH_ACT_SIGMOID;
+}
+
+template <int TM, int TN>
+__device__ __forceinline__ void direct_epilogue(const f32x4_t (&acc)[TM][TN], const GemmArgs& e, float* part,
+                                                uint64_t mw, uint64_t nw) {
+  const int lane = threadIdx.x & 63, l16 = lane & 15, lq = lane >> 4;
+  const uint64_t m0 = mw + l16, n0 = nw + lq * 4;
+  const uint64_t ld = part ? e.N : e.ldc;
+  float* cp = (part ? part : e.C) + m0 * ld + n0;
+  // raw sums (a partial, or nothing to apply)
+  const bool raw = part || (e.alpha == 1.f && e.beta == 0.f && !e.bias && e.act == VKH_ACT_NONE);
+  auto apply = [&](float acc1, float c, float b) {
+    float t = e.alpha * acc1;
+    if (e.beta != 0.f) t += e.beta * c;
+    if (e.bias) t += b;
+    return act_apply<false>(e.act, t);
+  };
+  // whole groups of 4 columns: 16-byte accesses at any 4-byte alignment
+  const bool inm = mw + TM * 16 <= e.M;  // every row in range
+  if (raw) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+      if (inm || m0 + i * 16 < e.M) {
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+          if (n0 + j * 16 + 3 < e.N) *reinterpret_cast<f32x4u_t*>(cp + i * 16 * ld + j * 16) = acc[i][j];
+      }
+  } else {
+    f32x4_t b[TN];
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+      b[j] = e.bias && n0 + j * 16 + 3 < e.N ? *reinterpret_cast<const f32x4u_t*>(e.bias + n0 + j * 16)
+                                             : f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+      if (inm || m0 + i * 16 < e.M) {
+        f32x4_t c[TN];
+        if (e.beta != 0.f)  // a block row's old values before its first store
+#pragma unroll
+          for (int j = 0; j < TN; ++j)
+            if (n0 + j * 16 + 3 < e.N) c[j] = *reinterpret_cast<const f32x4u_t*>(cp + i * 16 * ld + j * 16);
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+          if (n0 + j * 16 + 3 < e.N) {
+            f32x4_t v;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) v[q] = apply(acc[i][j][q], c[j][q], b[j][q]);
+            *reinterpret_cast<f32x4u_t*>(cp + i * 16 * ld + j * 16) = v;
+          }
+      }
+  }
+  // the group that straddles the last column: 1 to 3 elements
+  if (e.N % 4 != 0 && nw < e.N && e.N < nw + TN * 16) {
+    const int jt = (int)((e.N - nw) / 16);
+    f32x4_t v[TM];
+    static_for<TN>([&](auto jc) __attribute__((always_inline)) {
+      if (jt == decltype(jc)::value)
+#pragma unroll
+        for (int i = 0; i < TM; ++i) v[i] = acc[i][decltype(jc)::value];
+    });
+    const uint64_t n = n0 + jt * 16;
+    if (n < e.N && n + 3 >= e.N) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int q = 0; q < 3; ++q)
+          if (m0 + i * 16 < e.M && n + q < e.N) {
+            float* d = cp + i * 16 * ld + jt * 16 + q;
+            *d = raw ? v[i][q] : apply(v[i][q], e.beta != 0.f ? *d : 0.f, e.bias ? e.bias[n + q] : 0.f);
+          }
+    }
   }
 }
 
@@ -868,7 +935,7 @@ k_gemm_f32(GemmArgs p, float* part, uint64_t kc) {
     frags(cur, 0, 0);
   }
   __syncthreads();  // every wave is done with the operand tiles before staging
-  staged_epilogue<TM, TN, WM, WN, TST>(smem, acc, p, part ? part + (uint64_t)blockIdx.y * p.M * p.N : nullptr,
+  staged_epilogue<WM, WN, TST>(smem, acc, p, part ? part + (uint64_t)blockIdx.y * p.M * p.N : nullptr,
                                        m0, n0, wm, wn, reinterpret_cast<uint16_t*>(smem + STAGE));
 }
 
@@ -939,276 +1006,235 @@ k_splitk_combine(const float* part, uint64_t S, GemmArgs e) {
   }
 }
 
-// BM x BN tile, WGM x WGN waves of (BM/WGM) x (BN/WGN), double-buffered LDS
-// and register prefetch of the next BK-deep K slice; one barrier per slice.
-// After the K loop the LDS holds each wave's accumulators, 32 rows at a time,
-// so the epilogue reads and writes whole row segments of C.
-template <int BM, int BN, int BK, bool SPLIT, int WGM, int WGN>
-__global__ void __launch_bounds__(64 * WGM * WGN)
-k_gemm_packed(PackedArgs p) {
-  static_assert(PK_KALIGN % BK == 0, "Kp must be a multiple of the k slice");
-  constexpr int THREADS = 64 * WGM * WGN, WAVES = WGM * WGN;
-  constexpr int WM = BM / WGM, WN = BN / WGN;
-  static_assert(WM % 32 == 0 && WN % 32 == 0 && WN <= 256, "32 x 32 MFMA blocks per wave");
-  constexpr int TM = WM / 32, TN = WN / 32;
-  constexpr int PARTS = SPLIT ? 2 : 1;
-  constexpr int PK_LDK = BK + 8;
-  constexpr int A_TILE = BM * PK_LDK, B_TILE = BN * PK_LDK;        // BF16 elements
-  constexpr int MAIN_BYTES = 2 * PARTS * (A_TILE + B_TILE) * 2;
-  constexpr int SROW = WN + 4;                                      // staging row (floats)
-  constexpr int STAGE_BYTES = WAVES * 32 * SROW * 4;
-  constexpr int SMEM_BYTES = MAIN_BYTES > STAGE_BYTES ? MAIN_BYTES : STAGE_BYTES;
-  constexpr bool TST = STAGE_BYTES + tt_bytes<WAVES, WN>() <= SMEM_BYTES;
-  __shared__ __attribute__((aligned(16))) uint16_t smem[SMEM_BYTES / 2];
-  // operand tile (buffer, part): As(buf, q) / Bs(buf, q)
-  auto As = [&](int buf, int q) { return smem + (buf * PARTS + q) * A_TILE; };
-  auto Bs = [&](int buf, int q) { return smem + 2 * PARTS * A_TILE + (buf * PARTS + q) * B_TILE; };
-
-  const GemmArgs& e = p.e;
-  uint32_t tm, tn;
-  tile_coords(e, tm, tn);
-  const uint64_t m0 = (uint64_t)tm * BM, n0 = (uint64_t)tn * BN;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int wm = wave / WGN, wn = wave % WGN;
-  const int l32 = lane & 31, lhi = lane >> 5;
-  const uint64_t Kp = p.Kp;
-
-  PackedStager<BM, BK, SPLIT, THREADS> sa;
-  PackedStager<BN, BK, SPLIT, THREADS> sb;
-
-  f32x16_t acc[TM][TN];
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-
-  // Operand fragments of one 16-deep MFMA k-step, double-buffered in
-  // registers: the fragments of step s+1 are read from LDS while the MFMAs
-  // of step s issue, so LDS latency hides behind matrix-core work.
-  constexpr int KS = BK / 16;
-  static_assert(KS % 2 == 0, "the first k-step of every slice uses fragment buffer 0");
-  constexpr int NM = TM * TN * (SPLIT ? 3 : 1);  // MFMAs per k-step
-  constexpr int NDS = (TM + TN) * PARTS;         // fragment reads per k-step
-  constexpr int NVM = (PackedStager<BM, BK, SPLIT, THREADS>::NV + PackedStager<BN, BK, SPLIT, THREADS>::NV) * PARTS;
-  constexpr int VPP = (NVM + NDS - 1) / NDS;     // global loads per MFMA of the first step
-  constexpr int WPM = (NVM + NM - 1) / NM;       // LDS stores per MFMA of the last step
-  bf16x8_t fa[2][TM], fb[2][TN], fal[2][TM], fbl[2][TN];
-  const int arow = wm * WM + l32, brow = wn * WN + l32, kcol = lhi * 8;
-  auto frags = [&](int buf, int fb_idx, int k) {
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-      const int off = (arow + i * 32) * PK_LDK + k + kcol;
-      fa[fb_idx][i] = *reinterpret_cast<const bf16x8_t*>(As(buf, 0) + off);
-      if constexpr (SPLIT) fal[fb_idx][i] = *reinterpret_cast<const bf16x8_t*>(As(buf, 1) + off);
-    }
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      const int off = (brow + j * 32) * PK_LDK + k + kcol;
-      fb[fb_idx][j] = *reinterpret_cast<const bf16x8_t*>(Bs(buf, 0) + off);
-      if constexpr (SPLIT) fbl[fb_idx][j] = *reinterpret_cast<const bf16x8_t*>(Bs(buf, 1) + off);
-    }
-  };
-
-  const uint64_t kb = p.part ? (uint64_t)blockIdx.y * p.kc : 0;
-  const uint64_t nk = ((p.part ? min(kb + p.kc, Kp) : Kp) - kb) / BK;
-  sa.load(p.Ah, p.Al, m0, Kp, kb);
-  sb.load(p.Bh, p.Bl, n0, Kp, kb);
-  sa.store(As(0, 0), As(0, PARTS - 1));
-  sb.store(Bs(0, 0), Bs(0, PARTS - 1));
-  __syncthreads();
-  frags(0, 0, 0);
-  int cur = 0;
-  for (uint64_t kt = 0; kt < nk; ++kt) {
-    // Prefetch of the next slice into registers.  The final iteration loads
-    // the last slice again (in bounds, never read): the body has no branch,
-    // so the scheduler sees one region.
-    const uint64_t kn = kb + (kt + 1 < nk ? kt + 1 : kt) * BK;
-    sa.load(p.Ah, p.Al, m0, Kp, kn);
-    sb.load(p.Bh, p.Bl, n0, Kp, kn);
-#pragma unroll
-    for (int s = 0; s < KS; ++s) {
-      const int c = s & 1;
-      if (s + 1 < KS) frags(cur, c ^ 1, (s + 1) * 16);
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) {
-          if constexpr (SPLIT) {
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fal[c][i], fb[c][j], acc[i][j], 0, 0, 0);
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[c][i], fbl[c][j], acc[i][j], 0, 0, 0);
-          }
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[c][i], fb[c][j], acc[i][j], 0, 0, 0);
-        }
-      // Issue order within the slice: every k-step but the last alternates
-      // one MFMA with one fragment read for the next step (the first step
-      // also issues the next slice's global loads, VPP per pair, so that
-      // they have the whole slice to arrive); the last step alternates its
-      // MFMAs with the LDS stores of the prefetched slice.
-      if (s + 1 < KS) {
-#pragma unroll
-        for (int q = 0; q < NDS; ++q) {
-          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
-          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // DS read
-          if (s == 0) __builtin_amdgcn_sched_group_barrier(0x020, VPP, 0);  // VMEM read
-        }
-        if constexpr (NM > NDS) __builtin_amdgcn_sched_group_barrier(0x008, NM - NDS, 0);
-      }
-    }
-    sa.store(As(cur ^ 1, 0), As(cur ^ 1, PARTS - 1));
-    sb.store(Bs(cur ^ 1, 0), Bs(cur ^ 1, PARTS - 1));
-#pragma unroll
-    for (int q = 0; q < NM; ++q) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);    // MFMA
-      __builtin_amdgcn_sched_group_barrier(0x200, WPM, 0);  // DS write
-    }
-    __syncthreads();
-    cur ^= 1;
-    if (kt + 1 < nk) frags(cur, 0, 0);
-  }
-  __syncthreads();  // every wave is done with the operand tiles before staging
-  staged_epilogue<TM, TN, WM, WN, TST>(reinterpret_cast<float*>(smem), acc, e,
-                                       p.part ? p.part + (uint64_t)blockIdx.y * e.M * e.N : nullptr,
-                                       m0, n0, wm, wn, reinterpret_cast<uint16_t*>(smem) + STAGE_BYTES / 2);
+// ---- pipelined BF16 products ----------------------------------------------------
+// C from packed operands on v_mfma_f32_16x16x32_bf16, for products with enough
+// tiles to fill the chip.  PARTS BF16 values stand for each operand element
+// (1: BF16 mode, 2: split mode); a packed row holds its k in groups of KG,
+// the parts of a group one after another, so a slice of every row is ROWB
+// contiguous bytes in every mode.
+//
+// What bounds a loop that fills LDS, waits at a barrier and multiplies is the
+// wait: with the next slice requested at the start of a slice and awaited at
+// its end, 8192^3 ran at 1.04-1.19 PFLOP/s (matrix cores 58% busy).  Here:
+//  * slices go from global memory straight into LDS (no staging registers), a
+//    slice and a half ahead: a wave reads its sub-tile in quarters (halves of
+//    its rows and of its columns), and each half's LDS is refilled with the
+//    slice after next as soon as every wave has read it, so a load has six
+//    phases (about 3000 cycles) to arrive.  Waits count the loads still in
+//    flight (vmcnt) instead of draining them;
+//  * the two waves of a SIMD run half a phase apart (one extra barrier at the
+//    start for the second half of the block): while one reads fragments, the
+//    other multiplies;
+//  * 16-byte chunks of an LDS row sit XOR-swizzled by row so that the 16 rows
+//    of a fragment read fall on 16 different 16-byte banks.
+// Measured on the loop alone (same operands, interleaved): 8192^3 761-790 us
+// against 928-1062 us for the loop it replaces (1.45 PFLOP/s; 864 us with the
+// staggered waves but loads one slice ahead, 855 us without the stagger, 955 us
+// with 32 x 32 x 16 instructions), 16384 x 4096 x 4096 405-430 against 490-583 us.
+// One 16 x 16 x 32 instruction gives the bits of the two 32 x 32 x 16 ones it
+// replaces, so results equal k_gemm_packed's.
+__device__ __forceinline__ void load_lds16(const char* src, char* dst) {
+#ifdef __HIP_DEVICE_COMPILE__  // (the host pass would drop the launch stub of a template that uses the builtin)
+  __builtin_amdgcn_global_load_lds(src, dst, 16, 0, 0);
+#endif
 }
 
-// BF16 variant whose operand slices go from global memory straight into LDS
-// (global_load_lds_dwordx4: no VGPR staging, no LDS store instructions).  A
-// wave instruction fills 8 unpadded rows of 128 B (one BK = 64 slice of 8
-// rows): lane l writes row l / 8, 16-byte position l % 8, and fetches the
-// global chunk (l % 8) ^ (row & 7) of that row.  The XOR swizzle takes the
-// place of the row padding: a fragment read of 8 consecutive rows at one
-// chunk touches 8 distinct positions.  The next slice is requested at the
-// start of a slice and awaited, with one barrier, at its end.  Every output
-// accumulates k in the same order as k_gemm_packed.
-constexpr int DIRECT_SMEM_BYTES = 128 * 1024;  // (with 144 KB, room for the transposed staging tile, 1-4% slower)
+// waits until at most N global loads are in flight / a block barrier, neither
+// of which the scheduler moves anything across
+template <int N>
+__device__ __forceinline__ void wait_loads() {
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x0f70);
+  __builtin_amdgcn_sched_barrier(0);
+}
+__device__ __forceinline__ void phase_barrier() {
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_sched_barrier(0);
+}
 
-template <int BM, int BN, int WGM, int WGN>
-__global__ void __launch_bounds__(64 * WGM * WGN)
-k_gemm_direct(PackedArgs p) {
-  constexpr int BK = 64, ROWB = BK * 2;  // a slice row: 64 BF16 = 128 B
-  constexpr int WAVES = WGM * WGN;
+template <int PARTS>
+struct PipeSlice {
+  static constexpr int KG = PARTS == 1 ? 64 : 32;  // k of a slice
+  static constexpr int ROWB = KG * 2 * PARTS;      // bytes of a slice row
+  static constexpr int NF = ROWB / 64;             // 64-byte fragments of a row: k steps, or parts
+  static constexpr int CPR = ROWB / 16;            // 16-byte chunks of a row
+  // LDS position of chunk c of row r: rows of 128 bytes alternate between the
+  // halves of the 256-byte bank line, so 8 row pairs permute 8 positions
+  __device__ __forceinline__ static int pos(int r, int c) { return c ^ ((r >> 1) & 7); }
+};
+
+// DIRECT: the operands are exchanged and the accumulators stored without
+// staging (no C^T copy, no column sums)
+template <int BM, int BN, int WGM, int WGN, int PARTS, bool DIRECT>
+__global__ void __launch_bounds__(64 * WGM * WGN, 2)
+k_gemm_pipe(PackedArgs p) {
+  using S = PipeSlice<PARTS>;
+  constexpr int ROWB = S::ROWB, NF = S::NF, WAVES = WGM * WGN;
+  constexpr bool STAGGER = WAVES == 8;  // two waves a SIMD
   constexpr int WM = BM / WGM, WN = BN / WGN;
-  static_assert(WM % 32 == 0 && WN % 32 == 0, "32 x 32 MFMA blocks per wave");
-  static_assert(BM % (8 * WAVES) == 0 && BN % (8 * WAVES) == 0, "whole 8-row loads per wave");
-  constexpr int TM = WM / 32, TN = WN / 32;
+  constexpr int HM = WM / 2, HN = WN / 2;  // rows / columns of a half
+  static_assert(HM % 16 == 0 && HN % 16 == 0, "16 x 16 MFMA blocks per quarter");
+  constexpr int TMH = HM / 16, TNH = HN / 16;
+  // 1 KB loads (one wave instruction) of one wave row's half, and per wave
+  constexpr int GA = HM * ROWB / 1024, GB = HN * ROWB / 1024;
+  constexpr int LA = WGM * GA / WAVES, LB = WGN * GB / WAVES;
+  static_assert(LA * WAVES == WGM * GA && LB * WAVES == WGN * GB, "whole loads per wave and half");
   constexpr int A_BYTES = BM * ROWB, B_BYTES = BN * ROWB;
   constexpr int MAIN_BYTES = 2 * (A_BYTES + B_BYTES);
-  constexpr int SROW = WN + 4;
-  constexpr int STAGE_BYTES = WAVES * 32 * SROW * 4;
-  constexpr int SMEM_BYTES = MAIN_BYTES > STAGE_BYTES ? MAIN_BYTES : STAGE_BYTES;
-  constexpr int A_LOADS = BM / 8 / WAVES, B_LOADS = BN / 8 / WAVES;  // per wave per slice
-  // The array's size must not depend on the template parameters: with a
-  // dependent size, the host pass of this template emits no launch stub once
-  // the LDS-load builtin writes into the array.
-  static_assert(SMEM_BYTES <= DIRECT_SMEM_BYTES, "LDS of the direct-load kernel");
-  constexpr bool TST = STAGE_BYTES + tt_bytes<WAVES, WN>() <= DIRECT_SMEM_BYTES;
-  __shared__ __attribute__((aligned(16))) char smem[DIRECT_SMEM_BYTES];
-  auto Abuf = [&](int b) { return smem + b * A_BYTES; };
-  auto Bbuf = [&](int b) { return smem + 2 * A_BYTES + b * B_BYTES; };
+  constexpr int STAGE_BYTES = WAVES * 32 * (WN + 4) * 4;
+  constexpr int TT = tt_bytes<WAVES, WN>();
+  constexpr bool TST = STAGE_BYTES + TT <= 160 * 1024 && WAVES == 8;
+  constexpr int EPI_BYTES = DIRECT ? 0 : STAGE_BYTES + (TST ? TT : 0);
+  constexpr int SMEM_BYTES = MAIN_BYTES > EPI_BYTES ? MAIN_BYTES : EPI_BYTES;
+  __shared__ __attribute__((aligned(16))) char smem[SMEM_BYTES];
 
   const GemmArgs& e = p.e;
   uint32_t tm, tn;
   tile_coords(e, tm, tn);
   const uint64_t m0 = (uint64_t)tm * BM, n0 = (uint64_t)tn * BN;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = wave / WGN, wn = wave % WGN;
-  const int l32 = lane & 31, lhi = lane >> 5;
-  const int lrow = lane >> 3, lpos = lane & 7;
-  const uint64_t Kp = p.Kp;
 
-  auto load_slice = [&](int b, uint64_t k0) {
-#pragma unroll
-    for (int i = 0; i < A_LOADS; ++i) {
-      const int r0 = (i * WAVES + wave) * 8, row = r0 + lrow;
-      const uint16_t* src = p.Ah + (m0 + row) * Kp + k0 + ((lpos ^ (row & 7)) << 3);
-      __builtin_amdgcn_global_load_lds(src, smem + b * A_BYTES + r0 * ROWB, 16, 0, 0);
-    }
-#pragma unroll
-    for (int i = 0; i < B_LOADS; ++i) {
-      const int r0 = (i * WAVES + wave) * 8, row = r0 + lrow;
-      const uint16_t* src = p.Bh + (n0 + row) * Kp + k0 + ((lpos ^ (row & 7)) << 3);
-      __builtin_amdgcn_global_load_lds(src, smem + 2 * A_BYTES + b * B_BYTES + r0 * ROWB, 16, 0, 0);
-    }
-  };
-  // fragment of tile row `row`, 16-byte chunk c (k = 8c .. 8c + 7 of the slice)
-  auto frag = [&](const char* buf, int row, int c) {
-    return *reinterpret_cast<const bf16x8_t*>(buf + row * ROWB + ((c ^ (row & 7)) << 4));
-  };
-
-  f32x16_t acc[TM][TN];
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-
-  constexpr int KS = BK / 16;
-  constexpr int NM = TM * TN, NDS = TM + TN;
-  bf16x8_t fa[2][TM], fb[2][TN];
-  const int arow = wm * WM + l32, brow = wn * WN + l32;
-  auto frags = [&](int buf, int fi, int s) {
-#pragma unroll
-    for (int i = 0; i < TM; ++i) fa[fi][i] = frag(Abuf(buf), arow + i * 32, 2 * s + lhi);
-#pragma unroll
-    for (int j = 0; j < TN; ++j) fb[fi][j] = frag(Bbuf(buf), brow + j * 32, 2 * s + lhi);
-  };
-
+  // Slice kt of this block's k range starts kt * ROWB bytes into each row.
+  const uint64_t rowp = p.Kp * 2 * PARTS;  // bytes of a packed row
   const uint64_t kb = p.part ? (uint64_t)blockIdx.y * p.kc : 0;
-  const uint64_t nk = ((p.part ? min(kb + p.kc, Kp) : Kp) - kb) / BK;
-  load_slice(0, kb);
-  __builtin_amdgcn_s_waitcnt(0);
-  __syncthreads();
-  frags(0, 0, 0);
-  int cur = 0;
-  for (uint64_t kt = 0; kt < nk; ++kt) {
-    if (kt + 1 < nk) load_slice(cur ^ 1, kb + (kt + 1) * BK);
+  const uint64_t nk = ((p.part ? min(kb + p.kc, p.Kp) : p.Kp) - kb) / S::KG;
+  const char* ga = reinterpret_cast<const char*>(p.A) + m0 * rowp + kb * 2 * PARTS;
+  const char* gb = reinterpret_cast<const char*>(p.B) + n0 * rowp + kb * 2 * PARTS;
+
+  // 1 KB load q of a wave for half h of A (B): LDS offset within the operand's
+  // slice (wave-uniform) and this lane's source offset in 16-byte chunks
+  auto half_off = [&](int q, int g, int h, int wrows, int hrows) {
+    const int idx = q * WAVES + wave;
+    return (idx / g) * wrows * ROWB + h * hrows * ROWB + (idx % g) * 1024;
+  };
+  auto src_off = [&](int lds_off) {
+    const int c = (lds_off >> 4) + lane, r = c / S::CPR;
+    return (uint32_t)r * (uint32_t)(rowp >> 4) + S::pos(r, c % S::CPR);
+  };
+  uint32_t oa[2][LA], ob[2][LB];
 #pragma unroll
-    for (int s = 0; s < KS; ++s) {
-      const int c = s & 1;
-      if (s + 1 < KS) frags(cur, c ^ 1, s + 1);
+  for (int h = 0; h < 2; ++h) {
 #pragma unroll
-      for (int i = 0; i < TM; ++i)
+    for (int q = 0; q < LA; ++q) oa[h][q] = src_off(half_off(q, GA, h, WM, HM));
 #pragma unroll
-        for (int j = 0; j < TN; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[c][i], fb[c][j], acc[i][j], 0, 0, 0);
-      if (s + 1 < KS) {
-#pragma unroll
-        for (int q = 0; q < NDS; ++q) {
-          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
-          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // DS read
-        }
-        if constexpr (NM > NDS) __builtin_amdgcn_sched_group_barrier(0x008, NM - NDS, 0);
-      }
-    }
-    // the next slice has landed in LDS and every wave is done with this one
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-    cur ^= 1;
-    if (kt + 1 < nk) frags(cur, 0, 0);
+    for (int q = 0; q < LB; ++q) ob[h][q] = src_off(half_off(q, GB, h, WN, HN));
   }
-  __syncthreads();  // every wave is done with the operand tiles before staging
-  staged_epilogue<TM, TN, WM, WN, TST>(reinterpret_cast<float*>(smem), acc, e,
-                                       p.part ? p.part + (uint64_t)blockIdx.y * e.M * e.N : nullptr,
-                                       m0, n0, wm, wn, reinterpret_cast<uint16_t*>(smem) + STAGE_BYTES / 2);
+  // slices past the end load the last one again (in range, never read)
+  auto slice = [&](uint64_t kt) { return (kt < nk ? kt : nk - 1) * ROWB; };
+  auto load_a = [&](int b, uint64_t ks, int h) {
+#pragma unroll
+    for (int q = 0; q < LA; ++q) load_lds16(ga + ks + ((uint64_t)oa[h][q] << 4), smem + b * A_BYTES + half_off(q, GA, h, WM, HM));
+  };
+  auto load_b = [&](int b, uint64_t ks, int h) {
+#pragma unroll
+    for (int q = 0; q < LB; ++q)
+      load_lds16(gb + ks + ((uint64_t)ob[h][q] << 4), smem + 2 * A_BYTES + b * B_BYTES + half_off(q, GB, h, WN, HN));
+  };
+
+  f32x4_t acc[2 * TMH][2 * TNH];
+#pragma unroll
+  for (int i = 0; i < 2 * TMH; ++i)
+#pragma unroll
+    for (int j = 0; j < 2 * TNH; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+  // fragment f (64 bytes: 32 k of one part) of 16 rows: lane l holds row
+  // l % 16, 16-byte chunk l / 16
+  const int l16 = lane & 15, lq = lane >> 4;
+  auto frag = [&](const char* buf, int row, int f) {
+    return *reinterpret_cast<const bf16x8_t*>(buf + row * ROWB + S::pos(row, 4 * f + lq) * 16);
+  };
+  bf16x8_t fa[TMH][NF], fb[2][TNH][NF];
+  auto read_a = [&](int b, int h) {
+#pragma unroll
+    for (int f = 0; f < NF; ++f)
+#pragma unroll
+      for (int i = 0; i < TMH; ++i) fa[i][f] = frag(smem + b * A_BYTES, wm * WM + h * HM + i * 16 + l16, f);
+  };
+  auto read_b = [&](int b, int h) {
+#pragma unroll
+    for (int f = 0; f < NF; ++f)
+#pragma unroll
+      for (int j = 0; j < TNH; ++j)
+        fb[h][j][f] = frag(smem + 2 * A_BYTES + b * B_BYTES, wn * WN + h * HN + j * 16 + l16, f);
+  };
+  auto mul = [&](int h, int g, int f, int q) {
+#pragma unroll
+    for (int i = 0; i < TMH; ++i)
+#pragma unroll
+      for (int j = 0; j < TNH; ++j)
+        acc[h * TMH + i][g * TNH + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+            DIRECT ? fb[g][j][q] : fa[i][f], DIRECT ? fa[i][f] : fb[g][j][q], acc[h * TMH + i][g * TNH + j], 0, 0, 0);
+  };
+  // quarter (h, g): every product of its fragments, k in order (split mode:
+  // lo * hi, hi * lo, hi * hi of 32 k at a time)
+  auto quarter = [&](int h, int g) {
+    phase_barrier();
+    if constexpr (PARTS == 1) {
+      mul(h, g, 0, 0);
+      mul(h, g, 1, 1);
+    } else {
+      mul(h, g, 1, 0);
+      mul(h, g, 0, 1);
+      mul(h, g, 0, 0);
+    }
+    // (without the stagger every wave has read a half before any wave passes
+    // the next phase's barrier, which is before its refill is requested)
+    if constexpr (STAGGER) phase_barrier();
+    else __builtin_amdgcn_sched_barrier(0);
+  };
+
+  load_a(0, slice(0), 0);
+  load_b(0, slice(0), 0);
+  load_b(0, slice(0), 1);
+  load_a(0, slice(0), 1);
+  load_a(1, slice(1), 0);
+  load_b(1, slice(1), 0);
+  load_b(1, slice(1), 1);
+  wait_loads<2 * LA + 3 * LB>();
+  phase_barrier();
+  if (STAGGER && wave >= WAVES / 2) phase_barrier();
+  for (uint64_t kt = 0; kt < nk; ++kt) {
+    const int cur = (int)(kt & 1);
+    const uint64_t k1 = slice(kt + 1), k2 = slice(kt + 2);
+    read_b(cur, 0);
+    read_a(cur, 0);
+    load_a(cur ^ 1, k1, 1);
+    wait_loads<3 * LA + 2 * LB>();  // this slice's second half of B has landed
+    quarter(0, 0);
+    read_b(cur, 1);
+    wait_loads<2 * LA + 2 * LB>();  // this slice's second half of A has landed
+    quarter(0, 1);
+    read_a(cur, 1);
+    load_a(cur, k2, 0);
+    load_b(cur, k2, 0);
+    quarter(1, 1);
+    load_b(cur, k2, 1);
+    wait_loads<2 * LA + 3 * LB>();  // the next slice's first halves have landed
+    quarter(1, 0);
+  }
+  if (STAGGER && wave < WAVES / 2) phase_barrier();
+  wait_loads<0>();  // the last loads no longer write LDS
+  float* part = p.part ? p.part + (uint64_t)blockIdx.y * e.M * e.N : nullptr;
+  if constexpr (DIRECT) {
+    direct_epilogue(acc, e, part, m0 + wm * WM, n0 + wn * WN);
+  } else {
+    __syncthreads();
+    staged_epilogue<WM, WN, TST>(reinterpret_cast<float*>(smem), acc, e, part, m0, n0, wm, wn,
+                                 reinterpret_cast<uint16_t*>(smem + STAGE_BYTES));
+  }
 }
 
-// Tile choice of the packed kernel: 256 x 256 when both sides fill at least
-// one such tile (4 waves of 128 x 128), 128 x 128 otherwise and in split mode
-// (whose two BF16 parts double the LDS footprint).
-// Kernel configurations of the packed path: tile, k slice and wave grid.
-// BF16 keeps one part per operand; split mode (two parts) needs twice the
-// LDS per slice, hence its smaller k slice.
+// Kernel configurations of the packed path: tile, k slice, waves and the rows
+// of a wave's slab.  Split mode has two parts in a slice row, so half the k.
 typedef void (*PackedLaunch)(dim3, hipStream_t, const PackedArgs&);
-template <int BM, int BN, int BK, bool SPLIT, int WGM, int WGN>
-static void launch_packed(dim3 grid, hipStream_t s, const PackedArgs& pa) {
-  hipLaunchKernelGGL((k_gemm_packed<BM, BN, BK, SPLIT, WGM, WGN>), grid, dim3(64 * WGM * WGN), 0, s, pa);
-}
-template <int BM, int BN, int WGM, int WGN>
-static void launch_direct(dim3 grid, hipStream_t s, const PackedArgs& pa) {
-  hipLaunchKernelGGL((k_gemm_direct<BM, BN, WGM, WGN>), grid, dim3(64 * WGM * WGN), 0, s, pa);
+template <int BM, int BN, int WGM, int WGN, int PARTS>
+static void launch_pipe(dim3 grid, hipStream_t s, const PackedArgs& pa) {
+  if (pa.part || direct_ok(pa.e))
+    hipLaunchKernelGGL((k_gemm_pipe<BM, BN, WGM, WGN, PARTS, true>), grid, dim3(64 * WGM * WGN), 0, s, pa);
+  else
+    hipLaunchKernelGGL((k_gemm_pipe<BM, BN, WGM, WGN, PARTS, false>), grid, dim3(64 * WGM * WGN), 0, s, pa);
 }
 struct PackedCfg {
   int bm, bn, bk, waves, wm;  // wm: rows of a wave's slab (BM / WGM)
@@ -1216,27 +1242,15 @@ struct PackedCfg {
   int direct = 0;  // operand slices loaded from global memory straight into LDS
 };
 static const PackedCfg BF16_CFGS[] = {
-    {256, 256, 64, 4, 128, launch_packed<256, 256, 64, false, 2, 2>},
-    {256, 256, 64, 8, 128, launch_packed<256, 256, 64, false, 2, 4>},
-    {128, 128, 64, 4, 64, launch_packed<128, 128, 64, false, 2, 2>},
-    {256, 128, 64, 4, 128, launch_packed<256, 128, 64, false, 2, 2>},
-    {128, 256, 64, 4, 64, launch_packed<128, 256, 64, false, 2, 2>},
-    {256, 256, 64, 8, 128, launch_direct<256, 256, 2, 4>, 1},
-    // 8 waves of 64 x 32: twice the waves of configuration 2 in the same
-    // LDS, for short k, where the operand latency of each tile's few slices
-    // is exposed (16384 x 4096 x 256 with its BF16 row and transposed
-    // copies: 109 against 143-151 us)
-    {128, 128, 64, 8, 64, launch_packed<128, 128, 64, false, 2, 4>},
-    // (128 x 256 with 8 waves of 64 x 64: 110 KB of LDS, one block a
-    // compute unit, fastest on none of the MLP shapes, so not kept;
-    // direct loads with 4 waves of 128 x 128, a third less LDS fragment
-    // traffic, one wave per SIMD: 894 against 977 TFLOP/s at 8192^3 and
-    // slower on every MLP shape, so not kept)
+    {256, 256, 64, 8, 128, launch_pipe<256, 256, 2, 4, 1>, 1},
+    {128, 128, 64, 4, 64, launch_pipe<128, 128, 2, 2, 1>, 1},
+    {64, 64, 64, 4, 32, launch_pipe<64, 64, 2, 2, 1>, 1},
+    // (256 x 128 and 128 x 256 with 8 waves were fastest on none of 16 shapes)
 };
 static const PackedCfg SPLIT_CFGS[] = {
-    {128, 128, 32, 4, 64, launch_packed<128, 128, 32, true, 2, 2>},
-    {256, 128, 32, 8, 64, launch_packed<256, 128, 32, true, 4, 2>},
-    {128, 128, 32, 8, 64, launch_packed<128, 128, 32, true, 2, 4>},
+    {256, 256, 32, 8, 128, launch_pipe<256, 256, 2, 4, 2>, 1},
+    {128, 128, 32, 4, 64, launch_pipe<128, 128, 2, 2, 2>, 1},
+    {64, 64, 32, 4, 32, launch_pipe<64, 64, 2, 2, 2>, 1},
 };
 constexpr int PK_MAXTILE = 256;  // largest bm / bn of any configuration
 
@@ -1246,19 +1260,37 @@ static const PackedCfg* packed_cfgs(int mode, int& count) {
   return SPLIT_CFGS;
 }
 
-// Configuration without tuning, from measurements on MI355X: BF16 uses the
-// 8-wave 256 x 256 tile when both sides fill it (8192^3: 1.24 ms against
-// 1.43 ms for 4 waves; 65536 x 1024 x 1024: 0.294 against 0.348 ms), split
-// mode the 8-wave 256 x 128 tile for long K (8192^3: 3.55 against 4.18 ms)
-// and 128 x 128 otherwise (K = 1024: 0.59 against 0.74 ms).
+// Configuration without tuning, from measurements on MI355X.  The pipelined
+// kernels: the tile with the least estimated time, blocks of a CU times the
+// measured time of a tile per k (ns; alone on its CU / sharing it) plus a
+// fixed part (us).  Measured us for the tiles 256 / 128 / 64: 512^3 19 / 8.5 /
+// 5.2, 1024^3 28 / 12.7 / 7.6, 4096 x 1024 x 1024 30 / 15.2 / 16.3,
+// 3000^3 72 / 69 / 127, 16384 x 4096 x 4096 402 / 504 / 792, 65536 x 1024 x
+// 1024 150 / 212 / 288.
+// Split mode, packing included: 1024^3 68 / 36 / 26, 4096 x 1024 x 1024 75 /
+// 46 / 47, 3000^3 194 / 195 / 284, 8192^3 2172 / 2697 / 3508.
 // FP32 takes the 256 x 256 tile when at least 512 such tiles cover C (8192^3:
 // 141 against 126-135 TFLOP/s for the other tiles; 65536 x 1024 x 1024: 124
 // against 100-113), the 128 x 128 tile otherwise (4096 x 1024 x 784: 92
 // against 31 TFLOP/s for 256 x 256, which leaves most CUs idle).
+static uint64_t splitk_chunk(uint64_t M, uint64_t N, uint64_t Kp);
+
 static int default_cfg(int mode, uint64_t M, uint64_t N, uint64_t K) {
   if (mode == VKH_GEMM_FP32) return ceil_div(M, (uint64_t)256) * ceil_div(N, (uint64_t)256) >= 512 ? 3 : 0;
-  if (mode == VKH_GEMM_BF16) return (M >= 256 && N >= 256) ? 1 : 2;
-  return (M >= 256 && N >= 128 && K >= 4096) ? 1 : 0;
+  static const struct { uint64_t tile; double fixed_us, alone_ns, shared_ns; } COST[2][3] = {
+      {{256, 4.0, 22.9, 22.9}, {128, 3.5, 8.2, 7.5}, {64, 2.5, 4.7, 3.5}},
+      {{256, 4.0, 59.5, 59.5}, {128, 3.5, 22.0, 18.9}, {64, 2.5, 11.0, 6.3}}};
+  const auto& T = COST[mode == VKH_GEMM_BF16X3];
+  const uint64_t Kp = ceil_div(std::max<uint64_t>(K, 1), (uint64_t)PK_KALIGN) * PK_KALIGN;
+  const uint64_t kc = splitk_chunk(M, N, Kp), S = ceil_div(Kp, kc);
+  int best = 0;
+  double bt = 0;
+  for (int i = 0; i < 3; ++i) {
+    const uint64_t n = ceil_div(ceil_div(M, T[i].tile) * ceil_div(N, T[i].tile) * S, (uint64_t)256);
+    const double t = T[i].fixed_us + 1e-3 * (double)kc * std::max(T[i].alone_ns, T[i].shared_ns * (double)n);
+    if (i == 0 || t < bt) { best = i; bt = t; }
+  }
+  return best;
 }
 
 // number of kernel configurations of a mode
@@ -1343,21 +1375,18 @@ static uint16_t* pack_area(vkh_gpu* g, size_t bytes) {
   return (uint16_t*)g->pack;
 }
 
-template <bool SPLIT>
+template <int PARTS>
 static void pack_operand(vkh_gpu* g, const float* src, uint64_t ld, bool trans, uint64_t R,
-                         uint64_t K, uint16_t* hi, uint16_t* lo, uint64_t Rp, uint64_t Kp) {
+                         uint64_t K, uint16_t* dst, uint64_t Rp, uint64_t Kp) {
   if (!trans) {
-    const int vec = ((uintptr_t)src & 15u) == 0 && ld % 4 == 0;
     const uint64_t total4 = Rp * (Kp / 4);
     VKH_REQUIRE(total4 < (uint64_t(1) << 31), "gemm pack: operand too large");
-    hipLaunchKernelGGL((k_pack_rows<SPLIT>), dim3((unsigned)ceil_div(total4, 256)), dim3(256), 0, g->stream,
-                       src, ld, R, K, hi, lo, (uint32_t)total4, FastDiv((uint32_t)(Kp / 4)), Kp, vec);
+    hipLaunchKernelGGL((k_pack_rows<PARTS>), dim3((unsigned)ceil_div(total4, 256)), dim3(256), 0, g->stream,
+                       src, ld, R, K, dst, (uint32_t)total4, FastDiv((uint32_t)(Kp / 4)), Kp);
   } else {
-    const int vec = ((uintptr_t)src & 15u) == 0 && ld % 4 == 0;
     VKH_REQUIRE(Rp % PK_TR == 0, "gemm pack: padded rows not a multiple of the tile");
     dim3 grid((unsigned)(Rp / PK_TR), (unsigned)ceil_div(Kp, PK_TK));
-    hipLaunchKernelGGL((k_pack_cols<SPLIT>), grid, dim3(256), 0, g->stream, src, ld, R, K, hi, lo,
-                       Rp, Kp, vec);
+    hipLaunchKernelGGL((k_pack_cols<PARTS>), grid, dim3(256), 0, g->stream, src, ld, R, K, dst, Rp, Kp);
   }
   check_launch("gemm pack");
 }
@@ -1373,33 +1402,30 @@ static void gemm_packed(vkh_gpu* g, int mode, bool ta, bool tb, GemmArgs& a, int
   const PackedCfg* cfgs = packed_cfgs(mode, ncfg);
   VKH_REQUIRE(cfg >= 0 && cfg < ncfg, "gemm: configuration index out of range");
   const PackedCfg& s = cfgs[cfg];
-  const uint64_t Mp = ceil_div(a.M, s.bm) * s.bm, Np = ceil_div(a.N, s.bn) * s.bn;
+  // rows padded to the tile, and to the transposing pack's
+  const uint64_t pm = std::max(s.bm, PK_TR), pn = std::max(s.bn, PK_TR);
+  const uint64_t Mp = ceil_div(a.M, pm) * pm, Np = ceil_div(a.N, pn) * pn;
   const uint64_t Kp = ceil_div(std::max<uint64_t>(a.K, 1), PK_KALIGN) * PK_KALIGN;
   uint16_t* base = pack_area(g, packed_bytes(mode, a.M, a.N, a.K));
-  const uint16_t* Ah = base;
-  uint16_t* Al = split ? base + Mp * Kp : nullptr;
-  uint16_t* Bp = split ? Al + Mp * Kp : base + Mp * Kp;
-  const uint16_t* Bh = Bp;
-  uint16_t* Bl = split ? Bp + Np * Kp : nullptr;
+  const int parts = split ? 2 : 1;
+  uint16_t* Bp = base + Mp * Kp * parts;
   // op(A)[m][k] and op(B)^T[n][k] = op(B)[k][n]
   if (split) {
-    pack_operand<true>(g, a.A, a.lda, ta, a.M, a.K, base, Al, Mp, Kp);
-    pack_operand<true>(g, a.B, a.ldb, !tb, a.N, a.K, Bp, Bl, Np, Kp);
+    pack_operand<2>(g, a.A, a.lda, ta, a.M, a.K, base, Mp, Kp);
+    pack_operand<2>(g, a.B, a.ldb, !tb, a.N, a.K, Bp, Np, Kp);
   } else {
-    if (!a_pre) pack_operand<false>(g, a.A, a.lda, ta, a.M, a.K, base, nullptr, Mp, Kp);
-    if (!b_pre) pack_operand<false>(g, a.B, a.ldb, !tb, a.N, a.K, Bp, nullptr, Np, Kp);
+    if (!a_pre) pack_operand<1>(g, a.A, a.lda, ta, a.M, a.K, base, Mp, Kp);
+    if (!b_pre) pack_operand<1>(g, a.B, a.ldb, !tb, a.N, a.K, Bp, Np, Kp);
   }
-  if (a_pre) Ah = a_pre;
-  if (b_pre) Bh = b_pre;
-  a.tiles_m = (uint32_t)(Mp / s.bm);
-  a.tiles_n = (uint32_t)(Np / s.bn);
+  a.tiles_m = (uint32_t)ceil_div(a.M, (uint64_t)s.bm);
+  a.tiles_n = (uint32_t)ceil_div(a.N, (uint64_t)s.bn);
   const uint64_t nb = (uint64_t)a.tiles_m * a.tiles_n;
   VKH_REQUIRE(nb < (uint64_t(1) << 31), "GEMM too large");
   const uint64_t kc = splitk_chunk(a.M, a.N, Kp);
   const uint64_t S = ceil_div(Kp, kc);
   float* part = nullptr;
   if (S > 1) part = reinterpret_cast<float*>(reinterpret_cast<char*>(base) + operand_bytes(mode, a.M, a.N, Kp));
-  PackedArgs pa{Ah, Al, Bh, Bl, Kp, kc, part, a};
+  PackedArgs pa{a_pre ? a_pre : base, b_pre ? b_pre : Bp, Kp, kc, part, a};
   s.launch(dim3((unsigned)nb, (unsigned)S), g->stream, pa);
   check_launch("gemm (packed)");
   if (S > 1) {
@@ -2074,8 +2100,8 @@ int vkh_gemm_autotune(vkh_gpu* g, int mode, int trans_a, int trans_b, uint64_t M
     uint16_t* pa = pre ? (uint16_t*)wpa.get() : nullptr;
     uint16_t* pb = pre ? (uint16_t*)wpb.get() : nullptr;
     if (pre) {
-      pack_operand<false>(g, A, a.lda, trans_a, M, K, pa, nullptr, Mp, Kp);
-      pack_operand<false>(g, B, a.ldb, !trans_b, N, K, pb, nullptr, Np, Kp);
+      pack_operand<1>(g, A, a.lda, trans_a, M, K, pa, Mp, Kp);
+      pack_operand<1>(g, B, a.ldb, !trans_b, N, K, pb, Np, Kp);
     }
     hipEvent_t e0, e1;
     VKH_HIP(hipEventCreate(&e0));
