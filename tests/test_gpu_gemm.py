@@ -586,3 +586,110 @@ def test_pipelined_tile_edges(gpu, mode, M, N, K):
             np.testing.assert_array_equal(np.asarray(gC), P * (aux > 0))
     finally:
         _lib.call("vkh_gemm_set_config", h, md, 0, 1, M, N, K, -1)
+
+
+# Large FP32 products run from three BF16 parts (by sizes only; 4001 x 2047 x
+# 1030 is such a product, with ragged edges in every dimension), unless an
+# operand holds values out of their range; then the FP32 kernel runs.
+F32X3 = (4001, 2047, 1030)
+
+
+def f32x3_operands(seed, exact=False):
+    M, N, K = F32X3
+    rng = np.random.default_rng(seed)
+    if exact:  # products and sums are whole numbers below 2^24
+        return rng.integers(-60, 61, (M, K)).astype(np.float32), rng.integers(-60, 61, (K, N)).astype(np.float32)
+    return rng.standard_normal((M, K)).astype(np.float32), rng.standard_normal((K, N)).astype(np.float32)
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_fp32_parts_exact(gpu, ta, tb):
+    A, B = f32x3_operands(60, exact=True)
+    M, N, _ = F32X3
+    P = (A.astype(np.float64) @ B.astype(np.float64)).astype(np.float32)
+    got = run_gemm(gpu, "fp32", ta, tb, A.T.copy() if ta else A, B.T.copy() if tb else B)
+    np.testing.assert_array_equal(got, P)
+    if not ta and tb:
+        rng = np.random.default_rng(61)
+        C0 = rng.integers(-9, 10, (M, N)).astype(np.float32)
+        bias = rng.integers(-9, 10, N).astype(np.float32)
+        got = run_gemm(gpu, "fp32", 0, 1, A, B.T.copy(), C0=C0, alpha=2.0, beta=-1.0, bias=bias, act="relu")
+        np.testing.assert_array_equal(got, np.maximum(2 * P - C0 + bias, 0))
+
+
+def test_fp32_parts_error_not_larger(gpu):
+    """Against FP64, no further off than the FP32 kernel, which the same
+    product takes when one element is a denormal (all other rows compared)."""
+    A, B = f32x3_operands(62)
+    ref, bound = ref_gemm(0, 0, A, B)
+    parts = run_gemm(gpu, "fp32", 0, 0, A, B)
+    A2 = A.copy()
+    A2[0, 0] = 1e-40
+    native = run_gemm(gpu, "fp32", 0, 0, A2, B)
+    assert (np.abs(parts - ref) / bound).max() <= TOL["fp32"]
+    err = [np.linalg.norm((v - ref)[1:]) for v in (parts, native)]
+    assert not np.array_equal(parts[1:], native[1:])  # (two kernels)
+    assert err[0] <= err[1], err
+
+
+@pytest.mark.parametrize("where", ["A", "B"])
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan, 3e38, 1e-40, 2.0 ** -90])
+def test_fp32_parts_out_of_range(gpu, where, value):
+    A, B = f32x3_operands(63)
+    (A if where == "A" else B)[7, 9] = value
+    with np.errstate(invalid="ignore", over="ignore"):
+        ref = A.astype(np.float64) @ B.astype(np.float64)
+        ref32 = ref.astype(np.float32)  # overflow to infinity
+    bound = np.abs(A).astype(np.float64) @ np.abs(B).astype(np.float64)
+    got = run_gemm(gpu, "fp32", 0, 0, A, B)
+    fin = np.isfinite(ref32)
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(ref32))
+    assert (np.abs(got[fin] - ref[fin]) <= TOL["fp32"] * bound[fin]).all()
+
+
+def test_fp32_parts_small_products(gpu):
+    """Both operands near 2^-48: their products are near 2^-96 and keep the
+    FP32 accuracy."""
+    A, B = f32x3_operands(64)
+    A, B = A * np.float32(2.0 ** -48), B * np.float32(2.0 ** -48)
+    ref, bound = ref_gemm(0, 0, A, B)
+    got = run_gemm(gpu, "fp32", 0, 0, A, B)
+    assert (np.abs(got - ref) / bound).max() <= TOL["fp32"]
+
+
+@pytest.mark.parametrize("reserve", [True, False])
+def test_fp32_parts_in_a_graph(gpu, reserve):
+    """Captured, with and without a reserved packing region (without room the
+    FP32 kernel runs): replays follow the operands' values, back and forth
+    between the two kernels."""
+    import ctypes
+    M, N, K = F32X3
+    h = gpu._handle
+    A, B = f32x3_operands(65)
+    bad = A.copy()
+    bad[3, 4] = np.inf
+    want = {n: run_gemm(gpu, "fp32", 0, 0, v, B) for n, v in (("good", A), ("bad", bad))}
+    small = A.copy()
+    small[0, 0] = 1e-40  # the FP32 kernel's results in every other row
+    want["small"] = run_gemm(gpu, "fp32", 0, 0, small, B)
+    src = {"good": vk.Array(gpu, data=A), "bad": vk.Array(gpu, data=bad), "small": vk.Array(gpu, data=small)}
+    gA, gB, gC = vk.Array(gpu, data=A), vk.Array(gpu, data=B), vk.Array(gpu, shape=(M, N))
+    gpu.wait()
+    if reserve:
+        _lib.call("vkh_gemm_reserve", h, 0, M, N, K)
+    _lib.call("vkh_graph_begin", h)
+    _lib.call("vkh_gemm", h, 0, 0, 0, M, N, K, 1.0, gA._ptr, K, gB._ptr, N, 0.0, gC._ptr, N, None, 0, None)
+    ex = ctypes.c_void_p()
+    _lib.call("vkh_graph_end", h, ctypes.byref(ex))
+    try:
+        for name in ("good", "bad", "good", "small", "good"):
+            _lib.call("vkh_copy", h, gA._ptr, src[name]._ptr, gA.buffer.nbytes)
+            _lib.call("vkh_graph_launch", h, ex.value)
+            gC._set_job()
+            got = np.asarray(gC)
+            if reserve or name != "good":
+                np.testing.assert_array_equal(got, want[name])
+            else:  # (an earlier reservation on this context may have left room)
+                assert np.array_equal(got, want["good"]) or np.array_equal(got[1:], want["small"][1:])
+    finally:
+        _lib.call("vkh_graph_destroy", ex.value)
