@@ -554,16 +554,16 @@ def test_every_bf16_configuration_with_bf16_copies(gpu, M, N, K):
     assert (np.abs(outs[0] - ref) / bound).max() <= (K + 2) * 2.0 ** -24
 
 
-# The pipelined tiles: one to three k slices (64 deep in BF16 mode, 32 in
-# split mode), output edges just below, at and past a tile, odd leading
+# Every tile: one to three k slices (64 deep in BF16 mode, 32 in split mode, 32
+# or 64 in FP32), output edges just below, at and past a tile, odd leading
 # dimensions (16-byte stores at 4-byte alignment, 1 to 3 columns past the last
 # whole group), both epilogues (straight from the accumulators; staged, taken
 # for the activation derivative).  Integer-valued operands make every product
 # and sum exact, so the results must equal NumPy's bit for bit.
-@pytest.mark.parametrize("mode", ["bf16", "bf16x3"])
+@pytest.mark.parametrize("mode", ["bf16", "bf16x3", "fp32"])
 @pytest.mark.parametrize("M,N,K", [(17, 17, 17), (63, 65, 64), (64, 64, 65), (129, 127, 128), (257, 255, 129),
                                    (256, 256, 192), (300, 515, 33), (511, 513, 200), (130, 66, 4160)])
-def test_pipelined_tile_edges(gpu, mode, M, N, K):
+def test_tile_edges(gpu, mode, M, N, K):
     rng = np.random.default_rng(M + 3 * N + 7 * K)
     h, md = gpu._handle, _lib.GEMM_MODE[mode]
     A = rng.integers(-3, 4, (M, K)).astype(np.float32)
@@ -577,6 +577,11 @@ def test_pipelined_tile_edges(gpu, mode, M, N, K):
         for i in range(len(vk.gemm_configs(mode))):
             _lib.call("vkh_gemm_set_config", h, md, 0, 1, M, N, K, i)
             np.testing.assert_array_equal(run_gemm(gpu, mode, 0, 1, A, B), P)
+            for ta, tb in ((0, 0), (1, 0), (1, 1)) if mode == "fp32" else ():
+                _lib.call("vkh_gemm_set_config", h, md, ta, tb, M, N, K, i)
+                got = run_gemm(gpu, mode, ta, tb, A.T.copy() if ta else A, B if tb else B.T.copy())
+                _lib.call("vkh_gemm_set_config", h, md, ta, tb, M, N, K, -1)
+                np.testing.assert_array_equal(got, P)
             got = run_gemm(gpu, mode, 0, 1, A, B, C0=C0, alpha=2.0, beta=-1.0, bias=bias, act="relu")
             np.testing.assert_array_equal(got, np.maximum(2 * P - C0 + bias, 0))
             gC = vk.Array(gpu, shape=(M, N))

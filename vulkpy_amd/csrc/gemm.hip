@@ -801,19 +801,24 @@ constexpr int F32_BK = 32;
 
 static __device__ __attribute__((aligned(16))) float k_f32_zeros[4];
 
-template <int ROWS, bool KMAJ, int THREADS>
+//
+// VEC: the operand's contiguous extent is a multiple of 4, so a run of 4 is
+// wholly in or out of range.  Otherwise a run that crosses the end is read from
+// 4 elements before the end (the extent is more than 4) and shifted into place
+// at the LDS store.  16-byte loads need 4-byte alignment only.
+template <int ROWS, bool KMAJ, int THREADS, bool VEC, int BK = F32_BK>
 struct F32Stager {
-  static constexpr int NV = ROWS * F32_BK / 4 / THREADS;  // float4 per thread
-  static_assert(NV * 4 * THREADS == ROWS * F32_BK, "whole float4 per thread");
-  static constexpr int LD = KMAJ ? F32_BK : ROWS + 8;     // LDS row (floats)
-  static constexpr int FLOATS = KMAJ ? ROWS * F32_BK : F32_BK * LD;
+  static constexpr int NV = ROWS * BK / 4 / THREADS;  // float4 per thread
+  static_assert(NV * 4 * THREADS == ROWS * BK, "whole float4 per thread");
+  static constexpr int R4 = KMAJ ? BK / 4 : ROWS / 4;  // runs of a row
+  // LDS row (floats); tiles of up to 64 rows are read by 16-row fragments, four
+  // k rows (0, 4, 1, 5 apart) at a time, which 36 more floats keep apart
+  static constexpr int LD = KMAJ ? BK : ROWS > 64 ? ROWS + 8 : ROWS == 64 ? 100 : 36;
+  static constexpr int FLOATS = KMAJ ? ROWS * BK : BK * LD;
   f32x4_t r[NV];
 
   // Rows row0.. (K-major: the operand's rows; otherwise its columns) at k0,
-  // as runs of 4 elements along the contiguous dimension.  VEC: the operand
-  // is 16-byte aligned, its leading dimension and its contiguous extent are
-  // multiples of 4, so a run is wholly in or out of range.
-  template <bool VEC>
+  // as runs of 4 elements along the contiguous dimension.
   __device__ __forceinline__ void load(const float* P, uint64_t ld, uint64_t row0, uint64_t nrows,
                                        uint64_t k0, uint64_t K) {
 #pragma unroll
@@ -821,36 +826,40 @@ struct F32Stager {
       const int idx = threadIdx.x + i * THREADS;
       uint64_t gr, gc, rlim, clim;  // run row, first column, and their limits
       if constexpr (KMAJ) {
-        gr = row0 + idx / 8; gc = k0 + (idx % 8) * 4; rlim = nrows; clim = K;
+        gr = row0 + idx / R4; gc = k0 + (idx % R4) * 4; rlim = nrows; clim = K;
       } else {
-        gr = k0 + idx / (ROWS / 4); gc = row0 + (idx % (ROWS / 4)) * 4; rlim = K; clim = nrows;
+        gr = k0 + idx / R4; gc = row0 + (idx % R4) * 4; rlim = K; clim = nrows;
       }
-      if constexpr (VEC) {
-        const bool ok = gr < rlim && gc < clim;
-        r[i] = *reinterpret_cast<const f32x4_t*>(ok ? P + (gr * ld + gc) : k_f32_zeros);
-      } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const bool ok = gr < rlim && gc + e < clim;
-          r[i][e] = *(ok ? P + (gr * ld + gc + e) : k_f32_zeros);
-        }
-      }
+      const bool ok = gr < rlim && gc < clim;
+      if constexpr (!VEC) gc = min(gc, clim - 4);
+      r[i] = *reinterpret_cast<const f32x4u_t*>(ok ? P + (gr * ld + gc) : k_f32_zeros);
     }
   }
 
-  __device__ __forceinline__ void store(float* s) const {
+  // into LDS; row0, nrows, k0, K as given to load
+  __device__ __forceinline__ void store(float* s, uint64_t row0, uint64_t nrows, uint64_t k0, uint64_t K) const {
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
       const int idx = threadIdx.x + i * THREADS;
       int off;
       if constexpr (KMAJ) {
-        const int row = idx / 8, c = idx % 8;
-        off = row * F32_BK + ((c ^ (row & 7)) << 2);
+        const int row = idx / R4, c = idx % R4;
+        off = row * BK + ((c ^ (row & 7)) << 2);
       } else {
-        const int kr = idx / (ROWS / 4), c4 = idx % (ROWS / 4);
-        off = kr * LD + c4 * 4;
+        off = (idx / R4) * LD + (idx % R4) * 4;
       }
-      *reinterpret_cast<f32x4_t*>(s + off) = r[i];
+      f32x4_t v = r[i];
+      if constexpr (!VEC) {
+        const uint64_t gc = (KMAJ ? k0 : row0) + (idx % R4) * 4, last = (KMAJ ? K : nrows) - 4;
+        if (gc > last) {  // shifted down by the elements before the run (or out of range: zeros)
+          const uint64_t sh = gc - last;
+          v[0] = sh == 1 ? v[1] : sh == 2 ? v[2] : sh == 3 ? v[3] : 0.f;
+          v[1] = sh == 1 ? v[2] : sh == 2 ? v[3] : 0.f;
+          v[2] = sh == 1 ? v[3] : 0.f;
+          v[3] = 0.f;
+        }
+      }
+      *reinterpret_cast<f32x4_t*>(s + off) = v;
     }
   }
 
@@ -858,10 +867,25 @@ struct F32Stager {
   __device__ __forceinline__ static f32x4_t frag(const float* s, int row, int g, int h) {
     if constexpr (KMAJ) {
       const int c = 2 * g + h;
-      return *reinterpret_cast<const f32x4_t*>(s + row * F32_BK + ((c ^ (row & 7)) << 2));
+      return *reinterpret_cast<const f32x4_t*>(s + row * BK + ((c ^ (row & 7)) << 2));
     } else {
       const float* q = s + (8 * g + 4 * h) * LD + row;
       return f32x4_t{q[0], q[LD], q[2 * LD], q[3 * LD]};
+    }
+  }
+
+  // values of tile row `row` for the two 16 x 16 x 4 MFMAs of k group g: lanes
+  // 16 q .. 16 q + 15 supply k = 0, 4, 1, 5 [q] of the group, then 2, 6, 3, 7,
+  // the order in which four 32 x 32 x 2 MFMAs add them
+  __device__ __forceinline__ static void frag16(const float* s, int row, int g, int q, float (&v)[2]) {
+    if constexpr (KMAJ) {
+      const f32x4_t f = frag(s, row, g, q & 1);
+      v[0] = q & 2 ? f[1] : f[0];
+      v[1] = q & 2 ? f[3] : f[2];
+    } else {
+      const float* p = s + (8 * g + 4 * (q & 1) + (q >> 1)) * LD + row;
+      v[0] = p[0];
+      v[1] = p[2 * LD];
     }
   }
 };
@@ -874,8 +898,8 @@ k_gemm_f32(GemmArgs p, float* part, uint64_t kc) {
   constexpr int WM = BM / WGM, WN = BN / WGN;
   static_assert(WM % 32 == 0 && WN % 32 == 0, "32 x 32 MFMA blocks per wave");
   constexpr int TM = WM / 32, TN = WN / 32;
-  using SA = F32Stager<BM, AK, THREADS>;
-  using SB = F32Stager<BN, BKM, THREADS>;
+  using SA = F32Stager<BM, AK, THREADS, VEC>;
+  using SB = F32Stager<BN, BKM, THREADS, VEC>;
   constexpr int MAIN = 2 * (SA::FLOATS + SB::FLOATS), STAGE = WAVES * 32 * (WN + 4);
   constexpr int SMEM_FLOATS = MAIN > STAGE ? MAIN : STAGE;
   constexpr bool TST = 4 * STAGE + tt_bytes<WAVES, WN>() <= 4 * SMEM_FLOATS;
@@ -922,18 +946,18 @@ k_gemm_f32(GemmArgs p, float* part, uint64_t kc) {
   const uint64_t kb = part ? (uint64_t)blockIdx.y * kc : 0;
   const uint64_t ke = part ? min(kb + kc, K) : K;
   const uint64_t nk = (ke - kb + F32_BK - 1) / F32_BK;
-  sa.template load<VEC>(p.A, p.lda, m0, p.M, kb, K);
-  sb.template load<VEC>(p.B, p.ldb, n0, p.N, kb, K);
-  sa.store(As(0));
-  sb.store(Bs(0));
+  sa.load(p.A, p.lda, m0, p.M, kb, K);
+  sb.load(p.B, p.ldb, n0, p.N, kb, K);
+  sa.store(As(0), m0, p.M, kb, K);
+  sb.store(Bs(0), n0, p.N, kb, K);
   __syncthreads();
   frags(0, 0, 0);
   int cur = 0;
   for (uint64_t kt = 0; kt < nk; ++kt) {
     // the next slice (past K: zeros) into registers
     // (the prefetch after a chunk's last slice is stored but never used)
-    sa.template load<VEC>(p.A, p.lda, m0, p.M, kb + (kt + 1) * F32_BK, K);
-    sb.template load<VEC>(p.B, p.ldb, n0, p.N, kb + (kt + 1) * F32_BK, K);
+    sa.load(p.A, p.lda, m0, p.M, kb + (kt + 1) * F32_BK, K);
+    sb.load(p.B, p.ldb, n0, p.N, kb + (kt + 1) * F32_BK, K);
     // keep the loads here: left to itself the scheduler sinks them to the
     // LDS store at the end of the slice, where their latency is exposed
     __builtin_amdgcn_sched_barrier(0);
@@ -960,8 +984,8 @@ k_gemm_f32(GemmArgs p, float* part, uint64_t kc) {
       }
     }
     // the last group's MFMAs alternate with the LDS stores of the next slice
-    sa.store(As(cur ^ 1));
-    sb.store(Bs(cur ^ 1));
+    sa.store(As(cur ^ 1), m0, p.M, kb + (kt + 1) * F32_BK, K);
+    sb.store(Bs(cur ^ 1), n0, p.N, kb + (kt + 1) * F32_BK, K);
 #pragma unroll
     for (int q = 0; q < NM; ++q) {
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);    // MFMA
@@ -976,16 +1000,95 @@ k_gemm_f32(GemmArgs p, float* part, uint64_t kc) {
                                        m0, n0, wm, wn, reinterpret_cast<uint16_t*>(smem + STAGE));
 }
 
+// Small FP32 tiles (T x T, four waves of T/2 x T/2) for products with few
+// outputs, on 16 x 16 x 4 MFMAs: an FP32 MFMA adds its k terms one after the
+// other, so in the k order of frag16 every output has the bits of the larger
+// tiles.  A 128 x 128 tile takes 128 matrix-core cycles a k on its CU however
+// few tiles there are (512^3: 16 CUs busy, 43 us); 64 x 64 takes 32 and 32 x 32
+// takes 8 (9.6 us), bound by the latency of a slice's loads.  Slices are 32 and
+// 64 deep: 64 and 128 are no faster alone (9.1-9.5 us) and leave one block a CU
+// (5137 x 586 x 270 52 against 35 us).  The code is small and the accumulators
+// are stored without staging (direct_epilogue): 150 x 32 x 32 3.3 against 12 us.
+template <bool AK, bool BKM, bool VEC, int T, int BK>
+__global__ void __launch_bounds__(256)
+k_gemm_f32_small(GemmArgs p, float* part, uint64_t kc) {
+  constexpr int W = T / 2, TM = W / 16;
+  using SA = F32Stager<T, AK, 256, VEC, BK>;
+  using SB = F32Stager<T, BKM, 256, VEC, BK>;
+  __shared__ __attribute__((aligned(16))) float smem[2 * (SA::FLOATS + SB::FLOATS)];
+  auto As = [&](int b) { return smem + b * SA::FLOATS; };
+  auto Bs = [&](int b) { return smem + 2 * SA::FLOATS + b * SB::FLOATS; };
+  uint32_t tm, tn;
+  tile_coords(p, tm, tn);
+  const uint64_t m0 = (uint64_t)tm * T, n0 = (uint64_t)tn * T;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wm = wave >> 1, wn = wave & 1;
+  const int l16 = lane & 15, lq = lane >> 4;
+  f32x4_t acc[TM][TM];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TM; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+  const uint64_t K = p.K;
+  const uint64_t kb = part ? (uint64_t)blockIdx.y * kc : 0;
+  const uint64_t ke = part ? min(kb + kc, K) : K;
+  const uint64_t nk = (ke - kb + BK - 1) / BK;
+  SA sa;
+  SB sb;
+  sa.load(p.A, p.lda, m0, p.M, kb, ke);
+  sb.load(p.B, p.ldb, n0, p.N, kb, ke);
+  sa.store(As(0), m0, p.M, kb, ke);
+  sb.store(Bs(0), n0, p.N, kb, ke);
+  __syncthreads();
+  for (uint64_t kt = 0; kt < nk; ++kt) {
+    const int cur = (int)(kt & 1);
+    const uint64_t k1 = kb + (kt + 1) * BK;
+    const bool more = kt + 1 < nk;
+    if (more) {
+      sa.load(p.A, p.lda, m0, p.M, k1, ke);
+      sb.load(p.B, p.ldb, n0, p.N, k1, ke);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int g = 0; g < BK / 8; ++g) {
+      float fa[TM][2], fb[TM][2];
+#pragma unroll
+      for (int i = 0; i < TM; ++i) SA::frag16(As(cur), wm * W + i * 16 + l16, g, lq, fa[i]);
+#pragma unroll
+      for (int j = 0; j < TM; ++j) SB::frag16(Bs(cur), wn * W + j * 16 + l16, g, lq, fb[j]);
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TM; ++j)  // (operands exchanged, for direct_epilogue)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fb[j][u], fa[i][u], acc[i][j], 0, 0, 0);
+    }
+    if (more) {
+      sa.store(As(cur ^ 1), m0, p.M, k1, ke);
+      sb.store(Bs(cur ^ 1), n0, p.N, k1, ke);
+    }
+    __syncthreads();
+  }
+  direct_epilogue(acc, p, part ? part + (uint64_t)blockIdx.y * p.M * p.N : nullptr, m0 + wm * W, n0 + wn * W);
+}
+
 // Kernel configurations of the FP32 path (tile and wave grid).  They differ
 // in how the output is tiled only: every output sums its k in the same order,
 // so the choice never changes a result.
 typedef void (*F32Launch)(dim3, hipStream_t, const GemmArgs&, bool ta, bool tb, bool vec, float* part,
                           uint64_t kc);
+#define VKH_F32_LAYOUTS(LAUNCH)                  \
+  do { /* A is K-major unless transposed, B when transposed */ \
+    if (!ta && !tb) LAUNCH(true, false);         \
+    else if (!ta && tb) LAUNCH(true, true);      \
+    else if (ta && !tb) LAUNCH(false, false);    \
+    else LAUNCH(false, true);                    \
+  } while (0)
 template <int BM, int BN, int WGM, int WGN>
 static void launch_f32(dim3 grid, hipStream_t s, const GemmArgs& a, bool ta, bool tb, bool vec, float* part,
                        uint64_t kc) {
   const dim3 block(64 * WGM * WGN);
-  // A is K-major unless transposed, B is K-major when transposed
 #define VKH_F32_LAUNCH(AK, BKM)                                                                   \
   do {                                                                                            \
     if (vec)                                                                                      \
@@ -993,21 +1096,32 @@ static void launch_f32(dim3 grid, hipStream_t s, const GemmArgs& a, bool ta, boo
     else                                                                                          \
       hipLaunchKernelGGL((k_gemm_f32<AK, BKM, false, BM, BN, WGM, WGN>), grid, block, 0, s, a, part, kc); \
   } while (0)
-  if (!ta && !tb) VKH_F32_LAUNCH(true, false);
-  else if (!ta && tb) VKH_F32_LAUNCH(true, true);
-  else if (ta && !tb) VKH_F32_LAUNCH(false, false);
-  else VKH_F32_LAUNCH(false, true);
+  VKH_F32_LAYOUTS(VKH_F32_LAUNCH);
 #undef VKH_F32_LAUNCH
 }
+template <int T, int BK>
+static void launch_f32_small(dim3 grid, hipStream_t s, const GemmArgs& a, bool ta, bool tb, bool vec, float* part,
+                             uint64_t kc) {
+#define VKH_F32_LAUNCH(AK, BKM)                                                                  \
+  do {                                                                                           \
+    if (vec)                                                                                     \
+      hipLaunchKernelGGL((k_gemm_f32_small<AK, BKM, true, T, BK>), grid, dim3(256), 0, s, a, part, kc); \
+    else                                                                                         \
+      hipLaunchKernelGGL((k_gemm_f32_small<AK, BKM, false, T, BK>), grid, dim3(256), 0, s, a, part, kc); \
+  } while (0)
+  VKH_F32_LAYOUTS(VKH_F32_LAUNCH);
+#undef VKH_F32_LAUNCH
+}
+#undef VKH_F32_LAYOUTS
 struct F32Cfg {
   int bm, bn, waves, wm;  // wm: rows of a wave's slab (BM / WGM)
   F32Launch launch;
 };
 static const F32Cfg F32_CFGS[] = {
     {128, 128, 4, 64, launch_f32<128, 128, 2, 2>},
-    {256, 128, 8, 64, launch_f32<256, 128, 4, 2>},
-    {128, 256, 8, 64, launch_f32<128, 256, 2, 4>},
     {256, 256, 8, 128, launch_f32<256, 256, 2, 4>},
+    {64, 64, 4, 32, launch_f32_small<64, 32>},
+    {32, 32, 4, 16, launch_f32_small<32, 64>},
 };
 constexpr int F32_NCFG = sizeof(F32_CFGS) / sizeof(F32_CFGS[0]);
 
@@ -1326,28 +1440,46 @@ static const PackedCfg* packed_cfgs(int mode, int& count) {
 // 1024 150 / 212 / 288.
 // Split mode, packing included: 1024^3 68 / 36 / 26, 4096 x 1024 x 1024 75 /
 // 46 / 47, 3000^3 194 / 195 / 284, 8192^3 2172 / 2697 / 3508.
-// FP32 takes the 256 x 256 tile when at least 512 such tiles cover C (8192^3:
-// 141 against 126-135 TFLOP/s for the other tiles; 65536 x 1024 x 1024: 124
-// against 100-113), the 128 x 128 tile otherwise (4096 x 1024 x 784: 92
-// against 31 TFLOP/s for 256 x 256, which leaves most CUs idle).
+// FP32 tiles likewise (the 256 x 256 tile only for its column sums and where
+// its blocks fill the chip evenly), us for 128 / 64 / 32: 150 x 32 x 32 12.2 /
+// 3.9 / 3.3, 512^3 43 / 19 / 9.6, 5137 x 586 x 270 44 / 35 / 35, 2048 x 2048 x
+// 512 50 / 54 / 63, 4096 x 1024 x 1024 92 / 102 / 123.
 static uint64_t splitk_chunk(uint64_t M, uint64_t N, uint64_t Kp);
+static uint64_t f32_splitk_chunk(uint64_t M, uint64_t N, uint64_t K);
+
+struct TileCost {
+  int cfg;
+  uint64_t tile;
+  // us once, and a block; ns a k of a block: alone on its CU, and sharing it
+  double fixed_us, block_us, alone_ns, shared_ns;
+};
+static const TileCost F32_COST[] = {{0, 128, 5.0, 3.0, 76.0, 61.0}, {2, 64, 3.0, 0.0, 32.0, 25.0},
+                                    {3, 32, 2.5, 0.0, 14.0, 9.0}, {1, 256, 8.0, 6.0, 239.0, 239.0}};
+static const TileCost BF16_COST[] = {{0, 256, 4.0, 0.0, 22.9, 22.9}, {1, 128, 3.5, 0.0, 8.2, 7.5},
+                                     {2, 64, 2.5, 0.0, 4.7, 3.5}};
+static const TileCost SPLIT_COST[] = {{0, 256, 4.0, 0.0, 59.5, 59.5}, {1, 128, 3.5, 0.0, 22.0, 18.9},
+                                      {2, 64, 2.5, 0.0, 11.0, 6.3}};
+
+// the least estimated time (us) and its configuration
+static double tile_estimate(int mode, uint64_t M, uint64_t N, uint64_t K, int& cfg) {
+  const bool f32 = mode == VKH_GEMM_FP32;
+  const TileCost* T = f32 ? F32_COST : mode == VKH_GEMM_BF16 ? BF16_COST : SPLIT_COST;
+  const uint64_t k = std::max<uint64_t>(K, 1), Kp = f32 ? k : ceil_div(k, (uint64_t)PK_KALIGN) * PK_KALIGN;
+  const uint64_t kc = f32 ? f32_splitk_chunk(M, N, Kp) : splitk_chunk(M, N, Kp), S = ceil_div(Kp, kc);
+  double bt = 0;
+  for (int i = 0; i < (f32 ? 4 : 3); ++i) {
+    const double n = (double)ceil_div(ceil_div(M, T[i].tile) * ceil_div(N, T[i].tile) * S, (uint64_t)256);
+    const double t = T[i].fixed_us + n * T[i].block_us +
+                     1e-3 * (double)kc * std::max(T[i].alone_ns, T[i].shared_ns * n);
+    if (i == 0 || t < bt) { cfg = T[i].cfg; bt = t; }
+  }
+  return bt;
+}
 
 static int default_cfg(int mode, uint64_t M, uint64_t N, uint64_t K) {
-  if (mode == VKH_GEMM_FP32) return ceil_div(M, (uint64_t)256) * ceil_div(N, (uint64_t)256) >= 512 ? 3 : 0;
-  static const struct { uint64_t tile; double fixed_us, alone_ns, shared_ns; } COST[2][3] = {
-      {{256, 4.0, 22.9, 22.9}, {128, 3.5, 8.2, 7.5}, {64, 2.5, 4.7, 3.5}},
-      {{256, 4.0, 59.5, 59.5}, {128, 3.5, 22.0, 18.9}, {64, 2.5, 11.0, 6.3}}};
-  const auto& T = COST[mode == VKH_GEMM_BF16X3];
-  const uint64_t Kp = ceil_div(std::max<uint64_t>(K, 1), (uint64_t)PK_KALIGN) * PK_KALIGN;
-  const uint64_t kc = splitk_chunk(M, N, Kp), S = ceil_div(Kp, kc);
-  int best = 0;
-  double bt = 0;
-  for (int i = 0; i < 3; ++i) {
-    const uint64_t n = ceil_div(ceil_div(M, T[i].tile) * ceil_div(N, T[i].tile) * S, (uint64_t)256);
-    const double t = T[i].fixed_us + 1e-3 * (double)kc * std::max(T[i].alone_ns, T[i].shared_ns * (double)n);
-    if (i == 0 || t < bt) { best = i; bt = t; }
-  }
-  return best;
+  int cfg = 0;
+  tile_estimate(mode, M, N, K, cfg);
+  return cfg;
 }
 
 // number of kernel configurations of a mode
@@ -1516,18 +1648,18 @@ static size_t f32_split_bytes(uint64_t M, uint64_t N, uint64_t K) {
 
 static void gemm_f32(vkh_gpu* g, bool ta, bool tb, GemmArgs& a, int cfg) {
   VKH_REQUIRE(cfg >= 0 && cfg < F32_NCFG, "gemm: configuration index out of range");
+  // (a small tile stores what direct_epilogue can; its partial sums always)
+  const uint64_t kc = f32_splitk_chunk(a.M, a.N, a.K);
+  const uint64_t S = ceil_div(a.K, kc);
+  if (F32_CFGS[cfg].bm < 128 && S == 1 && !direct_ok(a)) cfg = 0;
   const F32Cfg& c = F32_CFGS[cfg];
   a.tiles_m = (uint32_t)ceil_div(a.M, (uint64_t)c.bm);
   a.tiles_n = (uint32_t)ceil_div(a.N, (uint64_t)c.bn);
   const uint64_t nb = (uint64_t)a.tiles_m * a.tiles_n;
   VKH_REQUIRE(nb < (uint64_t(1) << 31), "GEMM too large");
-  // 16-byte runs: aligned operands whose leading dimension and contiguous
-  // extent (A: K unless transposed, else M; B: N unless transposed, else K)
-  // are multiples of 4
-  const bool vec = ((uintptr_t)a.A & 15u) == 0 && a.lda % 4 == 0 && (ta ? a.M : a.K) % 4 == 0 &&
-                   ((uintptr_t)a.B & 15u) == 0 && a.ldb % 4 == 0 && (tb ? a.K : a.N) % 4 == 0;
-  const uint64_t kc = f32_splitk_chunk(a.M, a.N, a.K);
-  const uint64_t S = ceil_div(a.K, kc);
+  // whole 4-element runs: contiguous extents (A: K unless transposed, else M;
+  // B: N unless transposed, else K) that are multiples of 4
+  const bool vec = (ta ? a.M : a.K) % 4 == 0 && (tb ? a.K : a.N) % 4 == 0;
   float* part = S > 1 ? reinterpret_cast<float*>(pack_area(g, f32_split_bytes(a.M, a.N, a.K))) : nullptr;
   c.launch(dim3((unsigned)nb, (unsigned)S), g->stream, a, ta, tb, vec, part, kc);
   check_launch("gemm");
@@ -1570,14 +1702,18 @@ static size_t f32x3_bytes(uint64_t M, uint64_t N, uint64_t K) {
 // By sizes only (so eager, captured and differently laid out calls agree):
 // where the estimated time, packing included, is below 0.85 of the FP32
 // kernel's.  A round of 256 tiles takes 66 ns a k and 6 us, packing moves 10
-// bytes an element, the four launches cost 15 us (2048^3, 128 tiles: 154 us
-// with the FP32 kernel, 164 estimated here).
+// bytes an element, the four launches cost 15 us; writing C costs both the
+// same.  (2048^3, 128 tiles: 154 us with the FP32 kernel, 164 estimated here;
+// 8192 x 2048 x 300 94 against 118 us.  A 128 x 128 tile of three parts was
+// slower everywhere: 4096 x 4096 x 1024 241 us.)
 static bool f32x3_route(uint64_t M, uint64_t N, uint64_t K) {
   if (f32_splitk_chunk(M, N, K) != K || f32x3_bytes(M, N, K) > F32X3_MAX_BYTES) return false;
   const double tiles = (double)(ceil_div(M, (uint64_t)F32X3_BM) * ceil_div(N, (uint64_t)F32X3_BN));
-  const double split_us = 15.0 + std::ceil(tiles / 256.0) * (6.0 + (double)K * 0.066) + (double)(M + N) * (double)K * 10.0 / 5e6;
-  const double fp32_us = 2.0 * (double)M * (double)N * (double)K / 135e6;
-  return split_us < 0.85 * fp32_us;
+  const double c_us = (double)M * (double)N * 4.0 / 5.5e6;
+  const double parts_us = 15.0 + std::ceil(tiles / 256.0) * (6.0 + (double)K * 0.066) +
+                          (double)(M + N) * (double)K * 10.0 / 5e6 + c_us;
+  int cfg = 0;
+  return parts_us < 0.85 * (tile_estimate(VKH_GEMM_FP32, M, N, K, cfg) + c_us);
 }
 
 __global__ void __launch_bounds__(64) k_clear_ranges(uint32_t* range) {
@@ -1749,14 +1885,38 @@ k_skinny_colwalk(SkinnyArgs a, uint64_t kchunk, float* part) {
   for (int q = 0; q < QB; ++q)
 #pragma unroll
     for (int w = 0; w < VW; ++w) acc[q][w] = 0.f;
-  for (uint64_t k = k0; k < k1; ++k) {
-    float x[VW];
+  // U terms at a time, all their loads issued before the first sum (one term at
+  // a time, each waited for its own loads: a 64-term chunk took 24 us, 8 now),
+  // added in k order
+  constexpr int U = QB <= 4 ? 8 : 4;
+  auto load_x = [&](uint64_t k, float (&x)[VW]) {
     if constexpr (VW == 4) {
       const float4 t = *reinterpret_cast<const float4*>(a.X + k * a.sxk + p);
       x[0] = t.x; x[1] = t.y; x[2] = t.z; x[3] = t.w;
     } else {
       x[0] = a.X[k * a.sxk + p];
     }
+  };
+  uint64_t k = k0;
+  for (; k + U <= k1; k += U) {
+    float x[U][VW], y[U][QB];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      load_x(k + u, x[u]);
+#pragma unroll
+      for (int q = 0; q < QB; ++q) y[u][q] = q < a.Q ? a.Y[(k + u) * a.syk + q * a.syq] : 0.f;
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int q = 0; q < QB; ++q)
+        if (q < a.Q)
+#pragma unroll
+          for (int w = 0; w < VW; ++w) acc[q][w] += x[u][w] * y[u][q];
+  }
+  for (; k < k1; ++k) {
+    float x[VW];
+    load_x(k, x);
 #pragma unroll
     for (int q = 0; q < QB; ++q) {
       if (q < a.Q) {
