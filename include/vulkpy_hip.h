@@ -478,6 +478,10 @@ int vkh_huber_rows(vkh_gpu* gpu, const float* x, const float* y, float* L,
  *        used by the autograd wrapper, no counterpart in the reference */
 int vkh_loss_grad(vkh_gpu* gpu, int kind, const float* x, const float* y,
                   float* dx, uint64_t n, float scale);
+/* vkh_loss_grad times the device scalar *grad (1 when null), after the scale:
+ * the autograd wrapper's incoming gradient.  No counterpart in the reference. */
+int vkh_loss_grad_scaled(vkh_gpu* gpu, int kind, const float* x, const float* y,
+                         float* dx, uint64_t n, float scale, const float* grad);
 /* vkh_mse_rows (kind 1) or vkh_huber_rows (kind 2) and vkh_loss_grad of the
  * same kind over the same [rows, cols] x, y, in one launch with the same
  * bits.  No counterpart in the reference (a captured training step's loss

@@ -384,3 +384,102 @@ def test_c4_reduced_training_matches_oracle(gpu):
                 bits_equal(p.value, w_new)
                 bits_equal(p.opt_state.m, m_new)
                 bits_equal(p.opt_state.v, v_new)
+
+
+# Row kernels of more than 64 columns: edges of the register rows (256, 512,
+# 1024, 2048 columns of one wave; 4096, 8192, 16384 of four; longer rows loop)
+# and rows that start off 16 bytes.  Sums of n terms go through chains of at
+# most 64 + 9 additions, so a softmax value is within (73 + 3 + |x - max|) 2^-24
+# of FP64's relatively, and a loss within the sum of |t| times that plus the
+# chain's rounding of its own terms.
+LONG_ROWS = [65, 67, 255, 256, 257, 513, 1000, 1024, 1025, 2048, 2049, 4096, 4097, 8193, 16384, 16386]
+
+
+@pytest.mark.parametrize("cols", LONG_ROWS)
+def test_long_row_softmax_and_cross_entropy(gpu, cols):
+    from vulkpy_amd._lib import call
+    rows = 7
+    rng = np.random.default_rng(cols)
+    x = (rng.standard_normal((rows, cols)) * 3).astype(f32)
+    x[1, 3:] = -np.inf                                   # masked
+    x[2, ::2] = np.finfo(f32).min
+    t = np.identity(cols, dtype=f32)[rng.integers(0, 3, rows)]
+    t[3] = rng.uniform(0, 1, cols) / cols                # dense targets
+    xd, td = x.astype(np.float64), t.astype(np.float64)
+    d = xd - xd.max(axis=1, keepdims=True)
+    p = np.exp(d)
+    p /= p.sum(axis=1, keepdims=True)
+    tol = (76 + np.where(p > 0, np.minimum(-d, 104.0), 0)) * 2.0 ** -24
+    L = -(td * np.log(p + 1e-8)).sum(axis=1)
+    Ltol = (td * (2 * tol + 80 * 2.0 ** -24 * np.abs(np.log(p + 1e-8)))).sum(axis=1)
+    gx, gt = A(gpu, x), A(gpu, t)
+    sm, sm2 = vk.Array(gpu, shape=x.shape), vk.Array(gpu, shape=x.shape)
+    gL, gL2 = vk.Array(gpu, shape=(rows,)), vk.Array(gpu, shape=(rows,))
+    call("vkh_softmax_cross_entropy", gpu._handle, gx._ptr, gt._ptr, sm._ptr, gL._ptr, rows, cols)
+    call("vkh_softmax", gpu._handle, gx._ptr, sm2._ptr, rows, cols)
+    call("vkh_cross_entropy", gpu._handle, sm2._ptr, gt._ptr, gL2._ptr, rows, cols)
+    for a in (sm, sm2, gL, gL2):
+        a._set_job()
+    for got in (np.asarray(sm), np.asarray(sm2)):
+        assert (np.abs(got - p) <= tol * p + 2.0 ** -126).all()
+    for got in (np.asarray(gL), np.asarray(gL2)):
+        assert (np.abs(got - L) <= Ltol + 1e-12).all()
+    dy = rng.standard_normal((rows, cols)).astype(f32)
+    y = np.asarray(sm)
+    y64, g64 = y.astype(np.float64), dy.astype(np.float64)
+    want = y64 * (g64 - (g64 * y64).sum(axis=1, keepdims=True))
+    bound = y64 * (np.abs(g64) + (np.abs(g64) * y64).sum(axis=1, keepdims=True))
+    gdy, dx = A(gpu, dy), vk.Array(gpu, shape=x.shape)
+    call("vkh_softmax_backward", gpu._handle, sm._ptr, gdy._ptr, dx._ptr, rows, cols)
+    dx._set_job([sm, gdy])
+    assert (np.abs(np.asarray(dx) - want) <= 80 * 2.0 ** -24 * bound + 1e-37).all()
+
+
+def test_long_row_softmax_nan_and_infinity(gpu):
+    """A NaN or +infinity spoils its own row only, as in NumPy; a NaN or a
+    non-finite log reaches the loss past targets of 0."""
+    from vulkpy_amd._lib import call
+    x = np.random.default_rng(3).standard_normal((4, 300)).astype(f32)
+    x[1, 299], x[2, 5] = np.nan, np.inf
+    t = np.zeros((4, 300), dtype=f32)
+    t[:, 0] = 1
+    gx, gt = A(gpu, x), A(gpu, t)
+    sm, L = vk.Array(gpu, shape=x.shape), vk.Array(gpu, shape=(4,))
+    call("vkh_softmax_cross_entropy", gpu._handle, gx._ptr, gt._ptr, sm._ptr, L._ptr, 4, 300)
+    sm._set_job()
+    L._set_job()
+    got, gL = np.asarray(sm), np.asarray(L)
+    assert np.isnan(got[1]).all() and np.isnan(gL[1])
+    assert np.isnan(got[2, 5]) and np.isnan(gL[2])
+    assert np.isfinite(got[[0, 3]]).all() and np.isfinite(gL[[0, 3]]).all()
+    p = np.full((4, 300), 0.5, dtype=f32)
+    p[1, 7], p[2, 7], p[3, 7] = np.nan, -1e-8, np.inf  # logs: NaN, -inf, inf, times a target of 0
+    gp = A(gpu, p)
+    call("vkh_cross_entropy", gpu._handle, gp._ptr, gt._ptr, L._ptr, 4, 300)
+    L._set_job([gp])
+    assert np.isnan(np.asarray(L)).tolist() == [False, True, True, True]
+
+
+@pytest.mark.parametrize("cols", [65, 68, 255, 1001])
+def test_long_row_losses(gpu, cols):
+    """MSE and Huber rows of more than 64 columns: one wave a row, the same
+    bits with and without the gradient."""
+    from vulkpy_amd._lib import call
+    rows = 9
+    rng = np.random.default_rng(cols)
+    x, t = (rng.standard_normal((rows, cols)).astype(f32) for _ in range(2))
+    d = t.astype(np.float64) - x
+    gx, gt = A(gpu, x), A(gpu, t)
+    for kind, name, want in ((1, "mse", d * d), (2, "huber", 0.5 * np.minimum(d * d, np.abs(d)))):
+        L, L2 = vk.Array(gpu, shape=(rows,)), vk.Array(gpu, shape=(rows,))
+        dx, dx2 = vk.Array(gpu, shape=x.shape), vk.Array(gpu, shape=x.shape)
+        call(f"vkh_{name}_rows", gpu._handle, gx._ptr, gt._ptr, L._ptr, rows, cols)
+        call("vkh_loss_rows_grad", gpu._handle, kind, gx._ptr, gt._ptr, L2._ptr, dx._ptr, rows, cols, 0.125)
+        call("vkh_loss_grad", gpu._handle, kind, gx._ptr, gt._ptr, dx2._ptr, x.size, 0.125)
+        for a in (L, L2, dx, dx2):
+            a._set_job()
+        bits_equal(L, np.asarray(L2))
+        bits_equal(dx, np.asarray(dx2))
+        # a lane adds at most 16 + 1 terms, the wave 6: relative to the positive sum
+        np.testing.assert_allclose(np.asarray(L), want.sum(axis=1), rtol=28 * 2.0 ** -24)
+        bits_equal(dx, O.loss_grad(name, x, t, 0.125))

@@ -146,6 +146,7 @@ _SIGNATURES = {
     "vkh_mse_rows": (c_int, [P, P, P, P, U64, U64]),
     "vkh_huber_rows": (c_int, [P, P, P, P, U64, U64]),
     "vkh_loss_grad": (c_int, [P, c_int, P, P, P, U64, c_float]),
+    "vkh_loss_grad_scaled": (c_int, [P, c_int, P, P, P, U64, c_float, P]),
     "vkh_loss_rows_grad": (c_int, [P, c_int, P, P, P, P, U64, U64, c_float]),
     "vkh_adam": (c_int, [P, P, P, P, P, U64, c_float, c_double, c_double, c_float, c_double, c_double]),
     "vkh_adam_pow_advance": (c_int, [P, P, c_double, c_double]),

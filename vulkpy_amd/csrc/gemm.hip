@@ -1886,7 +1886,7 @@ k_skinny_colwalk(SkinnyArgs a, uint64_t kchunk, float* part) {
 #pragma unroll
     for (int w = 0; w < VW; ++w) acc[q][w] = 0.f;
   // U terms at a time, all their loads issued before the first sum (one term at
-  // a time, each waited for its own loads: a 64-term chunk took 24 us, 8 now),
+  // a time, each waited for its own loads: a 50-term chunk took 24 us, 14 now),
   // added in k order
   constexpr int U = QB <= 4 ? 8 : 4;
   auto load_x = [&](uint64_t k, float (&x)[VW]) {

@@ -41,7 +41,7 @@ from typing import Dict, Optional, Tuple
 import numpy as np
 import torch
 
-from ._lib import ACT, BINOP, GEMM_MODE, REDOP, call, shape_array
+from ._lib import ACT, GEMM_MODE, REDOP, call
 
 __all__ = ["dense", "relu", "sigmoid", "softmax", "softmax_cross_entropy", "mse", "huber"]
 
@@ -73,14 +73,6 @@ def _f32(t: torch.Tensor, name: str) -> torch.Tensor:
 
 def _p(t: Optional[torch.Tensor]):
     return None if t is None else ctypes.c_void_p(t.data_ptr())
-
-
-def _scale_by(h: int, dx: torch.Tensor, g: torch.Tensor) -> None:
-    """dx *= g for a one-element device tensor g, without reading g on the host."""
-    g = _f32(g.reshape(1), "grad_output")
-    n = dx.numel()
-    call("vkh_binary_bcast", h, BINOP["mul"], _p(dx), _p(g), _p(dx), 1,
-         shape_array((n,)), shape_array((1,)), shape_array((n,)))
 
 
 class _Dense(torch.autograd.Function):
@@ -212,8 +204,9 @@ class _Loss(torch.autograd.Function):
         a, t = ctx.saved_tensors
         h = _ctx(a)
         dx = torch.empty_like(a)
-        call("vkh_loss_grad", h, _KIND[ctx.kind], _p(a), _p(t), _p(dx), a.numel(), ctx.scale)
-        _scale_by(h, dx, g)
+        # the incoming gradient is read on the device, not on the host
+        g = _f32(g.reshape(1), "grad_output")
+        call("vkh_loss_grad_scaled", h, _KIND[ctx.kind], _p(a), _p(t), _p(dx), a.numel(), ctx.scale, _p(g))
         return dx, None, None, None
 
 
