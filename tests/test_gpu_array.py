@@ -650,3 +650,39 @@ def test_timer_next_kernel(gpu):
     np.testing.assert_array_equal(np.asarray(r), a + c)
     np.testing.assert_array_equal(np.asarray(r2), a * np.float32(2.0))
     assert 0.0 < ms.value <= outer.value, (ms.value, outer.value)
+
+
+# Broadcasts over ragged rows (units of 4 columns, the last one moved back to
+# the row's end): row lengths around multiples of 4, up to 7 collapsed dims,
+# every operand order, broadcast copies, clamp bounds, and in place (where the
+# end of a row goes element by element).  Bit for bit against NumPy.
+ROWS_SHAPES = [
+    ((5, 4), (5, 1)), ((5, 5), (1, 5)), ((7, 6), (7, 1)), ((3, 7), (1, 7)), ((1000, 999), (1, 999)), ((1000, 999), (1000, 1)),
+    ((3, 1, 75), (1, 50, 75)), ((3, 1, 76), (1, 50, 76)), ((6, 1, 3), (1, 5, 3)), ((9, 1, 1), (1, 4, 6)),
+    ((4, 1, 5, 1), (1, 3, 1, 9)), ((2, 3, 1, 65), (2, 1, 4, 65)), ((1, 7, 30), (9, 1, 1)), ((2, 1, 3, 1, 2, 1, 5), (1, 4, 1, 2, 1, 3, 5)),
+    ((2, 1, 2, 1, 2, 1, 2, 1, 5), (1, 2, 1, 2, 1, 2, 1, 2, 5)), ((300, 301), (1, 301)), ((2, 100003), (2, 1)),
+]
+
+
+@pytest.mark.parametrize("sa,sb", ROWS_SHAPES)
+def test_ragged_row_broadcasts(gpu, sa, sb):
+    rng = np.random.default_rng(len(sa) * 100 + sa[-1])
+    a, b = rng.standard_normal(sa).astype(np.float32), rng.standard_normal(sb).astype(np.float32)
+    ga, gb = A(gpu, a), A(gpu, b)
+    for op in ("sub", "div"):
+        f = (lambda x, y: x - y) if op == "sub" else (lambda x, y: x / y)
+        assert_bits(f(ga, gb), f(a, b))
+        assert_bits(f(gb, ga), f(b, a))
+    so = np.broadcast_shapes(sa, sb)
+    assert_bits(ga.broadcast_to(so), np.broadcast_to(a, so))
+    assert_bits(gb.broadcast_to(so), np.broadcast_to(b, so))
+    x = rng.standard_normal(so).astype(np.float32)
+    for small, gs in ((a, ga), (b, gb)):
+        gx = A(gpu, x)
+        gx -= gs
+        assert_bits(gx, x - small)
+        gx = A(gpu, x)
+        gx.clamp(gs, 0.5, inplace=True)
+        assert_bits(gx, np.minimum(np.maximum(x, small), np.float32(0.5)))
+    assert_bits(A(gpu, x).clamp(ga, gb), np.minimum(np.maximum(x, a), b))
+    assert_bits(A(gpu, x).clamp(-0.25, gb), np.minimum(np.maximum(x, np.float32(-0.25)), b))

@@ -7,8 +7,10 @@
 // the host: size-1 dims are dropped and adjacent dims with compatible strides
 // are merged, so the common cases become a 2-D [rows, cols] traversal where
 // each operand is FULL (same layout as the output), ROW (indexed by column),
-// COL (indexed by row) or SCALAR.  Those run with 128-bit loads/stores and a
-// grid-stride loop; anything else takes a general strided N-d kernel.
+// COL (indexed by row) or SCALAR.  Those run with 128-bit loads/stores, one
+// unit a thread; ragged rows and up to 7 collapsed dims run in units of a row
+// (k_ew_rows), and what is left (more dims, rows of 1 to 3 columns, 2^31 units)
+// takes the general strided kernels.
 #include <hip/hip_ext.h>
 
 #include "bmath.h"
@@ -253,6 +255,92 @@ k_ewnd(F f, NdDesc d, float* out, uint64_t total) {
   }
 }
 
+// Broadcasts over rows: the output is [rows, cols] with rows split into up to
+// ROWS_MAXD outer dims, and each input is contiguous (K_FULL) or constant
+// (K_FIRST) along a row.  A unit is 4 consecutive columns of one row, whatever
+// the row's alignment (16-byte accesses need 4 bytes of it only): unit u of row
+// r starts at column 4u, the last one at cols - 4, so that no unit is partial
+// and no lane takes a branch; where the output overlaps an input (OVERLAP) the
+// last unit takes its cols % 4 elements one by one instead, since an element
+// must not be read after another unit wrote it.  The row's outer coordinates
+// come from one fast division each.  HBM-bound; against one element a thread
+// with a 64-bit division a dim: 50000 x 999 by a row or column 67 against 147
+// us, 8192 x 16383 179 against 394, (3000, 1, 75) - (1, 500, 75) 90 against
+// 413, with 76 columns 66 (nontemporal stores; with ordinary ones 106), (100,
+// 1, 200, 1) - (1, 300, 1, 50) 253 against 1374 us.
+constexpr int ROWS_MAXD = 6;
+struct RowsDesc {
+  int nd;                       // outer dims after the first (innermost last); the first needs no division
+  FastDiv dims[ROWS_MAXD - 1];  // their sizes
+  uint32_t st[3][ROWS_MAXD];    // element strides of every outer dim per input
+  const float* p[3];
+  float s[3];  // value of an input without a pointer (K_SCALAR)
+};
+typedef __attribute__((ext_vector_type(4), aligned(4))) float f32x4u_t;
+
+template <int KIND, bool NT>
+__device__ __forceinline__ f32x4u_t load_unit(const float* p, uint64_t off, uint32_t col, float s) {
+  if constexpr (KIND == K_FULL) {
+    const f32x4u_t* q = reinterpret_cast<const f32x4u_t*>(p + off + col);
+    return NT ? __builtin_nontemporal_load(q) : *q;
+  } else {
+    const float v = KIND == K_FIRST ? p[off] : s;
+    return f32x4u_t{v, v, v, v};
+  }
+}
+__device__ __forceinline__ f32x4u_t load_unit_any(int kind, const float* p, uint64_t off, uint32_t col, float s) {
+  if (kind == K_FULL) return load_unit<K_FULL, false>(p, off, col, s);
+  return kind == K_FIRST ? load_unit<K_FIRST, false>(p, off, col, s) : load_unit<K_SCALAR, false>(p, off, col, s);
+}
+
+// KA, KB: kinds of the first two inputs (-1: at run time, from kinds); NTA: the
+// first input is as large as the output (read once)
+template <class F, int KA, int KB, bool NTA, bool OVERLAP>
+__global__ void __launch_bounds__(EW_BLOCK)
+k_ew_rows(F f, RowsDesc d, float* out, uint32_t units, FastDiv upr, uint32_t cols, int kinds) {
+  const uint32_t stride = gridDim.x * EW_BLOCK;
+  for (uint32_t t = blockIdx.x * EW_BLOCK + threadIdx.x; t < units; t += stride) {
+    const uint32_t r = upr.div(t), u = t - r * upr.d;
+    const bool tail = OVERLAP && u * 4 + 3 >= cols;
+    const uint32_t col = OVERLAP ? u * 4 : min(u * 4, cols - 4);
+    uint64_t off[3] = {0, 0, 0};
+    uint32_t rem = r;
+    for (int k = d.nd; k > 0; --k) {
+      const uint32_t q = d.dims[k - 1].div(rem), c = rem - q * d.dims[k - 1].d;
+      rem = q;
+#pragma unroll
+      for (int i = 0; i < F::nin; ++i) off[i] += (uint64_t)c * d.st[i][k];
+    }
+#pragma unroll
+    for (int i = 0; i < F::nin; ++i) off[i] += (uint64_t)rem * d.st[i][0];
+    float* o = out + (uint64_t)r * cols + col;
+    if (OVERLAP && tail) {
+      for (uint32_t c = col; c < cols; ++c) {
+        float v[3];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+          const int kind = (kinds >> (4 * i)) & 15;
+          v[i] = i >= F::nin ? 0.f : kind == K_FULL ? d.p[i][off[i] + c] : kind == K_FIRST ? d.p[i][off[i]] : d.s[i];
+        }
+        o[c - col] = f(v[0], v[1], v[2]);
+      }
+      continue;
+    }
+    f32x4u_t a, b, c;
+    if constexpr (KA >= 0) a = load_unit<KA, NTA>(d.p[0], off[0], col, d.s[0]);
+    else a = load_unit_any(kinds & 15, d.p[0], off[0], col, d.s[0]);
+    if constexpr (F::nin < 2) b = a;
+    else if constexpr (KB >= 0) b = load_unit<KB, false>(d.p[1], off[1], col, d.s[1]);
+    else b = load_unit_any((kinds >> 4) & 15, d.p[1], off[1], col, d.s[1]);
+    if constexpr (F::nin < 3) c = a;
+    else c = load_unit_any((kinds >> 8) & 15, d.p[2], off[2], col, d.s[2]);
+    f32x4u_t v;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) v[q] = f(a[q], b[q], c[q]);
+    __builtin_nontemporal_store(v, reinterpret_cast<f32x4u_t*>(o));
+  }
+}
+
 // ---- host-side broadcast planning -----------------------------------------------
 struct InSpec {
   const float* p;           // null => scalar s
@@ -305,6 +393,68 @@ static Plan make_plan(const std::vector<InSpec>& ins, const std::vector<uint64_t
 
 static bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 
+// Launches k_ew_rows for a collapsed plan of 2 to ROWS_MAXD + 1 dims with at
+// least 4 columns and fewer than 2^31 units; returns false otherwise.
+template <class F>
+static bool run_rows(vkh_gpu* g, const F& f, const std::vector<InSpec>& ins, const Plan& pl, float* out) {
+  const int nd = (int)pl.dims.size(), od = nd - 1;  // outer dims
+  if (nd < 2 || od > ROWS_MAXD || pl.dims[nd - 1] < 4) return false;
+  const uint64_t cols = pl.dims[nd - 1], rows = pl.total / cols, upr = ceil_div(cols, 4);
+  const uint64_t lim = uint64_t(1) << 31;
+  if (cols >= lim || rows >= lim || rows * upr >= lim) return false;
+  RowsDesc d{};
+  d.nd = od - 1;
+  for (int k = 1; k < od; ++k) d.dims[k - 1] = FastDiv((uint32_t)pl.dims[k]);
+  int kinds = 0;
+  bool overlap = false;
+  for (size_t i = 0; i < ins.size(); ++i) {
+    d.p[i] = ins[i].p;
+    d.s[i] = ins[i].s;
+    int kind = K_SCALAR;
+    if (ins[i].p) {
+      kind = pl.st[i][nd - 1] ? K_FULL : K_FIRST;
+      uint64_t last = kind == K_FULL ? cols - 1 : 0;  // element offset of the input's last element
+      for (int k = 0; k < od; ++k) {
+        if (pl.st[i][k] >= (uint64_t(1) << 32)) return false;
+        d.st[i][k] = (uint32_t)pl.st[i][k];
+        last += (pl.dims[k] - 1) * pl.st[i][k];
+      }
+      const uintptr_t lo = (uintptr_t)ins[i].p, ob = (uintptr_t)out;
+      if (lo < ob + pl.total * sizeof(float) && ob < lo + (last + 1) * sizeof(float)) overlap = true;
+    }
+    kinds |= kind << (4 * i);
+  }
+  const int ka = kinds & 15, kb = (kinds >> 4) & 15;
+  const bool nta = ka == K_FULL && !overlap && [&] {
+    for (int k = 0; k < od; ++k)
+      if (pl.st[0][k] == 0) return false;
+    return true;
+  }();
+  const uint32_t units = (uint32_t)(rows * upr);
+  const dim3 grid(full_grid(units, EW_BLOCK));
+  const FastDiv fu((uint32_t)upr);
+  auto launch = [&](auto kernel) { ew_launch(g, kernel, grid, f, d, out, units, fu, (uint32_t)cols, kinds); };
+  // (overlapping operands and three inputs take their kinds at run time)
+  if constexpr (F::nin == 1) {
+    if (overlap) launch(k_ew_rows<F, -1, -1, false, true>);
+    else if (ka == K_FULL) launch(k_ew_rows<F, K_FULL, -1, false, false>);
+    else launch(k_ew_rows<F, K_FIRST, -1, false, false>);
+  } else if constexpr (F::nin == 2) {
+    if (overlap) launch(k_ew_rows<F, -1, -1, false, true>);
+    else if (nta && kb == K_FULL) launch(k_ew_rows<F, K_FULL, K_FULL, true, false>);
+    else if (nta && kb == K_FIRST) launch(k_ew_rows<F, K_FULL, K_FIRST, true, false>);
+    else if (ka == K_FULL && kb == K_FULL) launch(k_ew_rows<F, K_FULL, K_FULL, false, false>);
+    else if (ka == K_FULL && kb == K_FIRST) launch(k_ew_rows<F, K_FULL, K_FIRST, false, false>);
+    else if (ka == K_FIRST && kb == K_FULL) launch(k_ew_rows<F, K_FIRST, K_FULL, false, false>);
+    else launch(k_ew_rows<F, -1, -1, false, false>);
+  } else {
+    if (overlap) launch(k_ew_rows<F, -1, -1, false, true>);
+    else launch(k_ew_rows<F, -1, -1, false, false>);
+  }
+  check_launch("elementwise (rows)");
+  return true;
+}
+
 // Launch functor F over inputs (1..3) into out of shape oshape.
 template <class F>
 static void run_ew(vkh_gpu* g, const F& f, const std::vector<InSpec>& ins,
@@ -344,6 +494,8 @@ static void run_ew(vkh_gpu* g, const F& f, const std::vector<InSpec>& ins,
       if (rows == 1) vec_elems = (cols / 4) * 4;
       else if (cols % 4 == 0) vec_elems = rows * cols;
     }
+    // 2-D with a ragged or unaligned row
+    if (vec_elems == 0 && rows > 1 && run_rows(g, f, ins, pl, out)) return;
     const uint64_t total4 = vec_elems / 4;
     if (total4 > 0) {
       const uint64_t cols4 = rows == 1 ? total4 : cols / 4;
@@ -370,6 +522,7 @@ static void run_ew(vkh_gpu* g, const F& f, const std::vector<InSpec>& ins,
     return;
   }
   VKH_REQUIRE(nd <= MAXD, "too many dimensions after collapsing");
+  if (run_rows(g, f, ins, pl, out)) return;
   NdDesc d{};
   d.nd = nd;
   for (int k = 0; k < nd; ++k) d.dims[k] = pl.dims[k];
