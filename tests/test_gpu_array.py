@@ -686,3 +686,41 @@ def test_ragged_row_broadcasts(gpu, sa, sb):
         assert_bits(gx, np.minimum(np.maximum(x, small), np.float32(0.5)))
     assert_bits(A(gpu, x).clamp(ga, gb), np.minimum(np.maximum(x, a), b))
     assert_bits(A(gpu, x).clamp(-0.25, gb), np.minimum(np.maximum(x, np.float32(-0.25)), b))
+
+
+# Axis reductions around every kernel's edges: short rows (4 to 63 elements,
+# through LDS), medium rows (8 to 64 lanes a row), long ones (a block a row);
+# few columns (a block takes whole rows: 1 to 3 columns, ragged groups of 4, up
+# to 1023), many columns, several matrices, chunked and not.  max and min are
+# exact, sums of n positive terms within n 2^-24 relatively whatever their order.
+REDUCE_EDGES = [((r, n), 1) for n in (4, 5, 16, 31, 63, 64, 65, 75, 127, 131, 257, 513, 999, 1025, 2047, 2049, 4099)
+                for r in (1, 259)]
+REDUCE_EDGES += [((k, m), 0) for k, m in ((64, 2), (1000, 3), (70001, 3), (999, 5), (40000, 4), (5000, 75), (33000, 16),
+                                          (300, 1023), (12800, 32), (130, 1025), (70, 5003), (65, 100003))]
+REDUCE_EDGES += [((3, 20000, 7), 1), ((300, 65, 2), 1), ((5, 128, 96), 1), ((70000, 64, 3), 1)]
+
+
+@pytest.mark.parametrize("shape,axis", REDUCE_EDGES)
+def test_reduce_axis_edges(gpu, shape, axis):
+    rng = np.random.default_rng(sum(shape))
+    x = rng.uniform(0.5, 1.5, shape).astype(np.float32)
+    g = A(gpu, x)
+    n = shape[axis]
+    x64 = x.astype(np.float64)
+    np.testing.assert_allclose(np.asarray(g.sum(axis=axis)), x64.sum(axis=axis), rtol=n * 2.0 ** -24)
+    np.testing.assert_allclose(np.asarray(g.mean(axis=axis)), x64.mean(axis=axis), rtol=(n + 2) * 2.0 ** -24)
+    assert_bits(g.maximum(axis=axis), x.max(axis=axis))
+    assert_bits(g.minimum(axis=axis, rebroadcast=True), np.broadcast_to(x.min(axis=axis, keepdims=True), shape))
+    p = (1 + (x - 1) * np.float32(2.0 ** -10)).astype(np.float32)
+    np.testing.assert_allclose(np.asarray(A(gpu, p).prod(axis=axis)), p.astype(np.float64).prod(axis=axis),
+                               rtol=n * 2.0 ** -23)
+    # a NaN reaches its own output only; infinities and the lowest value stay
+    flat = [0] * len(shape)
+    flat[axis] = n - 1
+    x[tuple(flat)] = np.nan
+    np.testing.assert_array_equal(np.isnan(np.asarray(A(gpu, x).maximum(axis=axis))), np.isnan(x.max(axis=axis)))
+    np.testing.assert_array_equal(np.isnan(np.asarray(A(gpu, x).sum(axis=axis))), np.isnan(x.sum(axis=axis)))
+    low = np.full(shape, np.finfo(np.float32).min, dtype=np.float32)
+    assert_bits(A(gpu, low).maximum(axis=axis), low.max(axis=axis))
+    low[:] = -np.inf
+    assert_bits(A(gpu, low).maximum(axis=axis), low.max(axis=axis))

@@ -136,7 +136,7 @@ namespace vkh {
 // Makes the context's device current for the calling thread.
 // Column-sum order shared with vkh_bias_grad (reduce.hip): rows per chunk of
 // a [rows, cols] operand, and the in-order combine of chunk partials.
-uint64_t bias_grad_chunk(vkh_gpu* g, uint64_t rows, uint64_t cols, bool vec);
+uint64_t bias_grad_chunk(vkh_gpu* g, uint64_t rows, uint64_t cols);
 void sum_chunks(vkh_gpu* g, const float* part, float* out, uint64_t m, uint64_t nchunk);
 void sum_chunks_from_zero(vkh_gpu* g, const float* part, float* out, uint64_t m, uint64_t nchunk);
 

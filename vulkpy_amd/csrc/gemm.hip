@@ -2239,8 +2239,8 @@ static bool dense1_chunks(vkh_gpu* g, uint64_t B, uint64_t N, uint64_t& kc_dw, u
   if (B == 0 || B % D1_TR != 0 || N % D1_TC != 0 || B / D1_TR >= 65536 || N / D1_TC >= (uint64_t(1) << 31))
     return false;
   kc_dw = colwalk_chunk(g, N, B, true, ndw);
-  kc_db = bias_grad_chunk(g, B, N, true);
-  return kc_dw <= (uint64_t)D1_TR && D1_TR % kc_dw == 0 && kc_db <= (uint64_t)D1_TR && D1_TR % kc_db == 0;
+  kc_db = bias_grad_chunk(g, B, N);
+  return kc_db > 0 && kc_dw <= (uint64_t)D1_TR && D1_TR % kc_dw == 0 && kc_db <= (uint64_t)D1_TR && D1_TR % kc_db == 0;
 }
 
 static void gemm_impl(vkh_gpu* g, int mode, int trans_a, int trans_b, uint64_t M, uint64_t N,
@@ -2562,7 +2562,7 @@ int vkh_gemm_bf16io(vkh_gpu* g, int mode, int trans_a, int trans_b, uint64_t M, 
 static bool colsum_ok(vkh_gpu* g, int mode, int ta, int tb, uint64_t M, uint64_t N, uint64_t K) {
   if (std::min(M, N) <= SKINNY_MAX || K <= SMALLK_MAX) return false;
   if (mode < VKH_GEMM_FP32 || mode > VKH_GEMM_BF16X3) return false;
-  if (bias_grad_chunk(g, M, N, N % 4 == 0) != (uint64_t)CS_ROWS) return false;
+  if (bias_grad_chunk(g, M, N) != (uint64_t)CS_ROWS) return false;
   auto it = g->gemm_cfg.find(cfg_key(mode, ta, tb, M, N, K));
   const int cfg = it != g->gemm_cfg.end() ? it->second : default_cfg(mode, M, N, K);
   if (mode == VKH_GEMM_FP32)

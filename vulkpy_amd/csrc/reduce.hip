@@ -3,17 +3,26 @@
 // The reference reduces an axis with one thread per output element looping
 // sequentially over k (vulkpy/shader/sum_axis.comp:20-32) and the whole array
 // with a tree of ceil(n/64) passes (vulkpy/vkarray.py:1246-1274).  Here:
-//  * rows (post == 1): one block (long rows), one wave (medium) or one thread
-//    (short rows) per output, 128-bit loads, wave shuffle + LDS tree;
-//  * strided axes (post > 1): one thread per output column group (float4 when
-//    post % 4 == 0) looping sequentially over k -- the reference order -- and,
-//    when that leaves the GPU under-occupied, k is split into chunks whose
-//    partials are combined in chunk order by a second kernel;
+//  * rows (post == 1): one block (long rows), 8 to 64 lanes (medium) or one
+//    thread (short rows, through LDS) per output, 128-bit loads at any
+//    alignment, wave shuffle + LDS tree;
+//  * strided axes (post > 1): few columns take whole rows a block and a tree over
+//    them; otherwise one thread per group of 4 columns loops sequentially over
+//    k -- the reference order -- and, when that leaves the GPU under-occupied, k
+//    is split into chunks whose partials are combined in chunk order by a
+//    second kernel;
 //  * full reductions: grid-stride FP64 accumulation per thread, FP64 block
 //    tree, FP64 cross-block combine, one rounding to FP32 at the end.
 #include "common.h"
+#include "fastdiv.h"
 
 namespace vkh {
+
+// 16 bytes of memory at any 4-byte alignment
+typedef __attribute__((ext_vector_type(4), aligned(4))) float f32x4u_t;
+__device__ __forceinline__ f32x4u_t ld4u(const float* p) {
+  return __builtin_nontemporal_load(reinterpret_cast<const f32x4u_t*>(p));
+}
 
 template <int OP, typename T>
 struct Red;
@@ -73,63 +82,77 @@ constexpr int ROW_BLOCK = 256;
 // one block per row (long rows)
 // U: 128-bit loads in flight per thread (4 or 8); each thread still combines
 // its elements in index order, so U never changes the result
-template <int OP, bool VEC, int U>
+// (rows of any alignment: 16-byte groups, then the last L % 4 elements)
+template <int OP, int U>
 __global__ void __launch_bounds__(ROW_BLOCK)
 k_rows_block(const float* a, float* out, uint64_t rows, uint64_t L, int rebroadcast, float mul, float dv) {
   __shared__ float lds[ROW_BLOCK / 64];
+  using R = Red<OP, float>;
   for (uint64_t r = blockIdx.x; r < rows; r += gridDim.x) {
     const float* row = a + r * L;
-    float acc = Red<OP, float>::init();
-    if (VEC) {
-      using R = Red<OP, float>;
-      const float4* row4 = reinterpret_cast<const float4*>(row);
-      const uint64_t L4 = L / 4;
-      uint64_t i = threadIdx.x;
-      // U loads in flight, combined in the same order as the plain loop
-      for (; i + (U - 1) * ROW_BLOCK < L4; i += U * ROW_BLOCK) {
-        float4 v[U];
+    float acc = R::init();
+    const uint64_t L4 = L / 4;
+    uint64_t i = threadIdx.x;
+    // U loads in flight, combined in the same order as the plain loop
+    for (; i + (U - 1) * ROW_BLOCK < L4; i += U * ROW_BLOCK) {
+      f32x4u_t v[U];
 #pragma unroll
-        for (int q = 0; q < U; ++q) v[q] = ld_stream(row4 + i + q * ROW_BLOCK);
+      for (int q = 0; q < U; ++q) v[q] = ld4u(row + 4 * (i + q * ROW_BLOCK));
 #pragma unroll
-        for (int q = 0; q < U; ++q) acc = R::f(acc, R::f(R::f(v[q].x, v[q].y), R::f(v[q].z, v[q].w)));
-      }
-      for (; i < L4; i += ROW_BLOCK) {
-        const float4 v = ld_stream(row4 + i);
-        acc = R::f(acc, R::f(R::f(v.x, v.y), R::f(v.z, v.w)));
-      }
-    } else {
-      for (uint64_t i = threadIdx.x; i < L; i += ROW_BLOCK) acc = Red<OP, float>::f(acc, row[i]);
+      for (int q = 0; q < U; ++q) acc = R::f(acc, R::f(R::f(v[q][0], v[q][1]), R::f(v[q][2], v[q][3])));
     }
+    for (; i < L4; i += ROW_BLOCK) {
+      const f32x4u_t v = ld4u(row + 4 * i);
+      acc = R::f(acc, R::f(R::f(v[0], v[1]), R::f(v[2], v[3])));
+    }
+    if (threadIdx.x < L % 4) acc = R::f(acc, row[4 * L4 + threadIdx.x]);
     float res = epilogue(block_reduce<OP, float, ROW_BLOCK>(acc, lds), mul, dv);
     if (!rebroadcast) {
       if (threadIdx.x == 0) out[r] = res;
     } else {
       float* orow = out + r * L;
-      if (VEC) {
-        float4* o4 = reinterpret_cast<float4*>(orow);
-        for (uint64_t i = threadIdx.x; i < L / 4; i += ROW_BLOCK) o4[i] = make_float4(res, res, res, res);
-      } else {
-        for (uint64_t i = threadIdx.x; i < L; i += ROW_BLOCK) orow[i] = res;
-      }
+      for (uint64_t i = threadIdx.x; i < L4; i += ROW_BLOCK)
+        *reinterpret_cast<f32x4u_t*>(orow + 4 * i) = f32x4u_t{res, res, res, res};
+      if (threadIdx.x < L % 4) orow[4 * L4 + threadIdx.x] = res;
     }
   }
 }
 
-// one wave per row (medium rows); 4 rows per block
-template <int OP>
+// Medium rows (64 <= L < ROWS_BLOCK_MIN_L): LPR lanes a row, each with up to
+// NV 16-byte groups, all loaded before the first is combined (any alignment);
+// the last L % 4 elements go to the row's first lanes.  With a wave a row and
+// 4-byte loads 1500000 x 75 took 224 us, the second step of every row with 11 of
+// 64 lanes; 102 now (84 for 76 columns), 50000 x 999 29 against 41.
+template <int OP, int LPR, int NV>
 __global__ void __launch_bounds__(256)
-k_rows_wave(const float* a, float* out, uint64_t rows, uint64_t L, int rebroadcast, float mul, float dv) {
-  const int lane = threadIdx.x & 63;
-  const uint64_t nw_total = (uint64_t)gridDim.x * 4;
-  for (uint64_t r = (uint64_t)blockIdx.x * 4 + (threadIdx.x >> 6); r < rows; r += nw_total) {
+k_rows_lanes(const float* a, float* out, uint64_t rows, uint32_t L, int rebroadcast, float mul, float dv) {
+  using R = Red<OP, float>;
+  constexpr int RPB = 256 / LPR;
+  const int li = threadIdx.x % LPR;
+  const uint32_t L4 = L / 4;
+  for (uint64_t r = (uint64_t)blockIdx.x * RPB + threadIdx.x / LPR; r < rows; r += (uint64_t)gridDim.x * RPB) {
     const float* row = a + r * L;
-    float acc = Red<OP, float>::init();
-    for (uint64_t i = lane; i < L; i += 64) acc = Red<OP, float>::f(acc, row[i]);
-    float res = epilogue(wave_reduce<OP, float>(acc), mul, dv);
+    f32x4u_t v[NV];
+    float acc = R::init();
+#pragma unroll
+    for (int q = 0; q < NV; ++q)
+      if (li + q * LPR < L4) v[q] = ld4u(row + 4 * (li + q * LPR));
+    const bool tail = 4 * L4 + li < L;
+    const float tv = tail ? row[4 * L4 + li] : 0.f;
+#pragma unroll
+    for (int q = 0; q < NV; ++q)
+      if (li + q * LPR < L4) acc = R::f(acc, R::f(R::f(v[q][0], v[q][1]), R::f(v[q][2], v[q][3])));
+    if (tail) acc = R::f(acc, tv);
+#pragma unroll
+    for (int off = LPR / 2; off >= 1; off >>= 1) acc = R::f(acc, __shfl_xor(acc, off, 64));
+    const float res = epilogue(acc, mul, dv);
     if (!rebroadcast) {
-      if (lane == 0) out[r] = res;
+      if (li == 0) out[r] = res;
     } else {
-      for (uint64_t i = lane; i < L; i += 64) out[r * L + i] = res;
+      float* o = out + r * L;
+      for (uint32_t i = li; i < L4; i += LPR)
+        *reinterpret_cast<f32x4u_t*>(o + 4 * i) = f32x4u_t{res, res, res, res};
+      if (tail) o[4 * L4 + li] = res;
     }
   }
 }
@@ -149,53 +172,172 @@ k_rows_thread(const float* a, float* out, uint64_t rows, uint64_t L, int rebroad
   }
 }
 
+// the same sums, in the same order, for rows of 4 to 63 elements: a block's 256
+// rows come through LDS as one contiguous run (16 bytes a lane; a thread
+// walking its own row in memory touches a cache line a step), at an odd pitch
+// so that the 64 rows of a wave's step are in 64 banks.  1000000 x 16 12 against
+// 36 us, 200000 x 17 6 against 9.
+template <int OP>
+__global__ void __launch_bounds__(256)
+k_rows_short(const float* a, float* out, uint64_t rows, FastDiv L, float mul, float dv) {
+  extern __shared__ float sh[];
+  const uint32_t len = L.d, pitch = len | 1;
+  for (uint64_t r0 = (uint64_t)blockIdx.x * 256; r0 < rows; r0 += (uint64_t)gridDim.x * 256) {
+    const uint32_t nr = (uint32_t)min<uint64_t>(256, rows - r0), n = nr * len;
+    const float* src = a + r0 * len;
+    for (uint32_t i = threadIdx.x * 4; i < n; i += 1024) {
+      f32x4u_t v;
+      if (i + 3 < n) {
+        v = ld4u(src + i);
+      } else {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) v[q] = i + q < n ? src[i + q] : 0.f;
+      }
+      uint32_t r = L.div(i), c = i - r * len;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        if (i + q < n) sh[r * pitch + c] = v[q];
+        if (++c == len) { c = 0; ++r; }
+      }
+    }
+    __syncthreads();
+    if (threadIdx.x < nr) {
+      const float* row = sh + threadIdx.x * pitch;
+      float acc = row[0];
+      for (uint32_t i = 1; i < len; ++i) acc = Red<OP, float>::f(acc, row[i]);
+      out[r0 + threadIdx.x] = epilogue(acc, mul, dv);
+    }
+    __syncthreads();
+  }
+}
+
 // ---- strided axes: post > 1 ------------------------------------------------------
-// a viewed as [prev, K, post]; thread owns VW consecutive columns j of one p
+// k_cols: a viewed as [prev, K, post]; thread owns VW consecutive columns j of one p
 // and reduces k in [k0, k1) sequentially.  Result goes to dst[(c * prev + p) *
 // post + j] where c is the chunk index (blockIdx.y).  U rows are loaded at a
 // time (VW == 4) and still combined in row order, so U never changes the result.
+// With VW = 4 the last group of a row starts at post - 4 (the columns it shares
+// with the group before are written twice, with the same values), at any
+// alignment; VW = 1 is for fewer than 4 columns and where groups of 4 would
+// leave fewer than 64 K threads (2000 x 2047: 13 us by fours).
 template <int OP, int VW, int U>
 __global__ void __launch_bounds__(256)
 k_cols(const float* a, float* dst, uint64_t prev, uint64_t K, uint64_t post, uint64_t kchunk,
        int final_pass, float mul, float dv) {
-  const uint64_t groups = post / VW;
+  const uint64_t groups = (post + VW - 1) / VW;
   const uint64_t total = prev * groups;
   const uint64_t c = blockIdx.y;
   const uint64_t k0 = c * kchunk;
   const uint64_t k1 = (k0 + kchunk < K) ? k0 + kchunk : K;
   const uint64_t stride = (uint64_t)gridDim.x * 256;
   for (uint64_t t = (uint64_t)blockIdx.x * 256 + threadIdx.x; t < total; t += stride) {
-    const uint64_t p = t / groups, j = (t - p * groups) * VW;
+    const uint64_t p = t / groups, j = min((t - p * groups) * VW, post - VW);
     const float* base = a + (p * K) * post + j;
     if (VW == 4) {
       using R = Red<OP, float>;
-      auto comb = [](float4& acc, const float4& v) {
-        acc.x = R::f(acc.x, v.x);
-        acc.y = R::f(acc.y, v.y);
-        acc.z = R::f(acc.z, v.z);
-        acc.w = R::f(acc.w, v.w);
+      auto comb = [](f32x4u_t& acc, const f32x4u_t& v) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) acc[q] = R::f(acc[q], v[q]);
       };
-      float4 acc = ld_stream(reinterpret_cast<const float4*>(base + k0 * post));
+      f32x4u_t acc = ld4u(base + k0 * post);
       uint64_t k = k0 + 1;
       // U rows in flight, still combined in row order
       for (; k + (U - 1) < k1; k += U) {
-        float4 v[U];
+        f32x4u_t v[U];
 #pragma unroll
-        for (int q = 0; q < U; ++q) v[q] = ld_stream(reinterpret_cast<const float4*>(base + (k + q) * post));
+        for (int q = 0; q < U; ++q) v[q] = ld4u(base + (k + q) * post);
 #pragma unroll
         for (int q = 0; q < U; ++q) comb(acc, v[q]);
       }
-      for (; k < k1; ++k) comb(acc, ld_stream(reinterpret_cast<const float4*>(base + k * post)));
-      if (final_pass) {
-        acc.x = epilogue(acc.x, mul, dv); acc.y = epilogue(acc.y, mul, dv);
-        acc.z = epilogue(acc.z, mul, dv); acc.w = epilogue(acc.w, mul, dv);
-      }
-      *reinterpret_cast<float4*>(dst + (c * prev + p) * post + j) = acc;
+      for (; k < k1; ++k) comb(acc, ld4u(base + k * post));
+      if (final_pass)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) acc[q] = epilogue(acc[q], mul, dv);
+      *reinterpret_cast<f32x4u_t*>(dst + (c * prev + p) * post + j) = acc;
     } else {
       float acc = base[k0 * post];
-      for (uint64_t k = k0 + 1; k < k1; ++k) acc = Red<OP, float>::f(acc, base[k * post]);
+      uint64_t k = k0 + 1;
+      for (; k + (U - 1) < k1; k += U) {
+        float v[U];
+#pragma unroll
+        for (int q = 0; q < U; ++q) v[q] = base[(k + q) * post];
+#pragma unroll
+        for (int q = 0; q < U; ++q) acc = Red<OP, float>::f(acc, v[q]);
+      }
+      for (; k < k1; ++k) acc = Red<OP, float>::f(acc, base[k * post]);
       if (final_pass) acc = epilogue(acc, mul, dv);
       dst[(c * prev + p) * post + j] = acc;
+    }
+  }
+}
+
+// Few columns: a block takes whole rows, thread t column group t % G of rows
+// t / G, + R, + 2R ... of its chunk, so that a block reads its chunk as one
+// contiguous run; the R sums of a column are then combined by a tree in LDS.
+// Chunk partials dst[p][c][post] are reduced by the same kernel, in as many
+// more passes as leave each thread about 16 rows.  k_cols gives every chunk a block of which only G threads work (1000000
+// x 16: 4 of 256) and combines up to 1024 chunks one after the other.  Against
+// it: 1000000 x 16 18 against 161 us, 3000000 x 3 11 against 371, 1500000 x 75
+// 78 against 678, 50000 x 999 44 against 120 (element loads), 50000 x 1000 43
+// against 60 (87 with one last pass over all 1024 chunks).
+template <int OP, int VW, int U>
+__global__ void __launch_bounds__(256)
+k_cols_narrow(const float* a, float* dst, uint64_t K, uint32_t post, uint64_t kchunk, uint32_t G, uint32_t R,
+              int final_pass, float mul, float dv) {
+  using Rd = Red<OP, float>;
+  __shared__ float lds[256 * VW];
+  const uint64_t c = blockIdx.x, p = blockIdx.y;
+  const uint64_t k0 = c * kchunk, k1 = min(k0 + kchunk, K);
+  const uint32_t rr = threadIdx.x / G, g = threadIdx.x - rr * G;
+  const uint32_t j = min(g * VW, post - VW);
+  uint32_t n = (uint32_t)min<uint64_t>(R, k1 - k0);  // rows of threads that have a row
+  float acc[VW];
+  auto load = [&](uint64_t k, float (&v)[VW]) {
+    const float* q = a + (p * K + k) * post + j;
+    if constexpr (VW == 4) {
+      const f32x4u_t t = ld4u(q);
+      v[0] = t[0]; v[1] = t[1]; v[2] = t[2]; v[3] = t[3];
+    } else {
+      v[0] = *q;
+    }
+  };
+  if (rr < n) {
+    load(k0 + rr, acc);
+    uint64_t k = k0 + rr + R;
+    for (; k + (uint64_t)(U - 1) * R < k1; k += (uint64_t)U * R) {
+      float v[U][VW];
+#pragma unroll
+      for (int q = 0; q < U; ++q) load(k + (uint64_t)q * R, v[q]);
+#pragma unroll
+      for (int q = 0; q < U; ++q)
+#pragma unroll
+        for (int w = 0; w < VW; ++w) acc[w] = Rd::f(acc[w], v[q][w]);
+    }
+    for (; k < k1; k += R) {
+      float v[VW];
+      load(k, v);
+#pragma unroll
+      for (int w = 0; w < VW; ++w) acc[w] = Rd::f(acc[w], v[w]);
+    }
+#pragma unroll
+    for (int w = 0; w < VW; ++w) lds[w * 256 + threadIdx.x] = acc[w];
+  }
+  __syncthreads();
+  while (n > 1) {
+    const uint32_t h = (n + 1) / 2;
+    if (rr + h < n)
+#pragma unroll
+      for (int w = 0; w < VW; ++w)
+        lds[w * 256 + threadIdx.x] = Rd::f(lds[w * 256 + threadIdx.x], lds[w * 256 + threadIdx.x + h * G]);
+    __syncthreads();
+    n = h;
+  }
+  if (rr == 0) {
+    float* d = dst + (p * gridDim.x + c) * post + j;
+#pragma unroll
+    for (int w = 0; w < VW; ++w) {
+      const float r = lds[w * 256 + threadIdx.x];
+      d[w] = final_pass ? epilogue(r, mul, dv) : r;
     }
   }
 }
@@ -400,10 +542,10 @@ static void reduce_all_noalloc(vkh_gpu* g, const float* a, uint64_t n, float* ou
 // of 256 rows reach 6.4 TB/s, 64 chunks 6.1).  The chunk count fixes the
 // summation order of sums and products, so it is part of the shape's
 // configuration.
-static uint64_t cols_chunk(vkh_gpu* g, const RedCfg& cfg, uint64_t prev, uint64_t K, uint64_t post, bool vec,
+static uint64_t cols_chunk(vkh_gpu* g, const RedCfg& cfg, uint64_t prev, uint64_t K, uint64_t post,
                            uint64_t& nchunk_out) {
   const unsigned cus = g->num_cus > 0 ? g->num_cus : 256;
-  const uint64_t threads = prev * (post / (vec ? 4 : 1));
+  const uint64_t threads = prev * (post >= 4 ? ceil_div(post, 4) : post);
   const uint64_t want = (uint64_t)cus * (uint64_t)cfg.par;
   uint64_t nchunk = 1;
   if (threads < want && K >= 64) {
@@ -416,6 +558,45 @@ static uint64_t cols_chunk(vkh_gpu* g, const RedCfg& cfg, uint64_t prev, uint64_
   return kchunk;
 }
 
+// Shapes of k_cols_narrow: fewer than 1024 columns (a block holds a row) and
+// too few columns in all to fill the chip with one thread a column group.  The
+// column sums that the fused last-layer backward reproduces in order (one
+// matrix, rows a multiple of 128, columns of 32: dense1_chunks in gemm.hip)
+// keep k_cols.
+static bool cols_narrow(vkh_gpu* g, uint64_t prev, uint64_t K, uint64_t post) {
+  if (post >= 1024 || K < 64 || prev > 65535 || (prev == 1 && K % 128 == 0 && post % 32 == 0)) return false;
+  const uint64_t cus = g->num_cus > 0 ? g->num_cus : 256;
+  return prev * ceil_div(post, 4) < cus * 256;
+}
+
+template <int OP>
+static void reduce_cols_narrow(vkh_gpu* g, const float* a, float* out, uint64_t prev, uint64_t K, uint64_t post,
+                               float mul, float dv) {
+  const uint64_t cus = g->num_cus > 0 ? g->num_cus : 256;
+  const uint32_t G = (uint32_t)(post >= 4 ? ceil_div(post, 4) : post), R = 256 / G;
+  // about four blocks a CU, at least 16 rows a thread
+  uint64_t nchunk = std::max<uint64_t>(1, std::min(ceil_div(4 * cus, prev), K / (16 * (uint64_t)R)));
+  const uint64_t kchunk = ceil_div(K, nchunk);
+  nchunk = ceil_div(K, kchunk);
+  auto launch = [&](const float* src, float* dst, uint64_t k, uint64_t kc, uint64_t nc, int fin) {
+    const dim3 grid((unsigned)nc, (unsigned)prev);
+    if (post >= 4)
+      hipLaunchKernelGGL((k_cols_narrow<OP, 4, 8>), grid, dim3(256), 0, g->stream, src, dst, k, (uint32_t)post, kc, G, R,
+                         fin, mul, dv);
+    else
+      hipLaunchKernelGGL((k_cols_narrow<OP, 1, 8>), grid, dim3(256), 0, g->stream, src, dst, k, (uint32_t)post, kc, G, R,
+                         fin, mul, dv);
+    check_launch("reduce cols (narrow)");
+  };
+  if (nchunk == 1) {
+    launch(a, out, K, kchunk, 1, 1);
+    return;
+  }
+  Workspace ws(g, sizeof(float) * prev * nchunk * post);
+  launch(a, (float*)ws.get(), K, kchunk, nchunk, 0);
+  reduce_cols_narrow<OP>(g, (const float*)ws.get(), out, prev, nchunk, post, mul, dv);
+}
+
 template <int OP>
 static void reduce_axis(vkh_gpu* g, const float* a, float* out, uint64_t prev, uint64_t K,
                         uint64_t post, int rebroadcast, float mul, float dv, int index = -1) {
@@ -423,18 +604,28 @@ static void reduce_axis(vkh_gpu* g, const float* a, float* out, uint64_t prev, u
   const RedCfg cfg = red_cfg(g, red_family(1, K, post), prev, K, post, index);
   if (post == 1) {
     const uint64_t rows = prev, L = K;
-    const bool vec = (L % 4 == 0) && (((uintptr_t)a & 15u) == 0) && (((uintptr_t)out & 15u) == 0);
     if (L >= ROWS_BLOCK_MIN_L) {
       unsigned grid = (unsigned)std::min<uint64_t>(rows, (uint64_t)cus * cfg.par);
-      if (vec && cfg.unroll == 8)
-        hipLaunchKernelGGL((k_rows_block<OP, true, 8>), dim3(grid), dim3(ROW_BLOCK), 0, g->stream, a, out, rows, L, rebroadcast, mul, dv);
-      else if (vec)
-        hipLaunchKernelGGL((k_rows_block<OP, true, 4>), dim3(grid), dim3(ROW_BLOCK), 0, g->stream, a, out, rows, L, rebroadcast, mul, dv);
+      if (cfg.unroll == 8)
+        hipLaunchKernelGGL((k_rows_block<OP, 8>), dim3(grid), dim3(ROW_BLOCK), 0, g->stream, a, out, rows, L, rebroadcast, mul, dv);
       else
-        hipLaunchKernelGGL((k_rows_block<OP, false, 4>), dim3(grid), dim3(ROW_BLOCK), 0, g->stream, a, out, rows, L, rebroadcast, mul, dv);
+        hipLaunchKernelGGL((k_rows_block<OP, 4>), dim3(grid), dim3(ROW_BLOCK), 0, g->stream, a, out, rows, L, rebroadcast, mul, dv);
     } else if (L >= 64) {
-      unsigned grid = (unsigned)std::min<uint64_t>(ceil_div(rows, 4), (uint64_t)cus * 16);
-      hipLaunchKernelGGL(k_rows_wave<OP>, dim3(grid), dim3(256), 0, g->stream, a, out, rows, L, rebroadcast, mul, dv);
+      // lanes a row: up to 4 groups a lane, 8 of a whole wave
+      auto launch = [&](auto kernel, int lpr) {
+        const unsigned grid = (unsigned)std::min<uint64_t>(ceil_div(rows, 256 / lpr), (uint64_t)cus * 64);
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), 0, g->stream, a, out, rows, (uint32_t)L, rebroadcast, mul, dv);
+      };
+      const uint64_t L4 = L / 4;
+      if (L4 <= 32) launch(k_rows_lanes<OP, 8, 4>, 8);
+      else if (L4 <= 64) launch(k_rows_lanes<OP, 16, 4>, 16);
+      else if (L4 <= 128) launch(k_rows_lanes<OP, 32, 4>, 32);
+      else if (L4 <= 256) launch(k_rows_lanes<OP, 64, 4>, 64);
+      else launch(k_rows_lanes<OP, 64, 8>, 64);
+    } else if (L >= 4 && !rebroadcast) {
+      const size_t sh = sizeof(float) * 256 * (L | 1);
+      unsigned grid = (unsigned)std::min<uint64_t>(ceil_div(rows, 256), (uint64_t)cus * 16);
+      hipLaunchKernelGGL(k_rows_short<OP>, dim3(grid), dim3(256), sh, g->stream, a, out, rows, FastDiv((uint32_t)L), mul, dv);
     } else {
       unsigned grid = (unsigned)std::min<uint64_t>(ceil_div(rows, 256), (uint64_t)cus * 16);
       hipLaunchKernelGGL(k_rows_thread<OP>, dim3(grid), dim3(256), 0, g->stream, a, out, rows, L, rebroadcast, mul, dv);
@@ -442,25 +633,35 @@ static void reduce_axis(vkh_gpu* g, const float* a, float* out, uint64_t prev, u
     check_launch("reduce rows");
     return;
   }
-  const bool vec = (post % 4 == 0) && (((uintptr_t)a & 15u) == 0) && (((uintptr_t)out & 15u) == 0);
-  const int VW = vec ? 4 : 1;
-  const uint64_t threads = prev * (post / VW);
+  if (cols_narrow(g, prev, K, post)) {
+    if (!rebroadcast) {
+      reduce_cols_narrow<OP>(g, a, out, prev, K, post, mul, dv);
+      return;
+    }
+    Workspace red(g, sizeof(float) * prev * post);
+    reduce_cols_narrow<OP>(g, a, (float*)red.get(), prev, K, post, mul, dv);
+    hipLaunchKernelGGL(k_rebroadcast_cols, dim3(stream_grid(g, prev * K * post, 256, 8)), dim3(256), 0, g->stream,
+                       (const float*)red.get(), out, prev, K, post);
+    check_launch("reduce rebroadcast");
+    return;
+  }
   uint64_t nchunk = 0;
-  const uint64_t kchunk = cols_chunk(g, cfg, prev, K, post, vec, nchunk);
+  const uint64_t kchunk = cols_chunk(g, cfg, prev, K, post, nchunk);
   const uint64_t m = prev * post;
+  const bool quads = post >= 4 && prev * ceil_div(post, 4) * nchunk >= (uint64_t)cus * 256;
+  const uint64_t threads = prev * (quads ? ceil_div(post, 4) : post);
   Workspace ws(g, (nchunk > 1 || rebroadcast) ? sizeof(float) * nchunk * m : 1);
   float* dst = (nchunk > 1 || rebroadcast) ? (float*)ws.get() : out;
-  if (vec && !(nchunk > 1 || rebroadcast)) { /* out alignment already checked */ }
   unsigned gx = (unsigned)std::min<uint64_t>(ceil_div(threads, 256), (uint64_t)cus * 16);
   if (gx < 1) gx = 1;
   dim3 grid(gx, (unsigned)nchunk);
   const int final_pass = (nchunk == 1) ? 1 : 0;
-  if (VW == 4 && cfg.unroll == 8)
+  if (quads && cfg.unroll == 8)
     hipLaunchKernelGGL((k_cols<OP, 4, 8>), grid, dim3(256), 0, g->stream, a, dst, prev, K, post, kchunk, final_pass, mul, dv);
-  else if (VW == 4)
+  else if (quads)
     hipLaunchKernelGGL((k_cols<OP, 4, 4>), grid, dim3(256), 0, g->stream, a, dst, prev, K, post, kchunk, final_pass, mul, dv);
   else
-    hipLaunchKernelGGL((k_cols<OP, 1, 4>), grid, dim3(256), 0, g->stream, a, dst, prev, K, post, kchunk, final_pass, mul, dv);
+    hipLaunchKernelGGL((k_cols<OP, 1, 8>), grid, dim3(256), 0, g->stream, a, dst, prev, K, post, kchunk, final_pass, mul, dv);
   check_launch("reduce cols");
   float* red = dst;
   if (nchunk > 1) {
@@ -519,12 +720,13 @@ int vkh_reduce_all(vkh_gpu* g, int op, const float* a, uint64_t n, float* out, i
 
 namespace vkh {
 // chunk length of the column sums of a [rows, cols] operand (vkh_bias_grad's
-// reduction), for kernels that must sum in the same order; vec: the operand
-// and output allow 16-byte accesses
-uint64_t bias_grad_chunk(vkh_gpu* g, uint64_t rows, uint64_t cols, bool vec) {
+// reduction), for kernels that must sum in the same order; 0 where that order
+// is not one of row chunks
+uint64_t bias_grad_chunk(vkh_gpu* g, uint64_t rows, uint64_t cols) {
+  if (cols == 1 || cols_narrow(g, 1, rows, cols)) return 0;
   const RedCfg cfg = red_cfg(g, red_family(1, rows, cols), 1, rows, cols, -1);
   uint64_t nchunk = 0;
-  return cols_chunk(g, cfg, 1, rows, cols, vec, nchunk);
+  return cols_chunk(g, cfg, 1, rows, cols, nchunk);
 }
 
 // Chunk partials part[c][m] summed per output in chunk order: FROM_ZERO 0
