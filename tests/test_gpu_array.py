@@ -724,3 +724,26 @@ def test_reduce_axis_edges(gpu, shape, axis):
     assert_bits(A(gpu, low).maximum(axis=axis), low.max(axis=axis))
     low[:] = -np.inf
     assert_bits(A(gpu, low).maximum(axis=axis), low.max(axis=axis))
+
+
+@pytest.mark.parametrize("shape,axis", [((60, 784), 0), ((60, 785), 0), ((50, 3), 0), ((50, 4), 0), ((7, 9, 5), 1),
+                                        ((5, 30, 2), 1), ((6, 11), 1), ((3, 4, 17), 2), ((1, 1), 0), ((40,), 0)])
+@pytest.mark.parametrize("n", [1, 3, 257])
+def test_gather_axis_run_lengths(gpu, shape, axis, n):
+    """Runs of 1 to 785 elements (groups of 4, the last one moved back to the
+    run's end; 1 to 3 elements one by one), out-of-range indices clamped; bytes
+    as they are, NaN payloads and -0 included."""
+    rng = np.random.default_rng(n + shape[0])
+    a = rng.integers(0, 2 ** 32, shape, dtype=np.uint32).view(np.float32)
+    idx = rng.integers(0, shape[axis] + 2, n).astype(np.uint32)
+    got = np.asarray(A(gpu, a).gather(vk.U32Array(gpu, data=idx), axis=axis))
+    want = np.moveaxis(np.take(a, np.minimum(idx, shape[axis] - 1), axis=axis), axis, 0)
+    np.testing.assert_array_equal(got.view(np.uint32), np.ascontiguousarray(want).view(np.uint32).reshape(got.shape))
+
+
+@pytest.mark.parametrize("classes", [1, 2, 3, 4, 5, 10, 1001])
+@pytest.mark.parametrize("n", [1, 2, 5, 1024])
+def test_onehot_sizes(gpu, classes, n):
+    lab = np.random.default_rng(n).integers(0, classes + 2, n)
+    got = np.asarray(vk.U32Array(gpu, data=lab).to_onehot(classes))
+    np.testing.assert_array_equal(got, np.identity(classes, dtype=np.float32)[np.minimum(lab, classes - 1)])
