@@ -13,6 +13,7 @@ There is no fallback: if the library is missing the first use raises
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 from ctypes import (POINTER, c_char_p, c_double, c_float, c_int, c_size_t,
                     c_uint16, c_uint32, c_uint64, c_void_p)
@@ -225,13 +226,27 @@ def check(status: int, what: str = "") -> None:
     raise RuntimeError(msg)
 
 
+_functions = {}  # entry points called so far, by name
+
+
 def call(name: str, *args) -> None:
     """Call an int-status function and raise on failure."""
-    check(getattr(load(), name)(*args), name)
+    fn = _functions.get(name)
+    if fn is None:
+        fn = _functions[name] = getattr(load(), name)
+    status = fn(*args)
+    if status:
+        check(status, name)
 
 
 def shape_array(shape) -> ctypes.Array:
-    """uint64 array of a shape tuple (for the broadcast entry points)."""
+    """uint64 array of a shape tuple (for the broadcast entry points, which only
+    read it: equal shapes share one array)."""
+    return _shape_array(tuple(shape))
+
+
+@functools.lru_cache(maxsize=1024)
+def _shape_array(shape) -> ctypes.Array:
     arr = (c_uint64 * max(len(shape), 1))()
     for i, v in enumerate(shape):
         arr[i] = int(v)

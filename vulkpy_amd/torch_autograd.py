@@ -48,14 +48,24 @@ __all__ = ["dense", "relu", "sigmoid", "softmax", "softmax_cross_entropy", "mse"
 _contexts: Dict[Tuple[int, int], int] = {}
 
 
+def _raw_stream(dev: int) -> int:
+    """Handle of torch's current stream on a device."""
+    return int(torch.cuda.current_stream(dev).cuda_stream)
+
+
+# (the same handle without building the Stream object, where torch has it)
+if hasattr(torch._C, "_cuda_getCurrentRawStream"):
+    _raw_stream = torch._C._cuda_getCurrentRawStream
+
+
 def _ctx(t: torch.Tensor) -> int:
     """Library context bound to torch's current stream on t's device."""
     if not t.is_cuda:
         raise ValueError("vulkpy_amd.torch_autograd needs tensors on a ROCm GPU "
                          f"(got device {t.device})")
     dev = t.device.index if t.device.index is not None else torch.cuda.current_device()
-    stream = torch.cuda.current_stream(dev).cuda_stream
-    key = (dev, int(stream))
+    stream = _raw_stream(dev)
+    key = (dev, stream)
     h = _contexts.get(key)
     if h is None:
         out = ctypes.c_void_p()
@@ -72,7 +82,7 @@ def _f32(t: torch.Tensor, name: str) -> torch.Tensor:
 
 
 def _p(t: Optional[torch.Tensor]):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
 class _Dense(torch.autograd.Function):

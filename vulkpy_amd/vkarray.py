@@ -26,9 +26,10 @@ from __future__ import annotations
 import ctypes
 import functools
 import logging
+import math
 import os
 import weakref
-from typing import Iterable, List, Optional, Tuple, Union
+from typing import Iterable, List, Optional, Sequence, Tuple, Union
 
 import numpy as np
 
@@ -61,10 +62,6 @@ class _Context:
         self.ticket = 0
         self.done_ticket = 0
         self.latest: Optional[_Event] = None
-
-    def issue(self) -> int:
-        self.ticket += 1
-        return self.ticket
 
     def covering(self, ticket: int) -> "_Event":
         """A recorded event that completes after job `ticket`."""
@@ -168,7 +165,7 @@ class Job:
 
     def __init__(self, ctx: _Context):
         self._ctx = ctx
-        self._ticket = ctx.issue()
+        ctx.ticket = self._ticket = ctx.ticket + 1
 
     def wait(self, timeout_ns: Optional[int] = None):
         """
@@ -241,6 +238,7 @@ class GPU:
         """
         self._idx = idx
         self._ctx = _context(idx, priority)
+        self._handle = self._ctx.handle
         self.gpu = self._ctx
         self.canSubgroupArithmetic = True
         logger.info(f"GPU {idx}: Subgroup Arithmetic: {self.canSubgroupArithmetic}")
@@ -252,10 +250,6 @@ class GPU:
 
     def __hash__(self):
         return hash(self._idx)
-
-    @property
-    def _handle(self):
-        return self._ctx.handle
 
     def _job(self) -> Job:
         return Job(self._ctx)
@@ -291,6 +285,10 @@ class GPU:
         call("vkh_empty_cache", self._handle)
 
 
+_c_void_p, _byref = ctypes.c_void_p, ctypes.byref
+_DTYPES = {t: np.dtype(t) for t in (np.float32, np.uint32, np.uint16, np.float64)}
+
+
 class _DeviceBuffer:
     """Device allocation of ``n`` elements of ``dtype`` (Buffer<T>, _vkarray.cc:38-130)."""
 
@@ -298,11 +296,11 @@ class _DeviceBuffer:
 
     def __init__(self, gpu: GPU, n: int, dtype):
         self._gpu = gpu
-        self.n = int(n)
-        self.dtype = np.dtype(dtype)
-        self.nbytes = self.n * self.dtype.itemsize
-        out = ctypes.c_void_p()
-        call("vkh_alloc", gpu._handle, max(self.nbytes, 1), ctypes.byref(out))
+        self.n = n = int(n)
+        self.dtype = dt = _DTYPES.get(dtype) or np.dtype(dtype)
+        self.nbytes = nbytes = n * dt.itemsize
+        out = _c_void_p()
+        call("vkh_alloc", gpu._handle, nbytes if nbytes > 0 else 1, _byref(out))
         self.ptr = out.value
 
     def size(self) -> int:
@@ -311,13 +309,19 @@ class _DeviceBuffer:
     def __del__(self):
         try:
             if self.ptr:
-                _lib.lib.vkh_free(self._gpu._handle, self.ptr)
+                _lib.load().vkh_free(self._gpu._handle, self.ptr)
                 self.ptr = None
         except Exception:
             pass
 
 
 def _parse_shape(shape) -> Tuple[int, ...]:
+    if type(shape) is tuple:
+        for s in shape:
+            if type(s) is not int:
+                break
+        else:
+            return shape
     return tuple(int(s) for s in np.asarray(shape, dtype=int).reshape(-1))
 
 
@@ -386,18 +390,18 @@ class _GPUArray(Resource):
 
     _dtype = np.float32
 
+    # Pipeline job to write this Array.
+    job: Optional[Job] = None
+
+    # Hold temporary resources until pipeline job finish.
+    _keep: Sequence[Resource] = ()
+
+    _host: Optional[np.ndarray] = None
+    _host_valid = False
+    _upload_pending = False
+
     def __init__(self, gpu: GPU):
         self._gpu: GPU = gpu
-
-        # Pipeline job to write this Array.
-        self.job: Optional[Job] = None
-
-        # Hold temporary resources until pipeline job finish.
-        self._keep: List[Resource] = []
-
-        self._host: Optional[np.ndarray] = None
-        self._host_valid = False
-        self._upload_pending = False
 
     # ---- construction helpers -------------------------------------------------
     def _init_data(self, data, dtype):
@@ -429,7 +433,7 @@ class _GPUArray(Resource):
 
     def _init_shape(self, shape, dtype):
         self.shape = _parse_shape(shape)
-        self.buffer = _DeviceBuffer(self._gpu, int(np.prod(self.shape, dtype=np.int64)), dtype)
+        self.buffer = _DeviceBuffer(self._gpu, math.prod(self.shape), dtype)
 
     @property
     def _ptr(self) -> int:
@@ -467,7 +471,7 @@ class _GPUArray(Resource):
         # stream) is what __del__ must wait for before the mirror's pinned
         # block can go back to the pool.
         self.job = self._gpu._job()
-        self._keep = list(keep)
+        self._keep = keep if type(keep) is list else list(keep)
         self._host_valid = False
 
     def flush(self):
@@ -655,6 +659,8 @@ class Shape(U32Array):
 
 def _normalize_axes(axis, ndim: int) -> List[int]:
     """Flattened, unique, non-negative axes (NumPy rule; vkarray.py:1196)."""
+    if type(axis) is int and -ndim <= axis < ndim:
+        return [axis + ndim if axis < 0 else axis]
     axes = np.unique(np.asarray(axis, dtype=int).reshape(-1))
     out = []
     for a in axes:
@@ -677,7 +683,13 @@ def _axis_runs(axes: List[int]) -> List[Tuple[int, int]]:
 
 
 def _prod(s) -> int:
-    return int(np.prod(s, dtype=np.int64)) if len(s) else 1
+    return math.prod(s)
+
+
+@functools.lru_cache(maxsize=1024)
+def _broadcast(*shapes) -> Tuple[int, ...]:
+    """NumPy's broadcast of shape tuples (a ValueError is raised on every call)"""
+    return tuple(int(s) for s in np.broadcast_shapes(*shapes))
 
 
 class Array(_GPUArray):
@@ -719,7 +731,12 @@ class Array(_GPUArray):
         self._set_job()
 
     def _new(self, shape) -> "Array":
-        return Array(self._gpu, shape=shape)
+        # Array(self._gpu, shape=shape) without the constructor's chain
+        ret = Array.__new__(Array)
+        ret._gpu = gpu = self._gpu
+        ret.shape = shape = _parse_shape(shape)
+        ret.buffer = _DeviceBuffer(gpu, math.prod(shape), np.float32)
+        return ret
 
     def _check_shape(self, other):
         if tuple(self.shape) != tuple(other.shape):
@@ -739,7 +756,7 @@ class Array(_GPUArray):
             call("vkh_binary", h, BINOP[op], self._ptr, other._ptr, ret._ptr, self.size)
             ret._set_job([self, other])
             return ret
-        shape = tuple(np.broadcast_shapes(tuple(self.shape), tuple(other.shape)))
+        shape = _broadcast(tuple(self.shape), tuple(other.shape))
         ret = self._new(shape)
         nd = len(shape)
         sa = (1,) * (nd - len(self.shape)) + tuple(self.shape)
@@ -758,7 +775,7 @@ class Array(_GPUArray):
             call("vkh_binary", h, BINOP[op], self._ptr, other._ptr, self._ptr, self.size)
             self._set_job([other])
         else:
-            shape = tuple(np.broadcast_shapes(tuple(self.shape), tuple(other.shape)))
+            shape = _broadcast(tuple(self.shape), tuple(other.shape))
             if shape != tuple(self.shape):
                 raise ValueError(f"Incompatible shape. {shape} vs {self.shape}")
             # NumPy rule (len(shape)) instead of the reference's shape[0]
@@ -1029,7 +1046,7 @@ class Array(_GPUArray):
             shapes.append(tuple(min.shape))
         if hi_arr:
             shapes.append(tuple(max.shape))
-        shape = tuple(np.broadcast_shapes(*shapes)) if len(shapes) > 1 else tuple(self.shape)
+        shape = _broadcast(*shapes) if len(shapes) > 1 else tuple(self.shape)
         if inplace and shape != tuple(self.shape):
             raise ValueError(f"Incompatible shape")
         lo_s = 0.0 if lo_arr else float(min)
@@ -1171,7 +1188,7 @@ class Array(_GPUArray):
             If ``shape`` is not compatible (NumPy rule).
         """
         shape = _parse_shape(shape)
-        if tuple(np.broadcast_shapes(tuple(self.shape), shape)) != shape:
+        if _broadcast(tuple(self.shape), shape) != shape:
             raise ValueError(f"Cannot broadcast to {shape}")
         ret = self._new(shape)
         nd = len(shape)
