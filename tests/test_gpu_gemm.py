@@ -593,6 +593,59 @@ def test_tile_edges(gpu, mode, M, N, K):
         _lib.call("vkh_gemm_set_config", h, md, 0, 1, M, N, K, -1)
 
 
+# The BF16 copies of C and C^T (written through LDS a block row / 64 rows at a
+# time) at edges of the tiles, of their 16-byte runs and of their leading
+# dimensions, with the values the conversion handles apart: NaNs with a
+# payload, denormals, -0.  C is exact (whole numbers, or the bias alone where A's row is
+# zero); the copies are the library's rounding of it, bit for bit.
+@pytest.mark.parametrize("mode", ["bf16", "bf16x3"])
+@pytest.mark.parametrize("M,N,K", [(17, 72, 64), (64, 64, 64), (72, 129, 64), (128, 192, 100), (255, 200, 64),
+                                   (264, 257, 128), (520, 264, 64)])
+def test_copies_at_tile_edges(gpu, mode, M, N, K):
+    rng = np.random.default_rng(5 * M + N + K)
+    h, md = gpu._handle, _lib.GEMM_MODE[mode]
+    A = rng.integers(-3, 4, (M, K)).astype(np.float32)
+    A[::5] = 0
+    B = rng.integers(-3, 4, (N, K)).astype(np.float32)
+    bias = rng.integers(-9, 10, N).astype(np.float32)
+    odd = np.array([0x7fc12345, 0xffd00001, 0x00000001, 0x80000001, 0x00008000, 0x00012345, 0x80000000, 0x7f7fffff],
+                   dtype=np.uint32).view(np.float32)
+    bias[3:3 + 5 * len(odd):5] = odd
+    aux = np.maximum(rng.integers(-2, 3, (M, N)), 0).astype(np.float32)
+    P = A @ B.T
+    gA, gB, gb, gX = (vk.Array(gpu, data=v) for v in (A, B, bias, aux))
+    x16 = vk.U32Array(gpu, shape=((M * N + 1) // 2,))
+    _lib.call("vkh_to_bf16", h, gX._ptr, x16._ptr, M * N)
+    x16._set_job([gX])
+    one = A @ B.T + bias
+    with np.errstate(invalid="ignore"):
+        want = {"none": one, "relu": np.maximum(one, 0), "aux": P * (aux > 0)}
+    try:
+        for i in range(len(vk.gemm_configs(mode))):
+            _lib.call("vkh_gemm_set_config", h, md, 0, 1, M, N, K, i)
+            for kind in ("none", "relu", "aux", "aux16"):
+                plain = kind.startswith("aux")
+                for ldt in (M, M + 5, -(-M // 8) * 8):
+                    C = vk.Array(gpu, shape=(M, N))
+                    cbf = vk.U32Array(gpu, data=np.full((M * N + 1) // 2, 0x5a5a5a5a, dtype=np.uint32))
+                    cbt = vk.U32Array(gpu, data=np.full((N * ldt + 1) // 2, 0x5a5a5a5a, dtype=np.uint32))
+                    _lib.call("vkh_gemm_bf16io_ext", h, md, 0, 1, M, N, K, 1.0, gA._ptr, K, gB._ptr, K, 0.0, C._ptr, N,
+                              None if plain else gb._ptr, _lib.ACT["relu" if kind == "relu" else "none"], cbf._ptr,
+                              gX._ptr if kind == "aux" else None, x16._ptr if kind == "aux16" else None, N,
+                              _lib.ACT["relu"] if plain else 0, None, None, cbt._ptr, ldt, None, 1)
+                    for o in (C, cbf, cbt):
+                        o._set_job([gA, gB, gb, gX, x16])
+                    got = np.asarray(C)
+                    np.testing.assert_array_equal(got, want["aux" if plain else kind])
+                    bits = bf16_bits(got)
+                    np.testing.assert_array_equal(np.asarray(cbf).view(np.uint16)[:M * N].reshape(M, N), bits)
+                    t = np.asarray(cbt).view(np.uint16)[:N * ldt].reshape(N, ldt)
+                    np.testing.assert_array_equal(t[:, :M], bits.T)
+                    assert np.all(t[:, M:] == 0x5a5a)
+    finally:
+        _lib.call("vkh_gemm_set_config", h, md, 0, 1, M, N, K, -1)
+
+
 # Large FP32 products run from three BF16 parts (by sizes only; 4001 x 2047 x
 # 1030 is such a product, with ragged edges in every dimension), unless an
 # operand holds values out of their range; then the FP32 kernel runs.

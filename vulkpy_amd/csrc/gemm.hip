@@ -58,8 +58,8 @@ struct GemmArgs {
   uint16_t* Cbft;  // C^T as BF16: Cbft[n * ldt + m] (optional)
   uint64_t ldt;
   // column sums of the final C over each chunk of CS_ROWS rows, in row order
-  // from the chunk's first row: cs[(m / CS_ROWS) * N + n] (optional; staged
-  // epilogues with 128-row wave slabs only)
+  // from the chunk's first row: cs[(m / CS_ROWS) * N + n] (optional; waves
+  // with 128-row slabs only)
   float* cs;
   int no_c;  // 1: the FP32 C is not stored (only Cbf / Cbft / cs)
   // the aux activation's output as BF16 instead of aux (ReLU' only: the BF16
@@ -350,12 +350,9 @@ __device__ __forceinline__ f32x4_t aux4(const GemmArgs& e, uint64_t m, uint64_t 
 // transposed BF16 copy is written here, one element at a time, unless write_t
 // is false (the staged epilogue writes it in whole runs).
 // D: x holds the derivative factors themselves (ReLU' decoded from codes)
-// bf (full groups): receives the four values as BF16, two a word, when it
-// converts them for e.Cbf or when `want_bf` (the caller writes them again)
 template <bool SIG = true, bool D = false>
 __device__ __forceinline__ float4 finish4(const GemmArgs& e, uint64_t m, uint64_t n, float4 acc, bool full,
-                                          int cnt, f32x4_t c, f32x4_t b, f32x4_t x, bool write_t,
-                                          uint2* bf = nullptr, bool want_bf = false) {
+                                          int cnt, f32x4_t c, f32x4_t b, f32x4_t x, bool write_t) {
   float* cp = e.C + m * e.ldc + n;
   float v[4] = {acc.x, acc.y, acc.z, acc.w};
 #pragma unroll
@@ -369,12 +366,11 @@ __device__ __forceinline__ float4 finish4(const GemmArgs& e, uint64_t m, uint64_
   }
   if (full) {
     if (!e.no_c) *reinterpret_cast<float4*>(cp) = make_float4(v[0], v[1], v[2], v[3]);
-    if (e.Cbf || want_bf) {
+    if (e.Cbf) {
       uint2 h;
       h.x = f2bf(v[0]) | ((uint32_t)f2bf(v[1]) << 16);
       h.y = f2bf(v[2]) | ((uint32_t)f2bf(v[3]) << 16);
-      if (e.Cbf) *reinterpret_cast<uint2*>(e.Cbf + m * e.ldc + n) = h;
-      if (bf) *bf = h;
+      *reinterpret_cast<uint2*>(e.Cbf + m * e.ldc + n) = h;
     }
   } else {
 #pragma unroll
@@ -425,22 +421,13 @@ __device__ __forceinline__ void store_part4(float* part, uint64_t N, uint64_t m,
 // l32 (l32 = lane % 32, lhi = lane / 32).  Each wave writes rows i*32 .. i*32+31 of its sub-tile to its own
 // 32 x (WN+4) float staging slice of `smem`, then reads them back as 4-float
 // row segments (WN/4 lanes per row), so C is accessed in whole row segments.
-// With `part` the raw sums go to that k chunk's partial matrix instead.  The
-// transposed BF16 copy (e.Cbft): with TST (the caller's LDS holds a second
-// area `tbase` of WN x TT_PITCH BF16 a wave after the staging slices) the
-// row pass also writes each final value as BF16 into that wave's transposed
-// tile, and after every second pass each group of eight lanes writes one
-// column's 64 rows as one 128-byte run of C^T (16 bytes a lane).  Without
-// it the row pass puts the final values back into the slice and each group
-// of four lanes converts one column of 32 rows into a 64-byte run.  The
-// caller's operand tiles in `smem` must be dead (a barrier before the call).
-constexpr int TT_PITCH = 72;  // transposed tile row: 64 rows of C + 8, 16-byte aligned
-template <int WAVES, int WN>
-constexpr int tt_bytes() { return WAVES * WN * TT_PITCH * 2; }
+// With `part` the raw sums go to that k chunk's partial matrix instead.  For
+// the transposed BF16 copy (e.Cbft) the row pass puts the final values back
+// into the slice and each group of four lanes converts one column of 32 rows
+// into a 64-byte run.  The caller's operand tiles in `smem` must be dead (a
+// barrier before the call).
 
-// rows i*32 .. i*32+31 of a wave's accumulators into its staging slice: 32 x 32
-// blocks (acc[i][j][r] as above), or 16 x 16 blocks, where acc[i][j][r] is
-// row i*16 + (lane/16)*4 + r, column j*16 + lane%16
+// rows i*32 .. i*32+31 of a wave's accumulators into its staging slice
 template <int I, int SROW, int TM, int TN>
 __device__ __forceinline__ void stage_pass(float* st, const f32x16_t (&acc)[TM][TN]) {
   const int l32 = threadIdx.x & 31, lhi = (threadIdx.x >> 5) & 1;
@@ -449,21 +436,10 @@ __device__ __forceinline__ void stage_pass(float* st, const f32x16_t (&acc)[TM][
 #pragma unroll
     for (int r = 0; r < 16; ++r) st[((r / 4) * 8 + lhi * 4 + (r % 4)) * SROW + j * 32 + l32] = acc[I][j][r];
 }
-template <int I, int SROW, int TM, int TN>
-__device__ __forceinline__ void stage_pass(float* st, const f32x4_t (&acc)[TM][TN]) {
-  const int l16 = threadIdx.x & 15, lq = (threadIdx.x >> 4) & 3;
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) st[(i * 16 + lq * 4 + r) * SROW + j * 16 + l16] = acc[2 * I + i][j][r];
-}
 
-template <int WM, int WN, bool TST, typename Acc>
+template <int WM, int WN, typename Acc>
 __device__ __forceinline__ void staged_epilogue(float* smem, const Acc& acc, const GemmArgs& e,
-                                                float* part, uint64_t m0, uint64_t n0, int wm, int wn,
-                                                uint16_t* tbase = nullptr) {
+                                                float* part, uint64_t m0, uint64_t n0, int wm, int wn) {
   constexpr int TM = WM / 32;  // passes of 32 rows
   constexpr int SROW = WN + 4, F4R = WN / 4, RPI = 64 / F4R;
   static_assert(64 % F4R == 0, "whole rows per wave pass");
@@ -471,21 +447,6 @@ __device__ __forceinline__ void staged_epilogue(float* smem, const Acc& acc, con
   float* st = smem + wave * 32 * SROW;
   const uint64_t nb = n0 + wn * WN;
   const bool tr = e.Cbft && !part;
-  const bool tst = TST && tr;
-  uint16_t* tt = TST ? tbase + wave * WN * TT_PITCH : nullptr;
-  // the final values of row segment (rr, cc..cc+3) of pass i into the
-  // transposed tile, rows of even passes first (as BF16 pairs already
-  // converted, or converted here)
-  auto put_t_bf = [&](int i, int rr, int cc, uint2 h) {
-    uint16_t* d = tt + cc * TT_PITCH + (i & 1) * 32 + rr;
-    d[0] = (uint16_t)h.x;
-    d[TT_PITCH] = (uint16_t)(h.x >> 16);
-    d[2 * TT_PITCH] = (uint16_t)h.y;
-    d[3 * TT_PITCH] = (uint16_t)(h.y >> 16);
-  };
-  auto put_t = [&](int i, int rr, int cc, float4 f) {
-    put_t_bf(i, rr, cc, make_uint2(f2bf(f.x) | ((uint32_t)f2bf(f.y) << 16), f2bf(f.z) | ((uint32_t)f2bf(f.w) << 16)));
-  };
   const bool tr_vec = e.ldt % 8 == 0 && ((uintptr_t)e.Cbft & 15u) == 0;
   // column sums: the wave's WM = 128 rows are one chunk; lane c < WN walks
   // column c down the staged slices in row order, 32 rows per pass
@@ -595,13 +556,10 @@ __device__ __forceinline__ void staged_epilogue(float* smem, const Acc& acc, con
           const int rr = r0 + (k0 + k) * RPI;
           const float4 v = *reinterpret_cast<const float4*>(st + rr * SROW + cc);
           const f32x4_t c = e.beta != 0.f ? *reinterpret_cast<const f32x4_t*>(e.C + (mb + rr) * e.ldc + n) : z;
-          uint2 hb = make_uint2(0u, 0u);
           const float4 f = relu_codes
-                               ? finish4<false, true>(e, mb + rr, n, v, true, 4, c, bq, relu_x(k0 + k), false,
-                                                      &hb, tst)
-                               : finish4<false>(e, mb + rr, n, v, true, 4, c, bq, xq[k], false, &hb, tst);
-          if (tst) put_t_bf(i, rr, cc, hb);
-          if (csum || (tr && !tst)) *reinterpret_cast<float4*>(st + rr * SROW + cc) = f;
+                               ? finish4<false, true>(e, mb + rr, n, v, true, 4, c, bq, relu_x(k0 + k), false)
+                               : finish4<false>(e, mb + rr, n, v, true, 4, c, bq, xq[k], false);
+          if (csum || tr) *reinterpret_cast<float4*>(st + rr * SROW + cc) = f;
         }
       }
     } else {
@@ -613,8 +571,7 @@ __device__ __forceinline__ void staged_epilogue(float* smem, const Acc& acc, con
             store_part4(part, e.N, m, n, v);
           } else {
             const float4 f = epilogue4(e, m, n, v, false);
-            if (tst) put_t(i, rr, cc, f);
-            if (csum || (tr && !tst)) *reinterpret_cast<float4*>(st + rr * SROW + cc) = f;
+            if (csum || tr) *reinterpret_cast<float4*>(st + rr * SROW + cc) = f;
           }
         }
       }
@@ -640,27 +597,8 @@ __device__ __forceinline__ void staged_epilogue(float* smem, const Acc& acc, con
         }
       }
     }
-    if (tst && ((i & 1) || i == TM - 1)) {
-      // rows (i & ~1) * 32 .. of the slab: eight lanes a column, 16 bytes each
-      const uint64_t mp = m0 + wm * WM + (i & ~1) * 32;
-      const int q = lane & 7, rows = (i & 1) ? 64 : 32;
-      if (q * 8 < rows) {
-        for (int c = lane >> 3; c < WN; c += 8) {
-          const uint64_t nt = nb + c;
-          if (nt >= e.N) continue;
-          uint16_t* dst = e.Cbft + nt * e.ldt + mp + q * 8;
-          const uint16_t* src = tt + c * TT_PITCH + q * 8;
-          if (tr_vec && mp + q * 8 + 7 < e.M) {
-            *reinterpret_cast<uint4*>(dst) = *reinterpret_cast<const uint4*>(src);
-          } else {
-            for (int r = 0; r < 8; ++r)
-              if (mp + q * 8 + r < e.M) dst[r] = src[r];
-          }
-        }
-      }
-    }
-    if (csum && !(tr && !tst)) __syncthreads();  // st (and tt) are read before the next pass writes them
-    if (tr && !tst) {
+    if (csum && !tr) __syncthreads();  // st is read before the next pass writes it
+    if (tr) {
       // four lanes per column, 8 rows (16 bytes) each: one store covers 16
       // columns in whole 64-byte runs
       const int q = lane & 3;
@@ -693,7 +631,8 @@ __device__ __forceinline__ void staged_epilogue(float* smem, const Acc& acc, con
 // operands exchanged (each block of the accumulators is then C^T's, so a lane
 // holds 4 consecutive columns of a row): no LDS, 16-byte accesses, 64-byte runs
 // of a row an instruction.  For alpha, beta, bias and ReLU (and the split-k
-// partial sums); anything else takes the staged epilogue.  acc[i][j] is the
+// partial sums); anything else takes copies_epilogue (small FP32 tiles: the
+// 128 x 128 one's staged epilogue).  acc[i][j] is the
 // 16 x 16 block (i, j) of the wave's sub-tile: row l16 = lane % 16, columns
 // 4 (lane / 16) .. + 3.  65536 x 1024 x 1024 151 us against 200 us staged.
 static bool direct_ok(const GemmArgs& e) {
@@ -770,6 +709,278 @@ __device__ __forceinline__ void direct_epilogue(const f32x4_t (&acc)[TM][TN], co
           }
     }
   }
+}
+
+// ---- register epilogue of the pipelined kernel, with BF16 copies and column sums ----
+// For what direct_epilogue leaves: BF16 copies of C (Cbf) and of C^T (Cbft),
+// column sums, aux derivatives, sigmoid.  The operands are exchanged as there,
+// so a lane holds 4 consecutive columns of a row and the values become final
+// where they are.  Only the copies pass through LDS, each wave in its own
+// area, so no block barrier is needed: a block row's 16 x WN BF16 values for
+// whole runs of a row, 64 rows' transposed values for 128-byte runs of C^T,
+// and (column sums) a block row's floats, which a lane per column adds in row
+// order.  What bounds it is the count of vector instructions, about 10 an
+// element (a quarter of them the rounding to BF16), and the stores.
+template <int TM, int TN>
+struct CopyArea {
+  static constexpr int WM = TM * 16, WN = TN * 16;
+  static constexpr int TR = WM < 64 ? WM : 64;   // rows of a transposed tile
+  static constexpr int TP = TR + 8, RP = WN + 8, FP = WN + 4;
+  static constexpr bool CSUM = WM == CS_ROWS && WN == 64;
+  static constexpr int T_BYTES = WN * TP * 2, R_BYTES = 16 * RP * 2, F_BYTES = CSUM ? 16 * FP * 4 : 0;
+  static constexpr int BYTES = T_BYTES + R_BYTES + F_BYTES + WN * 4;  // of a wave
+  static_assert(T_BYTES % 16 == 0 && R_BYTES % 16 == 0, "16-byte accesses");
+};
+
+// Floats as BF16, two a word.  The conversion instruction rounds as f2bf does
+// except for NaNs (f2bf keeps the payload) and denormals (f2bf rounds none of
+// them to zero): rows with one of those are converted again by f2bf.
+template <int N>
+__device__ __forceinline__ void f2bf_pairs(const float (&v)[N], uint32_t (&h)[N / 2]) {
+  typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2_t;
+  constexpr int SPECIAL = 0x93;  // NaNs and denormals, for v_cmp_class
+  bool odd = false;
+#pragma unroll
+  for (int k = 0; k < N; k += 2) {
+    odd |= __builtin_amdgcn_classf(v[k], SPECIAL) | __builtin_amdgcn_classf(v[k + 1], SPECIAL);
+    const bf16x2_t t = {(__bf16)v[k], (__bf16)v[k + 1]};
+    h[k / 2] = __builtin_bit_cast(uint32_t, t);
+  }
+  if (__builtin_expect(odd, 0)) {
+#pragma unroll
+    for (int k = 0; k < N; k += 2) h[k / 2] = f2bf(v[k]) | ((uint32_t)f2bf(v[k + 1]) << 16);
+  }
+}
+
+// LDS of this wave written by other lanes of it is read after this (and the
+// other way round): the hardware keeps a wave's LDS accesses in order
+__device__ __forceinline__ void wave_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// AUX: 0 none, 1 e.aux16, 2 e.aux
+template <int AUX, int TM, int TN>
+__device__ __forceinline__ void copies_epilogue(char* area, const f32x4_t (&acc)[TM][TN], const GemmArgs& e,
+                                                uint64_t mw, uint64_t nw) {
+  using L = CopyArea<TM, TN>;
+  constexpr int WN = L::WN;
+  static_assert(TM % 2 == 0, "block rows in pairs");
+  uint16_t* tt = reinterpret_cast<uint16_t*>(area);
+  uint16_t* rt = reinterpret_cast<uint16_t*>(area + L::T_BYTES);
+  float* ft = reinterpret_cast<float*>(area + L::T_BYTES + L::R_BYTES);
+  float* bt = reinterpret_cast<float*>(area + L::T_BYTES + L::R_BYTES + L::F_BYTES);
+  int lane = threadIdx.x & 63, l16 = lane & 15, lq = lane >> 4;
+  // the lane's number anew, so that no address made from it is kept in a
+  // register from one block row to the next (the accumulators leave too few)
+  auto fresh = [&]() __attribute__((always_inline)) {
+    asm volatile("" : "+v"(lane));
+    l16 = lane & 15;
+    lq = lane >> 4;
+  };
+  // every column in range: groups of 4 at any 4-byte alignment, with the
+  // lane's place within 16 rows in 32 bits next to a wave-uniform address
+  const bool whole = nw + WN <= e.N && e.ldc < (1u << 26) && e.ldaux < (1u << 26);
+  // (no bias: -0, which changes no value)
+  if (lane < WN) bt[lane] = e.bias ? e.bias[nw + lane < e.N ? nw + lane : e.N - 1] : -0.f;
+  wave_order();
+  // Row m0 + l16 of a matrix, TN groups of 4 columns.  Rows and columns beyond
+  // the matrix read its last ones; what is made of them is not stored.
+  auto load_row = [&](float(&d)[TN * 4], const float* base, uint64_t ld, uint64_t m0) __attribute__((always_inline)) {
+    if (whole && m0 + 15 < e.M) {
+      const float* p = base + m0 * ld + nw;
+      const uint32_t off = l16 * (uint32_t)ld + lq * 4;
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        const f32x4_t t = *reinterpret_cast<const f32x4u_t*>(p + j * 16 + off);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) d[j * 4 + q] = t[q];
+      }
+    } else {
+      const float* p = base + min(m0 + l16, e.M - 1) * ld;
+#pragma unroll
+      for (int k = 0; k < TN * 4; ++k) d[k] = p[min(nw + lq * 4 + (k / 4) * 16 + k % 4, e.N - 1)];
+    }
+  };
+  // the aux activation's outputs, two block rows ahead (a BF16 aux as raw
+  // bits, two columns a register)
+  constexpr int NX = AUX == 2 ? TN * 4 : TN * 2;
+  float ring[2][NX];
+  const bool aux8 = whole && ((uintptr_t)e.aux16 & 7u) == 0 && e.ldaux % 4 == 0;
+  auto load_aux = [&](float(&d)[NX], int i) __attribute__((always_inline)) {
+    const uint64_t m0 = mw + i * 16;
+    if constexpr (AUX == 2) {
+      load_row(d, e.aux, e.ldaux, m0);
+    } else if constexpr (AUX == 1) {
+      if (aux8 && m0 + 15 < e.M) {
+        const uint16_t* p = e.aux16 + m0 * e.ldaux + nw;
+        const uint32_t off = l16 * (uint32_t)e.ldaux + lq * 4;
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          const uint2 t = *reinterpret_cast<const uint2*>(p + j * 16 + off);
+          d[2 * j] = __uint_as_float(t.x);
+          d[2 * j + 1] = __uint_as_float(t.y);
+        }
+      } else {
+        const uint16_t* p = e.aux16 + min(m0 + l16, e.M - 1) * e.ldaux;
+        auto at = [&](int k) { return (uint32_t)p[min(nw + lq * 4 + (k / 4) * 16 + k % 4, e.N - 1)]; };
+#pragma unroll
+        for (int k = 0; k < TN * 4; k += 2) d[k / 2] = __uint_as_float(at(k) | (at(k + 1) << 16));
+      }
+    }
+  };
+  if constexpr (AUX != 0) {
+    load_aux(ring[0], 0);
+    load_aux(ring[1], 1);
+  }
+  const bool row16 = ((uintptr_t)e.Cbf & 15u) == 0 && e.ldc % 8 == 0 && nw + WN <= e.N;
+  const bool col16 = ((uintptr_t)e.Cbft & 15u) == 0 && e.ldt % 8 == 0;
+  const bool csum = L::CSUM && e.cs;
+  // ReLU: what is less than this becomes 0 (nothing without it)
+  const float floor_v = e.act == VKH_ACT_RELU ? 0.f : -__builtin_inff();
+  float csacc = 0.f;
+  // one copy of the code for every two block rows (the ring's registers);
+  // only the choice of the accumulators, whose indices are constants, is
+  // unrolled further
+#pragma unroll 1
+  for (int i2 = 0; i2 < TM; i2 += 2) {
+    static_for<2>([&](auto hc) __attribute__((always_inline)) {
+      constexpr int H = decltype(hc)::value;
+      const int i = i2 + H;
+      const uint64_t m0 = mw + i * 16;
+      if (m0 >= e.M) return;
+      fresh();
+      float v[TN * 4];
+      static_for<TM / 2>([&](auto ic) __attribute__((always_inline)) {
+        if (i2 == 2 * decltype(ic)::value)
+#pragma unroll
+          for (int k = 0; k < TN * 4; ++k) v[k] = acc[2 * decltype(ic)::value + H][k / 4][k % 4];
+      });
+#pragma unroll
+      for (int k = 0; k < TN * 4; ++k) v[k] = e.alpha * v[k];
+      if (e.beta != 0.f) {
+        float c[TN * 4];
+        load_row(c, e.C, e.ldc, m0);
+#pragma unroll
+        for (int k = 0; k < TN * 4; ++k) v[k] += e.beta * c[k];
+      }
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        const f32x4_t b = *reinterpret_cast<const f32x4_t*>(bt + j * 16 + lq * 4);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const float t = v[j * 4 + q] + b[q];
+          v[j * 4 + q] = t < floor_v ? 0.f : t;
+        }
+      }
+      if (__builtin_expect(e.act == VKH_ACT_SIGMOID, 0)) {
+        // one copy of its FP64 code: the values move past it in turn
+#pragma unroll 1
+        for (int t = 0; t < TN * 4; ++t) {
+          const float y = act_apply(VKH_ACT_SIGMOID, v[0]);
+#pragma unroll
+          for (int k = 0; k + 1 < TN * 4; ++k) v[k] = v[k + 1];
+          v[TN * 4 - 1] = y;
+        }
+      }
+      if constexpr (AUX == 1) {
+        // (ReLU' only)
+#pragma unroll
+        for (int k = 0; k < TN * 4; ++k) {
+          const uint32_t w = __float_as_uint(ring[H][k / 2]);
+          v[k] = act_deriv_mul(VKH_ACT_RELU, __uint_as_float(k & 1 ? w & 0xffff0000u : w << 16), v[k]);
+        }
+      } else if constexpr (AUX == 2) {
+#pragma unroll
+        for (int k = 0; k < TN * 4; ++k) v[k] = act_deriv_mul(e.aux_act, ring[H][k], v[k]);
+      }
+      if (AUX != 0 && i + 2 < TM) load_aux(ring[H], i + 2);
+      if (!e.no_c) {
+        if (whole && m0 + 15 < e.M) {
+          float* p = e.C + m0 * e.ldc + nw;
+          const uint32_t off = l16 * (uint32_t)e.ldc + lq * 4;
+#pragma unroll
+          for (int j = 0; j < TN; ++j)
+            *reinterpret_cast<f32x4u_t*>(p + j * 16 + off) = f32x4_t{v[j * 4], v[j * 4 + 1], v[j * 4 + 2], v[j * 4 + 3]};
+        } else if (m0 + l16 < e.M) {
+          const uint64_t n = nw + lq * 4;
+          float* p = e.C + (m0 + l16) * e.ldc + n;
+#pragma unroll
+          for (int k = 0; k < TN * 4; ++k)
+            if (n + (k / 4) * 16 + k % 4 < e.N) p[(k / 4) * 16 + k % 4] = v[k];
+        }
+      }
+      wave_order();  // (the previous block row's reads come before these writes)
+      if (csum) {
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+          *reinterpret_cast<f32x4_t*>(ft + l16 * L::FP + j * 16 + lq * 4) =
+              f32x4_t{v[j * 4], v[j * 4 + 1], v[j * 4 + 2], v[j * 4 + 3]};
+      }
+      if (e.Cbf || e.Cbft) {
+        uint32_t h[TN * 2];
+        f2bf_pairs(v, h);
+        if (e.Cbf) {
+#pragma unroll
+          for (int j = 0; j < TN; ++j)
+            *reinterpret_cast<uint2*>(rt + l16 * L::RP + j * 16 + lq * 4) = make_uint2(h[2 * j], h[2 * j + 1]);
+        }
+        if (e.Cbft) {
+          uint16_t* d = tt + lq * 4 * L::TP + (i * 16) % L::TR + l16;
+#pragma unroll
+          for (int k = 0; k < TN * 4; ++k)
+            d[((k / 4) * 16 + k % 4) * L::TP] = (uint16_t)(k & 1 ? h[k / 2] >> 16 : h[k / 2]);
+        }
+      }
+      wave_order();
+      if (e.Cbf) {
+        constexpr int LPR = WN / 8, RPI = 64 / LPR;  // lanes of a row, rows an instruction
+        const int c = (lane % LPR) * 8, r0 = lane / LPR;
+        uint16_t* dst = e.Cbf + (m0 + r0) * e.ldc + nw + c;
+        const uint16_t* src = rt + r0 * L::RP + c;
+        if (row16 && m0 + 15 < e.M) {
+#pragma unroll
+          for (int r = 0; r < 16 / RPI; ++r)
+            *reinterpret_cast<uint4*>(dst + r * RPI * e.ldc) = *reinterpret_cast<const uint4*>(src + r * RPI * L::RP);
+        } else {
+#pragma unroll 1
+          for (int r = r0; r < 16 && m0 + r < e.M; r += RPI, dst += RPI * e.ldc, src += RPI * L::RP)
+            for (int q = 0; q < 8 && nw + c + q < e.N; ++q) dst[q] = src[q];
+        }
+      }
+      if (csum) {
+        // a chain in row order from the slab's first row (every lane a column)
+        float f[16];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) f[r] = ft[r * L::FP + lane];
+        csacc = i == 0 ? f[0] : csacc + f[0];
+        if (m0 + 15 < e.M) {
+#pragma unroll
+          for (int r = 1; r < 16; ++r) csacc = csacc + f[r];
+        } else {
+#pragma unroll
+          for (int r = 1; r < 16; ++r) csacc = m0 + r < e.M ? csacc + f[r] : csacc;
+        }
+      }
+      if (e.Cbft && ((i + 1) * 16 % L::TR == 0 || m0 + 16 >= e.M)) {
+        const uint64_t mt = mw + (i * 16) / L::TR * L::TR;   // first row of the tile
+        constexpr int LPC = L::TR / 8, CPI = 64 / LPC;       // lanes of a column, columns an instruction
+        const int r = (lane % LPC) * 8, c0 = lane / LPC;
+        uint16_t* dst = e.Cbft + (nw + c0) * e.ldt + mt + r;
+        const uint16_t* src = tt + c0 * L::TP + r;
+        if (col16 && nw + WN <= e.N && mt + L::TR <= e.M) {
+#pragma unroll
+          for (int c = 0; c < WN / CPI; ++c)
+            *reinterpret_cast<uint4*>(dst + c * CPI * e.ldt) = *reinterpret_cast<const uint4*>(src + c * CPI * L::TP);
+        } else {
+#pragma unroll 1
+          for (int c = c0; c < WN && nw + c < e.N; c += CPI, dst += CPI * e.ldt, src += CPI * L::TP)
+            for (int q = 0; q < 8 && mt + r + q < e.M; ++q) dst[q] = src[q];
+        }
+      }
+    });
+  }
+  if (csum && nw + lane < e.N) e.cs[(mw / CS_ROWS) * e.N + nw + lane] = csacc;
 }
 
 // ---- FP32 path ----------------------------------------------------------------------
@@ -902,7 +1113,6 @@ k_gemm_f32(GemmArgs p, float* part, uint64_t kc) {
   using SB = F32Stager<BN, BKM, THREADS, VEC>;
   constexpr int MAIN = 2 * (SA::FLOATS + SB::FLOATS), STAGE = WAVES * 32 * (WN + 4);
   constexpr int SMEM_FLOATS = MAIN > STAGE ? MAIN : STAGE;
-  constexpr bool TST = 4 * STAGE + tt_bytes<WAVES, WN>() <= 4 * SMEM_FLOATS;
   __shared__ __attribute__((aligned(16))) float smem[SMEM_FLOATS];
   auto As = [&](int b) { return smem + b * SA::FLOATS; };
   auto Bs = [&](int b) { return smem + 2 * SA::FLOATS + b * SB::FLOATS; };
@@ -996,8 +1206,8 @@ k_gemm_f32(GemmArgs p, float* part, uint64_t kc) {
     frags(cur, 0, 0);
   }
   __syncthreads();  // every wave is done with the operand tiles before staging
-  staged_epilogue<WM, WN, TST>(smem, acc, p, part ? part + (uint64_t)blockIdx.y * p.M * p.N : nullptr,
-                                       m0, n0, wm, wn, reinterpret_cast<uint16_t*>(smem + STAGE));
+  staged_epilogue<WM, WN>(smem, acc, p, part ? part + (uint64_t)blockIdx.y * p.M * p.N : nullptr,
+                          m0, n0, wm, wn);
 }
 
 // Small FP32 tiles (T x T, four waves of T/2 x T/2) for products with few
@@ -1218,8 +1428,8 @@ struct PipeSlice {
   }
 };
 
-// DIRECT: the operands are exchanged and the accumulators stored without
-// staging (no C^T copy, no column sums)
+// The operands are exchanged (each block of the accumulators is C^T's).
+// DIRECT: direct_epilogue, else copies_epilogue
 template <int BM, int BN, int WGM, int WGN, int PARTS, bool DIRECT>
 __global__ void __launch_bounds__(64 * WGM * WGN, 2)
 k_gemm_pipe(PackedArgs p) {
@@ -1241,10 +1451,7 @@ k_gemm_pipe(PackedArgs p) {
   static_assert(LA * WAVES == WGM * GA && LB * WAVES == (BWHOLE ? 2 : 1) * WGN * GB, "whole loads per wave and half");
   constexpr int A_BYTES = BM * ROWB, B_BYTES = BN * ROWB;
   constexpr int MAIN_BYTES = 2 * (A_BYTES + B_BYTES);
-  constexpr int STAGE_BYTES = WAVES * 32 * (WN + 4) * 4;
-  constexpr int TT = tt_bytes<WAVES, WN>();
-  constexpr bool TST = STAGE_BYTES + TT <= 160 * 1024 && WAVES == 8;
-  constexpr int EPI_BYTES = DIRECT ? 0 : STAGE_BYTES + (TST ? TT : 0);
+  constexpr int EPI_BYTES = DIRECT ? 0 : WAVES * CopyArea<2 * TMH, 2 * TNH>::BYTES;
   constexpr int SMEM_BYTES = MAIN_BYTES > EPI_BYTES ? MAIN_BYTES : EPI_BYTES;
   __shared__ __attribute__((aligned(16))) char smem[SMEM_BYTES];
 
@@ -1327,7 +1534,7 @@ k_gemm_pipe(PackedArgs p) {
 #pragma unroll
       for (int j = 0; j < TNH; ++j)
         acc[h * TMH + i][g * TNH + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-            DIRECT ? fb[g][j][q] : fa[i][f], DIRECT ? fa[i][f] : fb[g][j][q], acc[h * TMH + i][g * TNH + j], 0, 0, 0);
+            fb[g][j][q], fa[i][f], acc[h * TMH + i][g * TNH + j], 0, 0, 0);
   };
   // quarter (h, g): every product of its fragments, k in order (with several
   // parts the products of 32 k at a time, the smaller ones first)
@@ -1391,9 +1598,13 @@ k_gemm_pipe(PackedArgs p) {
   if constexpr (DIRECT) {
     direct_epilogue(acc, e, part, m0 + wm * WM, n0 + wn * WN);
   } else {
-    __syncthreads();
-    staged_epilogue<WM, WN, TST>(reinterpret_cast<float*>(smem), acc, e, part, m0, n0, wm, wn,
-                                 reinterpret_cast<uint16_t*>(smem + STAGE_BYTES));
+    __syncthreads();  // (the waves' areas lie over every wave's operands)
+    const uint64_t mw = m0 + wm * WM, nw = n0 + wn * WN;
+    char* area = smem + wave * CopyArea<2 * TMH, 2 * TNH>::BYTES;
+    if (mw >= e.M || nw >= e.N) return;
+    if (e.aux16) copies_epilogue<1>(area, acc, e, mw, nw);
+    else if (e.aux) copies_epilogue<2>(area, acc, e, mw, nw);
+    else copies_epilogue<0>(area, acc, e, mw, nw);
   }
 }
 
