@@ -593,6 +593,31 @@ def test_tile_edges(gpu, mode, M, N, K):
         _lib.call("vkh_gemm_set_config", h, md, 0, 1, M, N, K, -1)
 
 
+# The column walk's forms (one launch up to 2048 outputs by 16 and 32 chunks of
+# 64 terms; else chunks and a combine, Y through LDS or, for one output, not)
+# add each output's terms in chunks in k order and the chunks in order:
+# the sums of NumPy's float32 steps bit for bit, which the forms' edges must keep
+# (chunk and batch remainders, output groups past Q and P).
+@pytest.mark.parametrize("P,Q,K", [(32, 3, 150), (2, 1, 17), (63, 5, 64), (65, 16, 65), (130, 4, 33), (2048, 2, 97),
+                                   (2049, 3, 97), (96, 1, 150), (96, 1, 300), (61, 7, 2048), (61, 7, 2049),
+                                   (64, 13, 2100), (100, 2, 4100)])
+def test_column_walk_order(gpu, P, Q, K):
+    rng = np.random.default_rng(P + 5 * Q + K)
+    X = rng.standard_normal((K, P)).astype(np.float32)
+    Y = rng.standard_normal((K, Q)).astype(np.float32)
+    C0 = rng.standard_normal((Q, P)).astype(np.float32)
+    got = run_gemm(gpu, "fp32", 1, 0, Y, X, C0=C0, beta=1.0)
+    n = max(1, -(-K // 64))
+    kc = -(-K // n)
+    total = np.zeros((Q, P), dtype=np.float32)
+    for k0 in range(0, K, kc):
+        part = np.zeros((Q, P), dtype=np.float32)
+        for k in range(k0, min(K, k0 + kc)):
+            part += X[k][None, :] * Y[k][:, None]
+        total += part
+    np.testing.assert_array_equal(got, total + C0)
+
+
 # The BF16 copies of C and C^T (written through LDS a block row / 64 rows at a
 # time) at edges of the tiles, of their 16-byte runs and of their leading
 # dimensions, with the values the conversion handles apart: NaNs with a

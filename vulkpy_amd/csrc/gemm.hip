@@ -2089,17 +2089,13 @@ __global__ void __launch_bounds__(256)
 k_skinny_colwalk(SkinnyArgs a, uint64_t kchunk, float* part) {
   const uint64_t p = ((uint64_t)blockIdx.x * 256 + threadIdx.x) * VW;
   const uint64_t chunk = blockIdx.y;
-  if (p >= a.P) return;
+  const bool in = p < a.P;
   const uint64_t k0 = chunk * kchunk, k1 = min(a.K, k0 + kchunk);
   float acc[QB][VW];
 #pragma unroll
   for (int q = 0; q < QB; ++q)
 #pragma unroll
     for (int w = 0; w < VW; ++w) acc[q][w] = 0.f;
-  // U terms at a time, all their loads issued before the first sum (one term at
-  // a time, each waited for its own loads: a 50-term chunk took 24 us, 14 now),
-  // added in k order
-  constexpr int U = QB <= 4 ? 8 : 4;
   auto load_x = [&](uint64_t k, float (&x)[VW]) {
     if constexpr (VW == 4) {
       const float4 t = *reinterpret_cast<const float4*>(a.X + k * a.sxk + p);
@@ -2108,35 +2104,65 @@ k_skinny_colwalk(SkinnyArgs a, uint64_t kchunk, float* part) {
       x[0] = a.X[k * a.sxk + p];
     }
   };
-  uint64_t k = k0;
-  for (; k + U <= k1; k += U) {
-    float x[U][VW], y[U][QB];
+  constexpr int U = 8;  // terms of X requested at a time, before the first sum
+  if constexpr (QB == 1) {
+    if (!in) return;
+    uint64_t k = k0;
+    for (; k + U <= k1; k += U) {
+      float x[U][VW], y[U];
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      load_x(k + u, x[u]);
+      for (int u = 0; u < U; ++u) {
+        load_x(k + u, x[u]);
+        y[u] = a.Y[(k + u) * a.syk];
+      }
 #pragma unroll
-      for (int q = 0; q < QB; ++q) y[u][q] = q < a.Q ? a.Y[(k + u) * a.syk + q * a.syq] : 0.f;
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int w = 0; w < VW; ++w) acc[0][w] += x[u][w] * y[u];
     }
+    for (; k < k1; ++k) {
+      float x[VW];
+      load_x(k, x);
+      const float y = a.Y[k * a.syk];
 #pragma unroll
-    for (int u = 0; u < U; ++u)
+      for (int w = 0; w < VW; ++w) acc[0][w] += x[w] * y;
+    }
+  } else {
+    // Segments of KS terms, Y's read into LDS by the whole block.  (With Y read by
+    // every thread itself, a scalar load for each term and output, 4096 x 16
+    // outputs over 4096 terms took 79 us, 35 now; one output is faster without
+    // LDS: 4096 x 1 over 1024 terms 9.8 against 13.6.)
+    constexpr int KS = 64;
+    __shared__ __attribute__((aligned(16))) float ys[KS * QB];
+    for (uint64_t s0 = k0; s0 < k1; s0 += KS) {
+      const int n = (int)min<uint64_t>(KS, k1 - s0);
+      float r[(KS * QB + 255) / 256];
 #pragma unroll
-      for (int q = 0; q < QB; ++q)
-        if (q < a.Q)
+      for (int u = 0; u < (KS * QB + 255) / 256; ++u) {
+        const int t = min((int)threadIdx.x + u * 256, n * QB - 1);
+        r[u] = a.Y[(s0 + t / QB) * a.syk + min(t % QB, a.Q - 1) * a.syq];
+      }
+      if (s0 > k0) __syncthreads();
 #pragma unroll
-          for (int w = 0; w < VW; ++w) acc[q][w] += x[u][w] * y[u][q];
-  }
-  for (; k < k1; ++k) {
-    float x[VW];
-    load_x(k, x);
+      for (int u = 0; u < (KS * QB + 255) / 256; ++u)
+        if ((int)threadIdx.x + u * 256 < KS * QB) ys[threadIdx.x + u * 256] = r[u];
+      __syncthreads();
+      if (!in) continue;
+      for (int i = 0; i < n; i += U) {
+        float x[U][VW];
 #pragma unroll
-    for (int q = 0; q < QB; ++q) {
-      if (q < a.Q) {
-        const float y = a.Y[k * a.syk + q * a.syq];
+        for (int u = 0; u < U; ++u) load_x(s0 + min(i + u, n - 1), x[u]);
 #pragma unroll
-        for (int w = 0; w < VW; ++w) acc[q][w] += x[w] * y;
+        for (int u = 0; u < U; ++u)
+          if (i + u < n)
+#pragma unroll
+            for (int q = 0; q < QB; ++q)
+#pragma unroll
+              for (int w = 0; w < VW; ++w) acc[q][w] += x[u][w] * ys[(i + u) * QB + q];
       }
     }
   }
+  if (!in) return;
 #pragma unroll
   for (int q = 0; q < QB; ++q)
     if (q < a.Q)
@@ -2164,6 +2190,66 @@ k_skinny_combine(SkinnyArgs a, const float* part, uint64_t nchunk) {
     }
     for (; c < nchunk; ++c) s += pp[c * step];
     skinny_store(a, p, q, s);
+  }
+}
+
+// Column walk of few outputs over few chunks (the weight gradient of a narrow
+// layer) in one launch: a block takes 64 p and up to 4 q, a wave a chunk (its
+// terms added in k order from 0; X requested 32 terms at once, Y's columns read
+// into LDS by the whole block first), then the chunks' sums, kept in LDS, are added
+// in order from 0 as k_skinny_combine adds them: the same bits. What bounds it
+// is the latency of the loads. 32 x 3 outputs over 150 terms 6.5 us (column walk
+// and combine 15), 1024 x 16 over 1024 terms 10 (73), over 2048 terms 15.5 (73).
+constexpr uint64_t WALK_P = 2048, WALK_CHUNKS = 32, WALK_TERMS = 64;
+constexpr int WALK_Q = 4, WALK_U = 32;
+__global__ void __launch_bounds__(1024)
+k_skinny_walk(SkinnyArgs a, uint32_t kchunk, uint32_t nchunk) {
+  extern __shared__ __attribute__((aligned(16))) float walk_lds[];
+  float* parts = walk_lds;                         // [nchunk][WALK_Q][64]
+  float* ys = walk_lds + nchunk * WALK_Q * 64;     // [K][WALK_Q]
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int waves = blockDim.x >> 6, q0 = blockIdx.y * WALK_Q;
+  const uint32_t K = (uint32_t)a.K;
+  const uint64_t p0 = (uint64_t)blockIdx.x * 64, pl = min(p0 + lane, a.P - 1);
+  // (columns beyond Q read the last one)
+  for (uint32_t t0 = threadIdx.x; t0 < K * WALK_Q; t0 += 8 * blockDim.x) {
+    float r[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const uint32_t t = min(t0 + u * blockDim.x, K * WALK_Q - 1);
+      r[u] = a.Y[(t / WALK_Q) * a.syk + min(q0 + (int)(t % WALK_Q), a.Q - 1) * a.syq];
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (t0 + u * blockDim.x < K * WALK_Q) ys[t0 + u * blockDim.x] = r[u];
+  }
+  __syncthreads();
+  for (uint32_t c = wave; c < nchunk; c += waves) {
+    const uint32_t k0 = c * kchunk, k1 = min(K, k0 + kchunk);
+    float acc[WALK_Q] = {0.f, 0.f, 0.f, 0.f};
+    for (uint32_t k = k0; k < k1; k += WALK_U) {
+      float x[WALK_U];
+#pragma unroll
+      for (int u = 0; u < WALK_U; ++u) x[u] = a.X[min(k + u, k1 - 1) * a.sxk + pl];  // (past the chunk: its last term)
+#pragma unroll
+      for (int u = 0; u < WALK_U; ++u)
+        if (k + u < k1) {
+          const f32x4_t y = *reinterpret_cast<const f32x4_t*>(ys + (k + u) * WALK_Q);
+#pragma unroll
+          for (int q = 0; q < WALK_Q; ++q) acc[q] += x[u] * y[q];
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < WALK_Q; ++q) parts[(c * WALK_Q + q) * 64 + lane] = acc[q];
+  }
+  __syncthreads();
+  for (int t = threadIdx.x; t < WALK_Q * 64; t += blockDim.x) {
+    const int q = t >> 6;
+    const uint64_t p = p0 + (t & 63);
+    float s = 0.f;
+#pragma unroll 8
+    for (uint32_t c = 0; c < nchunk; ++c) s += parts[c * WALK_Q * 64 + t];
+    if (p < a.P && q0 + q < a.Q) skinny_store(a, p, q0 + q, s);
   }
 }
 
@@ -2239,6 +2325,17 @@ static void gemm_skinny(vkh_gpu* g, bool ta, bool tb, const GemmArgs& e) {
   const uint64_t pthreads = v4 ? a.P / 4 : a.P;
   uint64_t nchunk = 0;
   const uint64_t kchunk = colwalk_chunk(g, a.P, a.K, v4, nchunk);
+  // Few outputs, few short chunks: one launch.  Us of k_skinny_walk / column walk
+  // and combine: 2048 x 4 over 512 terms 8.9 / 19, 64 x 4 over 2048 15 / 14, 64 x
+  // 16 over 2048 15 / 30; one output 150 terms 6.5 / 7.7, 512 8.3 / 7.6, 2048
+  // 15 / 8.8.  Past 32 chunks a block would walk them in turn.
+  if (a.P <= WALK_P && nchunk <= WALK_CHUNKS && kchunk <= WALK_TERMS && (a.Q > 1 || nchunk <= 4)) {
+    const unsigned waves = (unsigned)std::max<uint64_t>(4, std::min<uint64_t>(16, nchunk));
+    hipLaunchKernelGGL(k_skinny_walk, dim3((unsigned)ceil_div(a.P, 64), (unsigned)ceil_div(a.Q, WALK_Q)), dim3(64 * waves),
+                       sizeof(float) * WALK_Q * (nchunk * 64 + a.K), g->stream, a, (uint32_t)kchunk, (uint32_t)nchunk);
+    check_launch("gemm (skinny walk)");
+    return;
+  }
   Workspace ws(g, sizeof(float) * nchunk * (uint64_t)a.Q * a.P);
   float* part = (float*)ws.get();
   const uint64_t bx = ceil_div(pthreads, 256);
