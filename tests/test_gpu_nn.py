@@ -7,6 +7,7 @@ import pytest
 
 import vulkpy_amd as vk
 from vulkpy_amd import nn
+from vulkpy_amd._lib import call
 from vulkpy_amd.nn.parameters import Parameter
 from oracle import oracle as O
 
@@ -483,3 +484,22 @@ def test_long_row_losses(gpu, cols):
         # a lane adds at most 16 + 1 terms, the wave 6: relative to the positive sum
         np.testing.assert_allclose(np.asarray(L), want.sum(axis=1), rtol=28 * 2.0 ** -24)
         bits_equal(dx, O.loss_grad(name, x, t, 0.125))
+
+
+# vkh_bias_grad with beta: the column sums of the plain reduction added to
+# beta * db in their last pass (fewer than 1024 columns) or after it; the same
+# bits at 1 to 3 columns, ragged column groups, one and several row chunks.
+@pytest.mark.parametrize("rows,cols", [(64, 2), (64, 3), (150, 5), (150, 32), (63, 9), (1000, 1023), (1000, 1024),
+                                       (5000, 33), (100000, 6), (128, 64)])
+def test_bias_grad_accumulates(gpu, rows, cols):
+    rng = np.random.default_rng(rows + cols)
+    dy = rng.standard_normal((rows, cols)).astype(np.float32)
+    db = rng.standard_normal(cols).astype(np.float32)
+    g, d0, d1, d2 = (vk.Array(gpu, data=v) for v in (dy, db, db, db))
+    for d, beta in ((d0, 0.0), (d1, 1.0), (d2, -0.5)):
+        call("vkh_bias_grad", gpu._handle, g._ptr, d._ptr, rows, cols, beta)
+        d._set_job([g])
+    sums = np.asarray(d0)
+    np.testing.assert_allclose(sums, dy.astype(np.float64).sum(0), rtol=0, atol=rows * 2.0 ** -24 * np.abs(dy).sum(0).max())
+    np.testing.assert_array_equal(np.asarray(d1), db + sums)
+    np.testing.assert_array_equal(np.asarray(d2), np.float32(-0.5) * db + sums)

@@ -137,6 +137,8 @@ namespace vkh {
 // Column-sum order shared with vkh_bias_grad (reduce.hip): rows per chunk of
 // a [rows, cols] operand, and the in-order combine of chunk partials.
 uint64_t bias_grad_chunk(vkh_gpu* g, uint64_t rows, uint64_t cols);
+// vkh_bias_grad with beta in the sums' own last pass, where they have one (reduce.hip)
+bool bias_grad_narrow(vkh_gpu* g, const float* a, float* db, uint64_t rows, uint64_t cols, float beta);
 void sum_chunks(vkh_gpu* g, const float* part, float* out, uint64_t m, uint64_t nchunk);
 void sum_chunks_from_zero(vkh_gpu* g, const float* part, float* out, uint64_t m, uint64_t nchunk);
 
