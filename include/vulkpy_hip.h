@@ -142,6 +142,16 @@ int vkh_copy(vkh_gpu* gpu, void* dst, const void* src, size_t nbytes);
 /* dst[0..n) = value (vkarray.py:1541 `z[:] = 0.0`, initializers.py:48) */
 int vkh_fill_f32(vkh_gpu* gpu, float* dst, float value, size_t n);
 int vkh_fill_u32(vkh_gpu* gpu, uint32_t* dst, uint32_t value, size_t n);
+/* vkh_fill_f32 on up to VKH_FILL_MULTI_MAX buffers in one launch (a training
+ * step zeroes its parameters' gradients with it).  No counterpart in the
+ * reference. */
+#define VKH_FILL_MULTI_MAX 16
+typedef struct vkh_span {
+  float* p;
+  uint64_t n;
+} vkh_span;
+int vkh_fill_multi(vkh_gpu* gpu, const vkh_span* spans, int count,
+                   float value);
 
 /* ---- jobs ---------------------------------------------------------------- */
 /* replaces Job (_vkarray.cc:392-457): an event recorded after the work
@@ -536,6 +546,24 @@ typedef struct vkh_adam_param {
  * (a captured training step updates its parameters in one kernel). */
 int vkh_adam_device_multi(vkh_gpu* gpu, const vkh_adam_param* params,
                           int count);
+/* one parameter of vkh_adam_multi: the arguments of vkh_adam */
+typedef struct vkh_adam_step {
+  float* w;
+  const float* g;
+  float* m;
+  float* v;
+  uint64_t n;
+  float lr;
+  float eps;
+  double beta1;
+  double beta2;
+  double b1t;
+  double b2t;
+} vkh_adam_step;
+/* vkh_adam on up to VKH_ADAM_MULTI_MAX parameters in one launch, each with
+ * the bits vkh_adam gives it; no two may share a buffer they write.  No
+ * counterpart in the reference. */
+int vkh_adam_multi(vkh_gpu* gpu, const vkh_adam_step* params, int count);
 /* SGD (nn/optimizers.py:53) and AdaGrad (nn/optimizers.py:134-140), with the
  * optional regularizer term of vkh_adam_device (reg_kind 0 = none) */
 int vkh_sgd(vkh_gpu* gpu, float* w, float* g, uint64_t n, float lr,

@@ -503,3 +503,58 @@ def test_bias_grad_accumulates(gpu, rows, cols):
     np.testing.assert_allclose(sums, dy.astype(np.float64).sum(0), rtol=0, atol=rows * 2.0 ** -24 * np.abs(dy).sum(0).max())
     np.testing.assert_array_equal(np.asarray(d1), db + sums)
     np.testing.assert_array_equal(np.asarray(d2), np.float32(-0.5) * db + sums)
+
+
+# A step zeroes and updates its Dense parameters several a launch: the same
+# bits as one by one, with frozen and shared parameters, tied values, other
+# optimizers and layers of the user's own between them.
+def test_step_in_batches_equals_single_calls(gpu):
+    rng = np.random.default_rng(3)
+
+    class Scale(nn.Module):  # a parameter of its own, updated by its own method
+        def __init__(self):
+            self.p = Parameter(gpu, (1, 8), initializer=lambda g, s: A(g, np.full((1, 8), 2)))
+
+        def forward(self, x):
+            return x * self.p.value
+
+        def backward(self, dy):
+            g = (self._x * dy).sum(axis=0)
+            g.reshape((1, 8))
+            self.p.add_grad(g)
+            return dy * self.p.value
+
+        def zero_grad(self):
+            self.p.zero_grad()
+
+        def update(self):
+            self.p.update()
+
+    def build(seed):
+        r = np.random.default_rng(seed)
+
+        def w(g, shape):
+            return vk.Array(g, data=r.standard_normal(tuple(shape)).astype(np.float32) * 0.3)
+        layers = [nn.Dense(gpu, 5, 8, w_init=w), nn.ReLU(), Scale()]
+        layers += [nn.Dense(gpu, 8, 8, w_init=w) for _ in range(5)]
+        layers += [nn.Dense(gpu, 8, 8, w_init=w, w_opt=nn.SGD(0.01)), nn.Dense(gpu, 8, 3, w_init=w)]
+        layers[4].w.value = layers[3].w.value       # tied values
+        layers[6] = layers[5]                       # one layer twice
+        layers[7].b.grad = None                     # frozen
+        return nn.Sequence(layers, nn.SoftmaxCrossEntropyLoss()), layers
+
+    def single(self, method, batch):
+        for layer in self.L:
+            getattr(layer, method)()
+    x = vk.Array(gpu, data=rng.standard_normal((20, 5)).astype(np.float32))
+    y = vk.Array(gpu, data=np.eye(3, dtype=np.float32)[rng.integers(0, 3, 20)])
+    one, a = build(1)
+    two, b = build(1)
+    two._each_parameter = single.__get__(two)
+    for _ in range(3):
+        one.train(x, y)
+        two.train(x, y)
+    for p, q in zip(one._parameters(), two._parameters()):
+        np.testing.assert_array_equal(np.asarray(p.value), np.asarray(q.value))
+        if p.grad is not None:
+            np.testing.assert_array_equal(np.asarray(p.grad), np.asarray(q.grad))

@@ -50,6 +50,10 @@ U64 = c_uint64
 _u64p = POINTER(c_uint64)
 
 ADAM_MULTI_MAX = 8  # VKH_ADAM_MULTI_MAX
+FILL_MULTI_MAX = 16  # VKH_FILL_MULTI_MAX
+# struct module formats of vkh_span and vkh_adam_step (native layout)
+SPAN_FORMAT = "PQ"
+ADAM_STEP_FORMAT = "PPPPQffdddd"
 
 
 class AdamParam(ctypes.Structure):
@@ -84,6 +88,7 @@ _SIGNATURES = {
     "vkh_host_stats": (c_int, [POINTER(c_size_t), POINTER(c_size_t)]),
     "vkh_copy": (c_int, [P, P, P, c_size_t]),
     "vkh_fill_f32": (c_int, [P, P, c_float, c_size_t]),
+    "vkh_fill_multi": (c_int, [P, P, c_int, c_float]),
     "vkh_fill_u32": (c_int, [P, P, c_uint32, c_size_t]),
     "vkh_event_record": (c_int, [P, POINTER(P)]),
     "vkh_event_wait": (c_int, [P, U64]),
@@ -150,6 +155,7 @@ _SIGNATURES = {
     "vkh_loss_grad_scaled": (c_int, [P, c_int, P, P, P, U64, c_float, P]),
     "vkh_loss_rows_grad": (c_int, [P, c_int, P, P, P, P, U64, U64, c_float]),
     "vkh_adam": (c_int, [P, P, P, P, P, U64, c_float, c_double, c_double, c_float, c_double, c_double]),
+    "vkh_adam_multi": (c_int, [P, P, c_int]),
     "vkh_adam_pow_advance": (c_int, [P, P, c_double, c_double]),
     "vkh_adam_device": (c_int, [P, P, P, P, P, U64, c_float, c_double, c_double, c_float, P, P,
                                 c_int, c_float, c_float]),

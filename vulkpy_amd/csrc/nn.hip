@@ -671,6 +671,16 @@ __global__ void __launch_bounds__(256) k_adam_multi(AdamMulti a) {
   }
 }
 
+// the launch of k parameters' table with their blocks so far
+static void adam_multi_launch(vkh_gpu* g, AdamMulti& a, int k, uint64_t blocks) {
+  if (k == 0) return;
+  VKH_REQUIRE(blocks < (uint64_t(1) << 31), "adam: too many blocks");
+  for (int p = k; p <= ADAM_MT; ++p) a.first[p] = (uint32_t)blocks;
+  a.count = k;
+  hipLaunchKernelGGL(k_adam_multi, dim3((unsigned)blocks), dim3(256), 0, g->stream, a);
+  check_launch("adam (several parameters)");
+}
+
 // nn/optimizers.py:53: w += (-lr) * g (g with the regularizer term added first)
 __global__ void __launch_bounds__(256)
 k_sgd(float* __restrict__ w, float* __restrict__ g, uint64_t n, uint64_t n4, float neg_lr, RegTerms r) {
@@ -1006,6 +1016,32 @@ int vkh_adam_device(vkh_gpu* g, float* w, float* gr, float* m, float* v, uint64_
   });
 }
 
+int vkh_adam_multi(vkh_gpu* g, const vkh_adam_step* params, int count) {
+  return guarded([&] {
+    use(g);
+    VKH_REQUIRE(count >= 0 && count <= ADAM_MT, "adam_multi: count out of range");
+    VKH_REQUIRE(count == 0 || params, "adam_multi: null pointer");
+    AdamMulti a{};
+    uint64_t blocks = 0;
+    int k = 0;
+    for (int p = 0; p < count; ++p) {
+      const vkh_adam_step& q = params[p];
+      if (q.n == 0) continue;
+      VKH_REQUIRE(q.w && q.g && q.m && q.v, "adam_multi: null pointer");
+      const uint64_t n4 = vec4_count(q.n, {q.w, q.g, q.m, q.v});
+      a.t[k] = AdamTensor{q.w, const_cast<float*>(q.g), q.m, q.v, q.n, n4,
+                          AdamScalars{(float)q.beta1, (float)(1.0 - q.beta1), (float)q.beta2,
+                                      (float)(1.0 - q.beta2), q.eps, -q.lr, (float)(1.0 - q.b1t),
+                                      (float)(1.0 - q.b2t)},
+                          nullptr, RegTerms{0, 0.f, 0.f}};
+      a.first[k] = (uint32_t)blocks;
+      blocks += grid_for(g, n4 ? n4 : q.n);
+      ++k;
+    }
+    adam_multi_launch(g, a, k, blocks);
+  });
+}
+
 int vkh_adam_device_multi(vkh_gpu* g, const vkh_adam_param* params, int count) {
   return guarded([&] {
     use(g);
@@ -1028,13 +1064,7 @@ int vkh_adam_device_multi(vkh_gpu* g, const vkh_adam_param* params, int count) {
       blocks += grid_for(g, n4 ? n4 : q.n);
       ++k;
     }
-    if (k == 0) return;
-    VKH_REQUIRE(blocks < (uint64_t(1) << 31), "adam_device_multi: too many blocks");
-    a.first[k] = (uint32_t)blocks;
-    for (int p = k + 1; p <= ADAM_MT; ++p) a.first[p] = (uint32_t)blocks;
-    a.count = k;
-    hipLaunchKernelGGL(k_adam_multi, dim3((unsigned)blocks), dim3(256), 0, g->stream, a);
-    check_launch("adam_device_multi");
+    adam_multi_launch(g, a, k, blocks);
   });
 }
 

@@ -132,6 +132,34 @@ static void fill(vkh_gpu* g, T* dst, T value, uint64_t n) {
   check_launch("fill");
 }
 
+// Several buffers in one launch, buffer q by blocks [first[q], first[q + 1]) as
+// k_fill with that many blocks: a step of a small network zeroes its
+// parameters' gradients in 2.5 us instead of 2 us for each of them (and a
+// launch for each on the host).
+constexpr int FILL_MT = VKH_FILL_MULTI_MAX;
+struct FillMulti {
+  float* dst[FILL_MT];
+  uint64_t n[FILL_MT];
+  uint32_t first[FILL_MT + 1];
+};
+__global__ void __launch_bounds__(256) k_fill_multi(FillMulti f, float value) {
+  // (constant indices only: a by-value argument indexed at run time would be
+  // copied to scratch memory)
+  float* dst = f.dst[0];
+  uint64_t n = f.n[0];
+  uint32_t b0 = 0, b1 = f.first[1];
+#pragma unroll
+  for (int q = 1; q < FILL_MT; ++q)
+    if (blockIdx.x >= f.first[q]) {
+      dst = f.dst[q];
+      n = f.n[q];
+      b0 = f.first[q];
+      b1 = f.first[q + 1];
+    }
+  const uint64_t stride = (uint64_t)(b1 - b0) * 256;
+  for (uint64_t i = (uint64_t)(blockIdx.x - b0) * 256 + threadIdx.x; i < n; i += stride) dst[i] = value;
+}
+
 static void init_props(vkh_gpu* g) {
   hipDeviceProp_t prop;
   VKH_HIP(hipGetDeviceProperties(&prop, g->device));
@@ -417,6 +445,30 @@ int vkh_copy(vkh_gpu* g, void* dst, const void* src, size_t nbytes) {
 
 int vkh_fill_f32(vkh_gpu* g, float* dst, float value, size_t n) {
   return guarded([&] { use(g); fill<float>(g, dst, value, n); });
+}
+
+int vkh_fill_multi(vkh_gpu* g, const vkh_span* spans, int count, float value) {
+  return guarded([&] {
+    use(g);
+    VKH_REQUIRE(count >= 0 && count <= FILL_MT, "fill_multi: count out of range");
+    VKH_REQUIRE(count == 0 || spans, "fill_multi: null pointer");
+    FillMulti f{};
+    uint64_t blocks = 0;
+    int k = 0;
+    for (int q = 0; q < count; ++q) {
+      if (spans[q].n == 0) continue;
+      VKH_REQUIRE(spans[q].p, "fill_multi: null pointer");
+      f.dst[k] = spans[q].p;
+      f.n[k] = spans[q].n;
+      f.first[k++] = (uint32_t)blocks;
+      blocks += stream_grid(g, spans[q].n, 256);
+    }
+    if (k == 0) return;
+    VKH_REQUIRE(blocks < (uint64_t(1) << 31), "fill_multi: too many blocks");
+    for (int q = k; q <= FILL_MT; ++q) f.first[q] = (uint32_t)blocks;
+    hipLaunchKernelGGL(k_fill_multi, dim3((unsigned)blocks), dim3(256), 0, g->stream, f, value);
+    check_launch("fill (several buffers)");
+  });
 }
 
 int vkh_fill_u32(vkh_gpu* g, uint32_t* dst, uint32_t value, size_t n) {

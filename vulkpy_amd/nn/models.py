@@ -21,7 +21,8 @@ from typing import Iterable, Iterator, Optional, Tuple, Union
 
 from vulkpy_amd.vkarray import Array
 from .core import Module, Loss
-from .parameters import Parameter
+from .layers import Dense
+from .parameters import Parameter, Updates, ZeroGrads, _plain
 
 
 __all__ = ["Sequence"]
@@ -65,16 +66,26 @@ class Sequence:
 
     def _learn(self):
         """stages 2-5 for the loss of the last forward"""
-        for layer in self.L:
-            layer.zero_grad()
+        self._each_parameter("zero_grad", ZeroGrads())
         g = self.loss.grad()
         for layer in reversed(self.L):
             g = layer.backward(g)
         if self.regularize:
             for p in self._parameters():
                 p.regular_grad()
+        self._each_parameter("update", Updates())
+
+    def _each_parameter(self, method: str, batch):
+        """``method`` of every layer in order, the parameters of Dense layers
+        collected in ``batch`` (one launch for several)"""
         for layer in self.L:
-            layer.update()
+            if isinstance(layer, Dense) and _plain(layer, Dense, method):
+                batch.add(layer.w)
+                batch.add(layer.b)
+            elif not _plain(layer, Module, method):
+                batch.flush()
+                getattr(layer, method)()
+        batch.flush()
 
     def train(self, x: Array, y: Array) -> Tuple[Array, Array]:
         """

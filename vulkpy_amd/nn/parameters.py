@@ -16,11 +16,13 @@ On this backend every method is stream ordered and none waits on the host:
   kernel for the penalties of :mod:`vulkpy_amd.nn.regularizers`.
 """
 from __future__ import annotations
-from typing import Callable, Iterable, Optional
+import struct
+from typing import Callable, Iterable, List, Optional
 
+from vulkpy_amd._lib import ADAM_MULTI_MAX, ADAM_STEP_FORMAT, FILL_MULTI_MAX, SPAN_FORMAT, call
 from vulkpy_amd.vkarray import GPU, Array, zeros
 from .core import Optimizer, OptimizerState, Regularizer
-from .optimizers import Adam
+from .optimizers import Adam, AdamState
 from .regularizers import _fused_penalty
 
 
@@ -117,3 +119,93 @@ class Parameter:
             self.R._add_grad(self.value, self.grad)
             return
         self.add_grad(self.R.grad(self.value))
+
+
+def _plain(obj, klass, method: str) -> bool:
+    """Whether ``obj.method`` is ``klass``'s own, neither overridden in a
+    subclass nor replaced on the object."""
+    return getattr(type(obj), method, None) is getattr(klass, method) and method not in getattr(obj, "__dict__", ())
+
+
+class ZeroGrads:
+    """``Parameter.zero_grad`` of many parameters, up to ``FILL_MULTI_MAX`` a
+    launch; ``flush`` issues what has been added."""
+
+    def __init__(self):
+        self._grads: List[Array] = []
+
+    def add(self, p: Parameter):
+        if type(p) is not Parameter or "zero_grad" in vars(p):
+            self.flush()
+            p.zero_grad()
+        elif p.grad is not None:
+            q = self._grads
+            if q and (len(q) == FILL_MULTI_MAX or q[0]._gpu is not p.grad._gpu):
+                self.flush()
+            self._grads.append(p.grad)
+
+    def flush(self):
+        grads, self._grads = self._grads, []
+        if len(grads) == 1:
+            grads[0]._fill(0.0)
+        elif grads:
+            spans = [x for a in grads for x in (a._ptr, a.buffer.n)]
+            call("vkh_fill_multi", grads[0]._gpu._handle, struct.pack(SPAN_FORMAT * len(grads), *spans),
+                 len(grads), 0.0)
+            for a in grads:
+                a._set_job()
+
+
+class Updates:
+    """``Parameter.update`` of many parameters: those with the framework's own
+    Adam state up to ``ADAM_MULTI_MAX`` a launch, with the bits of the single
+    updates; any other parameter, or one that shares its value or state with
+    one already added, comes after those added before it."""
+
+    def __init__(self):
+        self._params: List[Parameter] = []
+        self._written = set()
+
+    def add(self, p: Parameter):
+        if type(p) is not Parameter or "update" in vars(p):
+            self.flush()
+            p.update()
+            return
+        if p.grad is None:
+            return
+        state = p.opt_state
+        if (type(state) is not AdamState or "_update" in vars(state)
+                or not (abs(state.opt.lr) < 1e38 and abs(state.opt.eps) < 1e38)
+                or p.value._gpu is not p.grad._gpu or p.value.size == 0):
+            self.flush()
+            p.update()
+            return
+        mine = (p.value._ptr, state.m._ptr, state.v._ptr)
+        if (len(self._params) == ADAM_MULTI_MAX or not self._written.isdisjoint(mine)
+                or (self._params and self._params[0].value._gpu is not p.value._gpu)):
+            self.flush()
+        self._params.append(p)
+        self._written.update(mine)
+
+    def flush(self):
+        params, self._params = self._params, []
+        self._written.clear()
+        if len(params) == 1:
+            params[0].update()
+            return
+        if not params:
+            return
+        table = []
+        for p in params:
+            st = p.opt_state
+            st._advance_powers()
+            o = st.opt
+            table += (p.value._ptr, p.grad._ptr, st.m._ptr, st.v._ptr, p.value.size, o.lr, o.eps, o.beta1,
+                      o.beta2, st.beta1t, st.beta2t)
+        call("vkh_adam_multi", params[0].value._gpu._handle,
+             struct.pack(ADAM_STEP_FORMAT * len(params), *table), len(params))
+        for p in params:
+            st = p.opt_state
+            p.value._set_job([p.grad])
+            st.m._set_job()
+            st.v._set_job()
