@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 
 import vulkpy_amd as vk
+from vulkpy_amd._lib import call
 from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -747,3 +748,48 @@ def test_onehot_sizes(gpu, classes, n):
     lab = np.random.default_rng(n).integers(0, classes + 2, n)
     got = np.asarray(vk.U32Array(gpu, data=lab).to_onehot(classes))
     np.testing.assert_array_equal(got, np.identity(classes, dtype=np.float32)[np.minimum(lab, classes - 1)])
+
+
+# Rows of 4 to 63 elements, 64 a wave through its LDS (any row count below 16
+# elements, from 64 rows a compute unit on above) or a few lanes a row: tile
+# remainders, every width of an LDS read, row starts that share banks, a base
+# that is not 16-byte aligned, NaNs and infinities.  A sum's error is below
+# L - 1 roundings of the sum of magnitudes, whatever its order.
+@pytest.mark.parametrize("L,rows", [(4, 1), (4, 64), (5, 63), (6, 65), (7, 300), (8, 1000), (12, 129), (15, 64),
+                                    (16, 100), (63, 100), (16, 20011), (17, 16384), (18, 20000), (20, 30001),
+                                    (32, 20063), (34, 16385), (48, 20000), (62, 16449), (63, 20001), (64, 20001),
+                                    (96, 500), (127, 333)])
+def test_short_rows(gpu, L, rows):
+    rng = np.random.default_rng(L + rows)
+    for offset in (0, 1):
+        x = (1 + rng.standard_normal(rows * L + 1) * 0.1).astype(np.float32)
+        flat = vk.Array(gpu, data=x)
+        a = x[offset:offset + rows * L].reshape(rows, L)
+        for op, want in ((0, a.astype(np.float64).sum(1)), (1, a.astype(np.float64).prod(1)), (2, a.max(1)), (3, a.min(1))):
+            out = vk.Array(gpu, shape=(rows,))
+            call("vkh_reduce_axis", gpu._handle, op, flat._ptr + 4 * offset, out._ptr, rows, L, 1, 0, 1.0, 1.0)
+            out._set_job([flat])
+            got = np.asarray(out)
+            if op >= 2:
+                np.testing.assert_array_equal(got, want)
+            else:
+                scale = np.abs(a).astype(np.float64).sum(1) if op == 0 else np.abs(want)
+                assert np.all(np.abs(got - want) <= L * 2.0 ** -24 * scale * 1.01)
+    x = rng.standard_normal((rows, L)).astype(np.float32)
+    for i, v in enumerate((np.nan, np.inf, -np.inf)):
+        x[i::7, (3 * i) % L] = v
+    arr = vk.Array(gpu, data=x)
+    with np.errstate(invalid="ignore"):
+        np.testing.assert_array_equal(np.asarray(arr.maximum(axis=1)), x.max(1))
+        np.testing.assert_array_equal(np.asarray(arr.minimum(axis=1)), x.min(1))
+        np.testing.assert_array_equal(np.isnan(np.asarray(arr.sum(axis=1))), np.isnan(x.sum(1)))
+
+
+# The same for operands larger than the caches (nontemporal reads; rows up to
+# 96): small whole numbers, so every order gives NumPy's sum.
+@pytest.mark.parametrize("L,rows", [(4, 17000003), (50, 1400001), (75, 900001), (66, 1040000)])
+def test_short_rows_streamed(gpu, L, rows):
+    x = np.random.default_rng(L).integers(-3, 4, (rows, L), dtype=np.int8).astype(np.float32)
+    a = vk.Array(gpu, data=x)
+    np.testing.assert_array_equal(np.asarray(a.sum(axis=1)), x.sum(1))
+    np.testing.assert_array_equal(np.asarray(a.maximum(axis=1)), x.max(1))

@@ -18,10 +18,24 @@
 
 namespace vkh {
 
-// 16 bytes of memory at any 4-byte alignment
+// 16 bytes of memory at any 4-byte alignment. NT: nontemporal, which streams an
+// operand larger than the caches (256 MB) about 10% faster and reads one that
+// they hold slower: column sums of 200000 x 999 134 / 148 us (with / without),
+// of 200000 x 17 12.8 / 9.1, rows of 100 x 100000 28 / 18.
 typedef __attribute__((ext_vector_type(4), aligned(4))) float f32x4u_t;
+template <bool NT>
 __device__ __forceinline__ f32x4u_t ld4u(const float* p) {
-  return __builtin_nontemporal_load(reinterpret_cast<const f32x4u_t*>(p));
+  if constexpr (NT) return __builtin_nontemporal_load(reinterpret_cast<const f32x4u_t*>(p));
+  return *reinterpret_cast<const f32x4u_t*>(p);
+}
+static bool streams(uint64_t elements) { return elements > (uint64_t(256) << 20) / sizeof(float); }
+
+// 16 bytes of global memory straight into LDS (lane i's at dst + 16 i)
+template <bool NT>
+__device__ __forceinline__ void load_lds16(const float* src, float* dst) {
+#ifdef __HIP_DEVICE_COMPILE__  // (the host pass would drop the launch stub of a template that uses the builtin)
+  __builtin_amdgcn_global_load_lds(src, dst, 16, 0, NT ? 2 : 0);  // (2: nt)
+#endif
 }
 
 template <int OP, typename T>
@@ -83,7 +97,7 @@ constexpr int ROW_BLOCK = 256;
 // U: 128-bit loads in flight per thread (4 or 8); each thread still combines
 // its elements in index order, so U never changes the result
 // (rows of any alignment: 16-byte groups, then the last L % 4 elements)
-template <int OP, int U>
+template <int OP, int U, bool NT>
 __global__ void __launch_bounds__(ROW_BLOCK)
 k_rows_block(const float* a, float* out, uint64_t rows, uint64_t L, int rebroadcast, float mul, float dv) {
   __shared__ float lds[ROW_BLOCK / 64];
@@ -97,12 +111,12 @@ k_rows_block(const float* a, float* out, uint64_t rows, uint64_t L, int rebroadc
     for (; i + (U - 1) * ROW_BLOCK < L4; i += U * ROW_BLOCK) {
       f32x4u_t v[U];
 #pragma unroll
-      for (int q = 0; q < U; ++q) v[q] = ld4u(row + 4 * (i + q * ROW_BLOCK));
+      for (int q = 0; q < U; ++q) v[q] = ld4u<NT>(row + 4 * (i + q * ROW_BLOCK));
 #pragma unroll
       for (int q = 0; q < U; ++q) acc = R::f(acc, R::f(R::f(v[q][0], v[q][1]), R::f(v[q][2], v[q][3])));
     }
     for (; i < L4; i += ROW_BLOCK) {
-      const f32x4u_t v = ld4u(row + 4 * i);
+      const f32x4u_t v = ld4u<NT>(row + 4 * i);
       acc = R::f(acc, R::f(R::f(v[0], v[1]), R::f(v[2], v[3])));
     }
     if (threadIdx.x < L % 4) acc = R::f(acc, row[4 * L4 + threadIdx.x]);
@@ -122,8 +136,10 @@ k_rows_block(const float* a, float* out, uint64_t rows, uint64_t L, int rebroadc
 // NV 16-byte groups, all loaded before the first is combined (any alignment);
 // the last L % 4 elements go to the row's first lanes.  With a wave a row and
 // 4-byte loads 1500000 x 75 took 224 us, the second step of every row with 11 of
-// 64 lanes; 102 now (84 for 76 columns), 50000 x 999 29 against 41.
-template <int OP, int LPR, int NV>
+// 64 lanes; 77 now, 50000 x 999 29 against 41.  LINES: rows of whole 128-byte
+// lines are read nontemporally (1500000 x 64 57 us, 64 without); a line that two
+// rows share would then come from memory twice (1500000 x 75 102).
+template <int OP, int LPR, int NV, bool LINES>
 __global__ void __launch_bounds__(256)
 k_rows_lanes(const float* a, float* out, uint64_t rows, uint32_t L, int rebroadcast, float mul, float dv) {
   using R = Red<OP, float>;
@@ -136,7 +152,8 @@ k_rows_lanes(const float* a, float* out, uint64_t rows, uint32_t L, int rebroadc
     float acc = R::init();
 #pragma unroll
     for (int q = 0; q < NV; ++q)
-      if (li + q * LPR < L4) v[q] = ld4u(row + 4 * (li + q * LPR));
+      if (li + q * LPR < L4)
+        v[q] = ld4u<LINES>(row + 4 * (li + q * LPR));
     const bool tail = 4 * L4 + li < L;
     const float tv = tail ? row[4 * L4 + li] : 0.f;
 #pragma unroll
@@ -172,45 +189,6 @@ k_rows_thread(const float* a, float* out, uint64_t rows, uint64_t L, int rebroad
   }
 }
 
-// the same sums, in the same order, for rows of 4 to 63 elements: a block's 256
-// rows come through LDS as one contiguous run (16 bytes a lane; a thread
-// walking its own row in memory touches a cache line a step), at an odd pitch
-// so that the 64 rows of a wave's step are in 64 banks.  1000000 x 16 12 against
-// 36 us, 200000 x 17 6 against 9.
-template <int OP>
-__global__ void __launch_bounds__(256)
-k_rows_short(const float* a, float* out, uint64_t rows, FastDiv L, float mul, float dv) {
-  extern __shared__ float sh[];
-  const uint32_t len = L.d, pitch = len | 1;
-  for (uint64_t r0 = (uint64_t)blockIdx.x * 256; r0 < rows; r0 += (uint64_t)gridDim.x * 256) {
-    const uint32_t nr = (uint32_t)min<uint64_t>(256, rows - r0), n = nr * len;
-    const float* src = a + r0 * len;
-    for (uint32_t i = threadIdx.x * 4; i < n; i += 1024) {
-      f32x4u_t v;
-      if (i + 3 < n) {
-        v = ld4u(src + i);
-      } else {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) v[q] = i + q < n ? src[i + q] : 0.f;
-      }
-      uint32_t r = L.div(i), c = i - r * len;
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        if (i + q < n) sh[r * pitch + c] = v[q];
-        if (++c == len) { c = 0; ++r; }
-      }
-    }
-    __syncthreads();
-    if (threadIdx.x < nr) {
-      const float* row = sh + threadIdx.x * pitch;
-      float acc = row[0];
-      for (uint32_t i = 1; i < len; ++i) acc = Red<OP, float>::f(acc, row[i]);
-      out[r0 + threadIdx.x] = epilogue(acc, mul, dv);
-    }
-    __syncthreads();
-  }
-}
-
 // ---- strided axes: post > 1 ------------------------------------------------------
 // k_cols: a viewed as [prev, K, post]; thread owns VW consecutive columns j of one p
 // and reduces k in [k0, k1) sequentially.  Result goes to dst[(c * prev + p) *
@@ -220,7 +198,7 @@ k_rows_short(const float* a, float* out, uint64_t rows, FastDiv L, float mul, fl
 // with the group before are written twice, with the same values), at any
 // alignment; VW = 1 is for fewer than 4 columns and where groups of 4 would
 // leave fewer than 64 K threads (2000 x 2047: 13 us by fours).
-template <int OP, int VW, int U>
+template <int OP, int VW, int U, bool NT>
 __global__ void __launch_bounds__(256)
 k_cols(const float* a, float* dst, uint64_t prev, uint64_t K, uint64_t post, uint64_t kchunk,
        int final_pass, float mul, float dv) {
@@ -239,17 +217,17 @@ k_cols(const float* a, float* dst, uint64_t prev, uint64_t K, uint64_t post, uin
 #pragma unroll
         for (int q = 0; q < 4; ++q) acc[q] = R::f(acc[q], v[q]);
       };
-      f32x4u_t acc = ld4u(base + k0 * post);
+      f32x4u_t acc = ld4u<NT>(base + k0 * post);
       uint64_t k = k0 + 1;
       // U rows in flight, still combined in row order
       for (; k + (U - 1) < k1; k += U) {
         f32x4u_t v[U];
 #pragma unroll
-        for (int q = 0; q < U; ++q) v[q] = ld4u(base + (k + q) * post);
+        for (int q = 0; q < U; ++q) v[q] = ld4u<NT>(base + (k + q) * post);
 #pragma unroll
         for (int q = 0; q < U; ++q) comb(acc, v[q]);
       }
-      for (; k < k1; ++k) comb(acc, ld4u(base + k * post));
+      for (; k < k1; ++k) comb(acc, ld4u<NT>(base + k * post));
       if (final_pass)
 #pragma unroll
         for (int q = 0; q < 4; ++q) acc[q] = epilogue(acc[q], mul, dv);
@@ -271,6 +249,90 @@ k_cols(const float* a, float* dst, uint64_t prev, uint64_t K, uint64_t post, uin
   }
 }
 
+// Rows of 4 to ROWS_TILE_L elements: a wave takes 64 rows at a time straight into
+// its own LDS (contiguous memory: whole aligned lines at any row length, and no
+// registers for what is in flight), then each lane reduces a row, VW elements an
+// LDS read, into eight accumulators (VW = 4: two reads') that are combined in
+// pairs. ROT: lane l starts at its row's read l, where rows would start
+// on the same banks.  HBM-bound: 2000000 x 32 38 us, 1000000 x 50 29 (58 both for
+// a block's 256 rows through registers to LDS and a barrier), 4000000 x 5 16 (21).
+// From 16 elements a row on and under 64 rows a CU, too few waves have rows and
+// k_rows_lanes takes them: 500 x 63 4.9 against 7.8, 16000 x 63 5.1 against 12.
+// Rows of 64 to 96 come here where the operand is larger than the caches (NT)
+// and rows are not whole lines: 1500000 x 75 after the kernel that wrote it 78 us
+// and the next kernel 90; k_rows_lanes takes 106 and 82 with nontemporal
+// loads, 78 and 108 without.
+constexpr uint32_t ROWS_TILE_L = 63, ROWS_TILE_L_NT = 96;
+template <int OP, int VW, bool ROT, bool NT>
+__global__ void __launch_bounds__(256)
+k_rows_tile(const float* a, float* out, uint64_t rows, uint32_t L, float mul, float dv) {
+  using Rd = Red<OP, float>;
+  extern __shared__ __attribute__((aligned(16))) float tile_lds[];
+  constexpr int A = 8 / VW;  // reads in flight with accumulators of their own
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  float* t = tile_lds + wave * 64 * L;
+  const uint32_t n4 = 16 * L, U = L / VW;
+  const uint64_t tiles = (rows + 63) / 64;
+  const bool aligned = ((uintptr_t)a & 15u) == 0;
+  for (uint64_t tile = (uint64_t)blockIdx.x * 4 + wave; tile < tiles; tile += (uint64_t)gridDim.x * 4) {
+    const uint32_t nr = (uint32_t)min<uint64_t>(64, rows - tile * 64);
+    const float* src = a + tile * 64 * L;
+    if (nr == 64 && aligned) {
+      for (uint32_t i = 0; i < n4; i += 64)
+        if (i + lane < n4) load_lds16<NT>(src + (uint64_t)(i + lane) * 4, t + i * 4);
+    } else if (nr == 64) {
+      typedef __attribute__((ext_vector_type(4))) float f32x4_t;
+#pragma unroll 4
+      for (uint32_t i = lane; i < n4; i += 64) *reinterpret_cast<f32x4_t*>(t + i * 4) = ld4u<false>(src + i * 4);
+    } else {
+      for (uint32_t i = lane; i < nr * L; i += 64) t[i] = src[i];
+    }
+    __builtin_amdgcn_s_waitcnt(0);  // (a wave's own LDS: no barrier)
+    __builtin_amdgcn_wave_barrier();
+    if ((uint32_t)lane < nr) {
+      typedef __attribute__((ext_vector_type(VW))) float vec_t;
+      const vec_t* row = reinterpret_cast<const vec_t*>(t + lane * L);
+      uint32_t e = ROT ? lane % U : 0;
+      auto next = [&]() __attribute__((always_inline)) {
+        const vec_t v = row[e];
+        ++e;
+        if (ROT && e == U) e = 0;
+        return v;
+      };
+      vec_t acc[A];
+      auto fold = [&](vec_t& x, vec_t y) __attribute__((always_inline)) {
+        if constexpr (VW == 1) {
+          x = Rd::f(x[0], y[0]);
+        } else {
+#pragma unroll
+          for (int w = 0; w < VW; ++w) x[w] = Rd::f(x[w], y[w]);
+        }
+      };
+      uint32_t k = min(U, (uint32_t)A);
+#pragma unroll
+      for (int q = 0; q < A; ++q)
+        if (q < (int)k) acc[q] = next();
+      for (; k + A <= U; k += A)
+#pragma unroll
+        for (int q = 0; q < A; ++q) fold(acc[q], next());
+#pragma unroll
+      for (int q = 0; q < A; ++q)
+        if (k + q < U) fold(acc[q], next());
+#pragma unroll
+      for (int h = A / 2; h >= 1; h /= 2)
+#pragma unroll
+        for (int q = 0; q < h; ++q)
+          if (q + h < (int)min(U, (uint32_t)A)) fold(acc[q], acc[q + h]);
+      float r = acc[0][0];
+      if constexpr (VW == 2) r = Rd::f(r, acc[0][1]);
+      if constexpr (VW == 4) r = Rd::f(Rd::f(r, acc[0][1]), Rd::f(acc[0][2], acc[0][3]));
+      out[tile * 64 + lane] = epilogue(r, mul, dv);
+    }
+    __builtin_amdgcn_s_waitcnt(0);  // the reads are done before the next rows arrive
+    __builtin_amdgcn_wave_barrier();
+  }
+}
+
 // Few columns: a block takes whole rows, thread t column group t % G of rows
 // t / G, + R, + 2R ... of its chunk, so that a block reads its chunk as one
 // contiguous run; the R sums of a column are then combined by a tree in LDS.
@@ -280,7 +342,7 @@ k_cols(const float* a, float* dst, uint64_t prev, uint64_t K, uint64_t post, uin
 // it: 1000000 x 16 18 against 161 us, 3000000 x 3 11 against 371, 1500000 x 75
 // 78 against 678, 50000 x 999 44 against 120 (element loads), 50000 x 1000 43
 // against 60 (87 with one last pass over all 1024 chunks).
-template <int OP, int VW, int U>
+template <int OP, int VW, int U, bool NT>
 __global__ void __launch_bounds__(256)
 k_cols_narrow(const float* a, float* dst, uint64_t K, uint32_t post, uint64_t kchunk, uint32_t G, uint32_t R,
               int final_pass, float mul, float dv, float beta) {
@@ -295,7 +357,7 @@ k_cols_narrow(const float* a, float* dst, uint64_t K, uint32_t post, uint64_t kc
   auto load = [&](uint64_t k, float (&v)[VW]) {
     const float* q = a + (p * K + k) * post + j;
     if constexpr (VW == 4) {
-      const f32x4u_t t = ld4u(q);
+      const f32x4u_t t = ld4u<NT>(q);
       v[0] = t[0]; v[1] = t[1]; v[2] = t[2]; v[3] = t[3];
     } else {
       v[0] = *q;
@@ -582,12 +644,10 @@ static void reduce_cols_narrow(vkh_gpu* g, const float* a, float* out, uint64_t 
   nchunk = ceil_div(K, kchunk);
   auto launch = [&](const float* src, float* dst, uint64_t k, uint64_t kc, uint64_t nc, int fin) {
     const dim3 grid((unsigned)nc, (unsigned)prev);
-    if (post >= 4)
-      hipLaunchKernelGGL((k_cols_narrow<OP, 4, 8>), grid, dim3(256), 0, g->stream, src, dst, k, (uint32_t)post, kc, G, R,
-                         fin, mul, dv, fin ? beta : 0.f);
-    else
-      hipLaunchKernelGGL((k_cols_narrow<OP, 1, 8>), grid, dim3(256), 0, g->stream, src, dst, k, (uint32_t)post, kc, G, R,
-                         fin, mul, dv, fin ? beta : 0.f);
+    auto kernel = post < 4 ? k_cols_narrow<OP, 1, 8, false>
+                           : (streams(prev * K * post) ? k_cols_narrow<OP, 4, 8, true> : k_cols_narrow<OP, 4, 8, false>);
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, g->stream, src, dst, k, (uint32_t)post, kc, G, R, fin, mul, dv,
+                       fin ? beta : 0.f);
     check_launch("reduce cols (narrow)");
   };
   if (nchunk == 1) {
@@ -608,26 +668,43 @@ static void reduce_axis(vkh_gpu* g, const float* a, float* out, uint64_t prev, u
     const uint64_t rows = prev, L = K;
     if (L >= ROWS_BLOCK_MIN_L) {
       unsigned grid = (unsigned)std::min<uint64_t>(rows, (uint64_t)cus * cfg.par);
-      if (cfg.unroll == 8)
-        hipLaunchKernelGGL((k_rows_block<OP, 8>), dim3(grid), dim3(ROW_BLOCK), 0, g->stream, a, out, rows, L, rebroadcast, mul, dv);
-      else
-        hipLaunchKernelGGL((k_rows_block<OP, 4>), dim3(grid), dim3(ROW_BLOCK), 0, g->stream, a, out, rows, L, rebroadcast, mul, dv);
-    } else if (L >= 64) {
+      auto kernel = cfg.unroll == 8 ? (streams(rows * L) ? k_rows_block<OP, 8, true> : k_rows_block<OP, 8, false>)
+                                    : (streams(rows * L) ? k_rows_block<OP, 4, true> : k_rows_block<OP, 4, false>);
+      hipLaunchKernelGGL(kernel, dim3(grid), dim3(ROW_BLOCK), 0, g->stream, a, out, rows, L, rebroadcast, mul, dv);
+    } else if (L >= 4 && !rebroadcast &&
+               (L <= ROWS_TILE_L ? L < 16 || rows >= (uint64_t)cus * 64
+                                 : L <= ROWS_TILE_L_NT && L % 32 != 0 && streams(rows * L))) {
+      const uint32_t vw = L % 4 == 0 ? 4 : (L % 2 == 0 ? 2 : 1);
+      const size_t sh = sizeof(float) * 256 * L;
+      const unsigned grid = (unsigned)std::min<uint64_t>(ceil_div(rows, 256), (uint64_t)cus * 8);
+      auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), sh, g->stream, a, out, rows, (uint32_t)L, mul, dv);
+      };
+      const bool rot = (L / vw) % 2 == 0, nt = streams(rows * L);
+#define VKH_ROWS_TILE(VW, ROT) \
+  do { if (nt) launch(k_rows_tile<OP, VW, ROT, true>); else launch(k_rows_tile<OP, VW, ROT, false>); } while (0)
+      if (vw == 4 && rot) VKH_ROWS_TILE(4, true);
+      else if (vw == 4) VKH_ROWS_TILE(4, false);
+      else if (vw == 2 && rot) VKH_ROWS_TILE(2, true);
+      else if (vw == 2) VKH_ROWS_TILE(2, false);
+      else VKH_ROWS_TILE(1, false);
+#undef VKH_ROWS_TILE
+    } else if (L >= 64 || (L >= 16 && !rebroadcast)) {
       // lanes a row: up to 4 groups a lane, 8 of a whole wave
       auto launch = [&](auto kernel, int lpr) {
         const unsigned grid = (unsigned)std::min<uint64_t>(ceil_div(rows, 256 / lpr), (uint64_t)cus * 64);
         hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), 0, g->stream, a, out, rows, (uint32_t)L, rebroadcast, mul, dv);
       };
       const uint64_t L4 = L / 4;
-      if (L4 <= 32) launch(k_rows_lanes<OP, 8, 4>, 8);
-      else if (L4 <= 64) launch(k_rows_lanes<OP, 16, 4>, 16);
-      else if (L4 <= 128) launch(k_rows_lanes<OP, 32, 4>, 32);
-      else if (L4 <= 256) launch(k_rows_lanes<OP, 64, 4>, 64);
-      else launch(k_rows_lanes<OP, 64, 8>, 64);
-    } else if (L >= 4 && !rebroadcast) {
-      const size_t sh = sizeof(float) * 256 * (L | 1);
-      unsigned grid = (unsigned)std::min<uint64_t>(ceil_div(rows, 256), (uint64_t)cus * 16);
-      hipLaunchKernelGGL(k_rows_short<OP>, dim3(grid), dim3(256), sh, g->stream, a, out, rows, FastDiv((uint32_t)L), mul, dv);
+      const bool lines = L % 32 == 0 && ((uintptr_t)a & 127u) == 0;
+#define VKH_ROWS_LANES(LPR, NV) \
+  do { if (lines) launch(k_rows_lanes<OP, LPR, NV, true>, LPR); else launch(k_rows_lanes<OP, LPR, NV, false>, LPR); } while (0)
+      if (L4 <= 32) VKH_ROWS_LANES(8, 4);
+      else if (L4 <= 64) VKH_ROWS_LANES(16, 4);
+      else if (L4 <= 128) VKH_ROWS_LANES(32, 4);
+      else if (L4 <= 256) VKH_ROWS_LANES(64, 4);
+      else VKH_ROWS_LANES(64, 8);
+#undef VKH_ROWS_LANES
     } else {
       unsigned grid = (unsigned)std::min<uint64_t>(ceil_div(rows, 256), (uint64_t)cus * 16);
       hipLaunchKernelGGL(k_rows_thread<OP>, dim3(grid), dim3(256), 0, g->stream, a, out, rows, L, rebroadcast, mul, dv);
@@ -658,12 +735,11 @@ static void reduce_axis(vkh_gpu* g, const float* a, float* out, uint64_t prev, u
   if (gx < 1) gx = 1;
   dim3 grid(gx, (unsigned)nchunk);
   const int final_pass = (nchunk == 1) ? 1 : 0;
-  if (quads && cfg.unroll == 8)
-    hipLaunchKernelGGL((k_cols<OP, 4, 8>), grid, dim3(256), 0, g->stream, a, dst, prev, K, post, kchunk, final_pass, mul, dv);
-  else if (quads)
-    hipLaunchKernelGGL((k_cols<OP, 4, 4>), grid, dim3(256), 0, g->stream, a, dst, prev, K, post, kchunk, final_pass, mul, dv);
-  else
-    hipLaunchKernelGGL((k_cols<OP, 1, 8>), grid, dim3(256), 0, g->stream, a, dst, prev, K, post, kchunk, final_pass, mul, dv);
+  const bool nt = streams(prev * K * post);
+  auto kernel = !quads ? k_cols<OP, 1, 8, false>
+                : cfg.unroll == 8 ? (nt ? k_cols<OP, 4, 8, true> : k_cols<OP, 4, 8, false>)
+                                  : (nt ? k_cols<OP, 4, 4, true> : k_cols<OP, 4, 4, false>);
+  hipLaunchKernelGGL(kernel, grid, dim3(256), 0, g->stream, a, dst, prev, K, post, kchunk, final_pass, mul, dv);
   check_launch("reduce cols");
   float* red = dst;
   if (nchunk > 1) {
