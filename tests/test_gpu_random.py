@@ -163,3 +163,27 @@ def test_henormal_shape_chunked(gpu):
     assert np.all(np.abs(got - want) <= 4 * np.spacing(np.abs(want) + np.float32(0.0))
                   + 4 * np.spacing(np.float32(0.02))), np.abs(got - want).max()
     np.testing.assert_array_equal(r.state(), o.state)
+
+
+# Long draws from few states are cut into chunks that start from matrix powers
+# of the state (one matrix for each hexadecimal digit of the chunk's number; a block a
+# chunk from 64 states, or 16 where few chunks suffice, on). The outputs and the
+# states left behind equal those of short draws, which walk the states.
+@pytest.mark.parametrize("S,steps", [(1, 300), (1, 70000), (2, 5000), (15, 2500), (16, 2300), (32, 40000), (34, 12345),
+                                     (63, 1111), (64, 255), (64, 256), (64, 4200), (130, 20000), (1000, 513),
+                                     (4822, 300)])
+def test_chunks_continue_the_states(gpu, S, steps):
+    for kind, piece in (("u32", 200), ("normal", 100)):
+        whole, parts = (vk.random.Xoshiro128pp(gpu, size=S, seed=S + steps) for _ in range(2))
+
+        def draw(r, n):
+            return np.asarray(r.randint(shape=(n,)) if kind == "u32" else r.normal(shape=(n,)))
+        if kind == "normal" and S % 2:
+            continue  # (an odd number of states draws uniforms first)
+        n = S * steps + (S // 2 if kind == "u32" else 0)
+        got = draw(whole, n)
+        cuts = [S * piece] * (n // (S * piece)) + [n % (S * piece)]
+        want = np.concatenate([draw(parts, c) for c in cuts if c])
+        np.testing.assert_array_equal(got.view(np.uint32), want.view(np.uint32))
+        if n % S == 0:  # the next draw starts from the states as they were left
+            np.testing.assert_array_equal(draw(whole, S * 3), draw(parts, S * 3))

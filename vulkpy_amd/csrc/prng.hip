@@ -68,11 +68,36 @@ static St mat_apply(const Mat& M, const St& x) {
   return y;
 }
 
-static Mat compose(const Mat& A, const Mat& B) {  // A after B
-  Mat C;
-  for (int k = 0; k < 128; ++k) C[k] = mat_apply(A, B[k]);
-  return C;
-}
+// A's images of every byte at every place, for many products with A: 16 table
+// look-ups a vector instead of a test of 128 bits
+struct ByteTable {
+  std::vector<St> t;  // [16][256]
+  explicit ByteTable(const Mat& A) : t(16 * 256) {
+    for (int b = 0; b < 16; ++b) {
+      St* u = &t[b * 256];
+      u[0] = St{{0, 0, 0, 0}};
+      for (int v = 1; v < 256; ++v) {
+        const St& c = A[8 * b + __builtin_ctz(v)];
+        for (int q = 0; q < 4; ++q) u[v].w[q] = u[v & (v - 1)].w[q] ^ c.w[q];
+      }
+    }
+  }
+  St apply(const St& x) const {
+    St y{{0, 0, 0, 0}};
+    for (int b = 0; b < 16; ++b) {
+      const St& c = t[b * 256 + ((x.w[b >> 2] >> (8 * (b & 3))) & 255u)];
+      for (int q = 0; q < 4; ++q) y.w[q] ^= c.w[q];
+    }
+    return y;
+  }
+  Mat after(const Mat& B) const {  // A after B
+    Mat C;
+    for (int k = 0; k < 128; ++k) C[k] = apply(B[k]);
+    return C;
+  }
+};
+
+static Mat compose(const Mat& A, const Mat& B) { return ByteTable(A).after(B); }  // A after B
 
 static Mat identity() {
   Mat I;
@@ -117,30 +142,35 @@ static Mat step_matrix() {
   return M;
 }
 
-// P_j = M^(Lc * 2^j), j < nbits, as [nbits][128 columns][4 words].  Kept
-// per chunk length for the life of the process (generators made by the
-// same initializer shapes share chunk lengths).
-static void chunk_jumps(uint64_t Lc, int nbits, std::vector<uint32_t>& out) {
+// M^(Lc * d * 16^j), j < ndigits, d = 1 .. 15, as [ndigits][15][128 columns][4
+// words]: the start of chunk c takes one product for each hexadecimal digit of
+// c that is not 0.  Kept per chunk length (generators made by the same
+// initializer shapes share them), the last 32 lengths.
+static void chunk_jumps(uint64_t Lc, int ndigits, std::vector<uint32_t>& out) {
   static std::mutex mu;
   static std::unordered_map<uint64_t, std::vector<uint32_t>> cache;
   std::lock_guard<std::mutex> lock(mu);
+  if (cache.size() >= 32 && !cache.count(Lc)) cache.clear();
   std::vector<uint32_t>& v = cache[Lc];
-  int have = (int)(v.size() / 512);
-  if (have < nbits) {
+  constexpr size_t DIGIT = 15 * 512;
+  auto put = [&](int j, int d, const Mat& P) {
+    for (int k = 0; k < 128; ++k) std::memcpy(&v[j * DIGIT + (size_t)(d - 1) * 512 + 4 * k], P[k].w, 16);
+  };
+  auto get = [&](int j, int d) {
     Mat P;
-    if (have == 0) {
-      P = mat_pow(step_matrix(), Lc);
-    } else {
-      for (int k = 0; k < 128; ++k) std::memcpy(P[k].w, &v[((size_t)(have - 1) * 128 + k) * 4], 16);
-      P = compose(P, P);
-    }
-    v.resize((size_t)nbits * 512);
-    for (int j = have; j < nbits; ++j) {
-      if (j > have) P = compose(P, P);
-      for (int k = 0; k < 128; ++k) std::memcpy(&v[((size_t)j * 128 + k) * 4], P[k].w, 16);
-    }
+    for (int k = 0; k < 128; ++k) std::memcpy(P[k].w, &v[j * DIGIT + (size_t)(d - 1) * 512 + 4 * k], 16);
+    return P;
+  };
+  const int have = (int)(v.size() / DIGIT);
+  if (have < ndigits) v.resize(ndigits * DIGIT);
+  for (int j = have; j < ndigits; ++j) {
+    const Mat one = j == 0 ? mat_pow(step_matrix(), Lc) : compose(get(j - 1, 1), get(j - 1, 15));
+    const ByteTable t(one);
+    Mat P = one;
+    put(j, 1, P);
+    for (int d = 2; d < 16; ++d) put(j, d, P = t.after(P));
   }
-  out.assign(v.begin(), v.begin() + (size_t)nbits * 512);
+  out.assign(v.begin(), v.begin() + ndigits * DIGIT);
 }
 
 static void seed_states(uint32_t S, uint64_t seed, std::vector<uint32_t>& out) {
@@ -196,8 +226,18 @@ __device__ __forceinline__ float to_unit(uint32_t r) {
 
 constexpr int PRNG_BLOCK = 256;
 
+// NT: nontemporal stores, where the states' outputs of a step are whole 128-byte
+// lines (2^20 states, 2^28 outputs 201 us, 212 without, 2^22 6.7 and 7.5);
+// elsewhere they would write lines in parts (65534 states, 2^26 outputs 104 us,
+// 51 without, 500 states, 2^27 243 and 185).
+template <bool NT, typename T>
+__device__ __forceinline__ void store_out(T* p, T v) {
+  if constexpr (NT) __builtin_nontemporal_store(v, p);
+  else *p = v;
+}
+
 // OUT: 0 = uint32, 1 = float in [0, 1), 2 = randrange
-template <int OUT>
+template <int OUT, bool NT>
 __global__ void __launch_bounds__(PRNG_BLOCK)
 k_xoshiro(uint4* state, void* out, uint32_t S, uint64_t n, uint32_t low, uint32_t range) {
   const uint64_t i = (uint64_t)blockIdx.x * PRNG_BLOCK + threadIdx.x;
@@ -205,12 +245,12 @@ k_xoshiro(uint4* state, void* out, uint32_t S, uint64_t n, uint32_t low, uint32_
   uint4 s = state[i];
   for (uint64_t k = i; k < n; k += S) {
     const uint32_t r = dnext(s);
-    if (OUT == 0) st_stream1(static_cast<uint32_t*>(out) + k, r);
-    else if (OUT == 1) st_stream1(static_cast<float*>(out) + k, to_unit(r));
+    if (OUT == 0) store_out<NT>(static_cast<uint32_t*>(out) + k, r);
+    else if (OUT == 1) store_out<NT>(static_cast<float*>(out) + k, to_unit(r));
     else {
       // prng_randrange.comp:24-26: low + uint(float(range) * u)
       const float u = to_unit(r);
-      st_stream1(static_cast<uint32_t*>(out) + k, low + __float2uint_rz((float)range * u));
+      store_out<NT>(static_cast<uint32_t*>(out) + k, low + __float2uint_rz((float)range * u));
     }
   }
   state[i] = s;
@@ -221,10 +261,16 @@ k_xoshiro(uint4* state, void* out, uint32_t S, uint64_t n, uint32_t low, uint32_
 // steps; when S is small (the reference's HeNormal uses 64 states,
 // nn/initializers.py:75-89) that serial chain is the whole kernel.  Here
 // thread (i, c) produces steps [c*Lc, (c+1)*Lc) of state i: it starts from
-// M^(c*Lc) applied to the state (M = one next() step over GF(2)), built
-// from the precomputed P_j = M^(Lc * 2^j) for the set bits j of c.  Outputs
+// M^(c*Lc) applied to the state (M = one next() step over GF(2)), one
+// precomputed matrix M^(Lc * d * 16^j) for each hexadecimal digit d of c.  Outputs
 // keep the mapping k = t*S + i.  Start states are read from a copy of the
 // state buffer; the chunk holding a state's last step writes it back.
+// UNI (64 states, or pairs, and more): a block has one c, so the matrices come
+// by scalar loads, many columns ahead, and each column is a mask and four
+// ands and xors.  With a matrix for each bit of c, every column a branch and a
+// load, a start took longer than 256 steps. 64 states, 2^20 outputs 51 -> 14 us
+// (normal 138 -> 33), 4822 states, 12.2 million 45 -> 22 (125 -> 45), 64 states, 2^24
+// 75 -> 26 (188 -> 69). The matrices of a new chunk length take the host 0.1 ms (0.5).
 
 // y = P x for a 128x128 bit matrix given by its columns (4 words each)
 __device__ __forceinline__ uint4 gf2_apply(const uint32_t* __restrict__ P, uint4 x) {
@@ -232,22 +278,32 @@ __device__ __forceinline__ uint4 gf2_apply(const uint32_t* __restrict__ P, uint4
   const uint32_t w[4] = {x.x, x.y, x.z, x.w};
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
+#pragma unroll 8
     for (int b = 0; b < 32; ++b) {
-      if ((w[q] >> b) & 1u) {
-        const uint32_t* col = P + (q * 32 + b) * 4;
-        y.x ^= col[0]; y.y ^= col[1]; y.z ^= col[2]; y.w ^= col[3];
-      }
+      const uint4 col = *reinterpret_cast<const uint4*>(P + (q * 32 + b) * 4);
+      const uint32_t m = 0u - ((w[q] >> b) & 1u);
+      y.x ^= col.x & m; y.y ^= col.y & m; y.z ^= col.z & m; y.w ^= col.w & m;
     }
   }
   return y;
 }
 
-__device__ __forceinline__ uint4 chunk_start(const uint4* init, const uint32_t* jumps, uint64_t i,
-                                             uint64_t c) {
-  uint4 s = init[i];
-  for (int j = 0; (c >> j) != 0; ++j)
-    if ((c >> j) & 1u) s = gf2_apply(jumps + (size_t)j * 512, s);
+__device__ __forceinline__ uint4 chunk_start(uint4 s, const uint32_t* jumps, uint64_t c) {
+  for (int j = 0; (c >> (4 * j)) != 0; ++j) {
+    const uint32_t d = (uint32_t)(c >> (4 * j)) & 15u;
+    if (d) s = gf2_apply(jumps + ((size_t)j * 15 + d - 1) * 512, s);
+  }
   return s;
+}
+
+// the state (pair) and the chunk of a thread: UNI as a grid of blocks by chunks,
+// otherwise one after the other
+template <bool UNI>
+__device__ __forceinline__ bool chunk_of(uint64_t units, uint64_t nchunks, uint64_t& u, uint64_t& c) {
+  const uint64_t tid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  u = UNI ? tid : tid % units;
+  c = UNI ? blockIdx.y : tid / units;
+  return UNI ? tid < units : c < nchunks;
 }
 
 // steps of state i when n outputs are taken round-robin from S states
@@ -255,24 +311,23 @@ __device__ __forceinline__ uint64_t steps_of(uint64_t i, uint64_t S, uint64_t n)
   return n > i ? (n - 1 - i) / S + 1 : 0;
 }
 
-template <int OUT>
+template <int OUT, bool UNI, bool NT>
 __global__ void __launch_bounds__(PRNG_BLOCK)
 k_xoshiro_chunked(const uint4* init, uint4* state, const uint32_t* jumps, void* out, uint32_t S,
                   uint64_t n, uint64_t Lc, uint64_t nchunks, uint32_t low, uint32_t range) {
-  const uint64_t tid = (uint64_t)blockIdx.x * PRNG_BLOCK + threadIdx.x;
-  if (tid >= (uint64_t)S * nchunks) return;
-  const uint64_t i = tid % S, c = tid / S;
+  uint64_t i, c;
+  if (!chunk_of<UNI>(S, nchunks, i, c)) return;
   const uint64_t L = steps_of(i, S, n);
   const uint64_t t0 = c * Lc;
   if (t0 >= L) return;
   const uint64_t t1 = min(t0 + Lc, L);
-  uint4 s = chunk_start(init, jumps, i, c);
+  uint4 s = chunk_start(init[i], jumps, c);
   for (uint64_t t = t0; t < t1; ++t) {
     const uint64_t k = t * S + i;
     const uint32_t r = dnext(s);
-    if (OUT == 0) st_stream1(static_cast<uint32_t*>(out) + k, r);
-    else if (OUT == 1) st_stream1(static_cast<float*>(out) + k, to_unit(r));
-    else st_stream1(static_cast<uint32_t*>(out) + k, low + __float2uint_rz((float)range * to_unit(r)));
+    if (OUT == 0) store_out<NT>(static_cast<uint32_t*>(out) + k, r);
+    else if (OUT == 1) store_out<NT>(static_cast<float*>(out) + k, to_unit(r));
+    else store_out<NT>(static_cast<uint32_t*>(out) + k, low + __float2uint_rz((float)range * to_unit(r)));
   }
   if (t1 == L) state[i] = s;
 }
@@ -321,21 +376,22 @@ __device__ __forceinline__ void box_muller(float u1, float u2, float mean, float
 typedef float vkh_f2v __attribute__((ext_vector_type(2)));
 
 // out[j] (j < n) and out[j + 1] (j + 1 < n) of a normal pair; one 8-byte
-// nontemporal store when both are in range and out + j is 8-byte aligned
+// store when both are in range and out + j is 8-byte aligned
+template <bool NT>
 __device__ __forceinline__ void store_pair(float* out, uint64_t j, uint64_t n, float o1, float o2) {
   if (j + 1 < n && ((uintptr_t)(out + j) & 7u) == 0) {
     const vkh_f2v v = {o1, o2};
-    __builtin_nontemporal_store(v, reinterpret_cast<vkh_f2v*>(out + j));
+    store_out<NT>(reinterpret_cast<vkh_f2v*>(out + j), v);
   } else {
-    if (j < n) st_stream1(out + j, o1);
-    if (j + 1 < n) st_stream1(out + j + 1, o2);
+    if (j < n) store_out<NT>(out + j, o1);
+    if (j + 1 < n) store_out<NT>(out + j + 1, o2);
   }
 }
 
 // Fused uniform + Box-Muller: thread p owns states 2p and 2p+1 (S even) and
 // produces normal pairs at uniform indices j = c*S + 2p < nu (nu even).
 // PAIRED: n == nu and out 8-byte aligned, so every pair is one 8-byte store.
-template <bool PAIRED>
+template <bool PAIRED, bool NT>
 __global__ void __launch_bounds__(PRNG_BLOCK)
 k_xoshiro_normal(uint4* state, float* out, uint32_t S, uint64_t nu, uint64_t n, float mean, float sd) {
   const uint64_t p = (uint64_t)blockIdx.x * PRNG_BLOCK + threadIdx.x;
@@ -349,9 +405,9 @@ k_xoshiro_normal(uint4* state, float* out, uint32_t S, uint64_t nu, uint64_t n, 
     box_muller<true>(u1, u2, mean, sd, o1, o2);
     if constexpr (PAIRED) {
       const vkh_f2v v = {o1, o2};
-      __builtin_nontemporal_store(v, reinterpret_cast<vkh_f2v*>(out + j));
+      store_out<NT>(reinterpret_cast<vkh_f2v*>(out + j), v);
     } else {
-      store_pair(out, j, n, o1, o2);
+      store_pair<NT>(out, j, n, o1, o2);
     }
   }
   state[i] = s1;
@@ -361,26 +417,26 @@ k_xoshiro_normal(uint4* state, float* out, uint32_t S, uint64_t nu, uint64_t n, 
 // chunked form of k_xoshiro_normal: thread (p, c) advances states 2p and 2p+1
 // over steps [c*Lc, (c+1)*Lc); both take the same number of steps because S
 // and nu are even
+template <bool UNI, bool NT>
 __global__ void __launch_bounds__(PRNG_BLOCK)
 k_xoshiro_normal_chunked(const uint4* init, uint4* state, const uint32_t* jumps, float* out,
                          uint32_t S, uint64_t nu, uint64_t n, uint64_t Lc, uint64_t nchunks,
                          float mean, float sd) {
-  const uint64_t tid = (uint64_t)blockIdx.x * PRNG_BLOCK + threadIdx.x;
-  const uint64_t half = S / 2;
-  if (tid >= half * nchunks) return;
-  const uint64_t p = tid % half, c = tid / half, i = 2 * p;
+  uint64_t p, c;
+  if (!chunk_of<UNI>(S / 2, nchunks, p, c)) return;
+  const uint64_t i = 2 * p;
   const uint64_t L = steps_of(i, S, nu);
   const uint64_t t0 = c * Lc;
   if (t0 >= L) return;
   const uint64_t t1 = min(t0 + Lc, L);
-  uint4 s1 = chunk_start(init, jumps, i, c), s2 = chunk_start(init, jumps, i + 1, c);
+  uint4 s1 = chunk_start(init[i], jumps, c), s2 = chunk_start(init[i + 1], jumps, c);
   for (uint64_t t = t0; t < t1; ++t) {
     const uint64_t j = t * S + i;
     const float u1 = to_unit(dnext(s1));
     const float u2 = to_unit(dnext(s2));
     float o1, o2;
     box_muller<true>(u1, u2, mean, sd, o1, o2);
-    store_pair(out, j, n, o1, o2);
+    store_pair<NT>(out, j, n, o1, o2);
   }
   if (t1 == L) {
     state[i] = s1;
@@ -514,7 +570,7 @@ struct vkh_xoshiro {
   uint32_t* jumps = nullptr;
   size_t jumps_bytes = 0;
   uint64_t jumps_lc = 0;
-  int jumps_nbits = 0;
+  int jumps_ndigits = 0;
 };
 
 using namespace vkh;
@@ -526,33 +582,52 @@ namespace {
 struct ChunkPlan {
   bool use = false;
   uint64_t Lc = 0, C = 1;
-  int nbits = 0;
+  int ndigits = 0;
+  bool uni = false;  // one chunk a block
+  dim3 grid, block;
 };
 
+constexpr uint64_t CHUNK_FULL = 128, CHUNK_MIN = 64, CHUNK_MIN_NORMAL = 32;  // steps of a chunk, at least
+
 // Chunk the per-state chains when `units` parallel chains (states, or state
-// pairs) are too few to fill the GPU and each is long: about 1024 threads
-// per compute unit, and at least 256 steps per chunk so the start-state
-// matrix products stay small next to the generation.  Not during graph
-// capture (the jump matrices are uploaded synchronously).
-ChunkPlan plan_chunks(const vkh_gpu* g, uint64_t units, uint64_t steps) {
+// pairs) are too few to fill the GPU and each is long.  Up to 512 threads per
+// compute unit a chunk may be as short as `least` steps, its start-state products
+// hidden by other waves' work, up to 1024 as CHUNK_FULL; fewer than four chunks
+// do not pay for the copy of the states (65534 states, 2^23 outputs 14.6 us in
+// two chunks, 10.6 without; 64 states, 2^14 outputs 9.5 in four, 11.7).  Under
+// 64 units a block of one chunk has idle lanes, which only pays where the chip
+// has room for every such wave (32 pairs, 2^20 outputs 33 us against 53, 2^28 548
+// against 363).  Not during graph capture (the jump matrices are uploaded
+// synchronously).
+ChunkPlan plan_chunks(const vkh_gpu* g, uint64_t units, uint64_t steps, uint64_t least) {
   ChunkPlan p;
-  if (g->capturing) return p;
-  const uint64_t target = (uint64_t)(g->num_cus > 0 ? g->num_cus : 256) * 1024;
+  if (g->capturing || steps < 4 * least) return p;
+  const uint64_t cus = g->num_cus > 0 ? g->num_cus : 256, target = cus * 1024;
   if (units * 4 >= target) return p;
-  const uint64_t C = std::min<uint64_t>(ceil_div(target, units), steps / 256);
+  const uint64_t full = std::min(ceil_div(target, units), steps / CHUNK_FULL);
+  uint64_t C = std::max(full, std::min(ceil_div(target / 2, units), steps / least));
+  p.uni = units >= 64 ? C < 65536 : units >= 16 && C <= 4 * cus;
+  if (!p.uni) C = full;
   if (C < 2) return p;
   p.Lc = ceil_div(steps, C);
   p.C = ceil_div(steps, p.Lc);
   if (p.C < 2) return p;
   p.use = true;
-  while ((uint64_t(1) << p.nbits) < p.C) ++p.nbits;  // bits of c in [0, C)
+  while (((p.C - 1) >> (4 * p.ndigits)) != 0) ++p.ndigits;  // digits of c < C
+  if (p.uni) {
+    p.block = dim3((unsigned)std::min<uint64_t>(PRNG_BLOCK, ceil_div(units, 64) * 64));
+    p.grid = dim3((unsigned)ceil_div(units, p.block.x), (unsigned)p.C);
+  } else {
+    p.block = dim3(PRNG_BLOCK);
+    p.grid = dim3(prng_grid(units * p.C));
+  }
   return p;
 }
 
 const uint32_t* prepare_jumps(vkh_xoshiro* r, const ChunkPlan& p) {
-  if (r->jumps && r->jumps_lc == p.Lc && r->jumps_nbits >= p.nbits) return r->jumps;
+  if (r->jumps && r->jumps_lc == p.Lc && r->jumps_ndigits >= p.ndigits) return r->jumps;
   std::vector<uint32_t> host;
-  chunk_jumps(p.Lc, p.nbits, host);
+  chunk_jumps(p.Lc, p.ndigits, host);
   const size_t nbytes = host.size() * sizeof(uint32_t);
   vkh_gpu* g = r->gpu;
   if (nbytes > r->jumps_bytes) {
@@ -570,31 +645,39 @@ const uint32_t* prepare_jumps(vkh_xoshiro* r, const ChunkPlan& p) {
   VKH_HIP(hipStreamSynchronize(g->stream));
   VKH_HIP(hipMemcpy(r->jumps, host.data(), nbytes, hipMemcpyHostToDevice));
   r->jumps_lc = p.Lc;
-  r->jumps_nbits = p.nbits;
+  r->jumps_ndigits = p.ndigits;
   return r->jumps;
+}
+
+// the stores of store_out<true>: see there
+bool whole_lines(const vkh_xoshiro* r, const void* out) {
+  return r->size % 32 == 0 && ((uintptr_t)out & 127u) == 0;
 }
 
 template <int OUT>
 void launch_uniform(vkh_xoshiro* r, void* out, uint64_t n, uint32_t low, uint32_t range) {
   vkh_gpu* g = r->gpu;
-  const ChunkPlan cp = plan_chunks(g, r->size, ceil_div(n, r->size));
+  const bool nt = whole_lines(r, out);
+  const ChunkPlan cp = plan_chunks(g, r->size, ceil_div(n, r->size), CHUNK_MIN);
   if (cp.use) {
     const uint32_t* jumps = prepare_jumps(r, cp);
     const size_t sb = (size_t)16 * r->size;
     Workspace init(g, sb);
     VKH_HIP(hipMemcpyAsync(init.get(), r->state, sb, hipMemcpyDeviceToDevice, g->stream));
-    const uint64_t th = (uint64_t)r->size * cp.C;
-    hipLaunchKernelGGL(k_xoshiro_chunked<OUT>, dim3(prng_grid(th)), dim3(PRNG_BLOCK), 0, g->stream,
-                       (const uint4*)init.get(), (uint4*)r->state, jumps, out, r->size, n, cp.Lc, cp.C,
-                       low, range);
+    auto kernel = !cp.uni ? k_xoshiro_chunked<OUT, false, false>
+                  : nt    ? k_xoshiro_chunked<OUT, true, true>
+                          : k_xoshiro_chunked<OUT, true, false>;
+    hipLaunchKernelGGL(kernel, cp.grid, cp.block, 0, g->stream, (const uint4*)init.get(), (uint4*)r->state, jumps, out,
+                       r->size, n, cp.Lc, cp.C, low, range);
   } else {
     // one state per thread (measured 197 us for 2^28 outputs from 2^20 states;
     // four states per thread with 16-byte stores: 232 us; four steps of a
     // block's 256 states staged through LDS so that each wave stores one
     // 1 KB row segment with 16-byte stores: no faster)
     const uint64_t th = std::min<uint64_t>(r->size, n);
-    hipLaunchKernelGGL(k_xoshiro<OUT>, dim3(prng_grid(th)), dim3(PRNG_BLOCK), 0, g->stream,
-                       (uint4*)r->state, out, r->size, n, low, range);
+    auto kernel = nt ? k_xoshiro<OUT, true> : k_xoshiro<OUT, false>;
+    hipLaunchKernelGGL(kernel, dim3(prng_grid(th)), dim3(PRNG_BLOCK), 0, g->stream, (uint4*)r->state, out, r->size, n,
+                       low, range);
   }
   check_launch("xoshiro");
 }
@@ -708,24 +791,25 @@ int vkh_xoshiro_normal(vkh_xoshiro* r, float* out, uint64_t n, float mean, float
     VKH_REQUIRE(out, "null output");
     const uint64_t nu = n + (n & 1);  // random.py:105-123: n even, or n + 1 uniforms
     if (r->size % 2 == 0) {
-      const ChunkPlan cp = plan_chunks(g, r->size / 2, ceil_div(nu, r->size));
+      const bool nt = whole_lines(r, out);
+      const ChunkPlan cp = plan_chunks(g, r->size / 2, ceil_div(nu, r->size), CHUNK_MIN_NORMAL);
       if (cp.use) {
         const uint32_t* jumps = prepare_jumps(r, cp);
         const size_t sb = (size_t)16 * r->size;
         Workspace init(g, sb);
         VKH_HIP(hipMemcpyAsync(init.get(), r->state, sb, hipMemcpyDeviceToDevice, g->stream));
-        const uint64_t th = (uint64_t)(r->size / 2) * cp.C;
-        hipLaunchKernelGGL(k_xoshiro_normal_chunked, dim3(prng_grid(th)), dim3(PRNG_BLOCK), 0, g->stream,
-                           (const uint4*)init.get(), (uint4*)r->state, jumps, out, r->size, nu, n,
-                           cp.Lc, cp.C, mean, sd);
+        auto kernel = !cp.uni ? k_xoshiro_normal_chunked<false, false>
+                      : nt    ? k_xoshiro_normal_chunked<true, true>
+                              : k_xoshiro_normal_chunked<true, false>;
+        hipLaunchKernelGGL(kernel, cp.grid, cp.block, 0, g->stream, (const uint4*)init.get(), (uint4*)r->state, jumps,
+                           out, r->size, nu, n, cp.Lc, cp.C, mean, sd);
       } else {
         uint64_t th = std::min<uint64_t>(r->size, nu) / 2;
-        if (n == nu && ((uintptr_t)out & 7u) == 0)
-          hipLaunchKernelGGL(k_xoshiro_normal<true>, dim3(prng_grid(th)), dim3(PRNG_BLOCK), 0, g->stream,
-                             (uint4*)r->state, out, r->size, nu, n, mean, sd);
-        else
-          hipLaunchKernelGGL(k_xoshiro_normal<false>, dim3(prng_grid(th)), dim3(PRNG_BLOCK), 0, g->stream,
-                             (uint4*)r->state, out, r->size, nu, n, mean, sd);
+        const bool paired = n == nu && ((uintptr_t)out & 7u) == 0;
+        auto kernel = paired ? (nt ? k_xoshiro_normal<true, true> : k_xoshiro_normal<true, false>)
+                             : (nt ? k_xoshiro_normal<false, true> : k_xoshiro_normal<false, false>);
+        hipLaunchKernelGGL(kernel, dim3(prng_grid(th)), dim3(PRNG_BLOCK), 0, g->stream, (uint4*)r->state, out, r->size,
+                           nu, n, mean, sd);
       }
       check_launch("xoshiro normal");
       return;
