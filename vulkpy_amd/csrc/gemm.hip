@@ -167,12 +167,31 @@ __device__ __forceinline__ bool out_of_parts(const uint32_t* range) {
   return la + lb > 102u || ha + hb > 90u;
 }
 
-__device__ __forceinline__ uint32_t bf2x(float a, float b) { return f2bf(a) | ((uint32_t)f2bf(b) << 16); }
+// Floats as BF16, two a word.  The conversion instruction rounds as f2bf does
+// except for NaNs (f2bf keeps the payload) and denormals (f2bf rounds none of
+// them to zero): rows with one of those are converted again by f2bf.
+template <int N>
+__device__ __forceinline__ void f2bf_pairs(const float (&v)[N], uint32_t (&h)[N / 2]) {
+  typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2_t;
+  constexpr int SPECIAL = 0x93;  // NaNs and denormals, for v_cmp_class
+  bool odd = false;
+#pragma unroll
+  for (int k = 0; k < N; k += 2) {
+    odd |= __builtin_amdgcn_classf(v[k], SPECIAL) | __builtin_amdgcn_classf(v[k + 1], SPECIAL);
+    const bf16x2_t t = {(__bf16)v[k], (__bf16)v[k + 1]};
+    h[k / 2] = __builtin_bit_cast(uint32_t, t);
+  }
+  if (__builtin_expect(odd, 0)) {
+#pragma unroll
+    for (int k = 0; k < N; k += 2) h[k / 2] = f2bf(v[k]) | ((uint32_t)f2bf(v[k + 1]) << 16);
+  }
+}
 
 // Row-major source: 4 consecutive elements a thread, one thread per 4 of
 // the padded [Rp][Kp] (Rp * Kp / 4 < 2^31: the row from one 32-bit
 // multiply-high division), so that each load instruction reads one contiguous
-// 1 KB run and each store writes 512 B (64-byte runs with PARTS > 1).
+// 1 KB run and each store writes 512 B (64-byte runs with PARTS > 1).  HBM-bound:
+// 65536 x 1024 in two parts 84 us (96 with the rounding in integer steps).
 template <int PARTS>
 __global__ void __launch_bounds__(256)
 k_pack_rows(const float* src, uint64_t ld, uint64_t R, uint64_t K, uint16_t* dst, uint32_t total4, FastDiv kq,
@@ -196,9 +215,11 @@ k_pack_rows(const float* src, uint64_t ld, uint64_t R, uint64_t K, uint16_t* dst
     for (int q = 0; q < 4; ++q) note_range(range, v[q]);
 #pragma unroll
   for (int part = 0; part < PARTS; ++part) {
-    *reinterpret_cast<uint2*>(dst + off + part * 32) = make_uint2(bf2x(v[0], v[1]), bf2x(v[2], v[3]));
+    uint32_t h[2];
+    f2bf_pairs(v, h);
+    *reinterpret_cast<uint2*>(dst + off + part * 32) = make_uint2(h[0], h[1]);
 #pragma unroll
-    for (int q = 0; q < 4; ++q) v[q] = v[q] - bf2f(f2bf(v[q]));
+    for (int q = 0; q < 4; ++q) v[q] = v[q] - __uint_as_float(q & 1 ? h[q / 2] & 0xffff0000u : h[q / 2] << 16);
   }
 }
 
@@ -207,7 +228,9 @@ k_pack_rows(const float* src, uint64_t ld, uint64_t R, uint64_t K, uint16_t* dst
 // column reads of the second phase spread over the banks), so the reads are
 // 16-byte loads along r (512-byte row segments) and the writes 16-byte
 // stores along k (256-byte row segments of the packed buffer).  Rp is a
-// multiple of PK_TR; the last k tile may pass Kp.
+// multiple of PK_TR; the last k tile may pass Kp.  HBM-bound; with nontemporal
+// reads (the source is not needed again, the packed rows are) and the rounding by
+// the conversion instruction 4096 x 16384 and its like take 56 us, 69 without.
 template <int PARTS>
 __global__ void __launch_bounds__(256)
 k_pack_cols(const float* src, uint64_t ld, uint64_t R, uint64_t K, uint16_t* dst, uint64_t Rp, uint64_t Kp,
@@ -222,7 +245,7 @@ k_pack_cols(const float* src, uint64_t ld, uint64_t R, uint64_t K, uint16_t* dst
     const int kk = f / R4, rr = (f % R4) * 4;
     const uint64_t r = r0 + rr, k = k0 + kk;
     if (k < K && r + 3 < R) {
-      v[i] = *reinterpret_cast<const f32x4u_t*>(src + k * ld + r);
+      v[i] = __builtin_nontemporal_load(reinterpret_cast<const f32x4u_t*>(src + k * ld + r));
     } else {
 #pragma unroll
       for (int q = 0; q < 4; ++q) v[i][q] = (k < K && r + q < R) ? src[k * ld + r + q] : 0.f;
@@ -240,8 +263,11 @@ k_pack_cols(const float* src, uint64_t ld, uint64_t R, uint64_t K, uint16_t* dst
     for (int i = 0; i < NL; ++i) {
       const int f = threadIdx.x + i * 256;
       const int kk = f / R4, w = (f % R4) * 2;
-      tb[kk][w] = bf2x(v[i][0], v[i][1]);
-      tb[kk][w + 1] = bf2x(v[i][2], v[i][3]);
+      const float t[4] = {v[i][0], v[i][1], v[i][2], v[i][3]};
+      uint32_t h[2];
+      f2bf_pairs(t, h);
+      tb[kk][w] = h[0];
+      tb[kk][w + 1] = h[1];
     }
     __syncthreads();
     constexpr int KC = PK_TK / 8;
@@ -285,10 +311,11 @@ k_pack_cols(const float* src, uint64_t ld, uint64_t R, uint64_t K, uint16_t* dst
         for (int q = 0; q < 8; ++q) note_range(range, v[q]);
 #pragma unroll
       for (int part = 0; part < PARTS; ++part) {
-        *reinterpret_cast<uint4*>(dst + off + part * 32) =
-            make_uint4(bf2x(v[0], v[1]), bf2x(v[2], v[3]), bf2x(v[4], v[5]), bf2x(v[6], v[7]));
+        uint32_t h[4];
+        f2bf_pairs(v, h);
+        *reinterpret_cast<uint4*>(dst + off + part * 32) = make_uint4(h[0], h[1], h[2], h[3]);
 #pragma unroll
-        for (int q = 0; q < 8; ++q) v[q] = v[q] - bf2f(f2bf(v[q]));
+        for (int q = 0; q < 8; ++q) v[q] = v[q] - __uint_as_float(q & 1 ? h[q / 2] & 0xffff0000u : h[q / 2] << 16);
       }
     }
   }
@@ -731,26 +758,6 @@ struct CopyArea {
   static constexpr int BYTES = T_BYTES + R_BYTES + F_BYTES + WN * 4;  // of a wave
   static_assert(T_BYTES % 16 == 0 && R_BYTES % 16 == 0, "16-byte accesses");
 };
-
-// Floats as BF16, two a word.  The conversion instruction rounds as f2bf does
-// except for NaNs (f2bf keeps the payload) and denormals (f2bf rounds none of
-// them to zero): rows with one of those are converted again by f2bf.
-template <int N>
-__device__ __forceinline__ void f2bf_pairs(const float (&v)[N], uint32_t (&h)[N / 2]) {
-  typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2_t;
-  constexpr int SPECIAL = 0x93;  // NaNs and denormals, for v_cmp_class
-  bool odd = false;
-#pragma unroll
-  for (int k = 0; k < N; k += 2) {
-    odd |= __builtin_amdgcn_classf(v[k], SPECIAL) | __builtin_amdgcn_classf(v[k + 1], SPECIAL);
-    const bf16x2_t t = {(__bf16)v[k], (__bf16)v[k + 1]};
-    h[k / 2] = __builtin_bit_cast(uint32_t, t);
-  }
-  if (__builtin_expect(odd, 0)) {
-#pragma unroll
-    for (int k = 0; k < N; k += 2) h[k / 2] = f2bf(v[k]) | ((uint32_t)f2bf(v[k + 1]) << 16);
-  }
-}
 
 // LDS of this wave written by other lanes of it is read after this (and the
 // other way round): the hardware keeps a wave's LDS accesses in order

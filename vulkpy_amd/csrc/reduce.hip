@@ -19,16 +19,17 @@
 namespace vkh {
 
 // 16 bytes of memory at any 4-byte alignment. NT: nontemporal, which streams an
-// operand larger than the caches (256 MB) about 10% faster and reads one that
-// they hold slower: column sums of 200000 x 999 134 / 148 us (with / without),
-// of 200000 x 17 12.8 / 9.1, rows of 100 x 100000 28 / 18.
+// operand that the 256 MB cache cannot hold next to others (128 MB and more) about
+// 10% faster and reads one that it holds slower: column sums of 200000 x 999 134 /
+// 148 us (with / without), of a gradient of 16384 x 4096 49 / 58, of 200000 x 17
+// 12.8 / 9.1, rows of 100 x 100000 28 / 18.
 typedef __attribute__((ext_vector_type(4), aligned(4))) float f32x4u_t;
 template <bool NT>
 __device__ __forceinline__ f32x4u_t ld4u(const float* p) {
   if constexpr (NT) return __builtin_nontemporal_load(reinterpret_cast<const f32x4u_t*>(p));
   return *reinterpret_cast<const f32x4u_t*>(p);
 }
-static bool streams(uint64_t elements) { return elements > (uint64_t(256) << 20) / sizeof(float); }
+static bool streams(uint64_t elements) { return elements >= (uint64_t(128) << 20) / sizeof(float); }
 
 // 16 bytes of global memory straight into LDS (lane i's at dst + 16 i)
 template <bool NT>
