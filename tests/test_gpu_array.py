@@ -787,7 +787,7 @@ def test_short_rows(gpu, L, rows):
 
 # The same for operands larger than the caches (nontemporal reads; rows up to
 # 96): small whole numbers, so every order gives NumPy's sum.
-@pytest.mark.parametrize("L,rows", [(4, 17000003), (50, 1400001), (75, 900001), (66, 1040000)])
+@pytest.mark.parametrize("L,rows", [(4, 17000003), (50, 1400001), (75, 900001), (66, 1040000), (95, 400001)])
 def test_short_rows_streamed(gpu, L, rows):
     x = np.random.default_rng(L).integers(-3, 4, (rows, L), dtype=np.int8).astype(np.float32)
     a = vk.Array(gpu, data=x)

@@ -142,8 +142,7 @@ class _Plan:
         self.hs_bf: List[Optional[_DeviceBuffer]] = [None] * len(units)
         self.ds_bf: List[Optional[_DeviceBuffer]] = [None] * len(units)
         # ... and their transposes hs[i]^T and ds[i]^T, written by the same
-        # products (c_bf16t, one 64-byte run of C^T per column of each 32-row
-        # tile) for the weight-gradient products dW = ds[i]^T x, which take
+        # products (c_bf16t, in 128-byte runs of C^T) for the weight-gradient products dW = ds[i]^T x, which take
         # them as packed op(A) and op(B)^T (vkh_gemm_bf16io) instead of
         # packing with a transposing pass; only where the producer runs on
         # the matrix cores, whose epilogue writes C^T coalesced
