@@ -593,6 +593,19 @@ def test_tile_edges(gpu, mode, M, N, K):
         _lib.call("vkh_gemm_set_config", h, md, 0, 1, M, N, K, -1)
 
 
+# Transposed operands are packed in 64 x 64 tiles where 128 x 128 ones are fewer
+# than two a compute unit, else in 128 x 128 ones; ragged in both dimensions,
+# whole-valued operands, so the products are NumPy's bit for bit.
+@pytest.mark.parametrize("mode", ["bf16", "bf16x3"])
+@pytest.mark.parametrize("ta,tb,M,N,K", [(0, 0, 70, 4099, 2101), (0, 0, 70, 301, 131), (1, 0, 65, 127, 66),
+                                         (1, 1, 4099, 70, 2101)])
+def test_transposing_pack_tiles(gpu, mode, ta, tb, M, N, K):
+    rng = np.random.default_rng(M + N + K)
+    A = rng.integers(-3, 4, (K, M) if ta else (M, K)).astype(np.float32)
+    B = rng.integers(-3, 4, (N, K) if tb else (K, N)).astype(np.float32)
+    np.testing.assert_array_equal(run_gemm(gpu, mode, ta, tb, A, B), (A.T if ta else A) @ (B.T if tb else B))
+
+
 # The column walk's forms (one launch up to 2048 outputs by 16 and 32 chunks of
 # 64 terms; else chunks and a combine, Y through LDS or, for one output, not)
 # add each output's terms in chunks in k order and the chunks in order:

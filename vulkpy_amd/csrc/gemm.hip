@@ -128,8 +128,7 @@ __device__ __forceinline__ void tile_coords(const GemmArgs& p, uint32_t& tm, uin
 // main kernel's inner loop is 16-byte loads, 16-byte LDS stores and MFMAs with
 // no conversion and no bounds checks.
 constexpr int PK_KALIGN = 64;  // packed K (Kp) is a multiple of every kernel's k slice
-constexpr int PK_TR = 128;     // transpose tile rows (r) in k_pack_cols (divides every Rp)
-constexpr int PK_TK = 128;     // transpose tile k in k_pack_cols
+constexpr int PK_TR = 128;     // transpose tile (rows r and k) in k_pack_cols (divides every Rp)
 
 // dst[r][k] = bf16(op(src)[r][k]) for r < Rp, k < Kp, zero outside [R, K);
 // op(src)[r][k] = src[r*ld + k] (TRANS = false) or src[k*ld + r] (TRANS = true).
@@ -224,21 +223,21 @@ k_pack_rows(const float* src, uint64_t ld, uint64_t R, uint64_t K, uint16_t* dst
   }
 }
 
-// Transposed source: a PK_TK (k) x PK_TR (r) tile goes through LDS (BF16
-// pairs for the plain pack, rows of PK_TR + 1 floats for the split one: the
+// Transposed source: a T (k) x T (r) tile goes through LDS (BF16
+// pairs for the plain pack, rows of T + 1 floats for the split one: the
 // column reads of the second phase spread over the banks), so the reads are
 // 16-byte loads along r (512-byte row segments) and the writes 16-byte
-// stores along k (256-byte row segments of the packed buffer).  Rp is a
-// multiple of PK_TR; the last k tile may pass Kp.  HBM-bound; with nontemporal
+// stores along k (256-byte row segments of the packed buffer; lengths for T =
+// 128).  Rp is a multiple of T; the last k tile may pass Kp.  HBM-bound; with nontemporal
 // reads (the source is not needed again, the packed rows are) and the rounding by
 // the conversion instruction 4096 x 16384 and its like take 56 us, 69 without.
-template <int PARTS>
+template <int PARTS, int T>
 __global__ void __launch_bounds__(256)
 k_pack_cols(const float* src, uint64_t ld, uint64_t R, uint64_t K, uint16_t* dst, uint64_t Rp, uint64_t Kp,
             uint32_t* range) {
-  const uint64_t r0 = (uint64_t)blockIdx.x * PK_TR, k0 = (uint64_t)blockIdx.y * PK_TK;
-  constexpr int R4 = PK_TR / 4;
-  constexpr int NL = PK_TK * R4 / 256;  // 16-byte loads per thread, all issued before the LDS writes
+  const uint64_t r0 = (uint64_t)blockIdx.x * T, k0 = (uint64_t)blockIdx.y * T;
+  constexpr int R4 = T / 4;
+  constexpr int NL = T * R4 / 256;  // 16-byte loads per thread, all issued before the LDS writes
   vkh_f4v v[NL];
 #pragma unroll
   for (int i = 0; i < NL; ++i) {
@@ -258,8 +257,8 @@ k_pack_cols(const float* src, uint64_t ld, uint64_t R, uint64_t K, uint16_t* dst
     // a compute unit.  Word w of row kk holds r = 2w (low half) and 2w + 1;
     // a thread of the second phase reads one word of 8 consecutive k and
     // writes the packed rows of both r.
-    constexpr int PW = PK_TR / 2 + 1;  // words a row: odd, so the column reads spread over banks
-    __shared__ uint32_t tb[PK_TK][PW];
+    constexpr int PW = T / 2 + 1;  // words a row: odd, so the column reads spread over banks
+    __shared__ uint32_t tb[T][PW];
 #pragma unroll
     for (int i = 0; i < NL; ++i) {
       const int f = threadIdx.x + i * 256;
@@ -271,8 +270,8 @@ k_pack_cols(const float* src, uint64_t ld, uint64_t R, uint64_t K, uint16_t* dst
       tb[kk][w + 1] = h[1];
     }
     __syncthreads();
-    constexpr int KC = PK_TK / 8;
-    for (int f = threadIdx.x; f < (PK_TR / 2) * KC; f += 256) {
+    constexpr int KC = T / 8;
+    for (int f = threadIdx.x; f < (T / 2) * KC; f += 256) {
       const int rp = f / KC, kc = f % KC;
       const uint64_t k = k0 + kc * 8;
       if (k >= Kp) continue;
@@ -289,7 +288,7 @@ k_pack_cols(const float* src, uint64_t ld, uint64_t R, uint64_t K, uint16_t* dst
       *reinterpret_cast<uint4*>(dst + off + Kp) = od;
     }
   } else {  // FP32 tile: the lower parts need the values
-    __shared__ float t[PK_TK][PK_TR + 1];
+    __shared__ float t[T][T + 1];
 #pragma unroll
     for (int i = 0; i < NL; ++i) {
       const int f = threadIdx.x + i * 256;
@@ -298,8 +297,8 @@ k_pack_cols(const float* src, uint64_t ld, uint64_t R, uint64_t K, uint16_t* dst
       for (int q = 0; q < 4; ++q) t[kk][rr + q] = v[i][q];
     }
     __syncthreads();
-    constexpr int KC = PK_TK / 8;  // 8-element chunks per packed row in the tile
-    for (int f = threadIdx.x; f < PK_TR * KC; f += 256) {
+    constexpr int KC = T / 8;  // 8-element chunks per packed row in the tile
+    for (int f = threadIdx.x; f < T * KC; f += 256) {
       const int rr = f / KC, kc = f % KC;
       const uint64_t k = k0 + kc * 8;
       if (k >= Kp) continue;
@@ -1799,8 +1798,15 @@ static void pack_operand(vkh_gpu* g, const float* src, uint64_t ld, bool trans, 
                        src, ld, R, K, dst, (uint32_t)total4, FastDiv((uint32_t)(Kp / 4)), Kp, range);
   } else {
     VKH_REQUIRE(Rp % PK_TR == 0, "gemm pack: padded rows not a multiple of the tile");
-    dim3 grid((unsigned)(Rp / PK_TR), (unsigned)ceil_div(Kp, PK_TK));
-    hipLaunchKernelGGL((k_pack_cols<PARTS>), grid, dim3(256), 0, g->stream, src, ld, R, K, dst, Rp, Kp, range);
+    // Tiles of 64 x 64 where 128 x 128 ones are fewer than two a compute unit: 573 x
+    // 1301 and its like in two parts 4.7 us against 9.4, 500 x 500 2.9 against 6.0, 4000 x 1000
+    // 7.2 against 8.6; at four a unit (4096 x 2048) 9.4 against 10.2 in one part, 18.8
+    // against 16.9 in three.
+    const bool small = (Rp / PK_TR) * ceil_div(Kp, PK_TR) < 2 * (uint64_t)(g->num_cus > 0 ? g->num_cus : 256);
+    const unsigned t = small ? PK_TR / 2 : PK_TR;
+    const dim3 grid((unsigned)(Rp / t), (unsigned)ceil_div(Kp, (uint64_t)t));
+    auto kernel = small ? k_pack_cols<PARTS, PK_TR / 2> : k_pack_cols<PARTS, PK_TR>;
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, g->stream, src, ld, R, K, dst, Rp, Kp, range);
   }
   check_launch("gemm pack");
 }
