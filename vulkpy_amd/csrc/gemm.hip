@@ -5,8 +5,7 @@
 // Here a block computes a BM x BN tile: operand slices are staged through LDS
 // ahead of their use, and each wave owns a sub-tile of 32 x 32 or 16 x 16 MFMA
 // blocks:
-//   FP32    v_mfma_f32_32x32x2_f32, 16x16x4 for few outputs (operands as
-//           stored); large products as six products of three BF16 parts
+//   FP32    v_mfma_f32_32x32x2_f32    (operands as stored)
 //   BF16    v_mfma_f32_16x16x32_bf16  (operands rounded to nearest-even BF16)
 //   BF16X3  the same instruction three times: lo*hi + hi*lo + hi*hi, where
 //           x = hi + lo + O(2^-16 |x|) with hi = bf16(x), lo = bf16(x - hi)
@@ -1400,7 +1399,7 @@ k_splitk_combine(const float* part, uint64_t S, GemmArgs e) {
 // staggered waves but loads one slice ahead, 855 us without the stagger, 955 us
 // with 32 x 32 x 16 instructions), 16384 x 4096 x 4096 405-430 against 490-583 us.
 // One 16 x 16 x 32 instruction gives the bits of the two 32 x 32 x 16 ones it
-// replaces.
+// replaces, so results equal k_gemm_packed's.
 __device__ __forceinline__ void load_lds16(const char* src, char* dst) {
 #ifdef __HIP_DEVICE_COMPILE__  // (the host pass would drop the launch stub of a template that uses the builtin)
   __builtin_amdgcn_global_load_lds(src, dst, 16, 0, 0);
@@ -1429,15 +1428,9 @@ struct PipeSlice {
   static constexpr int CPR = ROWB / 16;            // 16-byte chunks of a row
   // LDS position of chunk c of row r.  Rows of 128 bytes alternate between the
   // halves of the 256-byte bank line, so 8 row pairs permute 8 positions; rows
-  // of 192 bytes start at 4 places of it, so 4 row quads permute 4 positions.  (A
-  // 16-byte read's first 16 lanes at a time are 0-3, 12-15, 20-23 and 24-27: quads 0
-  // and 3 of one chunk and 1 and 2 of the next, so the quad's number itself as the
-  // permutation collided in half of the reads: LDS active 40% of the cycles, 21% so,
-  // matrix cores busy 80.5 and 83%.)
+  // of 192 bytes start at 4 places of it, so 4 row quads permute 4 positions.
   __device__ __forceinline__ static int pos(int r, int c) {
-    if (PARTS != 3) return c ^ ((r >> 1) & 7);
-    const int a = (r >> 2) & 3;
-    return (c & ~3) | ((c & 3) ^ ((a ^ (a << 1)) & 3));
+    return PARTS == 3 ? (c & ~3) | ((c & 3) ^ ((r >> 2) & 3)) : c ^ ((r >> 1) & 7);
   }
 };
 
