@@ -350,9 +350,7 @@ def mlp_gemm_utilisation(vk, gpu, timer, B: int, dims, reps: int = 3) -> dict:
     over `reps` launches behind an untimed one, in the configuration the step
     uses (configurations chosen by autotuning stay on the context), operand
     packing included.  frac = TFLOP/s / the mode's dense peak (split-BF16: a
-    third of the BF16 peak, since it runs three products; FP32: the FP32 matrix
-    peak, which large products, run as six BF16 products of three-part
-    operands, can exceed).  Products with
+    third of the BF16 peak, since it runs three products).  Products with
     min(M, N) <= 16 or K <= 16 run on the vector units (path "vector").
     """
     from vulkpy_amd import _lib

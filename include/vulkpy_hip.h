@@ -342,10 +342,7 @@ int vkh_gemm(vkh_gpu* gpu, int mode, int trans_a, int trans_b,
  * M x N x K product ahead of time and records the size so that the next
  * vkh_graph_begin reserves a large enough region (a capture cannot allocate;
  * a captured GEMM that does not fit fails and records its size for the next
- * capture).  Large FP32 products pack their operands too (as three BF16 parts);
- * one captured without room for them, or called where the area cannot grow,
- * runs the FP32 kernel instead, so eager and captured calls give the same bits
- * only after this reservation.  Refused during a capture.  No counterpart in the reference. */
+ * capture).  Refused during a capture.  No counterpart in the reference. */
 int vkh_gemm_reserve(vkh_gpu* gpu, int mode, uint64_t M, uint64_t N,
                      uint64_t K);
 

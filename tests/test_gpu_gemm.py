@@ -789,3 +789,32 @@ def test_fp32_parts_in_a_graph(gpu, reserve):
                 assert np.array_equal(got, want["good"]) or np.array_equal(got[1:], want["small"][1:])
     finally:
         _lib.call("vkh_graph_destroy", ex.value)
+
+
+def test_fp32_single_terms_rounded_once(gpu):
+    """Outputs with one nonzero term: the exact product, rounded once."""
+    M, N, K = F32X3
+    rng = np.random.default_rng(69)
+    idx = rng.integers(0, K, M)
+    A = np.zeros((M, K), dtype=np.float32)
+    A[np.arange(M), idx] = a = rng.uniform(1, 2, M).astype(np.float32)
+    B = rng.uniform(1, 2, (K, N)).astype(np.float32)
+    exact = a.astype(np.float64)[:, None] * B[idx].astype(np.float64)
+    np.testing.assert_array_equal(run_gemm(gpu, "fp32", 0, 0, A, B), exact.astype(np.float32))
+
+
+@pytest.mark.parametrize("M,N,K,cfg", [(2176, 2048, 1024, -1), (4001, 2047, 1030, -1), (4001, 2047, 1030, 0),
+                                       (4001, 2047, 1030, 1), (4001, 2047, 1030, 2), (4001, 2047, 1030, 3)])
+def test_fp32_accumulates_once(gpu, M, N, K, cfg):
+    """Large products added to what C holds, as the weight gradient of a Dense
+    layer is, in every tile (whole numbers, exact)."""
+    rng = np.random.default_rng(68)
+    x = rng.integers(-60, 61, (K, N)).astype(np.float32)
+    dy = rng.integers(-60, 61, (K, M)).astype(np.float32)
+    C0 = rng.integers(-9, 10, (M, N)).astype(np.float32)
+    want = dy.astype(np.float64).T @ x.astype(np.float64) + C0
+    try:
+        _lib.call("vkh_gemm_set_config", gpu._handle, 0, 1, 0, M, N, K, cfg)
+        np.testing.assert_array_equal(run_gemm(gpu, "fp32", 1, 0, dy, x, C0=C0, beta=1.0), want.astype(np.float32))
+    finally:
+        _lib.call("vkh_gemm_set_config", gpu._handle, 0, 1, 0, M, N, K, -1)

@@ -13,7 +13,6 @@
 // bias[n] and an activation, and can also emit a BF16 copy of the result.
 // Blocks are remapped so that consecutive tiles land on the same XCD (each of
 // the 8 XCDs has its own L2) and grouped along M for L2 reuse of B.
-#include <cmath>
 #include <type_traits>
 #include <utility>
 
@@ -65,7 +64,6 @@ struct GemmArgs {
   // the aux activation's output as BF16 instead of aux (ReLU' only: the BF16
   // copy has the sign, zero-ness and NaN-ness of the value)
   const uint16_t* aux16;
-  const uint32_t* range;  // FP32 kernel: where given, runs only for operands out of three BF16 parts' range
 };
 constexpr int CS_ROWS = 128;
 
@@ -140,32 +138,6 @@ __device__ __forceinline__ uint64_t pack_off(uint64_t r, uint64_t k, uint64_t Kp
   return PARTS == 1 ? r * Kp + k : r * Kp * PARTS + (k / 32) * (32 * PARTS) + k % 32;
 }
 
-// Range of an FP32 operand that goes into three BF16 parts: range[0] is the
-// largest -exponent below 2^-20 (0 where there is none; an element of 0 does
-// not count), range[1] the largest exponent above 2^20 (128: an infinity or a
-// NaN).  Elements between take no memory access; others read the word and
-// raise it only where they exceed it.
-constexpr int RANGE_FREE = 20;
-__device__ __forceinline__ void note_range(uint32_t* range, float x) {
-  const uint32_t mag = __float_as_uint(x) & 0x7fffffffu;
-  const int e = (int)(mag >> 23) - 127;
-  if (mag == 0u || (e >= -RANGE_FREE && e <= RANGE_FREE)) return;
-  uint32_t* w = range + (e > 0);
-  const uint32_t v = (uint32_t)(e > 0 ? e : -e);
-  if (v > __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(w, v);
-}
-
-// Whether three parts and their six larger products may lose something that
-// FP32 keeps, from the ranges of the operands (A's two words, then B's).  They
-// do not while every part is 0 or normal (the lowest bit of 2^-102 is 2^-125),
-// every kept product is normal (at least 2^(-102 - 24)) and no product or sum
-// of products overflows.
-__device__ __forceinline__ bool out_of_parts(const uint32_t* range) {
-  const uint32_t la = max(range[0], (uint32_t)RANGE_FREE), ha = max(range[1], (uint32_t)RANGE_FREE);
-  const uint32_t lb = max(range[2], (uint32_t)RANGE_FREE), hb = max(range[3], (uint32_t)RANGE_FREE);
-  return la + lb > 102u || ha + hb > 90u;
-}
-
 // Floats as BF16, two a word.  The conversion instruction rounds as f2bf does
 // except for NaNs (f2bf keeps the payload) and denormals (f2bf rounds none of
 // them to zero): rows with one of those are converted again by f2bf.
@@ -194,7 +166,7 @@ __device__ __forceinline__ void f2bf_pairs(const float (&v)[N], uint32_t (&h)[N 
 template <int PARTS>
 __global__ void __launch_bounds__(256)
 k_pack_rows(const float* src, uint64_t ld, uint64_t R, uint64_t K, uint16_t* dst, uint32_t total4, FastDiv kq,
-            uint64_t Kp, uint32_t* range) {
+            uint64_t Kp) {
   const uint32_t t = blockIdx.x * 256 + threadIdx.x;
   if (t >= total4) return;
   const uint32_t r = kq.div(t);
@@ -209,9 +181,6 @@ k_pack_rows(const float* src, uint64_t ld, uint64_t R, uint64_t K, uint16_t* dst
     for (int q = 0; q < 4; ++q) v[q] = (r < R && k + q < K) ? src[r * ld + k + q] : 0.f;
   }
   const uint64_t off = pack_off<PARTS>(r, k, Kp);
-  if constexpr (PARTS == 3)
-#pragma unroll
-    for (int q = 0; q < 4; ++q) note_range(range, v[q]);
 #pragma unroll
   for (int part = 0; part < PARTS; ++part) {
     uint32_t h[2];
@@ -232,8 +201,7 @@ k_pack_rows(const float* src, uint64_t ld, uint64_t R, uint64_t K, uint16_t* dst
 // the conversion instruction 4096 x 16384 and its like take 56 us, 69 without.
 template <int PARTS, int T>
 __global__ void __launch_bounds__(256)
-k_pack_cols(const float* src, uint64_t ld, uint64_t R, uint64_t K, uint16_t* dst, uint64_t Rp, uint64_t Kp,
-            uint32_t* range) {
+k_pack_cols(const float* src, uint64_t ld, uint64_t R, uint64_t K, uint16_t* dst, uint64_t Rp, uint64_t Kp) {
   const uint64_t r0 = (uint64_t)blockIdx.x * T, k0 = (uint64_t)blockIdx.y * T;
   constexpr int R4 = T / 4;
   constexpr int NL = T * R4 / 256;  // 16-byte loads per thread, all issued before the LDS writes
@@ -305,9 +273,6 @@ k_pack_cols(const float* src, uint64_t ld, uint64_t R, uint64_t K, uint16_t* dst
 #pragma unroll
       for (int q = 0; q < 8; ++q) v[q] = t[kc * 8 + q][rr];
       const uint64_t off = pack_off<PARTS>(r0 + rr, k, Kp);
-      if constexpr (PARTS == 3)
-#pragma unroll
-        for (int q = 0; q < 8; ++q) note_range(range, v[q]);
 #pragma unroll
       for (int part = 0; part < PARTS; ++part) {
         uint32_t h[4];
@@ -330,7 +295,6 @@ struct PackedArgs {
   uint64_t kc;
   float* part;
   GemmArgs e;
-  const uint32_t* range = nullptr;  // three parts: the operands' ranges (out_of_parts)
 };
 
 // 4 consecutive floats p[0 .. cnt) (one 16-byte load when `full`), zeros beyond.
@@ -1110,7 +1074,6 @@ struct F32Stager {
 template <bool AK, bool BKM, bool VEC, int BM, int BN, int WGM, int WGN>
 __global__ void __launch_bounds__(64 * WGM * WGN, 2)
 k_gemm_f32(GemmArgs p, float* part, uint64_t kc) {
-  if (p.range && !out_of_parts(p.range)) return;
   constexpr int THREADS = 64 * WGM * WGN, WAVES = WGM * WGN;
   constexpr int WM = BM / WGM, WN = BN / WGN;
   static_assert(WM % 32 == 0 && WN % 32 == 0, "32 x 32 MFMA blocks per wave");
@@ -1374,9 +1337,9 @@ k_splitk_combine(const float* part, uint64_t S, GemmArgs e) {
 }
 
 // ---- pipelined BF16 products ----------------------------------------------------
-// C from packed operands on v_mfma_f32_16x16x32_bf16.  PARTS BF16 values stand
-// for each operand element (1: BF16 mode, 2: split mode, 3: FP32 products of
-// large operands); a packed row holds its k in groups of KG,
+// C from packed operands on v_mfma_f32_16x16x32_bf16, for products with enough
+// tiles to fill the chip.  PARTS BF16 values stand for each operand element
+// (1: BF16 mode, 2: split mode); a packed row holds its k in groups of KG,
 // the parts of a group one after another, so a slice of every row is ROWB
 // contiguous bytes in every mode.
 //
@@ -1426,12 +1389,9 @@ struct PipeSlice {
   static constexpr int ROWB = KG * 2 * PARTS;      // bytes of a slice row
   static constexpr int NF = ROWB / 64;             // 64-byte fragments of a row: k steps, or parts
   static constexpr int CPR = ROWB / 16;            // 16-byte chunks of a row
-  // LDS position of chunk c of row r.  Rows of 128 bytes alternate between the
-  // halves of the 256-byte bank line, so 8 row pairs permute 8 positions; rows
-  // of 192 bytes start at 4 places of it, so 4 row quads permute 4 positions.
-  __device__ __forceinline__ static int pos(int r, int c) {
-    return PARTS == 3 ? (c & ~3) | ((c & 3) ^ ((r >> 2) & 3)) : c ^ ((r >> 1) & 7);
-  }
+  // LDS position of chunk c of row r: rows of 128 bytes alternate between the
+  // halves of the 256-byte bank line, so 8 row pairs permute 8 positions
+  __device__ __forceinline__ static int pos(int r, int c) { return c ^ ((r >> 1) & 7); }
 };
 
 // The operands are exchanged (each block of the accumulators is C^T's).
@@ -1439,7 +1399,6 @@ struct PipeSlice {
 template <int BM, int BN, int WGM, int WGN, int PARTS, bool DIRECT>
 __global__ void __launch_bounds__(64 * WGM * WGN, 2)
 k_gemm_pipe(PackedArgs p) {
-  if (PARTS == 3 && out_of_parts(p.range)) return;  // (the FP32 kernel takes these operands)
   using S = PipeSlice<PARTS>;
   constexpr int ROWB = S::ROWB, NF = S::NF, WAVES = WGM * WGN;
   constexpr bool STAGGER = WAVES == 8;  // two waves a SIMD
@@ -1449,12 +1408,8 @@ k_gemm_pipe(PackedArgs p) {
   constexpr int TMH = HM / 16, TNH = HN / 16;
   // 1 KB loads (one wave instruction) of one wave row's half, and per wave
   constexpr int GA = HM * ROWB / 1024, GB = HN * ROWB / 1024;
-  constexpr int LA = WGM * GA / WAVES;
-  // B goes as a whole, once both halves have been read, where the halves are
-  // not whole loads of every wave
-  constexpr bool BWHOLE = WGN * GB % WAVES != 0;
-  constexpr int LB = (BWHOLE ? 2 : 1) * WGN * GB / WAVES;
-  static_assert(LA * WAVES == WGM * GA && LB * WAVES == (BWHOLE ? 2 : 1) * WGN * GB, "whole loads per wave and half");
+  constexpr int LA = WGM * GA / WAVES, LB = WGN * GB / WAVES;
+  static_assert(LA * WAVES == WGM * GA && LB * WAVES == WGN * GB, "whole loads per wave and half");
   constexpr int A_BYTES = BM * ROWB, B_BYTES = BN * ROWB;
   constexpr int MAIN_BYTES = 2 * (A_BYTES + B_BYTES);
   constexpr int EPI_BYTES = DIRECT ? 0 : WAVES * CopyArea<2 * TMH, 2 * TNH>::BYTES;
@@ -1481,9 +1436,6 @@ k_gemm_pipe(PackedArgs p) {
     const int idx = q * WAVES + wave;
     return (idx / g) * wrows * ROWB + h * hrows * ROWB + (idx % g) * 1024;
   };
-  auto boff = [&](int q, int h) {
-    return BWHOLE ? (q * WAVES + wave) * 1024 : half_off(q, GB, h, WN, HN);
-  };
   auto src_off = [&](int lds_off) {
     const int c = (lds_off >> 4) + lane, r = c / S::CPR;
     return (uint32_t)r * (uint32_t)(rowp >> 4) + S::pos(r, c % S::CPR);
@@ -1494,7 +1446,7 @@ k_gemm_pipe(PackedArgs p) {
 #pragma unroll
     for (int q = 0; q < LA; ++q) oa[h][q] = src_off(half_off(q, GA, h, WM, HM));
 #pragma unroll
-    for (int q = 0; q < LB; ++q) ob[h][q] = src_off(boff(q, h));
+    for (int q = 0; q < LB; ++q) ob[h][q] = src_off(half_off(q, GB, h, WN, HN));
   }
   // slices past the end load the last one again (in range, never read)
   auto slice = [&](uint64_t kt) { return (kt < nk ? kt : nk - 1) * ROWB; };
@@ -1505,7 +1457,7 @@ k_gemm_pipe(PackedArgs p) {
   auto load_b = [&](int b, uint64_t ks, int h) {
 #pragma unroll
     for (int q = 0; q < LB; ++q)
-      load_lds16(gb + ks + ((uint64_t)ob[h][q] << 4), smem + 2 * A_BYTES + b * B_BYTES + boff(q, h));
+      load_lds16(gb + ks + ((uint64_t)ob[h][q] << 4), smem + 2 * A_BYTES + b * B_BYTES + half_off(q, GB, h, WN, HN));
   };
 
   f32x4_t acc[2 * TMH][2 * TNH];
@@ -1542,19 +1494,14 @@ k_gemm_pipe(PackedArgs p) {
         acc[h * TMH + i][g * TNH + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
             fb[g][j][q], fa[i][f], acc[h * TMH + i][g * TNH + j], 0, 0, 0);
   };
-  // quarter (h, g): every product of its fragments, k in order (with several
-  // parts the products of 32 k at a time, the smaller ones first)
+  // quarter (h, g): every product of its fragments, k in order (split mode:
+  // lo * hi, hi * lo, hi * hi of 32 k at a time)
   auto quarter = [&](int h, int g) {
     phase_barrier();
     if constexpr (PARTS == 1) {
       mul(h, g, 0, 0);
       mul(h, g, 1, 1);
     } else {
-      if constexpr (PARTS == 3) {
-        mul(h, g, 2, 0);
-        mul(h, g, 1, 1);
-        mul(h, g, 0, 2);
-      }
       mul(h, g, 1, 0);
       mul(h, g, 0, 1);
       mul(h, g, 0, 0);
@@ -1565,18 +1512,14 @@ k_gemm_pipe(PackedArgs p) {
     else __builtin_amdgcn_sched_barrier(0);
   };
 
-  // loads in flight that a wait leaves: those issued after what it waits for
-  constexpr int W0 = BWHOLE ? 2 * LA + LB : 2 * LA + 3 * LB;  // slice kt + 1: first half of A (and of B, or B)
-  constexpr int W1 = 3 * LA + 2 * LB;                         // slice kt: second half of B
-  constexpr int W2 = BWHOLE ? 2 * LA + LB : 2 * LA + 2 * LB;  // slice kt: second half of A
   load_a(0, slice(0), 0);
   load_b(0, slice(0), 0);
-  if constexpr (!BWHOLE) load_b(0, slice(0), 1);
+  load_b(0, slice(0), 1);
   load_a(0, slice(0), 1);
   load_a(1, slice(1), 0);
   load_b(1, slice(1), 0);
-  if constexpr (!BWHOLE) load_b(1, slice(1), 1);
-  wait_loads<W0>();
+  load_b(1, slice(1), 1);
+  wait_loads<2 * LA + 3 * LB>();
   phase_barrier();
   if (STAGGER && wave >= WAVES / 2) phase_barrier();
   for (uint64_t kt = 0; kt < nk; ++kt) {
@@ -1585,17 +1528,17 @@ k_gemm_pipe(PackedArgs p) {
     read_b(cur, 0);
     read_a(cur, 0);
     load_a(cur ^ 1, k1, 1);
-    if constexpr (!BWHOLE) wait_loads<W1>();
+    wait_loads<3 * LA + 2 * LB>();  // this slice's second half of B has landed
     quarter(0, 0);
     read_b(cur, 1);
-    wait_loads<W2>();
+    wait_loads<2 * LA + 2 * LB>();  // this slice's second half of A has landed
     quarter(0, 1);
     read_a(cur, 1);
     load_a(cur, k2, 0);
-    if constexpr (!BWHOLE) load_b(cur, k2, 0);
+    load_b(cur, k2, 0);
     quarter(1, 1);
     load_b(cur, k2, 1);
-    wait_loads<W0>();
+    wait_loads<2 * LA + 3 * LB>();  // the next slice's first halves have landed
     quarter(1, 0);
   }
   if (STAGGER && wave < WAVES / 2) phase_barrier();
@@ -1783,23 +1726,22 @@ static uint16_t* pack_area(vkh_gpu* g, size_t bytes) {
 
 template <int PARTS>
 static void pack_operand(vkh_gpu* g, const float* src, uint64_t ld, bool trans, uint64_t R,
-                         uint64_t K, uint16_t* dst, uint64_t Rp, uint64_t Kp, uint32_t* range = nullptr) {
+                         uint64_t K, uint16_t* dst, uint64_t Rp, uint64_t Kp) {
   if (!trans) {
     const uint64_t total4 = Rp * (Kp / 4);
     VKH_REQUIRE(total4 < (uint64_t(1) << 31), "gemm pack: operand too large");
     hipLaunchKernelGGL((k_pack_rows<PARTS>), dim3((unsigned)ceil_div(total4, 256)), dim3(256), 0, g->stream,
-                       src, ld, R, K, dst, (uint32_t)total4, FastDiv((uint32_t)(Kp / 4)), Kp, range);
+                       src, ld, R, K, dst, (uint32_t)total4, FastDiv((uint32_t)(Kp / 4)), Kp);
   } else {
     VKH_REQUIRE(Rp % PK_TR == 0, "gemm pack: padded rows not a multiple of the tile");
     // Tiles of 64 x 64 where 128 x 128 ones are fewer than two a compute unit: 573 x
     // 1301 and its like in two parts 4.7 us against 9.4, 500 x 500 2.9 against 6.0, 4000 x 1000
-    // 7.2 against 8.6; at four a unit (4096 x 2048) 9.4 against 10.2 in one part, 18.8
-    // against 16.9 in three.
+    // 7.2 against 8.6; at four a unit (4096 x 2048) 9.4 against 10.2 in one part.
     const bool small = (Rp / PK_TR) * ceil_div(Kp, PK_TR) < 2 * (uint64_t)(g->num_cus > 0 ? g->num_cus : 256);
     const unsigned t = small ? PK_TR / 2 : PK_TR;
     const dim3 grid((unsigned)(Rp / t), (unsigned)ceil_div(Kp, (uint64_t)t));
     auto kernel = small ? k_pack_cols<PARTS, PK_TR / 2> : k_pack_cols<PARTS, PK_TR>;
-    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, g->stream, src, ld, R, K, dst, Rp, Kp, range);
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, g->stream, src, ld, R, K, dst, Rp, Kp);
   }
   check_launch("gemm pack");
 }
@@ -1893,92 +1835,6 @@ static void gemm_f32(vkh_gpu* g, bool ta, bool tb, GemmArgs& a, int cfg) {
                        (const float*)part, S, a);
     check_launch("gemm split-k combine");
   }
-}
-
-// ---- FP32 products from three BF16 parts ------------------------------------------
-// Large FP32 products run on the BF16 matrix cores.  An FP32 value is exactly
-// h + m + l, three BF16 values (h = bf16(x), m = bf16(x - h), l = x - h - m: 24
-// mantissa bits in three times 8), and the product keeps the six terms hh, hm,
-// mh, hl, mm, lh; the dropped ml, lm and ll are at most 2^-26 |a b|, below the
-// rounding of the FP32 product itself.  Sums are FP32 as before, with fewer
-// roundings (one a term per 32 k against one per 2 k), so the error against 64
-// bits is smaller: over seven shapes of K 300 to 16384 with normal, uniform and
-// wide-range operands, 0.5 to 0.92 of the FP32 kernel's normwise (8192^3 normal
-// 1.44e-6 against 1.62e-6) and 0.57 to 0.98 of its largest elementwise one.
-// BF16 MFMAs do 16 times the work of FP32 ones and six terms cost 6 of them, so
-// the bound rises from 157 to about 400 TFLOP/s.  Packing included: 8192^3 4.62
-// against 7.92 ms (238 TFLOP/s), 16384 x 4096 x 4096 2.40 against 4.05 ms,
-// 4096 x 4096 x 1024 180 against 300 us.
-// Operands with a NaN, an infinity or too wide a range (out_of_parts) keep the
-// FP32 kernel: the packing passes note the ranges in device words, and of the
-// two kernels launched the one that does not apply returns at once, with no
-// host wait and the same way in a captured graph.  Such operands pay for the
-// packing (8192^3: 0.3 of 8.2 ms).
-constexpr int F32X3_BM = 256, F32X3_BN = 128;
-constexpr size_t F32X3_HEAD = 256;                    // bytes of the ranges before the packed operands
-constexpr size_t F32X3_MAX_BYTES = size_t(8) << 30;  // larger packed operands: FP32 kernel
-
-static size_t f32x3_bytes(uint64_t M, uint64_t N, uint64_t K) {
-  const uint64_t Mp = ceil_div(M, (uint64_t)F32X3_BM) * F32X3_BM, Np = ceil_div(N, (uint64_t)F32X3_BN) * F32X3_BN;
-  return F32X3_HEAD + (size_t)((Mp + Np) * (ceil_div(K, (uint64_t)PK_KALIGN) * PK_KALIGN) * 6);
-}
-
-// By sizes only (so eager, captured and differently laid out calls agree):
-// where the estimated time, packing included, is below 0.85 of the FP32
-// kernel's.  A round of 256 tiles takes 66 ns a k and 6 us, packing moves 10
-// bytes an element, the four launches cost 15 us; writing C costs both the
-// same.  (2048^3, 128 tiles: 154 us with the FP32 kernel, 164 estimated here;
-// 8192 x 2048 x 300 94 against 118 us.  A 128 x 128 tile of three parts was
-// slower everywhere: 4096 x 4096 x 1024 241 us.)
-static bool f32x3_route(uint64_t M, uint64_t N, uint64_t K) {
-  if (f32_splitk_chunk(M, N, K) != K || f32x3_bytes(M, N, K) > F32X3_MAX_BYTES) return false;
-  const double tiles = (double)(ceil_div(M, (uint64_t)F32X3_BM) * ceil_div(N, (uint64_t)F32X3_BN));
-  const double c_us = (double)M * (double)N * 4.0 / 5.5e6;
-  const double parts_us = 15.0 + std::ceil(tiles / 256.0) * (6.0 + (double)K * 0.066) +
-                          (double)(M + N) * (double)K * 10.0 / 5e6 + c_us;
-  int cfg = 0;
-  return parts_us < 0.85 * (tile_estimate(VKH_GEMM_FP32, M, N, K, cfg) + c_us);
-}
-
-__global__ void __launch_bounds__(64) k_clear_ranges(uint32_t* range) {
-  if (threadIdx.x < 4) range[threadIdx.x] = 0u;
-}
-
-// false: no packing area for the operands (the caller runs the FP32 kernel)
-static bool gemm_f32x3(vkh_gpu* g, bool ta, bool tb, GemmArgs& a, int cfg) {
-  const size_t bytes = f32x3_bytes(a.M, a.N, a.K);
-  char* base = nullptr;
-  if (g->capturing) {
-    if (bytes > g->graph_pack_bytes) return false;
-    base = (char*)g->graph_pack;
-  } else {
-    if (!g->alloc) return false;
-    try {
-      base = (char*)pack_area(g, bytes);
-    } catch (const Error& err) {
-      if (err.code != VKH_OUT_OF_MEMORY) throw;
-      return false;
-    }
-  }
-  const uint64_t Mp = ceil_div(a.M, (uint64_t)F32X3_BM) * F32X3_BM;
-  const uint64_t Np = ceil_div(a.N, (uint64_t)F32X3_BN) * F32X3_BN;
-  const uint64_t Kp = ceil_div(a.K, (uint64_t)PK_KALIGN) * PK_KALIGN;
-  uint32_t* range = (uint32_t*)base;
-  uint16_t* Ap = (uint16_t*)(base + F32X3_HEAD);
-  uint16_t* Bp = Ap + Mp * Kp * 3;
-  hipLaunchKernelGGL(k_clear_ranges, dim3(1), dim3(64), 0, g->stream, range);
-  check_launch("gemm range");
-  pack_operand<3>(g, a.A, a.lda, ta, a.M, a.K, Ap, Mp, Kp, range);
-  pack_operand<3>(g, a.B, a.ldb, !tb, a.N, a.K, Bp, Np, Kp, range + 2);
-  GemmArgs t = a;
-  t.tiles_m = (uint32_t)(Mp / F32X3_BM);
-  t.tiles_n = (uint32_t)(Np / F32X3_BN);
-  PackedArgs pa{Ap, Bp, Kp, Kp, nullptr, t, range};
-  launch_pipe<F32X3_BM, F32X3_BN, 4, 2, 3>(dim3(t.tiles_m * t.tiles_n), g->stream, pa);
-  check_launch("gemm (FP32 from BF16 parts)");
-  a.range = range;
-  gemm_f32(g, ta, tb, a, cfg);
-  return true;
 }
 
 // ---- skinny products: min(M, N) <= 16 ------------------------------------------------
@@ -2611,8 +2467,7 @@ static void gemm_impl(vkh_gpu* g, int mode, int trans_a, int trans_b, uint64_t M
   switch (mode) {
     case VKH_GEMM_FP32: {
       auto it = g->gemm_cfg.find(cfg_key(mode, trans_a, trans_b, M, N, K));
-      const int cfg = it != g->gemm_cfg.end() ? it->second : default_cfg(mode, M, N, K);
-      if (!(f32x3_route(M, N, K) && gemm_f32x3(g, trans_a, trans_b, a, cfg))) gemm_f32(g, trans_a, trans_b, a, cfg);
+      gemm_f32(g, trans_a, trans_b, a, it != g->gemm_cfg.end() ? it->second : default_cfg(mode, M, N, K));
       break;
     }
     case VKH_GEMM_BF16:
@@ -2827,9 +2682,7 @@ int vkh_gemm_reserve(vkh_gpu* g, int mode, uint64_t M, uint64_t N, uint64_t K) {
     // skinny and short-k products pack nothing; FP32 needs room only for
     // split-k partials
     if (M == 0 || N == 0 || std::min(M, N) <= SKINNY_MAX || K <= SMALLK_MAX) return;
-    const size_t bytes = mode != VKH_GEMM_FP32  ? packed_bytes(mode, M, N, K)
-                         : f32x3_route(M, N, K) ? f32x3_bytes(M, N, K)
-                                                : f32_split_bytes(M, N, K);
+    const size_t bytes = mode == VKH_GEMM_FP32 ? f32_split_bytes(M, N, K) : packed_bytes(mode, M, N, K);
     if (bytes == 0) return;
     g->graph_pack_hint = std::max(g->graph_pack_hint, bytes);
     pack_area(g, bytes);
@@ -2887,7 +2740,7 @@ static bool colsum_ok(vkh_gpu* g, int mode, int ta, int tb, uint64_t M, uint64_t
   auto it = g->gemm_cfg.find(cfg_key(mode, ta, tb, M, N, K));
   const int cfg = it != g->gemm_cfg.end() ? it->second : default_cfg(mode, M, N, K);
   if (mode == VKH_GEMM_FP32)
-    return !f32x3_route(M, N, K) && F32_CFGS[cfg].wm == CS_ROWS && ceil_div(K, f32_splitk_chunk(M, N, K)) == 1;
+    return F32_CFGS[cfg].wm == CS_ROWS && ceil_div(K, f32_splitk_chunk(M, N, K)) == 1;
   int n = 0;
   const PackedCfg* c = packed_cfgs(mode, n);
   const uint64_t Kp = ceil_div(K, (uint64_t)PK_KALIGN) * PK_KALIGN;

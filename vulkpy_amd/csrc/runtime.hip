@@ -305,17 +305,7 @@ int vkh_alloc(vkh_gpu* g, size_t nbytes, void** out) {
     VKH_REQUIRE(out, "null out");
     VKH_REQUIRE(g->alloc, "context on an external stream has no allocator");
     VKH_REQUIRE(!g->capturing, "device allocation while a graph is being captured");
-    try {
-      *out = g->alloc->allocate(nbytes);
-    } catch (const Error& e) {
-      // give the GEMM packing area back (its users are earlier in the stream)
-      // and try once more
-      if (e.code != VKH_OUT_OF_MEMORY || !g->pack) throw;
-      g->alloc->release(g->pack);
-      g->pack = nullptr;
-      g->pack_bytes = 0;
-      *out = g->alloc->allocate(nbytes);
-    }
+    *out = g->alloc->allocate(nbytes);
   });
 }
 

@@ -853,9 +853,7 @@ class Array(_GPUArray):
             Right operand; ``self.shape[-1]`` must equal ``other.shape[0]``.
         precision : {"fp32", "bf16", "bf16x3"}, optional
             Product precision (FP32 accumulation in every mode).  Default is
-            ``vulkpy_amd.get_matmul_precision()`` (``"fp32"``: large products
-            run as products of three BF16 parts of each element, with an
-            error no larger than the FP32 kernel's).
+            ``vulkpy_amd.get_matmul_precision()`` (``"fp32"``).
 
         Notes
         -----
