@@ -818,3 +818,40 @@ def test_fp32_accumulates_once(gpu, M, N, K, cfg):
         np.testing.assert_array_equal(run_gemm(gpu, "fp32", 1, 0, dy, x, C0=C0, beta=1.0), want.astype(np.float32))
     finally:
         _lib.call("vkh_gemm_set_config", gpu._handle, 0, 1, 0, M, N, K, -1)
+
+
+def test_products_of_several_threads(gpu):
+    """Threads on one context share its packing area (operands, split-k sums);
+    each product uses it alone: the bits of the products issued by one thread."""
+    import threading
+    jobs = [("bf16", 700, 500, 900), ("bf16x3", 900, 300, 1300), ("fp32", 200, 150, 4096), ("bf16", 150, 100, 8192)]
+    h, reps = gpu._handle, 25
+    rng = np.random.default_rng(70)
+    work = []
+    for mode, M, N, K in jobs:
+        A, B = (vk.Array(gpu, data=rng.standard_normal(s).astype(np.float32)) for s in ((M, K), (N, K)))
+        want = vk.Array(gpu, shape=(M, N))
+        out = [vk.Array(gpu, shape=(M, N)) for _ in range(reps)]
+        work.append((_lib.GEMM_MODE[mode], M, N, K, A, B, want, out))
+
+    def product(md, M, N, K, A, B, C):
+        _lib.call("vkh_gemm", h, md, 0, 1, M, N, K, 1.0, A._ptr, K, B._ptr, K, 0.0, C._ptr, N, None, 0, None)
+
+    start = threading.Barrier(len(work))
+
+    def run(md, M, N, K, A, B, out):
+        start.wait()
+        for C in out:
+            product(md, M, N, K, A, B, C)
+
+    threads = [threading.Thread(target=run, args=(*w[:6], w[7])) for w in work]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for md, M, N, K, A, B, want, out in work:
+        product(md, M, N, K, A, B, want)
+        want._set_job([A, B])
+        for C in out:
+            C._set_job([A, B])
+            np.testing.assert_array_equal(np.asarray(C).view(np.uint32), np.asarray(want).view(np.uint32))

@@ -107,7 +107,10 @@ struct vkh_gpu {
   char* arena = nullptr;
   size_t arena_size = 0, arena_used = 0, arena_hint = 0;
   // grow-only BF16 packing area of the matrix-core GEMMs (gemm.hip) for
-  // eager calls
+  // eager calls.  pack_mu is held from its choice through the launch of the
+  // last kernel that reads it: another thread's product then comes after this
+  // one on the stream as a whole, and cannot give the area back in between.
+  std::mutex pack_mu;
   void* pack = nullptr;
   size_t pack_bytes = 0;
   // packing area of GEMMs captured into a graph: a region of that graph's

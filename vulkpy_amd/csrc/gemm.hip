@@ -1700,8 +1700,9 @@ static size_t packed_bytes(int mode, uint64_t M, uint64_t N, uint64_t K) {
   return operand_bytes(mode, M, N, Kp) + (S > 1 ? (size_t)(S * M * N * 4) : 0);
 }
 
-// Packing area.  Eager calls share a per-context grow-only area (stream order
-// keeps uses apart).  A captured GEMM uses its graph's packing region, which
+// Packing area.  Eager calls share a per-context grow-only area: stream order
+// keeps uses apart, and the caller holds pack_mu until the last kernel that
+// uses the area is launched.  A captured GEMM uses its graph's packing region, which
 // the graph owns for as long as it can be replayed; it is sized when the
 // capture begins from what vkh_gemm_reserve recorded, and a capture that
 // needs more fails and records the size for the next capture.
@@ -1761,6 +1762,7 @@ static void gemm_packed(vkh_gpu* g, int mode, bool ta, bool tb, GemmArgs& a, int
   const uint64_t pm = std::max(s.bm, PK_TR), pn = std::max(s.bn, PK_TR);
   const uint64_t Mp = ceil_div(a.M, pm) * pm, Np = ceil_div(a.N, pn) * pn;
   const uint64_t Kp = ceil_div(std::max<uint64_t>(a.K, 1), PK_KALIGN) * PK_KALIGN;
+  std::lock_guard<std::mutex> lock(g->pack_mu);
   uint16_t* base = pack_area(g, packed_bytes(mode, a.M, a.N, a.K));
   const int parts = split ? 2 : 1;
   uint16_t* Bp = base + Mp * Kp * parts;
@@ -1826,6 +1828,8 @@ static void gemm_f32(vkh_gpu* g, bool ta, bool tb, GemmArgs& a, int cfg) {
   // whole 4-element runs: contiguous extents (A: K unless transposed, else M;
   // B: N unless transposed, else K) that are multiples of 4
   const bool vec = (ta ? a.M : a.K) % 4 == 0 && (tb ? a.K : a.N) % 4 == 0;
+  std::unique_lock<std::mutex> lock(g->pack_mu, std::defer_lock);
+  if (S > 1) lock.lock();
   float* part = S > 1 ? reinterpret_cast<float*>(pack_area(g, f32_split_bytes(a.M, a.N, a.K))) : nullptr;
   c.launch(dim3((unsigned)nb, (unsigned)S), g->stream, a, ta, tb, vec, part, kc);
   check_launch("gemm");
@@ -2684,6 +2688,7 @@ int vkh_gemm_reserve(vkh_gpu* g, int mode, uint64_t M, uint64_t N, uint64_t K) {
     if (M == 0 || N == 0 || std::min(M, N) <= SKINNY_MAX || K <= SMALLK_MAX) return;
     const size_t bytes = mode == VKH_GEMM_FP32 ? f32_split_bytes(M, N, K) : packed_bytes(mode, M, N, K);
     if (bytes == 0) return;
+    std::lock_guard<std::mutex> lock(g->pack_mu);
     g->graph_pack_hint = std::max(g->graph_pack_hint, bytes);
     pack_area(g, bytes);
   });
