@@ -793,3 +793,18 @@ def test_short_rows_streamed(gpu, L, rows):
     a = vk.Array(gpu, data=x)
     np.testing.assert_array_equal(np.asarray(a.sum(axis=1)), x.sum(1))
     np.testing.assert_array_equal(np.asarray(a.maximum(axis=1)), x.max(1))
+
+
+@pytest.mark.parametrize("L", [65, 75, 79])
+def test_row_sums_of_large_operands_order(gpu, L):
+    """Odd rows of 65 to 79 elements of operands past the caches, from LDS by one
+    thread each: the sums of a wave a row (lane i has elements i and i + 64; lanes
+    i and i ^ 32 are added first), bit for bit."""
+    rows = (1 << 25) // L + 67
+    x = np.random.default_rng(L).random((rows, L), dtype=np.float32)
+    v = x[:, :64].copy()
+    v[:, :L - 64] += x[:, 64:]
+    while v.shape[1] > 1:
+        h = v.shape[1] // 2
+        v = v[:, :h] + v[:, h:]
+    assert_bits(A(gpu, x).sum(axis=1), v[:, 0])

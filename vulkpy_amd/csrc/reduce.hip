@@ -135,7 +135,10 @@ k_rows_block(const float* a, float* out, uint64_t rows, uint64_t L, int rebroadc
 
 // Medium rows (64 <= L < ROWS_BLOCK_MIN_L): LPR lanes a row, each with up to
 // NV 16-byte groups, all loaded before the first is combined (any alignment);
-// the last L % 4 elements go to the row's first lanes.  With a wave a row and
+// the last L % 4 elements go to the row's first lanes.  A lane combines its
+// groups in pairs too: no sum is longer than in a wave a row and 4-byte loads
+// (rms error over 20000 random rows 0.97 to 1.02 of that one's from 64 to 512 columns, less
+// beyond; up to 1.03 with the groups one after the other).  With a wave a row and
 // 4-byte loads 1500000 x 75 took 224 us, the second step of every row with 11 of
 // 64 lanes; 77 now, 50000 x 999 29 against 41.  LINES: rows of whole 128-byte
 // lines are read nontemporally (1500000 x 64 57 us, 64 without); a line that two
@@ -150,17 +153,22 @@ k_rows_lanes(const float* a, float* out, uint64_t rows, uint32_t L, int rebroadc
   for (uint64_t r = (uint64_t)blockIdx.x * RPB + threadIdx.x / LPR; r < rows; r += (uint64_t)gridDim.x * RPB) {
     const float* row = a + r * L;
     f32x4u_t v[NV];
-    float acc = R::init();
 #pragma unroll
     for (int q = 0; q < NV; ++q)
       if (li + q * LPR < L4)
         v[q] = ld4u<LINES>(row + 4 * (li + q * LPR));
     const bool tail = 4 * L4 + li < L;
     const float tv = tail ? row[4 * L4 + li] : 0.f;
+    float g[NV];
 #pragma unroll
     for (int q = 0; q < NV; ++q)
-      if (li + q * LPR < L4) acc = R::f(acc, R::f(R::f(v[q][0], v[q][1]), R::f(v[q][2], v[q][3])));
-    if (tail) acc = R::f(acc, tv);
+      g[q] = li + q * LPR < L4 ? R::f(R::f(v[q][0], v[q][1]), R::f(v[q][2], v[q][3])) : R::init();
+    if (tail) g[NV - 1] = R::f(g[NV - 1], tv);
+#pragma unroll
+    for (int h = NV / 2; h >= 1; h /= 2)
+#pragma unroll
+      for (int q = 0; q < h; ++q) g[q] = R::f(g[q], g[q + h]);
+    float acc = g[0];
 #pragma unroll
     for (int off = LPR / 2; off >= 1; off >>= 1) acc = R::f(acc, __shfl_xor(acc, off, 64));
     const float res = epilogue(acc, mul, dv);
@@ -259,12 +267,32 @@ k_cols(const float* a, float* dst, uint64_t prev, uint64_t K, uint64_t post, uin
 // a block's 256 rows through registers to LDS and a barrier), 4000000 x 5 16 (21).
 // From 16 elements a row on and under 64 rows a CU, too few waves have rows and
 // k_rows_lanes takes them: 500 x 63 4.9 against 7.8, 16000 x 63 5.1 against 12.
-// Rows of 64 to 96 come here where the operand is larger than the caches (NT)
-// and rows are not whole lines: 1500000 x 75 after the kernel that wrote it 78 us
-// and the next kernel 90; k_rows_lanes takes 106 and 82 with nontemporal
-// loads, 78 and 108 without.
-constexpr uint32_t ROWS_TILE_L = 63, ROWS_TILE_L_NT = 96;
-template <int OP, int VW, bool ROT, bool NT>
+// WIDE: rows of 65 to 79 elements come here where the operand is larger than the
+// caches (NT) and their length is odd (no bank conflicts for one row a lane), added in the
+// order of a wave a row (lane_tree), whose error eight accumulators of 8 to 10
+// elements exceed by 3 to 4%.  1500000 x 75 after the kernel that wrote it 78 us and the
+// next kernel 90; k_rows_lanes takes 106 and 82 with nontemporal loads, 78 and
+// 108 without.  Past 80 elements a compute unit has LDS for one block only: 1323529 x 85
+// and the write of the operand together 236 us, 224 with k_rows_lanes (75 columns: 226, 65: 220).
+constexpr uint32_t ROWS_TILE_L = 63, ROWS_TILE_L_NT = 79;
+
+// The tree a wave makes of a row of 64 to 127 elements, lane i holding elements
+// i and i + 64 (lanes i and i ^ 32 first, then i ^ 16, ...), by one thread.
+template <int OP, int I = 0, int OFF = 1>
+__device__ __forceinline__ float lane_tree(const float* row, uint32_t L) {
+  using R = Red<OP, float>;
+  if constexpr (OFF < 64) {
+    return R::f(lane_tree<OP, I, OFF * 2>(row, L), lane_tree<OP, I + OFF, OFF * 2>(row, L));
+  } else {
+    const float v = R::f(R::init(), row[I]);
+    if constexpr (I + 64 > ROWS_TILE_L_NT) return v;
+    const bool two = I + 64 < L;
+    const float w = R::f(v, row[two ? I + 64 : I]);
+    return two ? w : v;
+  }
+}
+
+template <int OP, int VW, bool ROT, bool NT, bool WIDE = false>
 __global__ void __launch_bounds__(256)
 k_rows_tile(const float* a, float* out, uint64_t rows, uint32_t L, float mul, float dv) {
   using Rd = Red<OP, float>;
@@ -290,7 +318,9 @@ k_rows_tile(const float* a, float* out, uint64_t rows, uint32_t L, float mul, fl
     }
     __builtin_amdgcn_s_waitcnt(0);  // (a wave's own LDS: no barrier)
     __builtin_amdgcn_wave_barrier();
-    if ((uint32_t)lane < nr) {
+    if (WIDE) {
+      if ((uint32_t)lane < nr) out[tile * 64 + lane] = epilogue(lane_tree<OP>(t + lane * L, L), mul, dv);
+    } else if ((uint32_t)lane < nr) {
       typedef __attribute__((ext_vector_type(VW))) float vec_t;
       const vec_t* row = reinterpret_cast<const vec_t*>(t + lane * L);
       uint32_t e = ROT ? lane % U : 0;
@@ -674,7 +704,7 @@ static void reduce_axis(vkh_gpu* g, const float* a, float* out, uint64_t prev, u
       hipLaunchKernelGGL(kernel, dim3(grid), dim3(ROW_BLOCK), 0, g->stream, a, out, rows, L, rebroadcast, mul, dv);
     } else if (L >= 4 && !rebroadcast &&
                (L <= ROWS_TILE_L ? L < 16 || rows >= (uint64_t)cus * 64
-                                 : L <= ROWS_TILE_L_NT && L % 32 != 0 && streams(rows * L))) {
+                                 : L <= ROWS_TILE_L_NT && L % 2 != 0 && streams(rows * L))) {
       const uint32_t vw = L % 4 == 0 ? 4 : (L % 2 == 0 ? 2 : 1);
       const size_t sh = sizeof(float) * 256 * L;
       const unsigned grid = (unsigned)std::min<uint64_t>(ceil_div(rows, 256), (uint64_t)cus * 8);
@@ -684,7 +714,8 @@ static void reduce_axis(vkh_gpu* g, const float* a, float* out, uint64_t prev, u
       const bool rot = (L / vw) % 2 == 0, nt = streams(rows * L);
 #define VKH_ROWS_TILE(VW, ROT) \
   do { if (nt) launch(k_rows_tile<OP, VW, ROT, true>); else launch(k_rows_tile<OP, VW, ROT, false>); } while (0)
-      if (vw == 4 && rot) VKH_ROWS_TILE(4, true);
+      if (L > ROWS_TILE_L) launch(k_rows_tile<OP, 1, false, true, true>);
+      else if (vw == 4 && rot) VKH_ROWS_TILE(4, true);
       else if (vw == 4) VKH_ROWS_TILE(4, false);
       else if (vw == 2 && rot) VKH_ROWS_TILE(2, true);
       else if (vw == 2) VKH_ROWS_TILE(2, false);
