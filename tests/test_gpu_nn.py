@@ -558,3 +558,30 @@ def test_step_in_batches_equals_single_calls(gpu):
         np.testing.assert_array_equal(np.asarray(p.value), np.asarray(q.value))
         if p.grad is not None:
             np.testing.assert_array_equal(np.asarray(p.grad), np.asarray(q.grad))
+
+
+@pytest.mark.parametrize("cols", [300, 1000, 2048, 4096])
+def test_softmax_backward_sum_error(gpu, cols):
+    """The row's sum of dy * y, read from an element with y = 1 and dy = 0: rms
+    error no larger than that of a block a row (256 threads in column order, a
+    tree a wave, the waves in order)."""
+    rows = 4000
+    rng = np.random.default_rng(cols)
+    y = rng.random((rows, cols), dtype=np.float32)
+    dy = rng.standard_normal((rows, cols), dtype=np.float32)
+    y[:, 0], dy[:, 0] = 1, 0
+    terms = y * dy
+    acc = np.zeros((rows, 256), dtype=np.float32)
+    for i in range(0, cols, 256):
+        acc[:, :min(256, cols - i)] += terms[:, i:i + 256]
+    v = acc.reshape(rows, 4, 64)
+    while v.shape[2] > 1:
+        h = v.shape[2] // 2
+        v = v[:, :, :h] + v[:, :, h:]
+    block = ((v[:, 0, 0] + v[:, 1, 0]) + v[:, 2, 0]) + v[:, 3, 0]
+    gy, gd, dx = vk.Array(gpu, data=y), vk.Array(gpu, data=dy), vk.Array(gpu, shape=y.shape)
+    call("vkh_softmax_backward", gpu._handle, gy._ptr, gd._ptr, dx._ptr, rows, cols)
+    dx._set_job([gy, gd])
+    exact = (y.astype(np.float64) * dy).sum(axis=1)
+    got, ref = (np.sqrt(((s - exact) ** 2).mean()) for s in (-np.asarray(dx)[:, 0], block))
+    assert got <= ref, (got, ref)
