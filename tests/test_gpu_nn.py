@@ -585,3 +585,21 @@ def test_softmax_backward_sum_error(gpu, cols):
     exact = (y.astype(np.float64) * dy).sum(axis=1)
     got, ref = (np.sqrt(((s - exact) ** 2).mean()) for s in (-np.asarray(dx)[:, 0], block))
     assert got <= ref, (got, ref)
+
+
+@pytest.mark.parametrize("cols", [100, 300, 1000, 2000, 5000])
+def test_softmax_long_rows_exp_in_fp64(gpu, cols):
+    """exp(-1.0149802) lies just above the middle of two FP32 values;
+    the sum of the row's four terms that are not 0 (3 in one wave's columns, one in
+    another's) is rounded once."""
+    v = np.float32(-1.0149802)
+    x = np.full((5, cols), -200, dtype=np.float32)
+    x[:, :3], x[:, 77] = 0, v
+    e = np.float32(np.exp(np.float64(v)))
+    s = np.float32(3) + e
+    gx, y = vk.Array(gpu, data=x), vk.Array(gpu, shape=x.shape)
+    call("vkh_softmax", gpu._handle, gx._ptr, y._ptr, 5, cols)
+    y._set_job([gx])
+    want = np.zeros_like(x)
+    want[:, :3], want[:, 77] = np.float32(1) / s, e / s
+    np.testing.assert_array_equal(np.asarray(y), want)

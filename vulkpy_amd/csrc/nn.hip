@@ -160,6 +160,7 @@ __device__ __forceinline__ float xent_term(float x, float y) { return (-y) * dlo
 
 // The same for long rows: a target of 0 contributes (-0) * log, a zero, wherever
 // that log is finite, so its log is not evaluated (of a one-hot row only one is).
+// (log_f32 gives dlog's value at every FP32 input but one, where it is the nearer.)
 __device__ __forceinline__ float xent_term_sparse(float x, float y) {
   const float a = x + 1e-8f;
   if (y == 0.0f && a > 0.0f && a <= 3.40282347e+38f) return 0.0f;
@@ -251,8 +252,8 @@ k_softmax_row(const float* __restrict__ x, const float* __restrict__ t, float* _
     for (int i = 0; i < NV; ++i)
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const float e = exp_f32(v[i][q] - m);
-        v[i][q] = (li + i * T) * 4 + q >= cols || e < 1.17549435e-38f ? 0.0f : e;  // (softmax_exp)
+        const float e = softmax_exp(v[i][q] - m);
+        v[i][q] = (li + i * T) * 4 + q >= cols ? 0.0f : e;
       }
     auto term = [&](int i, int q) { return v[i][q]; };
     float s;
