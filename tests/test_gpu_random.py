@@ -187,3 +187,44 @@ def test_chunks_continue_the_states(gpu, S, steps):
         np.testing.assert_array_equal(got.view(np.uint32), want.view(np.uint32))
         if n % S == 0:  # the next draw starts from the states as they were left
             np.testing.assert_array_equal(draw(whole, S * 3), draw(parts, S * 3))
+
+
+def test_alternating_draws_match_oracle(gpu):
+    """More sizes in turn than a generator keeps chunk lengths for, with longer
+    chains of a known length in between."""
+    r = vk.random.Xoshiro128pp(gpu, size=64, seed=21)
+    o = O.Xoshiro128pp(64, 21)
+    sizes = [64 * k for k in (511, 512, 600, 700, 800, 900, 1000, 1100, 1200, 1300)]
+    for n in sizes + sizes[1:4] + [64 * 4096, 64 * 64, 64 * 40000, 64 * 600] + sizes[::-1]:
+        np.testing.assert_array_equal(np.asarray(r.randint(shape=(n,))), o.randint(n))
+        assert np.isfinite(np.asarray(r.normal(shape=(n,)))).all()
+        o.normal(n)
+    np.testing.assert_array_equal(r.state(), o.state)
+
+
+def test_draws_in_turn_do_not_wait(gpu):
+    """Uniform and normal draws of one size in turn (two chunk lengths) are queued
+    behind the work of the stream, not after it."""
+    import ctypes
+    r = vk.random.Xoshiro128pp(gpu, size=64, seed=3)
+    n, m, h = 1 << 20, 8192, gpu._handle
+    u, z = vk.Array(gpu, shape=(n,)), vk.Array(gpu, shape=(n,))
+    A, C = vk.zeros(gpu, (m, m)), vk.Array(gpu, shape=(m, m))
+
+    def product():
+        call("vkh_gemm", h, 1, 0, 1, m, m, m, 1.0, A._ptr, m, A._ptr, m, 0.0, C._ptr, m, None, 0, None)
+
+    product()
+    r.random(buffer=u), r.normal(buffer=z)
+    gpu.wait()
+    for _ in range(40):  # 30 ms and more
+        product()
+    ev, done = ctypes.c_void_p(), ctypes.c_int(-1)
+    call("vkh_event_record", h, ctypes.byref(ev))
+    for _ in range(2):
+        call("vkh_xoshiro_float", r._rng, u._ptr, n)
+        call("vkh_xoshiro_normal", r._rng, z._ptr, n, 0.0, 1.0)
+    call("vkh_event_query", ev, ctypes.byref(done))
+    gpu.wait()
+    call("vkh_event_destroy", ev)
+    assert done.value == 0

@@ -16,6 +16,7 @@
 #include "fastdiv.h"
 #include "bmath.h"
 
+#include <algorithm>
 #include <array>
 #include <thread>
 
@@ -561,16 +562,21 @@ k_onehot(const uint32_t* idx, float* out, uint64_t n, uint32_t classes) {
 
 }  // namespace vkh
 
+struct JumpTable {
+  uint64_t lc = 0;  // chunk length
+  int ndigits = 0;
+  uint32_t* dev = nullptr;
+  uint64_t used = 0;  // number of the last draw that took it
+};
+
 struct vkh_xoshiro {
   vkh_gpu* gpu = nullptr;
   uint32_t size = 0;
   uint32_t* state = nullptr;  // [size][4]
   bool from_alloc = false;
-  // jump matrices of the chunked kernels, valid for chunk length jumps_lc
-  uint32_t* jumps = nullptr;
-  size_t jumps_bytes = 0;
-  uint64_t jumps_lc = 0;
-  int jumps_ndigits = 0;
+  // jump matrices of the chunked kernels, for the chunk lengths used last
+  std::vector<JumpTable> jumps;
+  uint64_t draws = 0;
 };
 
 using namespace vkh;
@@ -588,20 +594,23 @@ struct ChunkPlan {
 };
 
 constexpr uint64_t CHUNK_FULL = 128, CHUNK_MIN = 64, CHUNK_MIN_NORMAL = 32;  // steps of a chunk, at least
+constexpr uint64_t CHUNKED_MIN = 512, CHUNKED_MIN_NORMAL = 128;                       // steps of a chain, at least
 
 // Chunk the per-state chains when `units` parallel chains (states, or state
 // pairs) are too few to fill the GPU and each is long.  Up to 512 threads per
 // compute unit a chunk may be as short as `least` steps, its start-state products
 // hidden by other waves' work, up to 1024 as CHUNK_FULL; fewer than four chunks
 // do not pay for the copy of the states (65534 states, 2^23 outputs 14.6 us in
-// two chunks, 10.6 without; 64 states, 2^14 outputs 9.5 in four, 11.7).  Under
+// two chunks, 10.6 without), nor do uniform chains under eight chunks for the first
+// draws of new sizes (64 states, 8200 to 32700 outputs, no size twice: 24 us a draw in
+// chunks, 15 without; normal 23 and 71; 2^14 outputs again and again 9.6 and 12.5).  Under
 // 64 units a block of one chunk has idle lanes, which only pays where the chip
 // has room for every such wave (32 pairs, 2^20 outputs 33 us against 53, 2^28 548
 // against 363).  Not during graph capture (the jump matrices are uploaded
 // synchronously).
-ChunkPlan plan_chunks(const vkh_gpu* g, uint64_t units, uint64_t steps, uint64_t least) {
+ChunkPlan plan_chunks(const vkh_gpu* g, uint64_t units, uint64_t steps, uint64_t least, uint64_t chain) {
   ChunkPlan p;
-  if (g->capturing || steps < 4 * least) return p;
+  if (g->capturing || steps < chain) return p;
   const uint64_t cus = g->num_cus > 0 ? g->num_cus : 256, target = cus * 1024;
   if (units * 4 >= target) return p;
   const uint64_t full = std::min(ceil_div(target, units), steps / CHUNK_FULL);
@@ -624,29 +633,43 @@ ChunkPlan plan_chunks(const vkh_gpu* g, uint64_t units, uint64_t steps, uint64_t
   return p;
 }
 
+// At most 8 lengths a generator (30 to 120 KB each): uniform and normal draws of
+// a size have different ones, and draws of several sizes alternate.  A known length
+// costs nothing.  A new one goes to memory of its own, which no kernel reads yet, so
+// its copy waits for no queued work; only the memory of a length given up does.
+// 2^20 uniform and 2^20 normal draws from 64 states in turn 46 us the two, 105 with
+// one length a generator and a wait for every switch.
+constexpr size_t JUMP_TABLES = 8;
+
 const uint32_t* prepare_jumps(vkh_xoshiro* r, const ChunkPlan& p) {
-  if (r->jumps && r->jumps_lc == p.Lc && r->jumps_ndigits >= p.ndigits) return r->jumps;
+  const uint64_t now = ++r->draws;
+  auto& ts = r->jumps;
+  auto t = std::find_if(ts.begin(), ts.end(), [&](const JumpTable& x) { return x.lc == p.Lc; });
+  if (t != ts.end() && t->ndigits >= p.ndigits) {
+    t->used = now;
+    return t->dev;
+  }
+  if (t == ts.end() && ts.size() == JUMP_TABLES)
+    t = std::min_element(ts.begin(), ts.end(), [](const JumpTable& a, const JumpTable& b) { return a.used < b.used; });
   std::vector<uint32_t> host;
   chunk_jumps(p.Lc, p.ndigits, host);
-  const size_t nbytes = host.size() * sizeof(uint32_t);
-  vkh_gpu* g = r->gpu;
-  if (nbytes > r->jumps_bytes) {
-    if (r->jumps) {
-      VKH_HIP(hipStreamSynchronize(g->stream));
-      VKH_HIP(hipFree(r->jumps));
-      r->jumps = nullptr;
-      r->jumps_bytes = 0;
-    }
-    VKH_HIP(hipMalloc(&r->jumps, nbytes));
-    r->jumps_bytes = nbytes;
+  if (t != ts.end()) {  // too few digits, or the least recently used: queued draws may read it
+    VKH_HIP(hipStreamSynchronize(r->gpu->stream));
+    uint32_t* old = t->dev;
+    ts.erase(t);
+    VKH_HIP(hipFree(old));
   }
-  // synchronous: earlier chunked launches may still read the old matrices,
-  // and the host vector dies at the end of this call
-  VKH_HIP(hipStreamSynchronize(g->stream));
-  VKH_HIP(hipMemcpy(r->jumps, host.data(), nbytes, hipMemcpyHostToDevice));
-  r->jumps_lc = p.Lc;
-  r->jumps_ndigits = p.ndigits;
-  return r->jumps;
+  const size_t nbytes = host.size() * sizeof(uint32_t);
+  JumpTable n{p.Lc, p.ndigits, nullptr, now};
+  ts.reserve(JUMP_TABLES);
+  VKH_HIP(hipMalloc(&n.dev, nbytes));
+  const hipError_t e = hipMemcpy(n.dev, host.data(), nbytes, hipMemcpyHostToDevice);
+  if (e != hipSuccess) {
+    (void)hipFree(n.dev);
+    check_hip(e, "hipMemcpy");
+  }
+  ts.push_back(n);
+  return n.dev;
 }
 
 // the stores of store_out<true>: see there
@@ -658,7 +681,7 @@ template <int OUT>
 void launch_uniform(vkh_xoshiro* r, void* out, uint64_t n, uint32_t low, uint32_t range) {
   vkh_gpu* g = r->gpu;
   const bool nt = whole_lines(r, out);
-  const ChunkPlan cp = plan_chunks(g, r->size, ceil_div(n, r->size), CHUNK_MIN);
+  const ChunkPlan cp = plan_chunks(g, r->size, ceil_div(n, r->size), CHUNK_MIN, CHUNKED_MIN);
   if (cp.use) {
     const uint32_t* jumps = prepare_jumps(r, cp);
     const size_t sb = (size_t)16 * r->size;
@@ -723,10 +746,8 @@ int vkh_xoshiro_destroy(vkh_xoshiro* r) {
     VKH_REQUIRE(!r->gpu->capturing, "xoshiro_destroy: not allowed during graph capture");
     if (r->from_alloc) r->gpu->alloc->release(r->state);
     else { VKH_HIP(hipStreamSynchronize(r->gpu->stream)); VKH_HIP(hipFree(r->state)); }
-    if (r->jumps) {
-      VKH_HIP(hipStreamSynchronize(r->gpu->stream));
-      VKH_HIP(hipFree(r->jumps));
-    }
+    if (!r->jumps.empty()) VKH_HIP(hipStreamSynchronize(r->gpu->stream));
+    for (const JumpTable& t : r->jumps) VKH_HIP(hipFree(t.dev));
     delete r;
   });
 }
@@ -792,7 +813,7 @@ int vkh_xoshiro_normal(vkh_xoshiro* r, float* out, uint64_t n, float mean, float
     const uint64_t nu = n + (n & 1);  // random.py:105-123: n even, or n + 1 uniforms
     if (r->size % 2 == 0) {
       const bool nt = whole_lines(r, out);
-      const ChunkPlan cp = plan_chunks(g, r->size / 2, ceil_div(nu, r->size), CHUNK_MIN_NORMAL);
+      const ChunkPlan cp = plan_chunks(g, r->size / 2, ceil_div(nu, r->size), CHUNK_MIN_NORMAL, CHUNKED_MIN_NORMAL);
       if (cp.use) {
         const uint32_t* jumps = prepare_jumps(r, cp);
         const size_t sb = (size_t)16 * r->size;
