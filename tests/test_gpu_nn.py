@@ -603,3 +603,22 @@ def test_softmax_long_rows_exp_in_fp64(gpu, cols):
     want = np.zeros_like(x)
     want[:, :3], want[:, 77] = np.float32(1) / s, e / s
     np.testing.assert_array_equal(np.asarray(y), want)
+
+
+@pytest.mark.parametrize("klass,calls", [(nn.Dense, 2), (Parameter, 4), (nn.ReLU, 1)])
+@pytest.mark.parametrize("method", ["zero_grad", "update"])
+def test_methods_replaced_on_a_class_are_called(gpu, monkeypatch, klass, calls, method):
+    """A training step calls what a program puts in the place of a class's
+    zero_grad or update (gradient clipping, say)."""
+    net = nn.Sequence([nn.Dense(gpu, 3, 4), nn.ReLU(), nn.Dense(gpu, 4, 2)], nn.MSELoss())
+    seen = []
+    own = getattr(klass, method)
+
+    def other(self):
+        seen.append(self)
+        own(self)
+
+    monkeypatch.setattr(klass, method, other)
+    x, y = (vk.Array(gpu, data=np.ones((5, n), dtype=np.float32)) for n in (3, 2))
+    net.train(x, y)
+    assert len(seen) == calls

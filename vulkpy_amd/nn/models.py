@@ -27,6 +27,9 @@ from .parameters import Parameter, Updates, ZeroGrads, _plain
 
 __all__ = ["Sequence"]
 
+# the methods of Dense layers and of those without parameters, as defined here
+_DENSE, _MODULE = ({m: getattr(c, m) for m in ("zero_grad", "update")} for c in (Dense, Module))
+
 
 class Sequence:
     """
@@ -79,10 +82,10 @@ class Sequence:
         """``method`` of every layer in order, the parameters of Dense layers
         collected in ``batch`` (one launch for several)"""
         for layer in self.L:
-            if isinstance(layer, Dense) and _plain(layer, Dense, method):
+            if isinstance(layer, Dense) and _plain(layer, method, _DENSE[method]):
                 batch.add(layer.w)
                 batch.add(layer.b)
-            elif not _plain(layer, Module, method):
+            elif not _plain(layer, method, _MODULE[method]):
                 batch.flush()
                 getattr(layer, method)()
         batch.flush()

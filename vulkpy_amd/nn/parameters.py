@@ -121,10 +121,14 @@ class Parameter:
         self.add_grad(self.R.grad(self.value))
 
 
-def _plain(obj, klass, method: str) -> bool:
-    """Whether ``obj.method`` is ``klass``'s own, neither overridden in a
-    subclass nor replaced on the object."""
-    return getattr(type(obj), method, None) is getattr(klass, method) and method not in getattr(obj, "__dict__", ())
+def _plain(obj, method: str, own) -> bool:
+    """Whether ``obj.method`` is the function ``own``, neither overridden in a
+    subclass nor replaced on a class or on the object."""
+    return getattr(type(obj), method, None) is own and method not in getattr(obj, "__dict__", ())
+
+
+# what the batches below stand for, as defined here (a program may replace them)
+_ZERO_GRAD, _UPDATE, _ADAM_UPDATE = Parameter.zero_grad, Parameter.update, AdamState._update
 
 
 class ZeroGrads:
@@ -135,7 +139,7 @@ class ZeroGrads:
         self._grads: List[Array] = []
 
     def add(self, p: Parameter):
-        if type(p) is not Parameter or "zero_grad" in vars(p):
+        if type(p) is not Parameter or not _plain(p, "zero_grad", _ZERO_GRAD):
             self.flush()
             p.zero_grad()
         elif p.grad is not None:
@@ -167,14 +171,14 @@ class Updates:
         self._written = set()
 
     def add(self, p: Parameter):
-        if type(p) is not Parameter or "update" in vars(p):
+        if type(p) is not Parameter or not _plain(p, "update", _UPDATE):
             self.flush()
             p.update()
             return
         if p.grad is None:
             return
         state = p.opt_state
-        if (type(state) is not AdamState or "_update" in vars(state)
+        if (type(state) is not AdamState or not _plain(state, "_update", _ADAM_UPDATE)
                 or not (abs(state.opt.lr) < 1e38 and abs(state.opt.eps) < 1e38)
                 or p.value._gpu is not p.grad._gpu or p.value.size == 0):
             self.flush()
