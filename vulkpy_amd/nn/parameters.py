@@ -163,12 +163,14 @@ class ZeroGrads:
 class Updates:
     """``Parameter.update`` of many parameters: those with the framework's own
     Adam state up to ``ADAM_MULTI_MAX`` a launch, with the bits of the single
-    updates; any other parameter, or one that shares its value or state with
-    one already added, comes after those added before it."""
+    updates; any other parameter, or one that writes what one already added
+    reads or writes (a shared value or state), or reads what that one writes,
+    comes after those added before it."""
 
     def __init__(self):
         self._params: List[Parameter] = []
         self._written = set()
+        self._read = set()
 
     def add(self, p: Parameter):
         if type(p) is not Parameter or not _plain(p, "update", _UPDATE):
@@ -186,14 +188,17 @@ class Updates:
             return
         mine = (p.value._ptr, state.m._ptr, state.v._ptr)
         if (len(self._params) == ADAM_MULTI_MAX or not self._written.isdisjoint(mine)
+                or p.grad._ptr in self._written or not self._read.isdisjoint(mine)
                 or (self._params and self._params[0].value._gpu is not p.value._gpu)):
             self.flush()
         self._params.append(p)
         self._written.update(mine)
+        self._read.add(p.grad._ptr)
 
     def flush(self):
         params, self._params = self._params, []
         self._written.clear()
+        self._read.clear()
         if len(params) == 1:
             params[0].update()
             return
