@@ -256,14 +256,17 @@ int vkh_reduce_config_info(int family, int index, int* unroll, int* par);
 int vkh_reduce_get_config(vkh_gpu* gpu, int kind, uint64_t prev,
                           uint64_t axis, uint64_t post, int* index,
                           int* tuned);
-/* choose a configuration for a shape (index < 0 restores the default) */
+/* choose a configuration for a shape (index < 0 restores the default); one
+ * with a single kernel choice accepts and ignores it */
 int vkh_reduce_set_config(vkh_gpu* gpu, int kind, uint64_t prev,
                           uint64_t axis, uint64_t post, int index);
 /* times every configuration of the shape's family on scratch data (a sum;
  * one warm-up and `reps` timed runs each), keeps the fastest for the shape
  * and returns its index; ms_per_config (optional, vkh_reduce_configs
  * entries) receives each mean time in milliseconds (-1 for a configuration
- * not timed, and for a family with a single kernel choice).  same_order != 0
+ * not timed, and for a shape with a single kernel choice: VKH_RFAM_NONE, and
+ * strided axes of few columns, whose kernel has no configurations; then
+ * nothing is kept and the index is 0).  same_order != 0
  * times only the configurations that keep the default summation order, so
  * the choice cannot change a result whatever the timings.  Synchronises the
  * stream; refused during graph capture. */

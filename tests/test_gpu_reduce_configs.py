@@ -204,3 +204,11 @@ def test_autotune_same_order(gpu):
     finally:
         for problem in tuned:
             set_cfg(gpu, problem, -1)
+
+
+@pytest.mark.parametrize("shape", [(1000, 6), (5000, 999), (64, 2)])
+def test_autotune_few_columns(gpu, shape):
+    """Column sums of few columns have one kernel: nothing is timed or kept."""
+    (r,) = vk.autotune_reduce(gpu, shape, 0, reps=1)
+    assert r["family"] is None and r["config"] is None and r["best"] == 0 and set(r["ms"]) == {-1.0}
+    assert get_cfg(gpu, (1, 1, *shape)) == (0, 0)

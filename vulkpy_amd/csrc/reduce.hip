@@ -1024,8 +1024,9 @@ int vkh_reduce_autotune(vkh_gpu* g, int kind, uint64_t prev, uint64_t axis, uint
     const int fam = red_family(kind, axis, post);
     int n = 0;
     const RedCfg* cfgs = red_cfgs(fam, n);
-    if (fam == VKH_RFAM_NONE) {  // a single kernel choice
-      if (ms_per_config) ms_per_config[0] = -1.0f;
+    if (fam == VKH_RFAM_NONE || (fam == VKH_RFAM_COLS && cols_narrow(g, prev, axis, post))) {  // a single kernel choice
+      if (ms_per_config)
+        for (int i = 0; i < n; ++i) ms_per_config[i] = -1.0f;
       if (best) *best = 0;
       return;
     }

@@ -1370,7 +1370,8 @@ def autotune_reduce(gpu: GPU, shape, axis=None, *, reps: int = 3,
         best = ctypes.c_int()
         call("vkh_reduce_autotune", gpu._handle, kind, prev, K, post, int(reps), int(same_order),
              ctypes.byref(best), ms)
-        fam = REDUCE_FAMILY[f.value]
+        # (no configuration was timed: the shape has a single kernel choice)
+        fam = REDUCE_FAMILY[f.value] if any(x >= 0 for x in ms) else None
         out.append({"family": fam, "shape": (kind, prev, K, post), "best": best.value,
                     "config": reduce_configs(fam)[best.value] if fam else None,
                     "ms": [round(float(x), 5) for x in ms]})
