@@ -220,10 +220,6 @@ __device__ __forceinline__ void st_stream(float4* p, const float4& v) {
   vkh_f4v w = {v.x, v.y, v.z, v.w};
   __builtin_nontemporal_store(w, reinterpret_cast<vkh_f4v*>(p));
 }
-template <typename T>
-__device__ __forceinline__ void st_stream1(T* p, T v) {
-  __builtin_nontemporal_store(v, p);
-}
 
 // Fills p[0..n) with hashed values in [-0.5, 0.5): the scratch operands of
 // the autotuning runs (gemm.hip, block of 256 threads).
@@ -251,22 +247,6 @@ __device__ __forceinline__ float np_min(float a, float b) {
 // them within one rounding of the exact value (the FP64 oracle).
 __device__ __forceinline__ float dexp(float x) { return (float)exp((double)x); }
 __device__ __forceinline__ float dlog(float x) { return (float)log((double)x); }
-
-__device__ __forceinline__ float binop_apply(int op, float a, float b) {
-  switch (op) {
-    case VKH_ADD: return a + b;
-    case VKH_SUB: return a - b;
-    case VKH_MUL: return a * b;
-    case VKH_DIV: return a / b;
-    case VKH_MAX: return np_max(a, b);
-    case VKH_MIN: return np_min(a, b);
-    case VKH_POW: return pow_f32(a, b);
-    case VKH_RSUB: return b - a;
-    case VKH_RDIV: return b / a;
-    case VKH_RPOW: return pow_f32(b, a);
-  }
-  return 0.0f;
-}
 
 template <int OP>
 __device__ __forceinline__ float binop(float a, float b) {

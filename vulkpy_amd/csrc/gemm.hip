@@ -93,17 +93,6 @@ __device__ __forceinline__ float act_deriv_mul(int act, float y, float dy) {
   return dy;
 }
 
-// Reads 4 consecutive elements of a row (guarded at the row end).
-__device__ __forceinline__ float4 load_row4(const float* row, uint64_t c, uint64_t limit, bool vec) {
-  if (vec && c + 3 < limit) return *reinterpret_cast<const float4*>(row + c);
-  float4 v;
-  v.x = c < limit ? row[c] : 0.f;
-  v.y = c + 1 < limit ? row[c + 1] : 0.f;
-  v.z = c + 2 < limit ? row[c + 2] : 0.f;
-  v.w = c + 3 < limit ? row[c + 3] : 0.f;
-  return v;
-}
-
 // XCD-aware tile order: consecutive remapped ids share an XCD, then tiles are
 // grouped by GROUP_M rows of tiles.
 __device__ __forceinline__ void tile_coords(const GemmArgs& p, uint32_t& tm, uint32_t& tn) {
@@ -1337,10 +1326,9 @@ k_splitk_combine(const float* part, uint64_t S, GemmArgs e) {
 }
 
 // ---- pipelined BF16 products ----------------------------------------------------
-// C from packed operands on v_mfma_f32_16x16x32_bf16, for products with enough
-// tiles to fill the chip.  PARTS BF16 values stand for each operand element
-// (1: BF16 mode, 2: split mode); a packed row holds its k in groups of KG,
-// the parts of a group one after another, so a slice of every row is ROWB
+// C from packed operands on v_mfma_f32_16x16x32_bf16.  PARTS BF16 values stand
+// for each operand element (1: BF16 mode, 2: split mode); a packed row holds its
+// k in groups of KG, the parts of a group one after another, so a slice of every row is ROWB
 // contiguous bytes in every mode.
 //
 // What bounds a loop that fills LDS, waits at a barrier and multiplies is the
@@ -1570,18 +1558,17 @@ static void launch_pipe(dim3 grid, hipStream_t s, const PackedArgs& pa) {
 struct PackedCfg {
   int bm, bn, bk, waves, wm;  // wm: rows of a wave's slab (BM / WGM)
   PackedLaunch launch;
-  int direct = 0;  // operand slices loaded from global memory straight into LDS
 };
 static const PackedCfg BF16_CFGS[] = {
-    {256, 256, 64, 8, 128, launch_pipe<256, 256, 2, 4, 1>, 1},
-    {128, 128, 64, 4, 64, launch_pipe<128, 128, 2, 2, 1>, 1},
-    {64, 64, 64, 4, 32, launch_pipe<64, 64, 2, 2, 1>, 1},
+    {256, 256, 64, 8, 128, launch_pipe<256, 256, 2, 4, 1>},
+    {128, 128, 64, 4, 64, launch_pipe<128, 128, 2, 2, 1>},
+    {64, 64, 64, 4, 32, launch_pipe<64, 64, 2, 2, 1>},
     // (256 x 128 and 128 x 256 with 8 waves were fastest on none of 16 shapes)
 };
 static const PackedCfg SPLIT_CFGS[] = {
-    {256, 256, 32, 8, 128, launch_pipe<256, 256, 2, 4, 2>, 1},
-    {128, 128, 32, 4, 64, launch_pipe<128, 128, 2, 2, 2>, 1},
-    {64, 64, 32, 4, 32, launch_pipe<64, 64, 2, 2, 2>, 1},
+    {256, 256, 32, 8, 128, launch_pipe<256, 256, 2, 4, 2>},
+    {128, 128, 32, 4, 64, launch_pipe<128, 128, 2, 2, 2>},
+    {64, 64, 32, 4, 32, launch_pipe<64, 64, 2, 2, 2>},
 };
 constexpr int PK_MAXTILE = 256;  // largest bm / bn of any configuration
 
@@ -1620,12 +1607,13 @@ static const TileCost BF16_COST[] = {{0, 256, 4.0, 0.0, 22.9, 22.9}, {1, 128, 3.
 static const TileCost SPLIT_COST[] = {{0, 256, 4.0, 0.0, 59.5, 59.5}, {1, 128, 3.5, 0.0, 22.0, 18.9},
                                       {2, 64, 2.5, 0.0, 11.0, 6.3}};
 
-// the least estimated time (us) and its configuration
-static double tile_estimate(int mode, uint64_t M, uint64_t N, uint64_t K, int& cfg) {
+// the configuration with the least estimated time (us)
+static int default_cfg(int mode, uint64_t M, uint64_t N, uint64_t K) {
   const bool f32 = mode == VKH_GEMM_FP32;
   const TileCost* T = f32 ? F32_COST : mode == VKH_GEMM_BF16 ? BF16_COST : SPLIT_COST;
   const uint64_t k = std::max<uint64_t>(K, 1), Kp = f32 ? k : ceil_div(k, (uint64_t)PK_KALIGN) * PK_KALIGN;
   const uint64_t kc = f32 ? f32_splitk_chunk(M, N, Kp) : splitk_chunk(M, N, Kp), S = ceil_div(Kp, kc);
+  int cfg = 0;
   double bt = 0;
   for (int i = 0; i < (f32 ? 4 : 3); ++i) {
     const double n = (double)ceil_div(ceil_div(M, T[i].tile) * ceil_div(N, T[i].tile) * S, (uint64_t)256);
@@ -1633,12 +1621,6 @@ static double tile_estimate(int mode, uint64_t M, uint64_t N, uint64_t K, int& c
                      1e-3 * (double)kc * std::max(T[i].alone_ns, T[i].shared_ns * n);
     if (i == 0 || t < bt) { cfg = T[i].cfg; bt = t; }
   }
-  return bt;
-}
-
-static int default_cfg(int mode, uint64_t M, uint64_t N, uint64_t K) {
-  int cfg = 0;
-  tile_estimate(mode, M, N, K, cfg);
   return cfg;
 }
 
@@ -2509,7 +2491,7 @@ int vkh_gemm_config_info(int mode, int index, int* bm, int* bn, int* bk, int* wa
     const PackedCfg* c = packed_cfgs(mode, n);
     VKH_REQUIRE(index >= 0 && index < n, "configuration index out of range");
     *bm = c[index].bm; *bn = c[index].bn; *bk = c[index].bk; *waves = c[index].waves;
-    if (direct) *direct = c[index].direct;
+    if (direct) *direct = 1;  // (operand slices from global memory straight into LDS)
   });
 }
 
