@@ -855,3 +855,14 @@ def test_products_of_several_threads(gpu):
         for C in out:
             C._set_job([A, B])
             np.testing.assert_array_equal(np.asarray(C).view(np.uint32), np.asarray(want).view(np.uint32))
+
+
+@pytest.mark.parametrize("M,N,K,tile", [(4096, 16384, 256, 128), (16384, 16384, 64, 64), (16384, 4096, 4096, 256),
+                                        (8192, 8192, 8192, 256), (150, 32, 32, 32)])
+def test_fp32_default_tile(gpu, M, N, K, tile):
+    """Large outputs over short k take small tiles: a 256 x 256 one's epilogue
+    has no other block on its CU to hide behind."""
+    import ctypes
+    index = ctypes.c_int()
+    _lib.call("vkh_gemm_get_config", gpu._handle, 0, 0, 0, M, N, K, ctypes.byref(index), None)
+    assert vk.gemm_configs("fp32")[index.value]["bm"] == tile

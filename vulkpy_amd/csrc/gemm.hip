@@ -1587,10 +1587,12 @@ static const PackedCfg* packed_cfgs(int mode, int& count) {
 // 1024 150 / 212 / 288.
 // Split mode, packing included: 1024^3 68 / 36 / 26, 4096 x 1024 x 1024 75 /
 // 46 / 47, 3000^3 194 / 195 / 284, 8192^3 2172 / 2697 / 3508.
-// FP32 tiles likewise (the 256 x 256 tile only for its column sums and where
-// its blocks fill the chip evenly), us for 128 / 64 / 32: 150 x 32 x 32 12.2 /
-// 3.9 / 3.3, 512^3 43 / 19 / 9.6, 5137 x 586 x 270 44 / 35 / 35, 2048 x 2048 x
-// 512 50 / 54 / 63, 4096 x 1024 x 1024 92 / 102 / 123.
+// FP32 tiles likewise (the 256 x 256 tile for long k, where its blocks, whose
+// epilogue is not hidden by another block of the CU, fill the chip evenly), us for 128 / 64 / 32: 150 x 32
+// x 32 12.2 / 3.9 / 3.3, 512^3 43 / 19 / 9.6, 5137 x 586 x 270 44 / 35 / 35, 2048 x
+// 2048 x 512 50 / 54 / 63, 4096 x 1024 x 1024 92 / 102 / 123; for 256 / 128: 4096 x
+// 16384 x 256 362 / 314, 65536 x 1024 x 1024 1074 / 1054, 16384 x 4096 x 4096 3950 /
+// 4002, 8192^3 7759 / 7935.
 static uint64_t splitk_chunk(uint64_t M, uint64_t N, uint64_t Kp);
 static uint64_t f32_splitk_chunk(uint64_t M, uint64_t N, uint64_t K);
 
@@ -1600,8 +1602,8 @@ struct TileCost {
   // us once, and a block; ns a k of a block: alone on its CU, and sharing it
   double fixed_us, block_us, alone_ns, shared_ns;
 };
-static const TileCost F32_COST[] = {{0, 128, 5.0, 3.0, 76.0, 61.0}, {2, 64, 3.0, 0.0, 32.0, 25.0},
-                                    {3, 32, 2.5, 0.0, 14.0, 9.0}, {1, 256, 8.0, 6.0, 239.0, 239.0}};
+static const TileCost F32_COST[] = {{0, 128, 5.0, 4.2, 76.0, 60.0}, {2, 64, 3.0, 0.0, 32.0, 25.0},
+                                    {3, 32, 2.5, 0.0, 14.0, 9.0}, {1, 256, 8.0, 30.0, 233.0, 233.0}};
 static const TileCost BF16_COST[] = {{0, 256, 4.0, 0.0, 22.9, 22.9}, {1, 128, 3.5, 0.0, 8.2, 7.5},
                                      {2, 64, 2.5, 0.0, 4.7, 3.5}};
 static const TileCost SPLIT_COST[] = {{0, 256, 4.0, 0.0, 59.5, 59.5}, {1, 128, 3.5, 0.0, 22.0, 18.9},
