@@ -1291,7 +1291,7 @@ static const F32Cfg F32_CFGS[] = {
     {64, 64, 4, 32, launch_f32_small<64, 32>},
     {32, 32, 4, 16, launch_f32_small<32, 64>},
 };
-constexpr int F32_NCFG = sizeof(F32_CFGS) / sizeof(F32_CFGS[0]);
+constexpr int F32_NCFG = sizeof(F32_CFGS) / sizeof(F32_CFGS[0]), F32_CFG_256 = 1;
 
 // Sums the S k-chunk partials of each output in chunk order and applies the
 // GEMM epilogue (alpha, beta * C, bias, activation, aux derivative, BF16 copy).
@@ -1636,6 +1636,17 @@ static int mode_cfgs(int mode) {
 
 static std::array<uint64_t, 6> cfg_key(int mode, int ta, int tb, uint64_t M, uint64_t N, uint64_t K) {
   return {(uint64_t)mode, (uint64_t)(ta != 0), (uint64_t)(tb != 0), M, N, K};
+}
+
+// The configuration of a product on a context: the one chosen for it, else the
+// default.  With column sums, which need waves of 128-row slabs, large FP32
+// products default to their 256 x 256 tile whatever is faster without.
+static int product_cfg(const vkh_gpu* g, int mode, int ta, int tb, uint64_t M, uint64_t N, uint64_t K, bool colsum) {
+  auto it = g->gemm_cfg.find(cfg_key(mode, ta, tb, M, N, K));
+  if (it != g->gemm_cfg.end()) return it->second;
+  if (colsum && mode == VKH_GEMM_FP32 && ceil_div(M, (uint64_t)256) * ceil_div(N, (uint64_t)256) >= 512)
+    return F32_CFG_256;
+  return default_cfg(mode, M, N, K);
 }
 
 // Fills p[0..n) with values in [-0.5, 0.5) from a hash of the index (operands
@@ -2454,15 +2465,13 @@ static void gemm_impl(vkh_gpu* g, int mode, int trans_a, int trans_b, uint64_t M
   }
   switch (mode) {
     case VKH_GEMM_FP32: {
-      auto it = g->gemm_cfg.find(cfg_key(mode, trans_a, trans_b, M, N, K));
-      gemm_f32(g, trans_a, trans_b, a, it != g->gemm_cfg.end() ? it->second : default_cfg(mode, M, N, K));
+      gemm_f32(g, trans_a, trans_b, a, product_cfg(g, mode, trans_a, trans_b, M, N, K, cs != nullptr));
       break;
     }
     case VKH_GEMM_BF16:
     case VKH_GEMM_BF16X3: {
-      auto it = g->gemm_cfg.find(cfg_key(mode, trans_a, trans_b, M, N, K));
       const bool pre = mode == VKH_GEMM_BF16 && K % PK_KALIGN == 0;
-      gemm_packed(g, mode, trans_a, trans_b, a, it != g->gemm_cfg.end() ? it->second : default_cfg(mode, M, N, K),
+      gemm_packed(g, mode, trans_a, trans_b, a, product_cfg(g, mode, trans_a, trans_b, M, N, K, cs != nullptr),
                   pre ? a_bf16 : nullptr, pre ? b_bf16 : nullptr);
       break;
     }
@@ -2726,8 +2735,7 @@ static bool colsum_ok(vkh_gpu* g, int mode, int ta, int tb, uint64_t M, uint64_t
   if (std::min(M, N) <= SKINNY_MAX || K <= SMALLK_MAX) return false;
   if (mode < VKH_GEMM_FP32 || mode > VKH_GEMM_BF16X3) return false;
   if (bias_grad_chunk(g, M, N) != (uint64_t)CS_ROWS) return false;
-  auto it = g->gemm_cfg.find(cfg_key(mode, ta, tb, M, N, K));
-  const int cfg = it != g->gemm_cfg.end() ? it->second : default_cfg(mode, M, N, K);
+  const int cfg = product_cfg(g, mode, ta, tb, M, N, K, true);
   if (mode == VKH_GEMM_FP32)
     return F32_CFGS[cfg].wm == CS_ROWS && ceil_div(K, f32_splitk_chunk(M, N, K)) == 1;
   int n = 0;
