@@ -489,6 +489,10 @@ __device__ __forceinline__ void staged_epilogue(float* smem, const Acc& acc, con
   // it: 1 (positive), NaN (NaN) or 0
   constexpr int WPP = (ITER + 3) / 4;  // code words of a pass
   uint32_t cwp[WPP];
+  auto codes = [&](auto ic) __attribute__((always_inline)) {
+#pragma unroll
+    for (int w = 0; w < WPP; ++w) cwp[w] = cw[decltype(ic)::value * ITER / 4 + w];
+  };
   auto relu_x = [&](int k) {
     const uint32_t byte = (cwp[k / 4] >> (8 * (k % 4))) & 0xffu;
     f32x4_t xv;
@@ -510,20 +514,9 @@ __device__ __forceinline__ void staged_epilogue(float* smem, const Acc& acc, con
     }
   };
   if (xpre && AHEAD) load_aux(0, 0);
-  // Pass i: rows i*32 .. i*32+31 of the sub-tile.  One copy of the pass's code:
-  // only the staging of its accumulators (whose registers need constant
-  // indices) is unrolled.  With every pass unrolled the kernels took 64-128 KB,
-  // more than the instruction cache holds, and a block's epilogue waited for
-  // its instructions: a single 256 x 256 tile with K = 256 took 30-40 us.
-#pragma unroll 1
-  for (int i = 0; i < TM; ++i) {
-    static_for<TM>([&](auto ic) __attribute__((always_inline)) {
-      if (i == decltype(ic)::value) {
-        stage_pass<decltype(ic)::value, SROW>(st, acc);
-#pragma unroll
-        for (int w = 0; w < WPP; ++w) cwp[w] = cw[decltype(ic)::value * ITER / 4 + w];
-      }
-    });
+  // Pass i: rows i*32 .. i*32+31 of the sub-tile, its accumulators staged first
+  // (their registers need constant indices).
+  auto pass = [&](int i) __attribute__((always_inline)) {
     __syncthreads();
     const uint64_t mb = m0 + wm * WM + i * 32;
     if (lane_fast && mb + 31 < e.M) {
@@ -598,6 +591,28 @@ __device__ __forceinline__ void staged_epilogue(float* smem, const Acc& acc, con
         }
       }
       __syncthreads();
+    }
+  };
+  // Two passes (128 x 128 tiles) share one copy of the code: a block alone on its
+  // CU waits for its instructions otherwise.  The four of a 256 x 256 tile have
+  // one each, whose accumulators die with it: a loop over them spills 104
+  // registers (16384 x 4096 x 256 in such tiles 364 us, 351 so; x 4096 4045 and 4023).
+  if constexpr (TM > 2) {
+    static_for<TM>([&](auto ic) __attribute__((always_inline)) {
+      stage_pass<decltype(ic)::value, SROW>(st, acc);
+      codes(ic);
+      pass(decltype(ic)::value);
+    });
+  } else {
+#pragma unroll 1
+    for (int i = 0; i < TM; ++i) {
+      static_for<TM>([&](auto ic) __attribute__((always_inline)) {
+        if (i == decltype(ic)::value) {
+          stage_pass<decltype(ic)::value, SROW>(st, acc);
+          codes(ic);
+        }
+      });
+      pass(i);
     }
   }
   if (csum && lane < WN) {
@@ -1588,11 +1603,11 @@ static const PackedCfg* packed_cfgs(int mode, int& count) {
 // Split mode, packing included: 1024^3 68 / 36 / 26, 4096 x 1024 x 1024 75 /
 // 46 / 47, 3000^3 194 / 195 / 284, 8192^3 2172 / 2697 / 3508.
 // FP32 tiles likewise (the 256 x 256 tile for long k, where its blocks, whose
-// epilogue is not hidden by another block of the CU, fill the chip evenly), us for 128 / 64 / 32: 150 x 32
-// x 32 12.2 / 3.9 / 3.3, 512^3 43 / 19 / 9.6, 5137 x 586 x 270 44 / 35 / 35, 2048 x
-// 2048 x 512 50 / 54 / 63, 4096 x 1024 x 1024 92 / 102 / 123; for 256 / 128: 4096 x
-// 16384 x 256 362 / 314, 65536 x 1024 x 1024 1074 / 1054, 16384 x 4096 x 4096 3950 /
-// 4002, 8192^3 7759 / 7935.
+// epilogue is not hidden by another block of the CU, fill the chip evenly), us for
+// 128 / 64 / 32: 150 x 32 x 32 12.2 / 3.9 / 3.3, 512^3 43 / 19 / 9.6, 1024^3 33 / 36 /
+// 41, 5137 x 586 x 270 44 / 35 / 35, 2048 x 2048 x 512 50 / 54 / 63, 4096 x 1024 x 1024
+// 92 / 102 / 123; for 256 / 128: 16384 x 4096 x 256 351 / 317, 65536 x 1024 x 1024 1092 /
+// 1090, 8192 x 8192 x 2048 2064 / 2118, 16384 x 4096 x 4096 4023 / 4174, 8192^3 7935 / 8350.
 static uint64_t splitk_chunk(uint64_t M, uint64_t N, uint64_t Kp);
 static uint64_t f32_splitk_chunk(uint64_t M, uint64_t N, uint64_t K);
 
@@ -1602,8 +1617,8 @@ struct TileCost {
   // us once, and a block; ns a k of a block: alone on its CU, and sharing it
   double fixed_us, block_us, alone_ns, shared_ns;
 };
-static const TileCost F32_COST[] = {{0, 128, 5.0, 4.2, 76.0, 60.0}, {2, 64, 3.0, 0.0, 32.0, 25.0},
-                                    {3, 32, 2.5, 0.0, 14.0, 9.0}, {1, 256, 8.0, 30.0, 233.0, 233.0}};
+static const TileCost F32_COST[] = {{0, 128, 5.0, 3.0, 76.0, 61.0}, {2, 64, 3.0, 0.0, 32.0, 25.0},
+                                    {3, 32, 2.5, 0.0, 14.0, 9.0}, {1, 256, 8.0, 28.0, 233.0, 233.0}};
 static const TileCost BF16_COST[] = {{0, 256, 4.0, 0.0, 22.9, 22.9}, {1, 128, 3.5, 0.0, 8.2, 7.5},
                                      {2, 64, 2.5, 0.0, 4.7, 3.5}};
 static const TileCost SPLIT_COST[] = {{0, 256, 4.0, 0.0, 59.5, 59.5}, {1, 128, 3.5, 0.0, 22.0, 18.9},
