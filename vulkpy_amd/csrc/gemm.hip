@@ -394,35 +394,25 @@ __device__ __forceinline__ void store_part4(float* part, uint64_t N, uint64_t m,
   }
 }
 
-// Epilogue of a block whose waves each hold the accumulator blocks of a
-// WM x WN sub-tile at (wm, wn): with 32 x 32 blocks acc[i][j][r] is C[m, n],
-// m = m0 + wm*WM + i*32 + (r/4)*8 + lhi*4 + r%4 and n = n0 + wn*WN + j*32 +
-// l32 (l32 = lane % 32, lhi = lane / 32).  Each wave writes rows i*32 .. i*32+31 of its sub-tile to its own
-// 32 x (WN+4) float staging slice of `smem`, then reads them back as 4-float
+// Epilogue of a block whose waves each hold TM x TN 32 x 32 accumulator blocks
+// of a WM x WN sub-tile at (wm, wn): acc[i][j][r] is C[m, n] with m = m0 + wm*WM +
+// i*32 + (r/4)*8 + lhi*4 + r%4 and n = n0 + wn*WN + j*32 + l32 (l32 = lane % 32,
+// lhi = lane / 32).  Each wave writes rows i*32 .. i*32+31 of its sub-tile to its
+// own 32 x (WN+4) float staging slice of `smem`, then reads them back as 4-float
 // row segments (WN/4 lanes per row), so C is accessed in whole row segments.
 // With `part` the raw sums go to that k chunk's partial matrix instead.  For
 // the transposed BF16 copy (e.Cbft) the row pass puts the final values back
 // into the slice and each group of four lanes converts one column of 32 rows
 // into a 64-byte run.  The caller's operand tiles in `smem` must be dead (a
 // barrier before the call).
-
-// rows i*32 .. i*32+31 of a wave's accumulators into its staging slice
-template <int I, int SROW, int TM, int TN>
-__device__ __forceinline__ void stage_pass(float* st, const f32x16_t (&acc)[TM][TN]) {
-  const int l32 = threadIdx.x & 31, lhi = (threadIdx.x >> 5) & 1;
-#pragma unroll
-  for (int j = 0; j < TN; ++j)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) st[((r / 4) * 8 + lhi * 4 + (r % 4)) * SROW + j * 32 + l32] = acc[I][j][r];
-}
-
-template <int WM, int WN, typename Acc>
-__device__ __forceinline__ void staged_epilogue(float* smem, const Acc& acc, const GemmArgs& e,
+template <int WM, int WN, int TM, int TN>
+__device__ __forceinline__ void staged_epilogue(float* smem, const f32x16_t (&acc)[TM][TN], const GemmArgs& e,
                                                 float* part, uint64_t m0, uint64_t n0, int wm, int wn) {
-  constexpr int TM = WM / 32;  // passes of 32 rows
+  static_assert(TM * 32 == WM && TN * 32 == WN, "a pass is 32 rows");
   constexpr int SROW = WN + 4, F4R = WN / 4, RPI = 64 / F4R;
   static_assert(64 % F4R == 0, "whole rows per wave pass");
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int l32 = lane & 31, lhi = lane >> 5;
   float* st = smem + wave * 32 * SROW;
   const uint64_t nb = n0 + wn * WN;
   const bool tr = e.Cbft && !part;
@@ -485,16 +475,10 @@ __device__ __forceinline__ void staged_epilogue(float* smem, const Acc& acc, con
       }
     }
   }
-  // ReLU' of the aux values of the pass's row segment k, as act_deriv_mul finds
-  // it: 1 (positive), NaN (NaN) or 0
-  constexpr int WPP = (ITER + 3) / 4;  // code words of a pass
-  uint32_t cwp[WPP];
-  auto codes = [&](auto ic) __attribute__((always_inline)) {
-#pragma unroll
-    for (int w = 0; w < WPP; ++w) cwp[w] = cw[decltype(ic)::value * ITER / 4 + w];
-  };
-  auto relu_x = [&](int k) {
-    const uint32_t byte = (cwp[k / 4] >> (8 * (k % 4))) & 0xffu;
+  // ReLU' of segment seg's aux values, as act_deriv_mul finds it: 1 (positive),
+  // NaN (NaN) or 0
+  auto relu_x = [&](int seg) {
+    const uint32_t byte = (cw[seg / 4] >> (8 * (seg % 4))) & 0xffu;
     f32x4_t xv;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
@@ -514,9 +498,14 @@ __device__ __forceinline__ void staged_epilogue(float* smem, const Acc& acc, con
     }
   };
   if (xpre && AHEAD) load_aux(0, 0);
-  // Pass i: rows i*32 .. i*32+31 of the sub-tile, its accumulators staged first
-  // (their registers need constant indices).
-  auto pass = [&](int i) __attribute__((always_inline)) {
+  // pass i: rows i*32 .. i*32+31 of the sub-tile (a constant i: the registers of
+  // its accumulators need constant indices)
+  auto pass = [&](auto ic) __attribute__((always_inline)) {
+    constexpr int i = decltype(ic)::value;
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) st[((r / 4) * 8 + lhi * 4 + (r % 4)) * SROW + j * 32 + l32] = acc[i][j][r];
     __syncthreads();
     const uint64_t mb = m0 + wm * WM + i * 32;
     if (lane_fast && mb + 31 < e.M) {
@@ -529,7 +518,7 @@ __device__ __forceinline__ void staged_epilogue(float* smem, const Acc& acc, con
           const float4 v = *reinterpret_cast<const float4*>(st + rr * SROW + cc);
           const f32x4_t c = e.beta != 0.f ? *reinterpret_cast<const f32x4_t*>(e.C + (mb + rr) * e.ldc + n) : z;
           const float4 f = relu_codes
-                               ? finish4<false, true>(e, mb + rr, n, v, true, 4, c, bq, relu_x(k0 + k), false)
+                               ? finish4<false, true>(e, mb + rr, n, v, true, 4, c, bq, relu_x(i * ITER + k0 + k), false)
                                : finish4<false>(e, mb + rr, n, v, true, 4, c, bq, xq[k], false);
           if (csum || tr) *reinterpret_cast<float4*>(st + rr * SROW + cc) = f;
         }
@@ -593,28 +582,11 @@ __device__ __forceinline__ void staged_epilogue(float* smem, const Acc& acc, con
       __syncthreads();
     }
   };
-  // Two passes (128 x 128 tiles) share one copy of the code: a block alone on its
-  // CU waits for its instructions otherwise.  The four of a 256 x 256 tile have
-  // one each, whose accumulators die with it: a loop over them spills 104
-  // registers (16384 x 4096 x 256 in such tiles 364 us, 351 so; x 4096 4045 and 4023).
-  if constexpr (TM > 2) {
-    static_for<TM>([&](auto ic) __attribute__((always_inline)) {
-      stage_pass<decltype(ic)::value, SROW>(st, acc);
-      codes(ic);
-      pass(decltype(ic)::value);
-    });
-  } else {
-#pragma unroll 1
-    for (int i = 0; i < TM; ++i) {
-      static_for<TM>([&](auto ic) __attribute__((always_inline)) {
-        if (i == decltype(ic)::value) {
-          stage_pass<decltype(ic)::value, SROW>(st, acc);
-          codes(ic);
-        }
-      });
-      pass(i);
-    }
-  }
+  // A copy of the code for each pass, whose accumulators die with it: a loop over
+  // the passes of a 256 x 256 tile spills 104 registers (16384 x 4096 x 256 in such
+  // tiles 364 us, 351 so; x 4096 4045 and 4023), over those of a 128 x 128 tile it
+  // costs 2% at 2500^3 and saves 1.7% with B transposed.
+  static_for<TM>([&](auto ic) __attribute__((always_inline)) { pass(ic); });
   if (csum && lane < WN) {
     const uint64_t m = m0 + wm * WM, nc = nb + lane;
     if (m < e.M && nc < e.N) e.cs[(m / CS_ROWS) * e.N + nc] = csacc;
