@@ -5,7 +5,11 @@
 // Here a block computes a BM x BN tile: operand slices are staged through LDS
 // ahead of their use, and each wave owns a sub-tile of 32 x 32 or 16 x 16 MFMA
 // blocks:
-//   FP32    v_mfma_f32_32x32x2_f32    (operands as stored)
+//   FP32    v_mfma_f32_32x32x2_f32, 16x16x4 for few outputs (operands as stored;
+//           an FP32 MFMA adds its terms one after the other, each rounded once, as
+//           fma does.  Three BF16 parts of an element on the BF16 matrix cores took
+//           4.4 ms at 8192^3, 7.9 so, but those round their sums more coarsely: an
+//           output of one nonzero term was up to 1.42 ulp off, 0.5 so)
 //   BF16    v_mfma_f32_16x16x32_bf16  (operands rounded to nearest-even BF16)
 //   BF16X3  the same instruction three times: lo*hi + hi*lo + hi*hi, where
 //           x = hi + lo + O(2^-16 |x|) with hi = bf16(x), lo = bf16(x - hi)
@@ -1337,7 +1341,7 @@ k_splitk_combine(const float* part, uint64_t S, GemmArgs e) {
 // staggered waves but loads one slice ahead, 855 us without the stagger, 955 us
 // with 32 x 32 x 16 instructions), 16384 x 4096 x 4096 405-430 against 490-583 us.
 // One 16 x 16 x 32 instruction gives the bits of the two 32 x 32 x 16 ones it
-// replaces, so results equal k_gemm_packed's.
+// replaces.
 __device__ __forceinline__ void load_lds16(const char* src, char* dst) {
 #ifdef __HIP_DEVICE_COMPILE__  // (the host pass would drop the launch stub of a template that uses the builtin)
   __builtin_amdgcn_global_load_lds(src, dst, 16, 0, 0);
