@@ -808,3 +808,18 @@ def test_row_sums_of_large_operands_order(gpu, L):
         h = v.shape[1] // 2
         v = v[:, :h] + v[:, h:]
     assert_bits(A(gpu, x).sum(axis=1), v[:, 0])
+
+
+@pytest.mark.parametrize("cols", [508, 509, 700, 999, 1023])
+@pytest.mark.parametrize("rows", [200, 300, 400, 500, 1000])
+def test_column_sums_error_few_rows(gpu, rows, cols):
+    """Sums of some hundred rows of up to 1023 columns: no further from 64 bits than
+    chunks of 32 rows and more, each added in row order and then in chunk order."""
+    x = np.random.default_rng(rows * cols).random((8, rows, cols), dtype=np.float32)
+    exact = x.astype(np.float64).sum(axis=1)
+    step = -(-rows // (rows // 32))
+    part = [x[:, k:k + step].cumsum(axis=1, dtype=np.float32)[:, -1] for k in range(0, rows, step)]
+    ref = np.stack(part, axis=1).cumsum(axis=1, dtype=np.float32)[:, -1]
+    got = np.stack([np.asarray(A(gpu, m).sum(axis=0)) for m in x])
+    rms = lambda s: np.sqrt(((s.astype(np.float64) - exact) ** 2).mean())
+    assert rms(got) <= rms(ref)

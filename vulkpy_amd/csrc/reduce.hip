@@ -368,12 +368,17 @@ k_rows_tile(const float* a, float* out, uint64_t rows, uint32_t L, float mul, fl
 // t / G, + R, + 2R ... of its chunk, so that a block reads its chunk as one
 // contiguous run; the R sums of a column are then combined by a tree in LDS.
 // Chunk partials dst[p][c][post] are reduced by the same kernel, in as many
-// more passes as leave each thread about 16 rows.  k_cols gives every chunk a block of which only G threads work (1000000
-// x 16: 4 of 256) and combines up to 1024 chunks one after the other.  Against
-// it: 1000000 x 16 18 against 161 us, 3000000 x 3 11 against 371, 1500000 x 75
-// 78 against 678, 50000 x 999 44 against 120 (element loads), 50000 x 1000 43
-// against 60 (87 with one last pass over all 1024 chunks).
-template <int OP, int VW, int U, bool NT>
+// more passes as leave each thread about 16 rows.  Rows in flight are combined in
+// pairs, eight, then four, two and one: where a row takes more than half of the
+// block (513 columns and more), the last pass has up to 31 chunk sums a thread, and
+// one after the other these made the rms error of 200 to 500 rows 1.03 to 1.31
+// times that of k_cols (in pairs 0.71 to 0.95).  k_cols gives every chunk a block
+// of which only G threads work (1000000 x 16: 4 of 256) and combines up to 1024
+// chunks one after the other.  Against it: 1000000 x 16 18 against 161 us, 3000000
+// x 3 11 against 371, 1500000 x 75 78 against 678, 50000 x 999 44 against 120
+// (element loads), 50000 x 1000 43 against 60 (87 with one last pass over all 1024
+// chunks).
+template <int OP, int VW, bool NT>
 __global__ void __launch_bounds__(256)
 k_cols_narrow(const float* a, float* dst, uint64_t K, uint32_t post, uint64_t kchunk, uint32_t G, uint32_t R,
               int final_pass, float mul, float dv, float beta) {
@@ -397,21 +402,25 @@ k_cols_narrow(const float* a, float* dst, uint64_t K, uint32_t post, uint64_t kc
   if (rr < n) {
     load(k0 + rr, acc);
     uint64_t k = k0 + rr + R;
-    for (; k + (uint64_t)(U - 1) * R < k1; k += (uint64_t)U * R) {
-      float v[U][VW];
+    auto rows = [&](auto count) {  // rows in flight, combined in pairs
+      constexpr int N = decltype(count)::value;
+      float v[N][VW];
 #pragma unroll
-      for (int q = 0; q < U; ++q) load(k + (uint64_t)q * R, v[q]);
+      for (int q = 0; q < N; ++q) load(k + (uint64_t)q * R, v[q]);
 #pragma unroll
-      for (int q = 0; q < U; ++q)
+      for (int s = 1; s < N; s *= 2)
 #pragma unroll
-        for (int w = 0; w < VW; ++w) acc[w] = Rd::f(acc[w], v[q][w]);
-    }
-    for (; k < k1; k += R) {
-      float v[VW];
-      load(k, v);
+        for (int q = 0; q < N; q += 2 * s)
 #pragma unroll
-      for (int w = 0; w < VW; ++w) acc[w] = Rd::f(acc[w], v[w]);
-    }
+          for (int w = 0; w < VW; ++w) v[q][w] = Rd::f(v[q][w], v[q + s][w]);
+#pragma unroll
+      for (int w = 0; w < VW; ++w) acc[w] = Rd::f(acc[w], v[0][w]);
+      k += (uint64_t)N * R;
+    };
+    while (k + 7 * (uint64_t)R < k1) rows(std::integral_constant<int, 8>());
+    if (k + 3 * (uint64_t)R < k1) rows(std::integral_constant<int, 4>());
+    if (k + R < k1) rows(std::integral_constant<int, 2>());
+    if (k < k1) rows(std::integral_constant<int, 1>());
 #pragma unroll
     for (int w = 0; w < VW; ++w) lds[w * 256 + threadIdx.x] = acc[w];
   }
@@ -676,8 +685,8 @@ static void reduce_cols_narrow(vkh_gpu* g, const float* a, float* out, uint64_t 
   nchunk = ceil_div(K, kchunk);
   auto launch = [&](const float* src, float* dst, uint64_t k, uint64_t kc, uint64_t nc, int fin) {
     const dim3 grid((unsigned)nc, (unsigned)prev);
-    auto kernel = post < 4 ? k_cols_narrow<OP, 1, 8, false>
-                           : (streams(prev * K * post) ? k_cols_narrow<OP, 4, 8, true> : k_cols_narrow<OP, 4, 8, false>);
+    auto kernel = post < 4 ? k_cols_narrow<OP, 1, false>
+                           : (streams(prev * K * post) ? k_cols_narrow<OP, 4, true> : k_cols_narrow<OP, 4, false>);
     hipLaunchKernelGGL(kernel, grid, dim3(256), 0, g->stream, src, dst, k, (uint32_t)post, kc, G, R, fin, mul, dv,
                        fin ? beta : 0.f);
     check_launch("reduce cols (narrow)");
